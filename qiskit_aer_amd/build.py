@@ -5,6 +5,7 @@ Usage: ``python -m qiskit_aer_amd.build`` (also called by the repository's
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import pathlib
 import shutil
@@ -61,15 +62,17 @@ def build(verbose: bool = True) -> pathlib.Path:
         raise RuntimeError(f"hipcc not found at {HIPCC}")
     OBJ.mkdir(parents=True, exist_ok=True)
     OUT.parent.mkdir(parents=True, exist_ok=True)
-    objs = []
+    cmds, objs = [], []
     for src in sorted(CSRC.glob("*.hip")):
-        obj = OBJ / (src.stem + ".hip.o")
-        _run([HIPCC, *HIP_FLAGS, "-c", str(src), "-o", str(obj)], verbose)
-        objs.append(str(obj))
+        objs.append(str(OBJ / (src.stem + ".hip.o")))
+        cmds.append([HIPCC, *HIP_FLAGS, "-c", str(src), "-o", objs[-1]])
     for src in sorted(CSRC.glob("*.cpp")):
-        obj = OBJ / (src.stem + ".cpp.o")
-        _run(["g++", *CXX_FLAGS, "-c", str(src), "-o", str(obj)], verbose)
-        objs.append(str(obj))
+        objs.append(str(OBJ / (src.stem + ".cpp.o")))
+        cmds.append(["g++", *CXX_FLAGS, "-c", str(src), "-o", objs[-1]])
+    # The translation units are independent: one compiler per CPU, at most 8.
+    with concurrent.futures.ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        for f in [pool.submit(_run, cmd, verbose) for cmd in cmds]:
+            f.result()
     tmp = OUT.with_suffix(".so.tmp")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", *objs, "-o", str(tmp)], verbose)
     os.replace(tmp, OUT)

@@ -12,16 +12,12 @@
 #include "gate_matrices.hpp"
 #include "host_parallel.hpp"
 #include "kernels.hpp"
-#include "batch.hpp"
-#include "reg_pass.hpp"
-#include "tile_pass.hpp"
+#include "pass_kernels.hpp"
 
 namespace aerhip {
 
 namespace {
 
-constexpr uint32_t kTileBitsC128 = 11;  // 2^11 x 16 B = 32 KiB of LDS
-constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
 constexpr size_t kMaxQueue = 4096;      // flush threshold of the gate queue
 
 inline uint64_t bit(uint32_t q) { return 1ull << q; }
@@ -34,6 +30,17 @@ inline uint32_t grid_for(uint64_t work, uint32_t cap = 8192) {
 }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+// Sums `cols` consecutive partials of each of `rows` rows (one thread per row,
+// sequential order).
+__global__ void k_sum_rows(const double *__restrict__ partial, uint64_t rows, uint32_t cols,
+                           double *__restrict__ out) {
+  const uint64_t r = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
+  if (r >= rows) return;
+  double s = 0;
+  for (uint32_t c = 0; c < cols; ++c) s += partial[r * cols + c];
+  out[r] = s;
+}
 
 }  // namespace
 

@@ -186,17 +186,6 @@ __global__ __launch_bounds__(kThreads) void k_inner(const cx<TA> *__restrict__ a
   }
 }
 
-// Sums `cols` consecutive partials of each of `rows` rows (one thread per row,
-// sequential order).
-__global__ void k_sum_rows(const double *__restrict__ partial, uint64_t rows, uint32_t cols,
-                           double *__restrict__ out) {
-  const uint64_t r = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
-  if (r >= rows) return;
-  double s = 0;
-  for (uint32_t c = 0; c < cols; ++c) s += partial[r * cols + c];
-  out[r] = s;
-}
-
 template <typename T>
 __global__ void k_probs_all(const cx<T> *__restrict__ sv, uint64_t n, double *__restrict__ out) {
   for (uint64_t i = blockIdx.x * (uint64_t)kThreads + threadIdx.x; i < n;

@@ -1,0 +1,6 @@
+// complex128 register pass with 4 register bits: the full variant.
+#include "pass_kernels.hpp"
+
+namespace aerhip {
+AERHIP_REG_PASS(, double, kTileBitsC128, 4, true, false)
+}  // namespace aerhip

@@ -1,0 +1,6 @@
+// complex64 register pass with 5 register bits: the lean variant.
+#include "pass_kernels.hpp"
+
+namespace aerhip {
+AERHIP_REG_PASS(, float, kTileBitsC64, 5, false, false)
+}  // namespace aerhip

@@ -1,0 +1,37 @@
+// The pass kernels the engine launches, declared here and compiled in
+// translation units of their own (pass_*.hip), which hipcc builds in parallel.
+#pragma once
+
+#include "batch.hpp"
+#include "reg_pass.hpp"
+#include "tile_pass.hpp"
+
+namespace aerhip {
+
+constexpr uint32_t kTileBitsC128 = 11;  // 2^11 x 16 B = 32 KiB of LDS
+constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
+
+#define AERHIP_REG_PASS(EXT, T, B, R, FULL, WIDE)                                                        \
+  EXT template __global__ void k_reg_pass<T, B, R, FULL, WIDE>(                                          \
+      cx<T> *__restrict__, const PassDesc *__restrict__, const ROp<T> *__restrict__,                     \
+      const TileOp *__restrict__, const cx<double> *__restrict__, double *__restrict__, uint64_t,        \
+      uint32_t, uint32_t, uint32_t);
+#define AERHIP_BATCH(EXT, T, B, R)                                                                       \
+  EXT template __global__ void k_batch<T, B, R>(cx<T> *__restrict__, const BatchCircuit *__restrict__,   \
+                                                const PassDesc *__restrict__, const ROp<T> *__restrict__, \
+                                                const TileOp *__restrict__,                              \
+                                                const cx<double> *__restrict__, double *__restrict__);
+
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, false, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, false, true)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, true, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, false, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, true, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, false, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, true, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, false, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, true, false)
+AERHIP_BATCH(extern, double, kTileBitsC128, 3)
+AERHIP_BATCH(extern, float, kTileBitsC64, 4)
+
+}  // namespace aerhip
