@@ -13,6 +13,7 @@
 #include "host_parallel.hpp"
 #include "kernels.hpp"
 #include "pass_kernels.hpp"
+#include "readout.hpp"
 
 namespace aerhip {
 
@@ -30,17 +31,6 @@ inline uint32_t grid_for(uint64_t work, uint32_t cap = 8192) {
 }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
-
-// Sums `cols` consecutive partials of each of `rows` rows (one thread per row,
-// sequential order).
-__global__ void k_sum_rows(const double *__restrict__ partial, uint64_t rows, uint32_t cols,
-                           double *__restrict__ out) {
-  const uint64_t r = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
-  if (r >= rows) return;
-  double s = 0;
-  for (uint32_t c = 0; c < cols; ++c) s += partial[r * cols + c];
-  out[r] = s;
-}
 
 }  // namespace
 
@@ -191,13 +181,13 @@ void Engine::initialize_random(uint64_t seed) {
     auto *sv = static_cast<cx<double> *>(sv_);
     k_gaussian<double><<<grid_for(size_, 16384), kThreads, 0, stream_>>>(sv, size_, seed);
     k_sumsq<double><<<grid, kThreads, 0, stream_>>>(sv, size_, d_partial_);
-    k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 1, grid, d_partial_ + grid);
+    sum_rows(d_partial_, 1, grid, d_partial_ + grid, stream_);
     k_scale<double><<<grid_for(size_, 16384), kThreads, 0, stream_>>>(sv, size_, d_partial_ + grid);
   } else {
     auto *sv = static_cast<cx<float> *>(sv_);
     k_gaussian<float><<<grid_for(size_, 16384), kThreads, 0, stream_>>>(sv, size_, seed);
     k_sumsq<float><<<grid, kThreads, 0, stream_>>>(sv, size_, d_partial_);
-    k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 1, grid, d_partial_ + grid);
+    sum_rows(d_partial_, 1, grid, d_partial_ + grid, stream_);
     k_scale<float><<<grid_for(size_, 16384), kThreads, 0, stream_>>>(sv, size_, d_partial_ + grid);
   }
   AERHIP_CHECK(hipGetLastError());
@@ -2348,8 +2338,7 @@ void Engine::flush() {
   if (nprobes) {
     // Sum each probe's tile partials in tile order and fetch the values.
     double *sums = d_probes_ + nprobes * ntiles;
-    k_sum_rows<<<grid_for(nprobes, 1u << 30), kThreads, 0, stream_>>>(
-        d_probes_, nprobes, static_cast<uint32_t>(ntiles), sums);
+    sum_rows(d_probes_, nprobes, static_cast<uint32_t>(ntiles), sums, stream_);
     AERHIP_CHECK(hipGetLastError());
     const size_t base = saved_expvals_.size();
     saved_expvals_.resize(base + nprobes);
@@ -2425,7 +2414,7 @@ double Engine::norm_t() {
   const uint32_t grid = grid_for(size_, 4096);
   ensure_partial(grid + 1);
   k_sumsq<T><<<grid, kThreads, 0, stream_>>>(static_cast<const cx<T> *>(sv_), size_, d_partial_);
-  k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 1, grid, d_partial_ + grid);
+  sum_rows(d_partial_, 1, grid, d_partial_ + grid, stream_);
   AERHIP_CHECK(hipGetLastError());
   return fetch_scalar(d_partial_ + grid);
 }
@@ -2449,7 +2438,7 @@ double Engine::norm_matrix_t(const MarginalDesc &md, const std::vector<cd> &mat)
                                                   reinterpret_cast<const MarginalDesc *>(sc),
                                                   reinterpret_cast<const cx<double> *>(sc + mat_off),
                                                   d_partial_);
-  k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 1, grid, d_partial_ + grid);
+  sum_rows(d_partial_, 1, grid, d_partial_ + grid, stream_);
   AERHIP_CHECK(hipGetLastError());
   return fetch_scalar(d_partial_ + grid);
 }
@@ -2539,7 +2528,7 @@ cd Engine::inner_product(Engine &other) {
   else
     k_inner<float, float><<<grid, kThreads, 0, stream_>>>(static_cast<const cx<float> *>(sv_),
         static_cast<const cx<float> *>(other.sv_), size_, d_partial_);
-  k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 2, grid, d_partial_ + 2 * grid);
+  sum_rows(d_partial_, 2, grid, d_partial_ + 2 * grid, stream_);
   AERHIP_CHECK(hipGetLastError());
   const double re = fetch_scalar(d_partial_ + 2 * grid);
   const double im = fetch_scalar(d_partial_ + 2 * grid + 1);
@@ -2590,31 +2579,26 @@ void Engine::probabilities_t(const std::vector<uint32_t> &qubits, double *out) {
   std::memset(&md, 0, sizeof(md));
   md.nq = nq;
   md.inner = 1ull << (n_ - nq);
+  const uint32_t low = std::min<uint32_t>(6, n_);
+  uint32_t nh = 0;  // measured qubits above the lane qubits
   for (uint32_t i = 0; i < nq; ++i) {
     md.sorted[i] = static_cast<uint8_t>(sorted[i]);
     md.order[i] = static_cast<uint8_t>(qubits[i]);
+    if (sorted[i] >= low) ++nh;
   }
-  MarginalDesc *dmd = static_cast<MarginalDesc *>(scratch(sizeof(MarginalDesc)));
-  if (md.inner <= 256) {
-    AERHIP_CHECK(hipMemcpy(dmd, &md, sizeof(md), hipMemcpyHostToDevice));
-    ensure_partial(outcomes);
-    dout = d_partial_;
-    k_marginal_small<T><<<grid_for(outcomes, 1u << 30), kThreads, 0, stream_>>>(sv, dmd, outcomes,
-                                                                                 dout);
-  } else {
-    uint64_t nchunk = std::max<uint64_t>(1, 8192 / outcomes);
-    nchunk = std::min<uint64_t>(nchunk, std::max<uint64_t>(1, md.inner / 1024));
-    md.nchunk = static_cast<uint32_t>(nchunk);
-    AERHIP_CHECK(hipMemcpy(dmd, &md, sizeof(md), hipMemcpyHostToDevice));
-    ensure_partial(outcomes * nchunk + outcomes);
-    // outcomes is a power of two: grid.y * grid.z == outcomes exactly.
-    dim3 grid(static_cast<uint32_t>(nchunk), 1, 1);
-    grid.y = static_cast<uint32_t>(std::min<uint64_t>(outcomes, 32768));
-    grid.z = static_cast<uint32_t>(outcomes / grid.y);
-    k_marginal_chunks<T><<<grid, kThreads, 0, stream_>>>(sv, dmd, d_partial_);
+  // Chunks of the unmeasured high indices: enough waves to fill the device
+  // (2^14), each with at least 32 of those indices where there are as many.
+  const uint64_t inner_h = 1ull << (n_ - low - nh);
+  const uint64_t nchunk = std::min<uint64_t>(std::max<uint64_t>(1, inner_h / 32), std::max<uint64_t>(1, (1ull << 14) >> nh));
+  md.nchunk = static_cast<uint32_t>(nchunk);
+  const uint64_t items = nchunk << nh;
+  ensure_partial(outcomes * nchunk + outcomes);
+  k_marginal<T><<<static_cast<uint32_t>(std::min<uint64_t>((items + 3) / 4, 1u << 16)), kThreads, 0, stream_>>>(
+      sv, md, low, items, inner_h / nchunk, d_partial_);
+  dout = d_partial_;
+  if (nchunk > 1) {
     dout = d_partial_ + outcomes * nchunk;
-    k_sum_rows<<<grid_for(outcomes, 1u << 30), kThreads, 0, stream_>>>(
-        d_partial_, outcomes, static_cast<uint32_t>(nchunk), dout);
+    sum_rows(d_partial_, outcomes, static_cast<uint32_t>(nchunk), dout, stream_);
   }
   AERHIP_CHECK(hipGetLastError());
   AERHIP_CHECK(hipMemcpyAsync(out, dout, outcomes * sizeof(double), hipMemcpyDeviceToHost, stream_));
@@ -2652,15 +2636,18 @@ void Engine::sample_t(const std::vector<double> &rnds, uint64_t *out) {
     const uint32_t sbits = std::min<uint32_t>(blockbits, 10);
     const uint64_t nruns = size_ >> sbits;
     const uint64_t nblocks = 1ull << isz;
-    ensure_partial(nruns + nblocks);
+    ensure_partial(nruns + 2 * nblocks);
     double *runs = d_partial_;
     double *blocks = d_partial_ + nruns;
+    double *upto = blocks + nblocks;
     k_run_sums<T><<<static_cast<uint32_t>((nruns + 3) / 4), kThreads, 0, stream_>>>(sv, sbits, nruns,
                                                                                    runs);
-    k_sum_rows<<<grid_for(nblocks, 1u << 30), kThreads, 0, stream_>>>(
-        runs, nblocks, static_cast<uint32_t>(nruns / nblocks), blocks);
-    k_sample<T><<<grid_for(shots, 1u << 30), kThreads, 0, stream_>>>(sv, size_, isz, sbits, blocks,
-                                                                      runs, drnd, shots, dout);
+    const uint64_t rpb = nruns / nblocks;  // runs per index block
+    if (rpb > 1) k_block_sums<<<static_cast<uint32_t>(nblocks), kThreads, 0, stream_>>>(runs, rpb, blocks);
+    k_prefix_blocks<<<1, kThreads, 0, stream_>>>(rpb > 1 ? blocks : runs, nblocks, upto);
+    if (rpb > 1) k_prefix_runs<<<static_cast<uint32_t>(nblocks), kThreads, 0, stream_>>>(runs, rpb, upto);
+    k_sample<T><<<static_cast<uint32_t>((shots + kDraws - 1) / kDraws), 64, 0, stream_>>>(
+        sv, size_, isz, sbits, upto, runs, drnd, shots, dout);
   }
   AERHIP_CHECK(hipGetLastError());
   AERHIP_CHECK(hipMemcpyAsync(out, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_));
@@ -2687,7 +2674,7 @@ double Engine::expval_t(uint64_t xmask, uint64_t zmask, uint32_t xmax, cd ph) {
   ensure_partial(grid + 1);
   k_expval_pauli<T><<<grid, kThreads, 0, stream_>>>(static_cast<const cx<T> *>(sv_), size_, xmask,
                                                      zmask, xmax, ph.real(), ph.imag(), d_partial_);
-  k_sum_rows<<<1, kThreads, 0, stream_>>>(d_partial_, 1, grid, d_partial_ + grid);
+  sum_rows(d_partial_, 1, grid, d_partial_ + grid, stream_);
   AERHIP_CHECK(hipGetLastError());
   return fetch_scalar(d_partial_ + grid);
 }
@@ -3139,8 +3126,7 @@ class MultiState {
                   static_cast<uint32_t>(P), st_);
     if (pps) {
       double *sums = d_probes_ + cnt * pps * ntiles;
-      k_sum_rows<<<grid_for(cnt * pps, 1u << 30), kThreads, 0, st_>>>(d_probes_, cnt * pps,
-                                                                      static_cast<uint32_t>(ntiles), sums);
+      sum_rows(d_probes_, cnt * pps, static_cast<uint32_t>(ntiles), sums, st_);
       AERHIP_CHECK(hipGetLastError());
       AERHIP_CHECK(hipMemcpyAsync(values, sums, cnt * pps * sizeof(double), hipMemcpyDeviceToHost, st_));
     }
@@ -3741,7 +3727,7 @@ int aerhip_expval_pauli_noalloc(const void *sv, uint64_t num_qubits, int precisi
     else
       k_expval_pauli<float><<<grid, kThreads, 0, st>>>(static_cast<const cx<float> *>(sv), size, xm, zm,
                                                        xmax, ph.real(), ph.imag(), part);
-    k_sum_rows<<<1, kThreads, 0, st>>>(part, 1, grid, out);
+    aerhip::sum_rows(part, 1, grid, out, st);
     AERHIP_CHECK(hipGetLastError());
   });
 }

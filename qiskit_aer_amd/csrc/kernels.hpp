@@ -278,121 +278,6 @@ __global__ __launch_bounds__(kThreads) void k_norm_group(const cx<T> *__restrict
   }
 }
 
-// Block (c, m) sums |psi|^2 over inner indices k in chunk c for outcome m.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_marginal_chunks(const cx<T> *__restrict__ sv,
-                                                              const MarginalDesc *__restrict__ md,
-                                                              double *__restrict__ partial) {
-  const uint64_t m = blockIdx.y + (uint64_t)gridDim.y * blockIdx.z;
-  const uint32_t nq = md->nq;
-  uint64_t mbits = 0;
-  for (uint32_t i = 0; i < nq; ++i) mbits |= ((m >> i) & 1ull) << md->order[i];
-  const uint64_t inner = md->inner;
-  const uint64_t chunk = (inner + md->nchunk - 1) / md->nchunk;
-  const uint64_t k0 = blockIdx.x * chunk;
-  const uint64_t k1 = min(inner, k0 + chunk);
-  double acc = 0;
-  for (uint64_t k = k0 + threadIdx.x; k < k1; k += kThreads) {
-    uint64_t idx = k;
-    for (uint32_t j = 0; j < nq; ++j) idx = insert_zero64(idx, md->sorted[j]);
-    acc += prob(sv[idx | mbits]);
-  }
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partial[m * md->nchunk + blockIdx.x] = acc;
-}
-
-// One thread per outcome for marginals with few inner indices.
-template <typename T>
-__global__ void k_marginal_small(const cx<T> *__restrict__ sv, const MarginalDesc *__restrict__ md,
-                                 uint64_t outcomes, double *__restrict__ out) {
-  const uint64_t m = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
-  if (m >= outcomes) return;
-  const uint32_t nq = md->nq;
-  uint64_t mbits = 0;
-  for (uint32_t i = 0; i < nq; ++i) mbits |= ((m >> i) & 1ull) << md->order[i];
-  double acc = 0;
-  for (uint64_t k = 0; k < md->inner; ++k) {
-    uint64_t idx = k;
-    for (uint32_t j = 0; j < nq; ++j) idx = insert_zero64(idx, md->sorted[j]);
-    acc += prob(sv[idx | mbits]);
-  }
-  out[m] = acc;
-}
-
-// Sum of |psi|^2 over consecutive runs of 2^sbits amplitudes, one wave per run.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_run_sums(const cx<T> *__restrict__ sv,
-                                                       uint32_t sbits, uint64_t nruns,
-                                                       double *__restrict__ out) {
-  const uint64_t run = blockIdx.x * (uint64_t)(kThreads / 64) + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63;
-  if (run >= nruns) return;
-  const uint64_t len = 1ull << sbits;
-  const uint64_t b = run << sbits;
-  double acc = 0;
-  for (uint64_t j = lane; j < len; j += 64) acc += prob(sv[b + j]);
-  acc = wave_sum(acc);
-  if (lane == 0) out[run] = acc;
-}
-
-// Sampling by a three-level cumulative search in the order of the reference's
-// QubitVector::sample_measure (qubitvector.hpp:2149-2228): index blocks of
-// 2^(n-isz) amplitudes (the reference's idxs), sub-runs of 2^sbits
-// amplitudes inside a block, then amplitudes; comparisons are rnd < cumsum.
-template <typename T>
-__global__ void k_sample(const cx<T> *__restrict__ sv, uint64_t size, uint32_t isz,
-                         uint32_t sbits, const double *__restrict__ blocks,
-                         const double *__restrict__ runs, const double *__restrict__ rnds,
-                         uint64_t shots, uint64_t *__restrict__ out) {
-  const uint64_t s = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
-  if (s >= shots) return;
-  const double rnd = rnds[s];
-  const uint64_t nblocks = 1ull << isz;
-  const uint64_t loop = size >> isz;
-  double p = 0;
-  uint64_t sample = 0;
-  uint64_t j = 0;
-  for (; j < nblocks; ++j) {
-    if (rnd < p + blocks[j]) break;
-    p += blocks[j];
-    sample += loop;
-  }
-  if (j == nblocks) {  // rnd beyond the accumulated total: last amplitude
-    out[s] = size - 1;
-    return;
-  }
-  const uint64_t rpb = loop >> sbits;  // runs per block
-  const uint64_t r0 = sample >> sbits;
-  for (uint64_t r = 0; r + 1 < rpb; ++r) {
-    const double v = runs[r0 + r];
-    if (rnd < p + v) break;
-    p += v;
-    sample += 1ull << sbits;
-  }
-  for (; sample < size - 1; ++sample) {
-    p += prob(sv[sample]);
-    if (rnd < p) break;
-  }
-  out[s] = sample;
-}
-
-// Linear scan for small states (END < 2^isz in the reference).
-template <typename T>
-__global__ void k_sample_linear(const cx<T> *__restrict__ sv, uint64_t size,
-                                const double *__restrict__ rnds, uint64_t shots,
-                                uint64_t *__restrict__ out) {
-  const uint64_t s = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
-  if (s >= shots) return;
-  const double rnd = rnds[s];
-  double p = 0;
-  uint64_t sample = 0;
-  for (; sample < size - 1; ++sample) {
-    p += prob(sv[sample]);
-    if (rnd < p) break;
-  }
-  out[s] = sample;
-}
-
 struct PauliTerm {
   uint64_t x, z;  // flip and sign masks
   double cr, ci;  // coefficient times the Pauli phase (-i)^#Y
