@@ -1,6 +1,5 @@
 // Host implementation of the engine and its C ABI (include/aerhip.h).
 #include <algorithm>
-#include <array>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -813,8 +812,12 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
   std::vector<TileOp> out;
   out.reserve(in.size());
   auto emit = [&](Group &g) {
-    if (g.originals.size() == 1) {
-      out.push_back(g.originals[0]);
+    // A single op stays as it is, but for a diagonal on a qubit that the tile
+    // fixes: as a fused diagonal of one member it runs in every register
+    // variant, as a general one (Q_DIAG) only in those with 4x4 gates.
+    const TileOp &first = g.originals[0];
+    if (g.originals.size() == 1 && !(first.kind == K_DIAG && first.pos[0] == kNotLocal)) {
+      out.push_back(first);
       return;
     }
     TileOp op;
@@ -839,7 +842,7 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
     }
     op.nonunitary = g.nonunitary ? 1u : 0u;
     out.push_back(op);
-    if (fused_ops) *fused_ops += g.originals.size();
+    if (fused_ops && g.originals.size() > 1) *fused_ops += g.originals.size();
   };
   auto close_if = [&](uint64_t touch) {
     std::vector<Group> keep;
@@ -929,13 +932,13 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
 // program inside a concatenated one.
 void rebase_rop(ROp<double> &r, uint32_t pool_base, uint32_t op_base) {
   const uint32_t kk = r.kind & ~F_ALL;
-  if (kk == Q_U2 || kk == Q_DIAGF) r.extra += pool_base;
+  if (kk == Q_U2 || kk == Q_DIAGF || kk == Q_PROBE) r.extra += pool_base;
   else if (kk == Q_DIAG || kk == Q_LDS) r.extra += op_base;
   else if ((kk == Q_LOAD || kk == Q_FILL) && r.a) r.b += pool_base;
 }
 
 void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint32_t R,
-                               const uint8_t *spos, size_t ntops) {
+                               const uint8_t *spos, size_t ntops, const std::vector<cd> &pool) {
   auto fail = [](const char *what) { throw std::logic_error(std::string("aerhip: register program: ") + what); };
   auto check_layout = [&](const RLayout &L) {
     uint32_t seen = 0;
@@ -993,7 +996,14 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
           break;
         case Q_D1: if (r.a >= B) fail("diagonal bit"); break;
         case Q_DIAG: if (r.extra >= ntops) fail("diagonal index"); break;
-        case Q_PROBE: if (r.u.pr.xr >= (1u << R)) fail("probe mask"); break;
+        case Q_PROBE:
+          if (!r.a || r.extra + 3ull * r.a > pool.size()) fail("probe run");
+          for (uint32_t k = 0; k < r.a; ++k) {
+            RProbe pr;
+            std::memcpy(&pr, pool.data() + r.extra + 3 * k, sizeof(pr));
+            if (pr.xr >= (1u << R) || pr.idx >= kProbeBatch || pr.flush > kProbeBatch) fail("probe record");
+          }
+          break;
         case Q_PHASE: case Q_NOP: break;
         case Q_DIAGF:
           if ((r.a & 0xFFu) > 8 || (r.a & 0xFF00u) || (r.a >> 16) > e.a) fail("fused diagonal tables");
@@ -1020,7 +1030,7 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
 // double; converted for complex64 at upload), TileOps run on the LDS tile go to
 // `tops`.  `lowb`: tile bits that must be lane bits for a full 128-byte run per
 // HBM access.
-void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uint32_t lowb,
+void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uint32_t lowb, bool single,
                       const uint8_t *spos, std::vector<cd> &pool,
                       std::vector<ROp<double>> &rops, std::vector<TileOp> &tops,
                       uint64_t *relayouts) {
@@ -1254,6 +1264,8 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     emit(Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
   };
+  uint32_t nprobes = 0;   // register probes of the pass so far
+  size_t last_probe = 0;  // pool offset of the last one's record
   auto emit_gate = [&](const TileOp &op, uint32_t rs) {
     ROp<double> r;
     std::memset(&r, 0, sizeof(r));
@@ -1340,6 +1352,17 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         r.a = b0;
         r.b = b1;
         r.extra = op.off;
+        if (single) {
+          // rounded here: the kernel reads the entries as scalars, where
+          // rounding them would cost it a conversion and a register each
+          cx<float> m[16];
+          for (int e = 0; e < 16; ++e)
+            m[e] = to_t<float>(mk<double>(pool[op.off + e].real(), pool[op.off + e].imag()));
+          cd rec[8];
+          std::memcpy(rec, m, sizeof(rec));
+          r.extra = static_cast<uint32_t>(pool.size());
+          pool.insert(pool.end(), rec, rec + 8);
+        }
         break;
       }
       case K_DIAG:
@@ -1423,16 +1446,32 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       }
       case K_PROBE: {
         materialize(pend);
-        r.kind = Q_PROBE;
-        r.extra = op.npairs;
+        RProbe pr;
+        std::memset(&pr, 0, sizeof(pr));
         uint32_t xl = 0;
         for (uint32_t b = 0; b < B; ++b)
           if (op.xl & (1u << b)) xl |= 1u << regidx(rs, b);
-        r.u.pr.xr = phys_of(xl);
-        r.u.pr.zl = op.zl;
-        r.u.pr.zg = op.zg;
-        r.u.pr.pr = op.pr;
-        r.u.pr.pi = op.pi;
+        pr.xr = phys_of(xl);
+        pr.zl = op.zl;
+        pr.zg = op.zg;
+        pr.pr = op.pr;
+        pr.pi = op.pi;
+        pr.slot = op.npairs;
+        pr.idx = nprobes++ % kProbeBatch;
+        if (pr.idx == kProbeBatch - 1) pr.flush = kProbeBatch;
+        cd rec[3];
+        std::memcpy(rec, &pr, sizeof(rec));
+        last_probe = pool.size();
+        pool.insert(pool.end(), rec, rec + 3);
+        // the next record of the run that the last op holds, or a new run
+        if (!map_dirty && (rops.back().kind & ~F_ALL) == Q_PROBE && rops.size() - 1 > enter_at &&
+            rops.back().extra + 3ull * rops.back().a == last_probe) {
+          ++rops.back().a;
+          return;
+        }
+        r.kind = Q_PROBE;
+        r.a = 1;
+        r.extra = static_cast<uint32_t>(last_probe);
         break;
       }
       default:
@@ -1507,6 +1546,12 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     rs = fill(0);
     emit(lds_mode ? Q_FILL : Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
+  }
+  if (nprobes % kProbeBatch) {  // the last batch's entries go out with its last probe
+    RProbe pr;
+    std::memcpy(&pr, pool.data() + last_probe, sizeof(pr));
+    pr.flush = nprobes % kProbeBatch;
+    std::memcpy(pool.data() + last_probe, &pr, sizeof(pr));
   }
   emit(Q_STORE, rs);
 }
@@ -2054,10 +2099,11 @@ void Engine::emit_program(Program &prog) {
         pops = fuse_phase_runs(pops, pd.spos, ns, prog.pool, fusion_max_qubit_, &stats_.fused);
       pd.kind = 2;  // register-layout tile pass: op_begin/nops index the ROps
       pd.op_begin = static_cast<uint32_t>(rops.size());
-      register_program(pops, ns, reg_bits_, low_bits_, pd.spos, prog.pool, rops, ops, &stats_.gathers);
+      register_program(pops, ns, reg_bits_, low_bits_, prec_ == AERHIP_PRECISION_SINGLE, pd.spos, prog.pool, rops, ops, &stats_.gathers);
       pd.nops = static_cast<uint32_t>(rops.size()) - pd.op_begin;
       if (pd.readonly) rops.back().extra = 1;  // the final STORE writes nothing
-      validate_register_program(rops.data() + pd.op_begin, pd.nops, ns, reg_bits_, pd.spos, ops.size());
+      validate_register_program(rops.data() + pd.op_begin, pd.nops, ns, reg_bits_, pd.spos, ops.size(),
+                                prog.pool);
     } else {
       pd.nops = static_cast<uint32_t>(pops.size());
       ops.insert(ops.end(), pops.begin(), pops.end());
@@ -2087,33 +2133,41 @@ struct DeviceProgram {
   uint32_t probes_per_state;
 };
 
-template <typename T, int B, int R>
-void launch_reg_pass(bool lean, bool wide, bool diag, uint32_t grid, hipStream_t stream, cx<T> *sv,
-                     const PassDesc *pd, const ROp<T> *rops, const TileOp *tops, const cx<double> *pool,
-                     double *probes, uint64_t state_stride, uint32_t pd_stride, uint32_t tile_log,
-                     uint32_t pps) {
-  // the staged lane tables of fused diagonals, only for passes that have them
-  const size_t dyn = diag ? kDiagLdsBytes : 0;
-  if constexpr (sizeof(T) == 8 && R == 3) {
-    if (lean && wide) {
-      k_reg_pass<T, B, R, false, true><<<grid, 1 << (B - R), dyn, stream>>>(
-          sv, pd, rops, tops, pool, probes, state_stride, pd_stride, tile_log, pps);
-      return;
-    }
+// The kernel of a pass: its register-pass variant, whether the wide lean one,
+// and whether it needs the LDS of staged fused-diagonal lane tables.
+struct PassKernel {
+  int variant = V_LEAN;
+  bool wide = true, diag = false;
+  void add(const PassKernel &o) {  // one kernel for several states' programs
+    variant |= o.variant;
+    wide = wide && o.wide;
+    diag = diag || o.diag;
   }
-  if (lean)
-    k_reg_pass<T, B, R, false><<<grid, 1 << (B - R), dyn, stream>>>(sv, pd, rops, tops, pool, probes,
-                                                                    state_stride, pd_stride, tile_log, pps);
-  else
-    k_reg_pass<T, B, R, true><<<grid, 1 << (B - R), dyn, stream>>>(sv, pd, rops, tops, pool, probes,
-                                                                   state_stride, pd_stride, tile_log, pps);
+};
+
+template <typename T, int B, int R>
+void launch_reg_pass(const PassKernel &k, uint32_t grid, hipStream_t stream, cx<T> *sv, const PassDesc *pd,
+                     const ROp<T> *rops, const TileOp *tops, const cx<double> *pool, double *probes,
+                     uint64_t state_stride, uint32_t pd_stride, uint32_t tile_log, uint32_t pps) {
+  const size_t dyn = k.diag ? kDiagLdsBytes : 0;
+  auto go = [&](auto kernel) {
+    kernel<<<grid, 1 << (B - R), dyn, stream>>>(sv, pd, rops, tops, pool, probes, state_stride, pd_stride,
+                                                tile_log, pps);
+  };
+  if constexpr ((sizeof(T) == 8 && R == 3) || (sizeof(T) == 4 && R == 4)) {
+    if constexpr (sizeof(T) == 8)
+      if (k.variant == V_LEAN && k.wide) return go(k_reg_pass<T, B, R, V_LEAN, true>);
+    if (k.variant == V_GATES) return go(k_reg_pass<T, B, R, V_GATES, false>);
+    if (k.variant == V_PROBES) return go(k_reg_pass<T, B, R, V_PROBES, false>);
+  }
+  if (k.variant == V_LEAN) return go(k_reg_pass<T, B, R, V_LEAN, false>);
+  go(k_reg_pass<T, B, R, V_FULL, false>);
 }
 
 // Launches pass index i (host descriptor `pd`, the same pass of every state)
-// over `count` states; `lean` / `wide` pick the register-pass variant, `diag`
-// gives it the LDS of staged fused-diagonal lane tables.
+// over `count` states with the kernel `pk`.
 void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, const PassDesc &pd,
-                 uint32_t i, bool lean, bool wide, bool diag, const DeviceProgram &dp, void *sv,
+                 uint32_t i, const PassKernel &pk, const DeviceProgram &dp, void *sv,
                  uint64_t count, uint32_t pd_stride, hipStream_t stream) {
   const uint64_t state_stride = 1ull << n;
   const PassDesc *dpd = dp.passes + i;
@@ -2129,19 +2183,19 @@ void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, co
       auto *s = static_cast<cx<double> *>(sv);
       auto *ro = static_cast<const ROp<double> *>(dp.rops);
       if (reg_bits == 3)
-        launch_reg_pass<double, kTileBitsC128, 3>(lean, wide, diag, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
+        launch_reg_pass<double, kTileBitsC128, 3>(pk, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
                                                   dp.probes, state_stride, pd_stride, tl, pps);
       else
-        launch_reg_pass<double, kTileBitsC128, 4>(lean, wide, diag, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
+        launch_reg_pass<double, kTileBitsC128, 4>(pk, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
                                                   dp.probes, state_stride, pd_stride, tl, pps);
     } else {
       auto *s = static_cast<cx<float> *>(sv);
       auto *ro = static_cast<const ROp<float> *>(dp.rops);
       if (reg_bits == 4)
-        launch_reg_pass<float, kTileBitsC64, 4>(lean, wide, diag, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
+        launch_reg_pass<float, kTileBitsC64, 4>(pk, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
                                                 dp.probes, state_stride, pd_stride, tl, pps);
       else
-        launch_reg_pass<float, kTileBitsC64, 5>(lean, wide, diag, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
+        launch_reg_pass<float, kTileBitsC64, 5>(pk, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
                                                 dp.probes, state_stride, pd_stride, tl, pps);
     }
   } else if (pd.kind == 3) {
@@ -2201,20 +2255,18 @@ bool graphs_enabled() {
   return on;
 }
 
-// The register-pass variant of a pass: lean if every op is a lean kind, wide
-// if it also has at most kWidePassOps ops.
-void pass_variant(const PassDesc &pd, const std::vector<ROp<double>> &rops, bool &lean, bool &wide,
-                  bool &diag) {
-  lean = true;
-  wide = pd.nops <= kWidePassOps;
-  diag = false;
-  if (pd.kind != 2) return;
-  for (uint32_t k = 0; k < pd.nops; ++k) {
-    const ROp<double> &r = rops[pd.op_begin + k];
-    lean = lean && lean_kind(r.kind);
+// The kernel of a pass, from its ops.
+PassKernel pass_kernel(const PassDesc &pd, const std::vector<ROp<double>> &rops) {
+  PassKernel k;
+  k.wide = pd.nops <= kWidePassOps;
+  if (pd.kind != 2) return k;
+  for (uint32_t i = 0; i < pd.nops; ++i) {
+    const ROp<double> &r = rops[pd.op_begin + i];
+    k.variant |= variant_of(r.kind);
     const uint32_t kk = r.kind & ~F_ALL;
-    diag = diag || ((kk == Q_LOAD || kk == Q_FILL) && r.a != 0);
+    k.diag = k.diag || ((kk == Q_LOAD || kk == Q_FILL) && r.a != 0);
   }
+  return k;
 }
 }  // namespace
 
@@ -2293,19 +2345,17 @@ void Engine::flush() {
   std::vector<uint64_t> sig = {reinterpret_cast<uint64_t>(d_prog_), reinterpret_cast<uint64_t>(sv_),
                                reinterpret_cast<uint64_t>(dprobes), static_cast<uint64_t>(prec_),
                                reg_bits_, n_, tile_bits_, passes.size(), ops_off, rops_off, pool_off};
-  std::vector<std::array<bool, 3>> variant(passes.size());
+  std::vector<PassKernel> kernels(passes.size());
   for (size_t i = 0; i < passes.size(); ++i) {
-    bool lean = false, wide = false, diag = false;
-    pass_variant(passes[i], rops, lean, wide, diag);
-    variant[i] = {lean, wide, diag};
     const PassDesc &pd = passes[i];
+    const PassKernel &k = kernels[i] = pass_kernel(pd, rops);
     sig.push_back((uint64_t(pd.kind) << 48) | (uint64_t(pd.ncomp) << 32) | (uint64_t(pd.nb) << 16) |
-                  (uint64_t(diag) << 2) | (uint64_t(lean) << 1) | uint64_t(wide));
+                  (uint64_t(k.variant) << 2) | (uint64_t(k.diag) << 1) | uint64_t(k.wide));
   }
   auto launch_all = [&] {
     for (size_t i = 0; i < passes.size(); ++i)
-      launch_pass(prec_, reg_bits_, n_, tile_bits_, passes[i], static_cast<uint32_t>(i), variant[i][0],
-                  variant[i][1], variant[i][2], dp, sv_, 1, 0, stream_);
+      launch_pass(prec_, reg_bits_, n_, tile_bits_, passes[i], static_cast<uint32_t>(i), kernels[i], dp, sv_, 1, 0,
+                  stream_);
   };
   if (graphs_enabled() && graph_exec_ && sig == graph_sig_) {
     AERHIP_CHECK(hipGraphLaunch(graph_exec_, stream_));
@@ -3054,17 +3104,13 @@ class MultiState {
     std::vector<TileOp> ops;
     std::vector<ROp<double>> rops;
     std::vector<cd> pool;
-    std::vector<char> lean(P, 1), wide(P, 1), diag(P, 0);
+    std::vector<PassKernel> kernels(P);
     for (uint64_t b = first; b < first + cnt; ++b) {
       const Program &p = parts[b];
       const uint32_t ob = static_cast<uint32_t>(ops.size()), rb = static_cast<uint32_t>(rops.size()),
                      pb = static_cast<uint32_t>(pool.size());
       for (size_t k = 0; k < P; ++k) {
-        bool l = false, w = false, dg = false;
-        pass_variant(p.passes[k], p.rops, l, w, dg);
-        lean[k] = lean[k] && l;
-        wide[k] = wide[k] && w;
-        diag[k] = diag[k] || dg;
+        kernels[k].add(pass_kernel(p.passes[k], p.rops));
         PassDesc d = p.passes[k];
         d.op_begin += d.kind == 2 ? rb : ob;
         passes.push_back(d);
@@ -3122,7 +3168,7 @@ class MultiState {
     void *sv = static_cast<char *>(states_) + first * (1ull << n_) * amp_bytes();
     for (size_t k = 0; k < P; ++k)
       launch_pass(prec_, planners_[first]->reg_bits(), n_, tb, parts[first].passes[k],
-                  static_cast<uint32_t>(k), lean[k] != 0, wide[k] != 0, diag[k] != 0, dp, sv, cnt,
+                  static_cast<uint32_t>(k), kernels[k], dp, sv, cnt,
                   static_cast<uint32_t>(P), st_);
     if (pps) {
       double *sums = d_probes_ + cnt * pps * ntiles;

@@ -2,6 +2,6 @@
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_REG_PASS(, double, kTileBitsC128, 3, false, false)
-AERHIP_REG_PASS(, double, kTileBitsC128, 3, false, true)
+AERHIP_REG_PASS(, double, kTileBitsC128, 3, V_LEAN, false)
+AERHIP_REG_PASS(, double, kTileBitsC128, 3, V_LEAN, true)
 }  // namespace aerhip

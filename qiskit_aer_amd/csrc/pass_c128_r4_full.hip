@@ -2,5 +2,5 @@
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_REG_PASS(, double, kTileBitsC128, 4, true, false)
+AERHIP_REG_PASS(, double, kTileBitsC128, 4, V_FULL, false)
 }  // namespace aerhip

@@ -2,5 +2,5 @@
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_REG_PASS(, float, kTileBitsC64, 5, true, false)
+AERHIP_REG_PASS(, float, kTileBitsC64, 5, V_FULL, false)
 }  // namespace aerhip

@@ -11,8 +11,8 @@ namespace aerhip {
 constexpr uint32_t kTileBitsC128 = 11;  // 2^11 x 16 B = 32 KiB of LDS
 constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
 
-#define AERHIP_REG_PASS(EXT, T, B, R, FULL, WIDE)                                                        \
-  EXT template __global__ void k_reg_pass<T, B, R, FULL, WIDE>(                                          \
+#define AERHIP_REG_PASS(EXT, T, B, R, V, WIDE)                                                        \
+  EXT template __global__ void k_reg_pass<T, B, R, V, WIDE>(                                          \
       cx<T> *__restrict__, const PassDesc *__restrict__, const ROp<T> *__restrict__,                     \
       const TileOp *__restrict__, const cx<double> *__restrict__, double *__restrict__, uint64_t,        \
       uint32_t, uint32_t, uint32_t);
@@ -22,15 +22,19 @@ constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
                                                 const TileOp *__restrict__,                              \
                                                 const cx<double> *__restrict__, double *__restrict__);
 
-AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, false, false)
-AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, false, true)
-AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, true, false)
-AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, false, false)
-AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, true, false)
-AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, false, false)
-AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, true, false)
-AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, false, false)
-AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, true, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, true)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_GATES, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_PROBES, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_FULL, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, V_LEAN, false)
+AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, V_FULL, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_LEAN, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_GATES, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_PROBES, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_FULL, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_LEAN, false)
+AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_FULL, false)
 AERHIP_BATCH(extern, double, kTileBitsC128, 3)
 AERHIP_BATCH(extern, float, kTileBitsC64, 4)
 

@@ -40,13 +40,15 @@ enum RegPassOpKind : uint32_t {
   Q_U1C = 47,       // 2x2 matrix on register bit a where (l & cl) == cvl
   Q_X = 48,         // X on register bit a where (l & cl) == cvl
   Q_Y = 49,         // Y on register bit a where (l & cl) == cvl
-  Q_U2 = 50,        // 4x4 matrix pool[extra..] on register bits a (matrix bit 0), b (bit 1)
+  Q_U2 = 50,        // 4x4 matrix pool[extra..] on register bits a (matrix bit 0), b (bit 1);
+                    // 16 entries in the state's precision (complex64: two per pool entry)
   Q_D1 = 51,        // diag(u.m[0..1], u.m[2..3]) on local bit a where (l & cl) == cvl; bit j
                     // of b: tile bit a of register j is 1
   Q_PHASE = 52,     // multiply by u.m[0..1] where (l & cl) == cvl; bit j of b: register j
                     // meets the register part of the predicate
   Q_DIAG = 53,      // diagonal of TileOp extra (local and fixed bits)
-  Q_PROBE = 54,     // Pauli probe whose X/Y bits are register bits (u.pr)
+  Q_PROBE = 54,     // a run of a Pauli probes whose X/Y bits are register bits: RProbe
+                    // records at pool[extra..]
   Q_NOP = 55,       // keeps the amplitudes (pads a register phase to an even length)
   Q_U1M = 57,       // 2x2 matrix on the register pairs {j, j ^ a}; bit k of extra set:
                     // the k-th pair's lower register holds the |1> amplitude
@@ -88,11 +90,31 @@ constexpr uint32_t F_MAP = 0x80000000u;
 // 2x2 gate on its target this way.
 constexpr uint32_t F_ALL = F_MAP;
 
-// Kinds the lean register-pass variant runs.
-constexpr bool lean_kind(uint32_t kind) {
-  const uint32_t k = kind & ~F_ALL;
-  return k == Q_LOAD || k == Q_STORE || k == Q_RELAYOUT || k == Q_U1 || k == Q_U1X || k == Q_U1M ||
-         k == Q_U1MX || k == Q_X || k == Q_D1 || k == Q_PHASE || k == Q_NOP || k == Q_DIAGF;
+// Variants of the register pass.  The op loop is an interpreter: its register
+// allocation is that of its greediest op, so each variant compiles the ops of
+// the passes it is launched for and no others.  Lean: 2x2 gates, X, single-
+// qubit diagonals, phases, fused diagonals.  Gates: those with 4x4 gates,
+// controlled 2x2 gates, Y and diagonals.  Probes: the lean ops with Pauli probes.
+// Full: every op, and the tile in LDS for what does not run in registers.
+enum PassVariant : int { V_LEAN = 0, V_GATES = 1, V_PROBES = 2, V_FULL = 3 };
+constexpr bool has_gates(int v) { return v == V_GATES || v == V_FULL; }
+constexpr bool has_probes(int v) { return v == V_PROBES || v == V_FULL; }
+// Variants whose op heads hold the controls and the first payload words.
+constexpr bool head_payload(int v) { return v == V_LEAN || v == V_PROBES; }
+
+// The least variant that runs an op (the variants of a pass combine by OR).
+constexpr int variant_of(uint32_t kind) {
+  switch (kind & ~F_ALL) {
+    case Q_LOAD: case Q_STORE: case Q_RELAYOUT: case Q_U1: case Q_U1X: case Q_U1M: case Q_U1MX:
+    case Q_X: case Q_D1: case Q_PHASE: case Q_NOP: case Q_DIAGF:
+      return V_LEAN;
+    case Q_U2: case Q_U1C: case Q_Y: case Q_DIAG:
+      return V_GATES;
+    case Q_PROBE:
+      return V_PROBES;
+    default:
+      return V_FULL;
+  }
 }
 
 // Bit positions packed four to a word (byte i of word w is entry 4w+i), so
@@ -111,12 +133,25 @@ __host__ __device__ __forceinline__ void set_byte(uint32_t *w, int i, uint32_t v
   w[i >> 2] = (w[i >> 2] & ~(0xFFu << (8 * (i & 3)))) | ((v & 0xFFu) << (8 * (i & 3)));
 }
 
+// One Pauli probe of a run (three pool entries).  A probe's sum over each wave
+// goes to LDS entry idx; a record with flush = k hands the first k entries of
+// the pass on, after one barrier for all of them (the host sets it on every
+// kProbeBatch-th probe of the pass and on its last).
+constexpr uint32_t kProbeBatch = 64;
 struct RProbe {
-  uint32_t xr;  // X/Y mask in register-index space
-  uint32_t zl;  // Z mask over tile bits
-  uint64_t zg;  // Z mask over qubits fixed by the tile
+  uint32_t xr;     // X/Y mask in register-index space
+  uint32_t zl;     // Z mask over tile bits
+  uint64_t zg;     // Z mask over qubits fixed by the tile
   double pr, pi;
+  uint32_t slot;   // index of the saved value
+  uint32_t idx;    // entry of the batch
+  uint32_t flush;
+  uint32_t pad;
 };
+static_assert(sizeof(RProbe) == 3 * sizeof(cx<double>), "a probe record is three pool entries");
+// LDS doubles of a workgroup of nw waves: one per wave for the probes that run
+// on the LDS tile, then the batch's sums and its slots.
+constexpr uint32_t red_doubles(uint32_t nw) { return nw + kProbeBatch * nw + kProbeBatch / 2; }
 
 // 128-byte op record: a 64-byte header and a 64-byte payload, each read with
 // one scalar load (both issued together, so an op costs one load latency).
@@ -135,7 +170,6 @@ struct alignas(128) ROp {
     float mr[16];    // complex64 Q_U1 / Q_U1X / Q_U1M: the matrix as a real 4x4, rows over
                      // (re a0', im a0', re a1', im a1'), columns over (re a0, im a0, re a1, im a1)
     RLayout lay;
-    RProbe pr;
     uint8_t fq[32];  // Q_DIAGF: fixed qubits of the tables, four per table
   } u;
 };
@@ -514,7 +548,7 @@ __device__ __forceinline__ Amps<T, NR> q_xy(const Amps<T, NR> &a, uint32_t tlc,
 template <typename T, int NR, int b0, int b1>
 __device__ __forceinline__ Amps<T, NR> q_u2(const Amps<T, NR> &a, uint32_t tlc,
                                             const RegIdx<NR> &ri, uint32_t cl, uint32_t cvl,
-                                            const cx<double> *__restrict__ mp) {
+                                            const cx<T> *__restrict__ mp) {
   constexpr int lo = b0 < b1 ? b0 : b1, hi = b0 < b1 ? b1 : b0;
   Amps<T, NR> o;
   if (cl == 0) {
@@ -523,8 +557,7 @@ __device__ __forceinline__ Amps<T, NR> q_u2(const Amps<T, NR> &a, uint32_t tlc,
     if (cvl != 0) return pass_through(a);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const cx<T> c0 = to_t<T>(mp[r]), c1 = to_t<T>(mp[r + 4]);
-      const cx<T> c2 = to_t<T>(mp[r + 8]), c3 = to_t<T>(mp[r + 12]);
+      const cx<T> c0 = mp[r], c1 = mp[r + 4], c2 = mp[r + 8], c3 = mp[r + 12];
 #pragma unroll
       for (int p = 0; p < NR / 4; ++p) {
         const int j = pair_lo<hi>(pair_lo<lo>(p));
@@ -537,8 +570,7 @@ __device__ __forceinline__ Amps<T, NR> q_u2(const Amps<T, NR> &a, uint32_t tlc,
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const cx<T> c0 = to_t<T>(mp[r]), c1 = to_t<T>(mp[r + 4]);
-    const cx<T> c2 = to_t<T>(mp[r + 8]), c3 = to_t<T>(mp[r + 12]);
+    const cx<T> c0 = mp[r], c1 = mp[r + 4], c2 = mp[r + 8], c3 = mp[r + 12];
 #pragma unroll
     for (int p = 0; p < NR / 4; ++p) {
       const int j = pair_lo<hi>(pair_lo<lo>(p));
@@ -612,7 +644,7 @@ __device__ __forceinline__ Amps<T, NR> d_xy(uint32_t b, const Amps<T, NR> &a, ui
 template <typename T, int NR, int P = 1>
 __device__ __forceinline__ Amps<T, NR> d_u2(uint32_t p, const Amps<T, NR> &a, uint32_t tlc,
                                             const RegIdx<NR> &ri, uint32_t cl, uint32_t cvl,
-                                            const cx<double> *mp) {
+                                            const cx<T> *mp) {
   constexpr int R = reg_bits_of<NR>();
   constexpr int b0 = P / R, b1 = P % R;
   constexpr int last = (R - 1) * R + (R - 2);
@@ -626,36 +658,122 @@ __device__ __forceinline__ Amps<T, NR> d_u2(uint32_t p, const Amps<T, NR> &a, ui
   }
 }
 
-// sum_j sign_j * Re(phase * a[j ^ xr] * conj(a[j])), sign_j the parity of
-// (l_j & zl) xor sgb: the thread's share of Re<psi| phase P |psi>.
+// The wave's sum of v, valid in lane 63: DPP moves within rows of 16 lanes and
+// two row broadcasts, so that no step waits for LDS as a shuffle does.
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  auto step = [](double x, auto ctrl, auto rows) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), decltype(ctrl)::value, decltype(rows)::value, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, true);
+    return x + __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
+  };
+  using std::integral_constant;
+  v = step(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});  // row_shr 1
+  v = step(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});  // row_shr 2
+  v = step(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});  // row_shr 4
+  v = step(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});  // row_shr 8
+  v = step(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});  // row_bcast 15
+  v = step(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});  // row_bcast 31
+  return v;
+}
+
+// An amplitude's component in FP64.  The complex64 conversion is written out so
+// that it stays in the probe shape that uses it: shared by all of them it would
+// be moved ahead of their dispatch, 64 registers for the whole of it.
+__device__ __forceinline__ double wide(double v) { return v; }
+__device__ __forceinline__ double wide(float v) {
+  double d;
+  asm volatile("v_cvt_f64_f32 %0, %1" : "=v"(d) : "v"(v));
+  return d;
+}
+
+// The thread's share of Re<psi| phase P |psi> up to the sign of its thread
+// bits: sum_j s_j Re(phase conj(a_j) a[j ^ xr]), s_j the parity of the
+// register's tile bits with the Z mask.  Without X this is
+// Re(phase) sum_j s_j |a_j|^2.  With X the two members of a pair hold conjugate
+// products c, conj(c): equal signs add up to 2 Re(phase) Re(c), opposite ones
+// to -2 Im(phase) Im(c), so a pair costs three FMAs.
 template <typename T, int NR, int xr>
-__device__ __forceinline__ double q_probe(const Amps<T, NR> &a, uint32_t tl,
-                                          const RegIdx<NR> &ri, uint32_t zl, uint32_t sgb,
-                                          double pr, double pi) {
-  const uint32_t st = (__popc(tl & zl) & 1u) ^ sgb;
+__device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RegIdx<NR> &ri, const RProbe &pr) {
+  auto sign = [&](int j) { return (__popc(ri.at(j) & pr.zl) & 1u) ? -1.0 : 1.0; };
   double acc = 0;
+  if constexpr (xr == 0) {
 #pragma unroll
-  for (int j = 0; j < NR; ++j) {
-    const double x0 = a.v[j].x, y0 = a.v[j].y;
-    const double x1 = a.v[j ^ xr].x, y1 = a.v[j ^ xr].y;
-    const double px = pr * x1 - pi * y1, py = pr * y1 + pi * x1;
-    double v = px * x0 + py * y0;
-    if (st ^ (__popc(ri.at(j) & zl) & 1u)) v = -v;
-    acc += v;
+    for (int j = 0; j < NR; ++j) {
+      const double x = wide(a.v[j].x), y = wide(a.v[j].y);
+      acc = fma_t(sign(j), fma_t(x, x, y * y), acc);
+    }
+    return pr.pr * acc;
+  } else {
+    constexpr int hb = top_bit<xr>();
+    const bool odd = (__popc((ri.at(xr) ^ ri.t0) & pr.zl) & 1u) != 0;
+    if (odd) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        if (j & (1 << hb)) continue;
+        const double x0 = wide(a.v[j].x), y0 = wide(a.v[j].y), x1 = wide(a.v[j ^ xr].x), y1 = wide(a.v[j ^ xr].y);
+        acc = fma_t(sign(j), fma_t(y1, x0, -(x1 * y0)), acc);
+      }
+      return -2.0 * pr.pi * acc;
+    }
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      if (j & (1 << hb)) continue;
+      const double x0 = wide(a.v[j].x), y0 = wide(a.v[j].y), x1 = wide(a.v[j ^ xr].x), y1 = wide(a.v[j ^ xr].y);
+      acc = fma_t(sign(j), fma_t(x1, x0, y1 * y0), acc);
+    }
+    return 2.0 * pr.pr * acc;
   }
-  return acc;
 }
 
 template <typename T, int NR, int X>
-__device__ __forceinline__ double q_probe_dispatch(uint32_t xr, const Amps<T, NR> &a, uint32_t tl,
-                                                   const RegIdx<NR> &ri, uint32_t zl,
-                                                   uint32_t sgb, double pr, double pi) {
+__device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const RegIdx<NR> &ri, const RProbe &pr) {
   if constexpr (X < NR) {
-    if (xr == X) return q_probe<T, NR, X>(a, tl, ri, zl, sgb, pr, pi);
-    return q_probe_dispatch<T, NR, X + 1>(xr, a, tl, ri, zl, sgb, pr, pi);
+    if (pr.xr == X) return q_probe<T, NR, X>(a, ri, pr);
+    return q_probe_dispatch<T, NR, X + 1>(a, ri, pr);
   } else {
     return 0.0;
   }
+}
+
+// A run of probes on the amplitudes in registers.  What a probe needs is FMAs
+// and one sum over the workgroup; barriers per probe are what cost most, so the
+// waves leave their sums in LDS and one barrier serves a batch.  33 probes per
+// pass on 2^28 complex128 amplitudes: 7.6 ms with two barriers, shuffles and
+// both orders of every pair per probe, TIME here.
+template <typename T, int NR, int NT>
+__device__ __forceinline__ Amps<T, NR> q_probes(const RProbe *recs, uint32_t count, Amps<T, NR> a, uint32_t tl,
+                                                const RegIdx<NR> &ri, uint64_t base, uint32_t tid, double *red,
+                                                const ProbeSink &sink) {
+  constexpr uint32_t NW = NT / 64;
+  double *sums = red + NW;
+  uint32_t *slots = reinterpret_cast<uint32_t *>(sums + kProbeBatch * NW);
+  for (uint32_t k = 0; k < count; ++k) {
+    // complex128 amplitudes pass through the loop as values the compiler cannot
+    // know: it would compute the products of every probe shape ahead of it
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) asm volatile("" : "+v"(a.v[j].x), "+v"(a.v[j].y));
+    }
+    const RProbe pr = recs[k];
+    double v = q_probe_dispatch<T, NR, 0>(a, ri, pr);
+    if ((__popc(tl & pr.zl) ^ __popcll(base & pr.zg)) & 1u) v = -v;
+    v = wave_sum_dpp(v);
+    if ((tid & 63u) == 63u) {
+      sums[pr.idx * NW + (tid >> 6)] = v;
+      if (tid == 63u) slots[pr.idx] = pr.slot;
+    }
+    if (pr.flush) {
+      __syncthreads();
+      if (tid < pr.flush) {
+        double s = 0;
+        for (uint32_t w = 0; w < NW; ++w) s += sums[tid * NW + w];
+        sink.put(slots[tid], s);
+      }
+      __syncthreads();  // the entries are free for the next batch
+    }
+  }
+  return a;
 }
 
 // Layout state of a thread: tile index of its thread part and of each register.
@@ -838,8 +956,8 @@ __device__ __forceinline__ void u1_matrix(const ROp<T> &op, const OpHead<T, PF> 
   m3 = fx ? c1 : c3;
 }
 
-template <typename T, int B, int R, bool FULL>
-__device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<T, !FULL> &hd,
+template <typename T, int B, int R, int V>
+__device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<T, head_payload(V)> &hd,
                                                  const Amps<T, 1 << R> &a,
                                                  LayoutState<1 << R> &st, cx<T> *lds,
                                                  double *red, uint64_t base, uint32_t tid,
@@ -885,7 +1003,7 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     }
   }
   if (kind == Q_U1M) {  // relabelled pairs
-    if constexpr (sizeof(T) == 4 && !FULL) {
+    if constexpr (sizeof(T) == 4 && head_payload(V)) {
       return d_u1m_mfma<NR>(ra, extra, a, hd.arow, mfma_row_swapped(hd.arow));
     } else {
       cx<T> m0, m1, m2, m3;
@@ -895,7 +1013,7 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
   }
   if (kind == Q_U1MX) {  // the same, with an X folded in where its tile predicate holds
     const bool fx = op_tile_ok(op, hd, base);
-    if constexpr (sizeof(T) == 4 && !FULL) {
+    if constexpr (sizeof(T) == 4 && head_payload(V)) {
       const f32x4 An = fx ? f32x4{hd.arow.z, hd.arow.w, hd.arow.x, hd.arow.y} : hd.arow;
       return d_u1m_mfma<NR>(ra, extra, a, An, mfma_row_swapped(An));
     } else {
@@ -905,26 +1023,24 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     }
   }
   if (kind == Q_PROBE || kind == Q_NOP) {
-    if (FULL && kind == Q_PROBE) {
-      const RProbe &pr = op.u.pr;
-      const uint32_t sgb = __popcll(base & pr.zg) & 1u;
-      double acc = q_probe_dispatch<T, NR, 0>(pr.xr, a, st.tl, st.ri, pr.zl, sgb, pr.pr, pr.pi);
-      acc = block_sum_nt<(1 << TB)>(acc, red);
-      if (tid == 0) sink.put(extra, acc);
+    if constexpr (has_probes(V)) {
+      if (kind == Q_PROBE)
+        return q_probes<T, NR, 1 << TB>(reinterpret_cast<const RProbe *>(pool + extra), ra, a, st.tl, st.ri, base,
+                                        tid, red, sink);
     }
     return pass_through(a);
   }
   if (kind == Q_RELAYOUT) {
     // complex64: the tile passes through LDS in a swizzled order, slot x at
     // x ^ ((x >> 4) & 15), so that consecutive lanes reach distinct banks also
-    // when the register bits are the low tile bits; complex128 in the full
-    // variant (the passes with 4x4 gates, which change layout most): slot x at
+    // when the register bits are the low tile bits; complex128 in all
+    // but the lean variant (passes with 4x4 gates change layout most): slot x at
     // x ^ ((x >> 3) & 7).  Each swizzle is linear and the thread and register
     // parts of x are disjoint, so it splits into a per-lane and a per-register
     // term.
     auto swz = [](uint32_t x) {
       if (sizeof(T) == 4) return x ^ ((x >> 4) & 15u);
-      return FULL ? x ^ ((x >> 3) & 7u) : x;
+      return V != V_LEAN ? x ^ ((x >> 3) & 7u) : x;
     };
     __syncthreads();
     const uint32_t tw = swz(st.tl);
@@ -942,12 +1058,12 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
   const uint32_t cl = tile_ok ? op_cl(op, hd) : 0u;
   const uint32_t cvl = tile_ok ? op_cvl(op, hd) : 1u;
   const uint32_t tlc = st.tl & cl;
-  if (FULL && kind == Q_U1C) {
+  if (has_gates(V) && kind == Q_U1C) {
     const cx<T> m0 = mat_at<T>(op.u.m, 0), m1 = mat_at<T>(op.u.m, 1), m2 = mat_at<T>(op.u.m, 2), m3 = mat_at<T>(op.u.m, 3);
     return d_u1c<T, NR>(ra, a, tlc, st.ri, cl, cvl, m0, m1, m2, m3);
   }
-  if (kind == Q_X || (FULL && kind == Q_Y)) {
-    const bool isy = FULL && kind == Q_Y;
+  if (kind == Q_X || (has_gates(V) && kind == Q_Y)) {
+    const bool isy = has_gates(V) && kind == Q_Y;
     if (cl == 0) {
       // No local control: the gate acts on the whole tile or not at all, so
       // the registers are only moved (no per-lane selects).
@@ -956,7 +1072,8 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     }
     return d_xy<T, NR>(ra, a, tlc, st.ri, cl, cvl, isy);
   }
-  if (FULL && kind == Q_U2) return d_u2<T, NR>(ra * reg_bits_of<NR>() + rb, a, tlc, st.ri, cl, cvl, pool + extra);
+  if (has_gates(V) && kind == Q_U2) return d_u2<T, NR>(ra * reg_bits_of<NR>() + rb, a, tlc, st.ri, cl, cvl,
+                                                        reinterpret_cast<const cx<T> *>(pool + extra));
   const cx<T> one = mk<T>(1, 0);
   Amps<T, NR> o;
   if (kind == Q_DIAGF) {
@@ -1076,7 +1193,7 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     }
     return o;
   }
-  if constexpr (!FULL) return pass_through(a);  // not reached: lean programs hold no other kinds
+  if constexpr (!has_gates(V)) return pass_through(a);  // not reached: such programs hold no other kinds
   // Q_DIAG (the last kind, so that every path computes new amplitudes)
   const TileOp &top = tops[extra];
   const uint32_t k = top.k;
@@ -1136,7 +1253,7 @@ __device__ __forceinline__ void stage_diag_tables(uint2 drec, const cx<double> *
 // form
 //     LOAD  { register ops }  ( SPILL { LDS ops } FILL { register ops } )*  STORE
 // where each register phase holds an even number of ops (Q_NOP pads).
-template <typename T, int B, int R, int MATCAP, bool FULL>
+template <typename T, int B, int R, int MATCAP, int V>
 __device__ __forceinline__ void reg_tile(cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd,
                                          const ROp<T> *__restrict__ rops,
                                          const TileOp *__restrict__ tops,
@@ -1196,13 +1313,13 @@ __device__ __forceinline__ void reg_tile(cx<T> *__restrict__ sv, const PassDesc 
     // after the current one is loaded while the current op runs.
     const uint32_t cnt = e.extra;
     const ROp<T> *opp = opl + o;
-    OpHead<T, !FULL> h0 = load_head<!FULL>(opp[0]);
+    OpHead<T, head_payload(V)> h0 = load_head<head_payload(V)>(opp[0]);
     for (uint32_t i = 0; i < cnt; i += 2) {
-      const OpHead<T, !FULL> h1 = load_head<!FULL>(opp[1]);
+      const OpHead<T, head_payload(V)> h1 = load_head<head_payload(V)>(opp[1]);
       const Amps<T, NR> b =
-          rw_op<T, B, R, FULL>(opp[0], h0, a, st, lds, red, base, tid, tops, pool, sink, dlt);
-      h0 = load_head<!FULL>(opp[2]);
-      a = rw_op<T, B, R, FULL>(opp[1], h1, b, st, lds, red, base, tid, tops, pool, sink, dlt);
+          rw_op<T, B, R, V>(opp[0], h0, a, st, lds, red, base, tid, tops, pool, sink, dlt);
+      h0 = load_head<head_payload(V)>(opp[2]);
+      a = rw_op<T, B, R, V>(opp[1], h1, b, st, lds, red, base, tid, tops, pool, sink, dlt);
       opp += 2;
     }
     o += cnt;
@@ -1210,7 +1327,7 @@ __device__ __forceinline__ void reg_tile(cx<T> *__restrict__ sv, const PassDesc 
     if (l.kind & F_MAP) {
       load_map<R>(l, st.ri);
     }
-    if (!FULL || (l.kind & ~F_MAP) == Q_STORE) {
+    if (V != V_FULL || (l.kind & ~F_MAP) == Q_STORE) {
       if (l.extra) return;  // read-only pass
       const RegOff<NR> ro = reg_offset_mapped<R>(l.u.lay, st.ri);
       cx<T> *p = sv + base + thread_offset<TB>(l.u.lay, tid);
@@ -1218,6 +1335,7 @@ __device__ __forceinline__ void reg_tile(cx<T> *__restrict__ sv, const PassDesc 
       for (int j = 0; j < NR; ++j) st_stream(p + ro.gr[j], a.v[j]);
       return;
     }
+    if constexpr (V == V_FULL) {
     // SPILL: the tile goes to LDS in natural order for the LDS primitives.
     __syncthreads();
 #pragma unroll
@@ -1229,6 +1347,7 @@ __device__ __forceinline__ void reg_tile(cx<T> *__restrict__ sv, const PassDesc 
         lds_apply<T, NT, B, MATCAP>(top, lds, mat, doff, red, N, base, pool, sink);
       }
       ++o;
+    }
     }
   }
 }
@@ -1249,25 +1368,24 @@ constexpr int reg_pass_waves() {
   return waves < 1 ? 1 : waves > 8 ? 8 : waves;
 }
 
-// One workgroup per tile.  FULL = false: a lean variant for programs whose
-// ops are all LOAD, STORE, RELAYOUT, U1, U1M, X, D1, PHASE and NOP (a single
-// register phase); the smaller op loop keeps the frequent gates faster.
-template <typename T, int B, int R, bool FULL, bool WIDE = false>
+// One workgroup per tile.  All variants but the full one run programs of a
+// single register phase.
+template <typename T, int B, int R, int V, bool WIDE = false>
 __global__ __launch_bounds__(1 << (B - R))
 __attribute__((amdgpu_waves_per_eu(reg_pass_waves<T, B, R, WIDE>()))) void k_reg_pass(
     cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd, const ROp<T> *__restrict__ rops,
     const TileOp *__restrict__ tops, const cx<double> *__restrict__ pool,
     double *__restrict__ probes, uint64_t state_stride, uint32_t pd_stride, uint32_t tile_log,
     uint32_t probes_per_state) {
-  static_assert(!WIDE || (!FULL && sizeof(T) == 8), "the wide variant is the lean complex128 one");
+  static_assert(!WIDE || (V == V_LEAN && sizeof(T) == 8), "the wide variant is the lean complex128 one");
   __shared__ cx<T> lds[1 << B];
   __shared__ cx<T> mat[16];
   __shared__ uint32_t doff[32];
-  __shared__ double red[(1 << (B - R)) / 64];
+  __shared__ double red[red_doubles((1 << (B - R)) / 64)];
   const StateTile st = state_tile(tile_log);
   const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles, false};
   // kDiagLdsBytes of dynamic LDS when the pass has fused-diagonal slots
-  reg_tile<T, B, R, 16, FULL>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool,
+  reg_tile<T, B, R, 16, V>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool,
                               sink, st.t, lds, mat, doff, red, reinterpret_cast<cx<double> *>(aerhip_dyn_lds));
 }
 
