@@ -120,14 +120,14 @@ struct TileOp {
 
 struct PassDesc {
   uint32_t kind;      // 0 = tile pass, 1 = dense group pass, 2 = register pass,
-                      // 3 = probe sweep, 4 = qubit-permutation pass (K_QPERM)
+                      // 3 = probe sweep (nops K_PROBEs), 4 = qubit-permutation pass (K_QPERM)
   uint32_t nb;        // tile qubits
   uint32_t c;         // S contains qubits 0..c-1
   uint32_t op_begin;  // first TileOp of the pass
   uint32_t nops;
   uint32_t ncomp;     // number of qubits outside the tile
   uint32_t readonly;  // 1: the pass only reads the state (probes); nothing is written back
-  uint32_t pad;
+  uint32_t batch_class; // batched circuits: 0 = runs in k_batch<V_PROBES>, 1 = in k_batch<V_FULL>
   uint8_t spos[16];   // tile qubits, ascending
   uint8_t comp[64];   // qubits outside the tile, ascending
 };

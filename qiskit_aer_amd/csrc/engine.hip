@@ -1556,6 +1556,45 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   emit(Q_STORE, rs);
 }
 
+// Read-only passes that follow one another commute.  Of such a run, the probes
+// too wide for a tile become one sweep, and so do those of tile passes that
+// hold one or two where that reads less: a tile pass reads the whole state, a
+// sweep the state once and half of it per probe.  Measured on 28 qubits
+// (complex128): a tile pass of two probes 0.60 ms, a sweep of the two 1.09; 16
+// random Pauli strings on 20 qubits took 16 passes, now one or two.
+std::vector<PassPlan> Engine::gather_sweeps(std::vector<PassPlan> plans) const {
+  if (n_ <= tile_bits_) return plans;
+  std::vector<PassPlan> out;
+  for (size_t i = 0; i < plans.size();) {
+    auto readonly = [&](const PassPlan &pp) {
+      for (uint32_t idx : pp.prims)
+        if (queue_[idx].kind != K_PROBE) return false;
+      return true;
+    };
+    size_t j = i, wide = 0, ones = 0;
+    while (j < plans.size() && readonly(plans[j])) {
+      wide += plans[j].solo;
+      ones += !plans[j].solo && plans[j].prims.size() == 1;
+      ++j;
+    }
+    if (j == i) {
+      out.push_back(std::move(plans[i++]));
+      continue;
+    }
+    const bool sweeps = wide > 0 || ones > 2;  // 1 + ones / 2 reads against `ones`
+    PassPlan sweep{true, 0, {}};
+    for (; i < j; ++i) {
+      PassPlan &pp = plans[i];
+      if (pp.solo || (sweeps && pp.prims.size() <= 2))
+        sweep.prims.insert(sweep.prims.end(), pp.prims.begin(), pp.prims.end());
+      else
+        out.push_back(std::move(pp));
+    }
+    if (!sweep.prims.empty()) out.push_back(std::move(sweep));
+  }
+  return out;
+}
+
 std::vector<PassPlan> Engine::plan() const {
   std::vector<PassPlan> out;
   const uint32_t nb = tile_bits_;
@@ -1981,7 +2020,16 @@ void Engine::set_block_fusion(uint32_t width, bool cost_check) {
 void Engine::emit_program(Program &prog) {
   if (block_width_ >= 2 && n_ > fusion_threshold_) queue_ = fuse_blocks(queue_);
   queue_ = merge_swap_layers(queue_);
-  const std::vector<PassPlan> plans = plan();
+  // Of probes that follow one another, those a tile can hold come first: the
+  // others end the stretch of the queue that is planned together.
+  for (size_t i = 0; i < queue_.size();) {
+    size_t j = i;
+    while (j < queue_.size() && queue_[j].kind == K_PROBE) ++j;
+    if (j > i + 1)
+      std::stable_partition(queue_.begin() + i, queue_.begin() + j, [](const Prim &p) { return !p.solo; });
+    i = std::max(j, i + 1);
+  }
+  const std::vector<PassPlan> plans = gather_sweeps(plan());
   std::vector<PassDesc> &passes = prog.passes;
   std::vector<TileOp> &ops = prog.ops;
   std::vector<ROp<double>> &rops = prog.rops;
@@ -2008,17 +2056,7 @@ void Engine::emit_program(Program &prog) {
     }
     pd.kind = pp.solo ? 1u : 0u;
     if (pp.solo && queue_[pp.prims[0]].kind == K_PROBE) {
-      // probe sweep: one TileOp with the masks over all qubits
-      const Prim &p = queue_[pp.prims[0]];
-      TileOp op;
-      std::memset(&op, 0, sizeof(op));
-      op.kind = K_PROBE;
-      op.cg = p.xmask;
-      op.zg = p.zmask;
-      op.t = p.q.empty() ? 0u : p.q[0];
-      op.npairs = p.npairs;
-      op.pr = p.pr;
-      op.pi = p.pi;
+      // probe sweep: one TileOp per probe with the masks over all qubits
       PassDesc sd;
       std::memset(&sd, 0, sizeof(sd));
       sd.kind = 3;
@@ -2026,8 +2064,19 @@ void Engine::emit_program(Program &prog) {
       sd.nb = tile_bits_;
       sd.ncomp = n_ - tile_bits_;
       sd.op_begin = static_cast<uint32_t>(ops.size());
-      sd.nops = 1;
-      ops.push_back(op);
+      sd.nops = static_cast<uint32_t>(pp.prims.size());
+      for (uint32_t idx : pp.prims) {
+        const Prim &p = queue_[idx];
+        TileOp op;
+        std::memset(&op, 0, sizeof(op));
+        op.kind = K_PROBE;
+        op.cg = p.xmask;
+        op.zg = p.zmask;
+        op.npairs = p.npairs;
+        op.pr = p.pr;
+        op.pi = p.pi;
+        ops.push_back(op);
+      }
       passes.push_back(sd);
       continue;
     }
@@ -2199,16 +2248,14 @@ void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, co
                                                 dp.probes, state_stride, pd_stride, tl, pps);
     }
   } else if (pd.kind == 3) {
-    // probe sweep over the whole state, one workgroup per tile-sized slice
+    // probes over the whole state, one workgroup per tile-sized slice
     const uint32_t tl = n - tile_bits;
     if (prec == AERHIP_PRECISION_DOUBLE)
       k_probe_sweep<double><<<grid_of(tl), kThreads, 0, stream>>>(
-          static_cast<const cx<double> *>(sv), state_stride, dpd, dp.ops, dp.probes, state_stride, pd_stride,
-          tl, pps);
+          static_cast<const cx<double> *>(sv), dpd, dp.ops, dp.probes, state_stride, pd_stride, tl, pps);
     else
       k_probe_sweep<float><<<grid_of(tl), kThreads, 0, stream>>>(
-          static_cast<const cx<float> *>(sv), state_stride, dpd, dp.ops, dp.probes, state_stride, pd_stride,
-          tl, pps);
+          static_cast<const cx<float> *>(sv), dpd, dp.ops, dp.probes, state_stride, pd_stride, tl, pps);
   } else if (pd.kind == 4) {
     // qubit permutation (a layer of SWAPs): four tiles per workgroup, each
     // exchanged with its partner tile or skipped
@@ -2845,8 +2892,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   std::vector<uint64_t> pass_at(count + 1, 0), op_at(count + 1, 0), rop_at(count + 1, 0),
       pool_at(count + 1, 0);
   std::vector<BatchCircuit> circ(count);
-  std::vector<double> cost(count);
-  uint64_t sv_off = 0, probe_off = 0;
+  uint64_t sv_off = 0, probe_off = 0, part_off = 0;
   for (uint64_t i = 0; i < count; ++i) {
     const Program &p = parts[i];
     for (const PassDesc &d : p.passes)
@@ -2864,18 +2910,31 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     c.pass_count = static_cast<uint32_t>(p.passes.size());
     c.probe_base = static_cast<uint32_t>(probe_off);
     c.num_probes = nprobes[i];
-    cost[i] = static_cast<double>(c.pass_count + 1) * static_cast<double>(1ull << c.num_qubits);
+    c.tile_log = c.num_qubits - engines[i]->tile_bits();
+    c.part_off = part_off;
     sv_off += align_up(1ull << c.num_qubits, 256);
+    part_off += static_cast<uint64_t>(c.num_probes) << c.tile_log;
     probe_off += c.num_probes;
   }
   if (op_at[count] > UINT32_MAX || rop_at[count] > UINT32_MAX || pool_at[count] > UINT32_MAX)
     throw std::invalid_argument("aerhip: batch program too large");
-  // Largest circuits first: workgroups start in index order.
-  std::vector<uint64_t> order(count);
-  for (uint64_t i = 0; i < count; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return cost[a] > cost[b]; });
-  std::vector<BatchCircuit> sorted(count);
-  for (uint64_t i = 0; i < count; ++i) sorted[i] = circ[order[i]];
+  // By size, then by number of passes: the circuits of one size that have a
+  // pass p are a range for every p.
+  std::vector<BatchCircuit> sorted = circ;
+  std::stable_sort(sorted.begin(), sorted.end(), [](const BatchCircuit &a, const BatchCircuit &b) {
+    return a.num_qubits != b.num_qubits ? a.num_qubits > b.num_qubits : a.pass_count > b.pass_count;
+  });
+  uint32_t max_passes = 0;
+  for (const BatchCircuit &c : sorted) max_passes = std::max(max_passes, c.pass_count);
+  // Per pass index: which kernels its passes need (bit 0 k_batch<V_PROBES>,
+  // bit 1 k_batch<V_FULL>).
+  std::vector<uint32_t> classes(max_passes, 0);
+  for (Program &p : parts)
+    for (size_t k = 0; k < p.passes.size(); ++k) {
+      PassDesc &d = p.passes[k];
+      d.batch_class = d.kind == 2 && !has_gates(pass_kernel(d, p.rops).variant) ? 0u : 1u;
+      classes[k] |= 1u << d.batch_class;
+    }
 
   const size_t amp = prec == AERHIP_PRECISION_DOUBLE ? 16 : 8;
   const size_t circ_bytes = count * sizeof(BatchCircuit);
@@ -2940,23 +2999,49 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     AERHIP_CHECK(hipEventCreate(&e1));
     AERHIP_CHECK(hipMalloc(&d_states, sv_off * amp));
     AERHIP_CHECK(hipMalloc(&d_prog, total));
-    AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_probes), (probe_off + 1) * sizeof(double)));
+    AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_probes), (probe_off + part_off + 1) * sizeof(double)));
     AERHIP_CHECK(hipMemcpyAsync(d_prog, h.get(), total, hipMemcpyHostToDevice, st));
     char *d = static_cast<char *>(d_prog);
     const auto *dc = reinterpret_cast<const BatchCircuit *>(d);
-    const auto *dp = reinterpret_cast<const PassDesc *>(d + pass_off);
-    const auto *dops = reinterpret_cast<const TileOp *>(d + ops_off);
-    const auto *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
-    const uint32_t grid = static_cast<uint32_t>(count);
     AERHIP_CHECK(hipEventRecord(e0, st));
+    auto run = [&](auto zero, auto bits, auto regs) {
+      using T = decltype(zero);
+      constexpr int B = decltype(bits)::value, R = decltype(regs)::value;
+      auto *sv = static_cast<cx<T> *>(d_states);
+      const auto *dp = reinterpret_cast<const PassDesc *>(d + pass_off);
+      const auto *dr = reinterpret_cast<const ROp<T> *>(d + rops_off);
+      const auto *dops = reinterpret_cast<const TileOp *>(d + ops_off);
+      const auto *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
+      k_fill_basis<T><<<grid_for(sv_off, 16384), kThreads, 0, st>>>(sv, sv_off, ~0ull);
+      k_batch_ones<T><<<grid_for(count, 1u << 30), kThreads, 0, st>>>(sv, dc, count);
+      for (uint32_t p = 0; p < max_passes; ++p) {
+        BatchGroups gr;
+        std::memset(&gr, 0, sizeof(gr));
+        uint64_t wgs = 0;
+        for (uint64_t i = 0; i < count;) {
+          uint64_t j = i, end = i;  // [i, end): one size; [i, j): those with a pass p
+          while (end < count && sorted[end].num_qubits == sorted[i].num_qubits) ++end;
+          while (j < end && sorted[j].pass_count > p) ++j;
+          if (j > i) {
+            gr.g[gr.n++] = BatchGroup{static_cast<uint32_t>(i), static_cast<uint32_t>(wgs), sorted[i].tile_log};
+            wgs += (j - i) << sorted[i].tile_log;
+          }
+          i = end;
+        }
+        if (wgs > 0xFFFFFFFFull / kThreads) throw std::invalid_argument("aerhip: batch too large for one launch");
+        if (classes[p] & 1u)
+          k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops,
+                                                                                     dpool, d_probes + probe_off);
+        if (classes[p] & 2u)
+          k_batch<T, B, R, V_FULL><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops, dpool,
+                                                                                   d_probes + probe_off);
+      }
+      k_batch_sums<<<static_cast<uint32_t>(count), kThreads, 0, st>>>(dc, d_probes + probe_off, d_probes);
+    };
     if (prec == AERHIP_PRECISION_DOUBLE)
-      k_batch<double, kTileBitsC128, 3><<<grid, kThreads, 0, st>>>(
-          static_cast<cx<double> *>(d_states), dc, dp,
-          reinterpret_cast<const ROp<double> *>(d + rops_off), dops, dpool, d_probes);
+      run(0.0, std::integral_constant<int, kTileBitsC128>{}, std::integral_constant<int, 3>{});
     else
-      k_batch<float, kTileBitsC64, 4><<<grid, kThreads, 0, st>>>(
-          static_cast<cx<float> *>(d_states), dc, dp,
-          reinterpret_cast<const ROp<float> *>(d + rops_off), dops, dpool, d_probes);
+      run(0.0f, std::integral_constant<int, kTileBitsC64>{}, std::integral_constant<int, 4>{});
     AERHIP_CHECK(hipGetLastError());
     AERHIP_CHECK(hipEventRecord(e1, st));
     AERHIP_CHECK(hipMemcpyAsync(values, d_probes, probe_off * sizeof(double), hipMemcpyDeviceToHost, st));

@@ -162,6 +162,7 @@ class Engine {
   void apply_matrix_1(uint32_t q, const std::vector<cd> &mat);
   void apply_diagonal_1(uint32_t q, const cd *diag);
   std::vector<PassPlan> plan() const;
+  std::vector<PassPlan> gather_sweeps(std::vector<PassPlan> plans) const;
   std::vector<Prim> fuse_blocks(const std::vector<Prim> &in);
   std::vector<Prim> merge_swap_layers(const std::vector<Prim> &in) const;
   PassDesc qperm_pass(const Prim &p, std::vector<TileOp> &ops) const;

@@ -1,6 +1,6 @@
-// complex64 batched-circuit kernel.
+// complex64 batched-circuit kernel: every pass kind.
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_BATCH(, float, kTileBitsC64, 4)
+AERHIP_BATCH(, float, kTileBitsC64, 4, V_FULL)
 }  // namespace aerhip

@@ -16,11 +16,11 @@ constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
       cx<T> *__restrict__, const PassDesc *__restrict__, const ROp<T> *__restrict__,                     \
       const TileOp *__restrict__, const cx<double> *__restrict__, double *__restrict__, uint64_t,        \
       uint32_t, uint32_t, uint32_t);
-#define AERHIP_BATCH(EXT, T, B, R)                                                                       \
-  EXT template __global__ void k_batch<T, B, R>(cx<T> *__restrict__, const BatchCircuit *__restrict__,   \
-                                                const PassDesc *__restrict__, const ROp<T> *__restrict__, \
-                                                const TileOp *__restrict__,                              \
-                                                const cx<double> *__restrict__, double *__restrict__);
+#define AERHIP_BATCH(EXT, T, B, R, V)                                                                    \
+  EXT template __global__ void k_batch<T, B, R, V>(                                                      \
+      cx<T> *__restrict__, const BatchCircuit *__restrict__, const BatchGroups, uint32_t,                \
+      const PassDesc *__restrict__, const ROp<T> *__restrict__, const TileOp *__restrict__,              \
+      const cx<double> *__restrict__, double *__restrict__);
 
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, false)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, true)
@@ -35,7 +35,9 @@ AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_PROBES, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_FULL, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_LEAN, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_FULL, false)
-AERHIP_BATCH(extern, double, kTileBitsC128, 3)
-AERHIP_BATCH(extern, float, kTileBitsC64, 4)
+AERHIP_BATCH(extern, double, kTileBitsC128, 3, V_PROBES)
+AERHIP_BATCH(extern, double, kTileBitsC128, 3, V_FULL)
+AERHIP_BATCH(extern, float, kTileBitsC64, 4, V_PROBES)
+AERHIP_BATCH(extern, float, kTileBitsC64, 4, V_FULL)
 
 }  // namespace aerhip

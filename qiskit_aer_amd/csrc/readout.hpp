@@ -2,6 +2,7 @@
 // probabilities and the sampling index.  Included by engine.hip alone.
 #pragma once
 
+#include "batch.hpp"
 #include "kernels.hpp"
 #include "tile_pass.hpp"
 
@@ -49,6 +50,22 @@ inline void sum_rows(const double *partial, uint64_t rows, uint32_t cols, double
     k_sum_rows<kThreads><<<static_cast<uint32_t>(rows), kThreads, 0, stream>>>(partial, cols, out);
   else
     k_sum_rows<1024><<<static_cast<uint32_t>(rows), 1024, 0, stream>>>(partial, cols, out);
+}
+
+// values[probe_base + i] = sum of the tile partials of probe i: a workgroup per
+// circuit, a wave per probe.
+__global__ __launch_bounds__(kThreads) void k_batch_sums(const BatchCircuit *__restrict__ circ,
+                                                      const double *__restrict__ partial,
+                                                               double *__restrict__ values) {
+  const BatchCircuit &c = circ[blockIdx.x];
+  const uint64_t tiles = 1ull << c.tile_log;
+  for (uint32_t i = threadIdx.x >> 6; i < c.num_probes; i += kThreads / 64) {
+    const double *row = partial + c.part_off + i * tiles;
+    double s = 0;
+    for (uint64_t k = threadIdx.x & 63u; k < tiles; k += 64) s += row[k];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63u) == 0) values[c.probe_base + i] = s;
+  }
 }
 
 // Marginal probabilities, QubitVector::probabilities(qubits)

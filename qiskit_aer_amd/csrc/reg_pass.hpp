@@ -1383,10 +1383,91 @@ __attribute__((amdgpu_waves_per_eu(reg_pass_waves<T, B, R, WIDE>()))) void k_reg
   __shared__ uint32_t doff[32];
   __shared__ double red[red_doubles((1 << (B - R)) / 64)];
   const StateTile st = state_tile(tile_log);
-  const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles, false};
+  const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles};
   // kDiagLdsBytes of dynamic LDS when the pass has fused-diagonal slots
   reg_tile<T, B, R, 16, V>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool,
                               sink, st.t, lds, mat, doff, red, reinterpret_cast<cx<double> *>(aerhip_dyn_lds));
+}
+
+// Saved Pauli expectation values as a sweep, for probes that share no tile
+// pass: `op[0..nops)` K_PROBEs with cg = X mask, zg = Z mask over all qubits.
+// The workgroup holds the 2^nb amplitudes of its slice in registers for the
+// whole list; a probe reads the partners i ^ X, a permuted slice, and only in
+// the slices whose highest differing qubit outside the slice is 0 (the other
+// member of a pair adds the same or the opposite, see q_probe).  So a probe costs half a read of
+// the state, where a sweep of its own costs a whole one and a launch.
+template <typename T, int NT, int NR>
+__device__ __forceinline__ void probe_sweep(const cx<T> *__restrict__ sv, const TileOp *__restrict__ ops,
+                                            uint32_t nops, uint32_t nb, const ProbeSink &sink, uint64_t slice,
+                                            double *red) {
+  constexpr uint32_t NW = NT / 64;
+  double *sums = red + NW;
+  const uint32_t tid = threadIdx.x, N = 1u << nb;
+  const uint64_t base = slice << nb;
+  cx<T> a[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) {
+    const uint32_t i = static_cast<uint32_t>(j) * NT + tid;
+    a[j] = i < N ? sv[base + i] : mk<T>(0, 0);
+  }
+  for (uint32_t k = 0; k < nops; ++k) {
+    const TileOp &op = ops[k];
+    const uint64_t x = op.cg, z = op.zg, xh = x >> nb << nb;
+    const uint32_t xl = static_cast<uint32_t>(x) & (N - 1u);
+    const bool odd = (__popcll(x & z) & 1u) != 0;
+    double acc = 0;
+    if (!(xh & base) || !((base >> (63 - __clzll(xh))) & 1ull)) {
+      const cx<T> *other = sv + (base ^ xh);
+      cx<T> b[NR];
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        const uint32_t i = static_cast<uint32_t>(j) * NT + tid;
+        b[j] = i < N ? other[i ^ xl] : mk<T>(0, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        const double s = (__popcll(z & (static_cast<uint64_t>(j) * NT)) & 1u) ? -1.0 : 1.0;
+        const double x0 = a[j].x, y0 = a[j].y, x1 = b[j].x, y1 = b[j].y;
+        const double p = odd ? y1 : x1, q = odd ? -x1 : y1;
+        acc = fma_t(s, fma_t(p, x0, q * y0), acc);
+      }
+      acc *= (odd ? -op.pi : op.pr) * (xh ? 2.0 : 1.0);
+      if (__popcll(z & (base | (tid & (NT - 1u)))) & 1u) acc = -acc;
+    }
+    acc = wave_sum_dpp(acc);
+    const uint32_t idx = k % kProbeBatch;
+    if ((tid & 63u) == 63u) sums[idx * NW + (tid >> 6)] = acc;
+    if (idx == kProbeBatch - 1 || k + 1 == nops) {
+      __syncthreads();
+      if (tid <= idx) {
+        double t = 0;
+        for (uint32_t w = 0; w < NW; ++w) t += sums[tid * NW + w];
+        sink.put(ops[k - idx + tid].npairs, t);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+template <typename T>
+constexpr int probe_sweep_regs() {  // amplitudes per thread of the largest tile
+  return 32768 / static_cast<int>(sizeof(cx<T>)) / kThreads;
+}
+
+// One workgroup per slice (2^tile_log slices per state).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_probe_sweep(const cx<T> *__restrict__ sv,
+                                                          const PassDesc *__restrict__ pd,
+                                                          const TileOp *__restrict__ ops,
+                                                          double *__restrict__ probes,
+                                                          uint64_t state_stride, uint32_t pd_stride,
+                                                          uint32_t tile_log, uint32_t probes_per_state) {
+  __shared__ double red[red_doubles(kThreads / 64)];
+  const StateTile st = state_tile(tile_log);
+  const PassDesc *d = pd + st.b * pd_stride;
+  const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles};
+  probe_sweep<T, kThreads, probe_sweep_regs<T>()>(sv + st.b * state_stride, ops + d->op_begin, d->nops, d->nb, sink,
+                                                  st.t, red);
 }
 
 // A layer of SWAPs on disjoint qubit pairs permutes the index bits by an

@@ -39,17 +39,12 @@ __device__ __forceinline__ constexpr int pair_lo(int p) {
 }
 
 // Where a tile's share of a saved expectation value goes: p[slot * ntiles +
-// tile] (one workgroup per tile; the host sums the row in tile order), or,
-// with one workgroup walking every tile of a state, p[slot] += share.
+// tile] (one workgroup per tile; the rows are summed afterwards).
 struct ProbeSink {
   double *p;
   uint64_t tile, ntiles;
-  bool accumulate;
   __device__ __forceinline__ void put(uint32_t slot, double v) const {
-    if (accumulate)
-      p[slot] += v;
-    else
-      p[static_cast<uint64_t>(slot) * ntiles + tile] = v;
+    p[static_cast<uint64_t>(slot) * ntiles + tile] = v;
   }
 };
 
@@ -404,44 +399,6 @@ __device__ __forceinline__ void lds_tile(cx<T> *__restrict__ sv, const PassDesc 
   for (uint32_t l = tid; l < N; l += NT) sv[base + (l & cmask) + hioff[l >> c]] = tile[l];
 }
 
-// A saved Pauli expectation value whose X/Y qubits do not fit a tile: block
-// `blk` of `nblk` equal slices of k_expval_pauli's iteration space (pairs
-// idx0 = insert-0 at the pivot, idx1 = idx0 ^ X; or single amplitudes when X
-// is empty).  op: K_PROBE with cg = X mask, zg = Z mask (all qubits), t = the
-// pivot.  Returns the slice's share in thread 0.
-template <typename T, int NT>
-__device__ __forceinline__ double probe_sweep_block(const cx<T> *__restrict__ sv, uint64_t size,
-                                                    const TileOp &op, uint64_t blk,
-                                                    uint64_t nblk, double *red) {
-  const uint64_t xmask = op.cg, zmask = op.zg;
-  const uint32_t xmax = op.t;
-  const double pr = op.pr, pi = op.pi;
-  const uint64_t work = xmask ? size >> 1 : size;
-  const uint64_t chunk = (work + nblk - 1) / nblk;
-  const uint64_t lo = blk * chunk;
-  const uint64_t hi = lo + chunk < work ? lo + chunk : work;
-  double acc = 0;
-  for (uint64_t i = lo + threadIdx.x; i < hi; i += NT) {
-    if (xmask == 0) {
-      const double x = sv[i].x, y = sv[i].y;
-      double v = pr * (x * x + y * y);
-      if (__popcll(i & zmask) & 1) v = -v;
-      acc += v;
-    } else {
-      const uint64_t i0 = insert_zero64(i, xmax), i1 = i0 ^ xmask;
-      const double x0 = sv[i0].x, y0 = sv[i0].y, x1 = sv[i1].x, y1 = sv[i1].y;
-      const double a1x = pr * x1 - pi * y1, a1y = pr * y1 + pi * x1;
-      const double a0x = pr * x0 - pi * y0, a0y = pr * y0 + pi * x0;
-      double v0 = a1x * x0 + a1y * y0;
-      double v1 = a0x * x1 + a0y * y1;
-      if (__popcll(i0 & zmask) & 1) v0 = -v0;
-      if (__popcll(i1 & zmask) & 1) v1 = -v1;
-      acc += v0 + v1;
-    }
-  }
-  return block_sum_nt<NT>(acc, red);
-}
-
 // Workgroup -> (state, tile) of a pass over `count` states of one size that
 // run the same pass index: workgroup w (after the XCD-aware order) takes tile
 // w mod 2^tile_log of state w >> tile_log.  State b's amplitudes start at
@@ -454,25 +411,6 @@ struct StateTile {
 __device__ __forceinline__ StateTile state_tile(uint32_t tile_log) {
   const uint64_t w = xcd_tile(blockIdx.x, gridDim.x);
   return StateTile{w >> tile_log, w & ((1ull << tile_log) - 1ull), 1ull << tile_log};
-}
-
-// One workgroup per slice (2^tile_log slices per state):
-// probes[(b * probes_per_state + slot) * 2^tile_log + slice].  The probe of
-// state b is ops[pd_b->op_begin], pd_b = pd + b * pd_stride.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_probe_sweep(const cx<T> *__restrict__ sv,
-                                                          uint64_t size,
-                                                          const PassDesc *__restrict__ pd,
-                                                          const TileOp *__restrict__ ops,
-                                                          double *__restrict__ probes,
-                                                          uint64_t state_stride, uint32_t pd_stride,
-                                                          uint32_t tile_log, uint32_t probes_per_state) {
-  __shared__ double red[kThreads / 64];
-  const StateTile st = state_tile(tile_log);
-  const TileOp &o = ops[pd[st.b * pd_stride].op_begin];
-  const double v = probe_sweep_block<T, kThreads>(sv + st.b * state_stride, size, o, st.t, st.ntiles, red);
-  if (threadIdx.x == 0)
-    probes[(st.b * probes_per_state + o.npairs) * st.ntiles + st.t] = v;
 }
 
 // One workgroup per tile.
@@ -490,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_lds(cx<T> *__restrict__ sv,
   __shared__ uint32_t doff[32];
   __shared__ double red[kThreads / 64];
   const StateTile st = state_tile(tile_log);
-  const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles, false};
+  const ProbeSink sink{probes + st.b * probes_per_state * st.ntiles, st.t, st.ntiles};
   lds_tile<T, kThreads, BMAX, 1024>(sv + st.b * state_stride, pd + st.b * pd_stride, ops, pool,
                                     sink, st.t, tile, hioff, mat, doff, red);
 }
