@@ -19,6 +19,10 @@ namespace aerhip {
 namespace {
 
 constexpr size_t kMaxQueue = 4096;      // flush threshold of the gate queue
+// Gate passes from 2^9 tiles on (two workgroups per CU): 20 layers of brickwork at
+// fusion width 2 take 1.19 against 1.13 ms on 21 qubits, 1.65 against 1.30 on 22,
+// but 1.10 against 1.15 on 20.
+constexpr uint32_t kGateMinQubits = 21;
 
 inline uint64_t bit(uint32_t q) { return 1ull << q; }
 
@@ -54,7 +58,7 @@ Engine::Engine(uint32_t num_qubits, int precision, int device)
 }
 
 Engine::Engine(uint32_t num_qubits, int precision, int device, PlanOnly)
-    : n_(num_qubits), prec_(precision), device_(device), plan_only_(true) {
+    : n_(num_qubits), prec_(precision), device_(device), plan_only_(true), gate_passes_(false) {
   if (precision != AERHIP_PRECISION_DOUBLE && precision != AERHIP_PRECISION_SINGLE)
     throw std::invalid_argument("aerhip: invalid precision");
   if (num_qubits < 1 || num_qubits > 40)
@@ -669,6 +673,7 @@ struct RItem {
 };
 
 constexpr uint32_t kProbeSentinel = 1u << 31;
+constexpr size_t kMaxMoves = 4;  // register moves that still cost less than a layout change
 
 RItem classify_item(const TileOp &op, uint32_t R) {
   RItem it;
@@ -991,7 +996,7 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
         case Q_U1: case Q_U1X: case Q_U1C: case Q_X: case Q_Y:
           if (r.a >= R) fail("register bit of a gate");
           break;
-        case Q_U2:
+        case Q_U2: case Q_CXR:
           if (r.a >= R || r.b >= R || r.a == r.b) fail("register bits of a 2-qubit gate");
           break;
         case Q_D1: if (r.a >= B) fail("diagonal bit"); break;
@@ -1030,10 +1035,13 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
 // double; converted for complex64 at upload), TileOps run on the LDS tile go to
 // `tops`.  `lowb`: tile bits that must be lane bits for a full 128-byte run per
 // HBM access.
-void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uint32_t lowb, bool single,
+// `gate`: for a gate pass (gate_pass.hpp), which moves registers instead of
+// relabelling them and finds its ops by code.
+void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uint32_t lowb, bool single, bool gate,
                       const uint8_t *spos, std::vector<cd> &pool,
                       std::vector<ROp<double>> &rops, std::vector<TileOp> &tops,
                       uint64_t *relayouts) {
+  const size_t first_rop = rops.size();
   std::vector<RItem> rem;
   rem.reserve(in.size());
   for (const TileOp &op : in) rem.push_back(classify_item(op, R));
@@ -1221,6 +1229,46 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       if ((tmask & cur_rs & (1u << b))) r |= 1u << regidx(cur_rs, b);
     return r;
   };
+  // Ends the relabelling by moving the registers: content of register j goes to
+  // lin(j) ^ cinv, as a sequence of CX on register bits (Gauss-Jordan on the
+  // columns of lin: CX from s to t adds column t to column s) and X.  Returns
+  // false, with nothing done, where that takes more moves than a layout change
+  // is worth.
+  auto move_home = [&] {
+    uint32_t col[8];
+    std::vector<std::pair<uint32_t, uint32_t>> steps;
+    for (uint32_t q = 0; q < R; ++q) col[q] = colinv[q];
+    auto add = [&](uint32_t s, uint32_t t) {
+      col[s] ^= col[t];
+      steps.push_back({s, t});
+    };
+    for (uint32_t b = 0; b < R; ++b) {
+      for (uint32_t s = b + 1; s < R && !((col[b] >> b) & 1u); ++s)
+        if ((col[s] >> b) & 1u) add(b, s);
+      for (uint32_t s = 0; s < R; ++s)
+        if (s != b && ((col[s] >> b) & 1u)) add(s, b);
+    }
+    if (steps.size() + static_cast<size_t>(__builtin_popcount(cinv)) > kMaxMoves) return false;
+    for (const auto &st : steps) {
+      ROp<double> r;
+      std::memset(&r, 0, sizeof(r));
+      r.kind = Q_CXR;
+      r.a = st.first;
+      r.b = st.second;
+      rops.push_back(r);
+    }
+    for (uint32_t b = 0; b < R; ++b)
+      if ((cinv >> b) & 1u) {
+        ROp<double> r;
+        std::memset(&r, 0, sizeof(r));
+        r.kind = Q_X;
+        r.a = b;
+        rops.push_back(r);
+      }
+    map_reset();
+    map_dirty = true;  // the next op carries the layout's own order
+    return true;
+  };
   // X gates controlled only by qubits fixed by the tile, waiting on logical
   // register bits (pend) to fold into the next 2x2 gate on that bit (Q_U1X,
   // Q_U1MX);
@@ -1234,7 +1282,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     bool fresh = true;
     for (uint32_t b = 0; b < R; ++b)
       if ((bits >> b) & 1u) fresh = fresh && identity_on(b);
-    if (!fresh) {
+    if (!fresh && !move_home()) {
       emit_raw(Q_RELAYOUT, cur_rs);  // Q_X pairs the layout's own register bits
       if (relayouts) ++*relayouts;
     }
@@ -1260,7 +1308,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   auto need_identity = [&](uint32_t rs, std::initializer_list<uint32_t> bits) {
     bool ok = true;
     for (uint32_t b : bits) ok = ok && identity_on(b);
-    if (ok) return;
+    if (ok || move_home()) return;
     emit(Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
   };
@@ -1326,7 +1374,21 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         }
         materialize((1u << t) | reg_bits(op.cl));
         if (op.kind == K_MCX && op.cg == 0 && (op.cl & ~rs) == 0 && __builtin_popcount(op.cl) <= 1) {
-          // X with at most one register control: relabel the registers
+          // X with at most one register control: relabel the registers, or in
+          // a gate pass, whose ops work in place, move them
+          if (gate) {
+            auto move = [&](uint32_t kind, uint32_t a, uint32_t b) {
+              ROp<double> m;
+              std::memset(&m, 0, sizeof(m));
+              m.kind = kind;
+              m.a = a;
+              m.b = b;
+              rops.push_back(m);
+            };
+            if (op.cl) move(Q_CXR, regidx(rs, static_cast<uint32_t>(__builtin_ctz(op.cl))), t);
+            if (!op.cl || !(op.cvl & op.cl)) move(Q_X, t, 0);
+            return;
+          }
           if (op.cl == 0) {
             cinv ^= 1u << t;
           } else {
@@ -1352,6 +1414,15 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         r.a = b0;
         r.b = b1;
         r.extra = op.off;
+        if (gate && b0 > b1) {
+          // gate passes take the lower register bit as matrix bit 0
+          std::swap(r.a, r.b);
+          cd m[16];
+          auto sw = [](uint32_t i) { return (i >> 1) | (i & 1u) << 1; };
+          for (uint32_t e = 0; e < 16; ++e) m[sw(e & 3u) + 4 * sw(e >> 2)] = pool[op.off + e];
+          r.extra = static_cast<uint32_t>(pool.size());
+          pool.insert(pool.end(), m, m + 16);
+        }
         if (single) {
           // rounded here: the kernel reads the entries as scalars, where
           // rounding them would cost it a conversion and a register each
@@ -1554,6 +1625,13 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     std::memcpy(pool.data() + last_probe, &pr, sizeof(pr));
   }
   emit(Q_STORE, rs);
+  if (gate)
+    for (size_t i = first_rop; i < rops.size(); ++i) {
+      const uint32_t k = rops[i].kind;
+      rops[i].code = gate_code(rops[i]);
+      if (rops[i].code == C_NOP && k != Q_NOP && k != Q_LOAD && k != Q_STORE)
+        throw std::logic_error("aerhip: op outside the gate pass");
+    }
 }
 
 // Read-only passes that follow one another commute.  Of such a run, the probes
@@ -1582,7 +1660,8 @@ std::vector<PassPlan> Engine::gather_sweeps(std::vector<PassPlan> plans) const {
       continue;
     }
     const bool sweeps = wide > 0 || ones > 2;  // 1 + ones / 2 reads against `ones`
-    PassPlan sweep{true, 0, {}};
+    PassPlan sweep;
+    sweep.solo = true;
     for (; i < j; ++i) {
       PassPlan &pp = plans[i];
       if (pp.solo || (sweeps && pp.prims.size() <= 2))
@@ -1595,6 +1674,24 @@ std::vector<PassPlan> Engine::gather_sweeps(std::vector<PassPlan> plans) const {
   return out;
 }
 
+// Whether the handle's passes may use the gate pass's larger tiles: complex128
+// under the engine's own tile settings, with diagonal fusion (single diagonals
+// on fixed qubits run fused), and enough tiles to fill the device.
+bool Engine::gate_tiles() const {
+  return gate_passes_ && prec_ == AERHIP_PRECISION_DOUBLE && tile_bits_ == kTileBitsC128 && low_bits_ == 3 &&
+         reg_bits_ == 3 && fusion_enable_ && n_ > fusion_threshold_ && n_ >= kGateMinQubits;
+}
+
+// Whether the gate pass runs a primitive.
+bool Engine::gate_prim(const Prim &p) const {
+  switch (p.kind) {
+    case K_DENSE1: case K_MCX: case K_MCY: case K_MCPHASE: return true;
+    case K_DENSE: return p.q.size() == 2 && p.ctrl.empty();
+    case K_DIAG: return p.q.size() == 1 && p.ctrl.empty();
+    default: return false;
+  }
+}
+
 std::vector<PassPlan> Engine::plan() const {
   std::vector<PassPlan> out;
   const uint32_t nb = tile_bits_;
@@ -1603,6 +1700,7 @@ std::vector<PassPlan> Engine::plan() const {
   for (const Prim &p : queue_)
     if (!p.solo && static_cast<uint32_t>(__builtin_popcountll(p.tmask | lowmask)) > nb)
       throw std::logic_error("aerhip: a primitive mixes more qubits than a tile holds");
+  const bool gates = gate_tiles();
   while (seg_begin < queue_.size()) {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
@@ -1615,7 +1713,8 @@ std::vector<PassPlan> Engine::plan() const {
       // primitives touch is blocked.
       uint64_t active = 0;
       for (uint32_t idx : remaining) active |= queue_[idx].touch;
-      auto scan = [&](uint64_t s0, PassPlan *take, std::vector<uint32_t> *rest) {
+      // A gate pass (`cap` qubits) takes only what its kernel runs.
+      auto scan = [&](uint32_t cap, uint64_t s0, PassPlan *take, std::vector<uint32_t> *rest) {
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
@@ -1623,10 +1722,11 @@ std::vector<PassPlan> Engine::plan() const {
         for (size_t r = 0; r < remaining.size(); ++r) {
           const uint32_t idx = remaining[r];
           const Prim &p = queue_[idx];
-          bool fits = !(p.touch & blocked) && !(p.kind == K_PROBE && nonunitary_blocked);
+          bool fits = !(p.touch & blocked) && !(p.kind == K_PROBE && nonunitary_blocked) &&
+                      (cap == nb || gate_prim(p));
           if (fits) {
             const uint64_t ns = s | p.tmask;
-            fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= nb;
+            fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
             if (fits) s = ns;
           }
           if (fits) {
@@ -1648,25 +1748,36 @@ std::vector<PassPlan> Engine::plan() const {
       // (the 30-qubit U3+CX brickwork takes 29 passes instead of 66); the
       // pass keeps the candidate that takes the most primitives, the first
       // on ties.
+      // A pass on the small tile runs every primitive; a gate pass is taken
+      // where it holds more of them, or as many but more than a few: a pass of
+      // one gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.
       uint64_t seed = lowmask;
-      size_t best = scan(lowmask, nullptr, nullptr);
-      const uint32_t w = nb - low_bits_;
-      if (n_ > nb && w > 0)
-        for (uint32_t a = 0; a + w <= n_; ++a) {
-          const uint64_t s0 = lowmask | (((1ull << w) - 1ull) << a);
-          const size_t c = scan(s0, nullptr, nullptr);
-          if (c > best) {
-            best = c;
+      uint32_t cap = nb;
+      size_t best = 0;
+      auto try_tile = [&](uint32_t c) {
+        auto candidate = [&](uint64_t s0) {
+          const size_t k = scan(c, s0, nullptr, nullptr);
+          if (k > best || (k == best && k > 4 && c > cap)) {
+            best = k;
             seed = s0;
+            cap = c;
           }
-        }
+        };
+        candidate(lowmask);
+        const uint32_t w = c - low_bits_;
+        if (n_ > c && w > 0)
+          for (uint32_t a = 0; a + w <= n_; ++a) candidate(lowmask | (((1ull << w) - 1ull) << a));
+      };
+      try_tile(nb);
+      if (gates) try_tile(kGateTileC128);
       PassPlan pp;
       pp.solo = false;
+      pp.gate = cap != nb;
       std::vector<uint32_t> rest;
-      scan(seed, &pp, &rest);
+      scan(cap, seed, &pp, &rest);
       uint64_t s = pp.smask;
       // Complete the tile with the lowest free qubits (longer contiguous runs).
-      for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < nb; ++q)
+      for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < cap; ++q)
         s |= bit(q);
       pp.smask = s;
       out.push_back(std::move(pp));
@@ -2141,17 +2252,18 @@ void Engine::emit_program(Program &prog) {
       }
       pops.push_back(op);
     }
-    const uint32_t full_bits =
-        prec_ == AERHIP_PRECISION_DOUBLE ? kTileBitsC128 : kTileBitsC64;
+    const uint32_t full_bits = pp.gate ? kGateTileC128 : prec_ == AERHIP_PRECISION_DOUBLE ? kTileBitsC128 : kTileBitsC64;
+    const uint32_t R = pp.gate ? kGateRegBits : reg_bits_;
     if (!pp.solo && reg_bits_ > 0 && ns == full_bits) {
       if (fusion_enable_ && n_ > fusion_threshold_)
         pops = fuse_phase_runs(pops, pd.spos, ns, prog.pool, fusion_max_qubit_, &stats_.fused);
-      pd.kind = 2;  // register-layout tile pass: op_begin/nops index the ROps
+      pd.kind = pp.gate ? 5 : 2;  // register-layout tile pass: op_begin/nops index the ROps
       pd.op_begin = static_cast<uint32_t>(rops.size());
-      register_program(pops, ns, reg_bits_, low_bits_, prec_ == AERHIP_PRECISION_SINGLE, pd.spos, prog.pool, rops, ops, &stats_.gathers);
+      register_program(pops, ns, R, low_bits_, prec_ == AERHIP_PRECISION_SINGLE, pp.gate, pd.spos, prog.pool, rops,
+                       ops, &stats_.gathers);
       pd.nops = static_cast<uint32_t>(rops.size()) - pd.op_begin;
       if (pd.readonly) rops.back().extra = 1;  // the final STORE writes nothing
-      validate_register_program(rops.data() + pd.op_begin, pd.nops, ns, reg_bits_, pd.spos, ops.size(),
+      validate_register_program(rops.data() + pd.op_begin, pd.nops, ns, R, pd.spos, ops.size(),
                                 prog.pool);
     } else {
       pd.nops = static_cast<uint32_t>(pops.size());
@@ -2247,6 +2359,12 @@ void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, co
         launch_reg_pass<float, kTileBitsC64, 5>(pk, grid_of(tl), stream, s, dpd, ro, dp.ops, dp.pool,
                                                 dp.probes, state_stride, pd_stride, tl, pps);
     }
+  } else if (pd.kind == 5) {
+    const uint32_t tl = pd.ncomp;
+    k_gate_pass<double, kGateTileC128, kGateRegBits>
+        <<<grid_of(tl), 1 << (kGateTileC128 - kGateRegBits), pk.diag ? kDiagLdsBytes : 0, stream>>>(
+            static_cast<cx<double> *>(sv), dpd, static_cast<const ROp<double> *>(dp.rops), dp.ops, dp.pool,
+            state_stride, pd_stride, tl);
   } else if (pd.kind == 3) {
     // probes over the whole state, one workgroup per tile-sized slice
     const uint32_t tl = n - tile_bits;
@@ -2306,7 +2424,7 @@ bool graphs_enabled() {
 PassKernel pass_kernel(const PassDesc &pd, const std::vector<ROp<double>> &rops) {
   PassKernel k;
   k.wide = pd.nops <= kWidePassOps;
-  if (pd.kind != 2) return k;
+  if (pd.kind != 2 && pd.kind != 5) return k;
   for (uint32_t i = 0; i < pd.nops; ++i) {
     const ROp<double> &r = rops[pd.op_begin + i];
     k.variant |= variant_of(r.kind);
@@ -2957,7 +3075,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
                    pb = static_cast<uint32_t>(pool_at[i]);
     for (size_t k = 0; k < p.passes.size(); ++k) {
       PassDesc d = p.passes[k];
-      d.op_begin += d.kind == 2 ? rb : ob;
+      d.op_begin += d.kind == 2 || d.kind == 5 ? rb : ob;
       hp[pass_at[i] + k] = d;
     }
     for (size_t k = 0; k < p.ops.size(); ++k) {
@@ -3073,6 +3191,7 @@ class MultiState {
     for (Engine *e : planners_)
       if (!e->plan_only() || e->num_qubits() != n || e->precision() != prec)
         throw std::invalid_argument("aerhip: states need planning handles of one size and precision");
+    for (Engine *e : planners_) e->use_gate_passes();
     AERHIP_CHECK(hipSetDevice(device_));
     AERHIP_CHECK(hipStreamCreate(&st_));
     AERHIP_CHECK(hipEventCreate(&e0_));
@@ -3197,7 +3316,7 @@ class MultiState {
       for (size_t k = 0; k < P; ++k) {
         kernels[k].add(pass_kernel(p.passes[k], p.rops));
         PassDesc d = p.passes[k];
-        d.op_begin += d.kind == 2 ? rb : ob;
+        d.op_begin += d.kind == 2 || d.kind == 5 ? rb : ob;
         passes.push_back(d);
       }
       for (TileOp t : p.ops) {

@@ -32,8 +32,9 @@ struct Prim {
 };
 
 struct PassPlan {
-  bool solo;
-  uint64_t smask;              // tile qubits
+  bool solo = false;
+  bool gate = false;           // runs as a gate pass
+  uint64_t smask = 0;          // tile qubits
   std::vector<uint32_t> prims; // indices into the queue
 };
 
@@ -149,6 +150,9 @@ class Engine {
   uint32_t tile_bits() const { return tile_bits_; }
   uint32_t reg_bits() const { return reg_bits_; }
   uint64_t probes_queued() const { return probes_queued_; }
+  // Gate passes for a planning handle (its program then runs through
+  // launch_pass; the batched-circuit kernels do not hold them).
+  void use_gate_passes() { gate_passes_ = true; }
 
  private:
   void check_qubits(const std::vector<uint32_t> &qubits) const;
@@ -162,6 +166,8 @@ class Engine {
   void apply_matrix_1(uint32_t q, const std::vector<cd> &mat);
   void apply_diagonal_1(uint32_t q, const cd *diag);
   std::vector<PassPlan> plan() const;
+  bool gate_tiles() const;
+  bool gate_prim(const Prim &p) const;
   std::vector<PassPlan> gather_sweeps(std::vector<PassPlan> plans) const;
   std::vector<Prim> fuse_blocks(const std::vector<Prim> &in);
   std::vector<Prim> merge_swap_layers(const std::vector<Prim> &in) const;
@@ -179,6 +185,7 @@ class Engine {
   int prec_;
   int device_;
   bool plan_only_ = false;
+  bool gate_passes_ = true;
   uint64_t size_;
   void *sv_ = nullptr;
   hipStream_t stream_ = nullptr;

@@ -1,0 +1,426 @@
+// Gate pass on large tiles (gfx950): the register pass for long programs of
+// gates, with twice the amplitudes per thread.
+//
+// A pass is one read and one write of the state for as many gates as its tile
+// qubits allow, so a tile of one more qubit means fewer passes, and one more
+// register bit means fewer layout changes.  Both cost registers: 2^R complex128
+// amplitudes are 64 VGPRs at R = 4, so ops work in place on the one copy (no
+// second bank), each on a few amplitudes at a time.  Layout changes go through
+// LDS one component after the other, so a tile of 2^12 complex128 amplitudes
+// needs 32 KiB and the occupancy is that of the smaller tile.
+//
+// The op loop is an interpreter: host-computed codes name the op together with
+// its register bits, and one comparison tree finds it.
+//
+// Bound by the FP64 units: the 30-qubit brickwork at fusion width 2 runs 24
+// passes of 11.1 ms, 91 % of whose cycles issue vector instructions (4663 per
+// wave, 3140 of them FMAs of 4x4 gates), at 118 VGPRs and four waves per SIMD.
+// Register passes on 2^11 tiles take 29 passes of 13.6 ms for it: 403 against
+// 269 ms a step.  Three waves (150 VGPRs) 281 ms; five (96 VGPRs) spill: 390 ms.
+#pragma once
+
+#include "reg_pass.hpp"
+
+namespace aerhip {
+
+// Code of an op (ROp::code): group and register bits.
+enum GateCode : uint32_t {
+  C_NOP = 0x00,
+  C_U1 = 0x10,       // + b: 2x2 gate on register bit b
+  C_U2 = 0x20,       // + index of the register bits b0 < b1
+  C_X = 0x30,        // + b: X on register bit b of every lane
+  C_XC = 0x38,       // + b: X where the lane's predicate holds
+  C_U1C = 0x40,      // + b: 2x2 gate where the predicate holds
+  C_Y = 0x48,        // + b: Y where the predicate holds
+  C_CXR = 0x50,      // + 4 c + t: register moves
+  C_PHASE = 0x60,
+  C_D1 = 0x61,
+  C_DIAGF = 0x62,
+  C_RELAYOUT = 0x63,
+};
+
+// Index of a pair of register bits b0 < b1.
+constexpr uint32_t pair_index(uint32_t b0, uint32_t b1) { return b1 * (b1 - 1) / 2 + b0; }
+
+// Whether a gate pass runs this op.
+constexpr bool gate_kind(uint32_t kind) {
+  const int v = variant_of(kind);
+  return v == V_LEAN || v == V_GATES;
+}
+
+// The code of a register op; U2 ops come with a < b.
+inline uint32_t gate_code(const ROp<double> &r) {
+  switch (r.kind & ~F_ALL) {
+    case Q_U1: case Q_U1X: return C_U1 + r.a;
+    case Q_U2: return C_U2 + pair_index(r.a, r.b);
+    case Q_X: return (r.cl ? C_XC : C_X) + r.a;
+    case Q_U1C: return C_U1C + r.a;
+    case Q_Y: return C_Y + r.a;
+    case Q_CXR: return C_CXR + 4 * r.a + r.b;
+    case Q_PHASE: return C_PHASE;
+    case Q_D1: return C_D1;
+    case Q_DIAGF: return C_DIAGF;
+    case Q_RELAYOUT: return C_RELAYOUT;
+    default: return C_NOP;
+  }
+}
+
+// (p, q) <- M (p, q), M column major (u00, u10, u01, u11).  The last FMA of
+// each component writes over the amplitude it reads, so the pair needs four
+// temporaries and no moves.
+template <typename T>
+__device__ __forceinline__ void g_u1(cx<T> &p, cx<T> &q, const cx<T> (&m)[4]) {
+  T tx = -m[2].x * q.x, ty = -m[2].x * q.y, ux = -m[1].x * p.x, uy = -m[1].x * p.y;
+  tx = fma_t(m[2].y, q.y, tx);
+  ty = fma_t(-m[2].y, q.x, ty);
+  ux = fma_t(m[1].y, p.y, ux);
+  uy = fma_t(-m[1].y, p.x, uy);
+  tx = fma_t(m[0].y, p.y, tx);
+  ty = fma_t(-m[0].y, p.x, ty);
+  ux = fma_t(m[3].y, q.y, ux);
+  uy = fma_t(-m[3].y, q.x, uy);
+  p.x = fma_t(m[0].x, p.x, -tx);
+  p.y = fma_t(m[0].x, p.y, -ty);
+  q.x = fma_t(m[3].x, q.x, -ux);
+  q.y = fma_t(m[3].x, q.y, -uy);
+}
+
+template <typename T, int NR, int b>
+__device__ __forceinline__ void g_u1b(Amps<T, NR> &a, const cx<T> (&u)[4]) {
+#pragma unroll
+  for (int k = 0; k < NR / 2; ++k) g_u1(a.v[pair_lo<b>(k)], a.v[pair_lo<b>(k) | (1 << b)], u);
+}
+
+// 4x4 gate on register bits b0 (matrix bit 0) < b1, column major.
+template <typename T, int NR, int b0, int b1>
+__device__ __forceinline__ void g_u2(Amps<T, NR> &a, const cx<T> (&m)[16]) {
+#pragma unroll
+  for (int p = 0; p < NR / 4; ++p) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int j = pair_lo<b1>(pair_lo<b0>(p));
+    const int i[4] = {j, j | (1 << b0), j | (1 << b1), j | (1 << b0) | (1 << b1)};
+    T tx[4], ty[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int f = r == 0 ? 1 : 0;
+      tx[r] = -m[r + 4 * f].x * a.v[i[f]].x;
+      ty[r] = -m[r + 4 * f].x * a.v[i[f]].y;
+      tx[r] = fma_t(m[r + 4 * f].y, a.v[i[f]].y, tx[r]);
+      ty[r] = fma_t(-m[r + 4 * f].y, a.v[i[f]].x, ty[r]);
+#pragma unroll
+      for (int c = f + 1; c < 4; ++c) {
+        if (c == r) continue;
+        tx[r] = fma_t(-m[r + 4 * c].x, a.v[i[c]].x, tx[r]);
+        ty[r] = fma_t(-m[r + 4 * c].x, a.v[i[c]].y, ty[r]);
+        tx[r] = fma_t(m[r + 4 * c].y, a.v[i[c]].y, tx[r]);
+        ty[r] = fma_t(-m[r + 4 * c].y, a.v[i[c]].x, ty[r]);
+      }
+      tx[r] = fma_t(m[5 * r].y, a.v[i[r]].y, tx[r]);
+      ty[r] = fma_t(-m[5 * r].y, a.v[i[r]].x, ty[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      a.v[i[r]].x = fma_t(m[5 * r].x, a.v[i[r]].x, -tx[r]);
+      a.v[i[r]].y = fma_t(m[5 * r].x, a.v[i[r]].y, -ty[r]);
+    }
+  }
+}
+
+// Exchanges two components.  Written out, because as a permutation of values it
+// would tie the registers of the op loop's paths in knots: the compiler then
+// keeps a second copy of the amplitudes and moves between the two at every op.
+__device__ __forceinline__ void g_swap(double &x, double &y) {
+  double t;
+  asm volatile("v_mov_b64 %2, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2" : "+v"(x), "+v"(y), "=&v"(t));
+}
+__device__ __forceinline__ void g_swap(float &x, float &y) { asm volatile("v_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
+template <typename T>
+__device__ __forceinline__ void g_swap(cx<T> &p, cx<T> &q) {
+  g_swap(p.x, q.x);
+  g_swap(p.y, q.y);
+}
+
+// a <- f a
+template <typename T>
+__device__ __forceinline__ void g_mul(cx<T> &a, cx<T> f) {
+  T t = f.y * a.y, u = -f.y * a.x;
+  asm volatile("" : "+v"(t), "+v"(u));  // keeps the negation in the last FMA
+  a.x = fma_t(f.x, a.x, -t);
+  a.y = fma_t(f.x, a.y, -u);
+}
+
+template <typename T, int NR, int b>
+__device__ __forceinline__ void g_x(Amps<T, NR> &a) {
+#pragma unroll
+  for (int k = 0; k < NR / 2; ++k) {
+    const int j = pair_lo<b>(k);
+    g_swap(a.v[j], a.v[j | (1 << b)]);
+  }
+}
+
+template <typename T, int NR, int b, bool isy>
+__device__ __forceinline__ void g_xc(Amps<T, NR> &a, uint32_t tlc, const RegIdx<NR> &ri, uint32_t cl, uint32_t cvl) {
+#pragma unroll
+  for (int k = 0; k < NR / 2; ++k) {
+    const int j = pair_lo<b>(k), jj = j | (1 << b);
+    const bool on = (tlc | (ri.at(j) & cl)) == cvl;
+    const cx<T> p = a.v[j], q = a.v[jj];
+    a.v[j] = csel(on, isy ? mk<T>(q.y, -q.x) : q, p);
+    a.v[jj] = csel(on, isy ? mk<T>(-p.y, p.x) : p, q);
+  }
+}
+
+template <typename T, int NR, int b>
+__device__ __forceinline__ void g_u1c(Amps<T, NR> &a, uint32_t tlc, const RegIdx<NR> &ri, uint32_t cl, uint32_t cvl,
+                                      const cx<T> (&m)[4]) {
+#pragma unroll
+  for (int k = 0; k < NR / 2; ++k) {
+    const int j = pair_lo<b>(k), jj = j | (1 << b);
+    const bool on = (tlc | (ri.at(j) & cl)) == cvl;
+    cx<T> p = a.v[j], q = a.v[jj];
+    g_u1(p, q, m);
+    a.v[j] = csel(on, p, a.v[j]);
+    a.v[jj] = csel(on, q, a.v[jj]);
+  }
+}
+
+template <typename T, int NR, int c, int t>
+__device__ __forceinline__ void g_cxr(Amps<T, NR> &a) {
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    if (((j >> c) & 1) && !((j >> t) & 1)) g_swap(a.v[j], a.v[j | (1 << t)]);
+}
+
+// The four matrix entries of a 2x2 gate, its columns exchanged where an X is
+// folded in (fx).
+template <typename T>
+__device__ __forceinline__ void g_load_u1(const ROp<T> &op, bool fx, cx<T> (&m)[4]) {
+  const T *c0 = op.u.m + (fx ? 4 : 0), *c1 = op.u.m + (fx ? 0 : 4);
+  m[0] = mk<T>(c0[0], c0[1]);
+  m[1] = mk<T>(c0[2], c0[3]);
+  m[2] = mk<T>(c1[0], c1[1]);
+  m[3] = mk<T>(c1[2], c1[3]);
+}
+
+// One component of every amplitude moves from slots ws ^ rw(j) to rs ^ rr(j).
+template <typename T, int NR, bool im>
+__device__ __forceinline__ void g_exchange(Amps<T, NR> &a, T *xch, const uint32_t (&w)[NR], const uint32_t (&r)[NR]) {
+#pragma unroll
+  for (int j = 0; j < NR; ++j) xch[w[j]] = im ? a.v[j].y : a.v[j].x;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NR; ++j) (im ? a.v[j].y : a.v[j].x) = xch[r[j]];
+}
+
+template <typename T, int B, int R>
+__device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd,
+                                          const ROp<T> *__restrict__ rops, const TileOp *__restrict__ tops,
+                                          const cx<double> *__restrict__ pool, uint64_t tile_id, T *xch,
+                                          cx<double> *dlt) {
+  constexpr int TB = B - R, NT = 1 << TB, NR = 1 << R;
+  const uint32_t tid = threadIdx.x;
+  uint64_t base = tile_id;
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const uint32_t q = pd->spos[i];
+    base = ((base >> q) << (q + 1)) | (base & ((1ull << q) - 1ull));
+  }
+  base = uniform64(base);
+  const ROp<T> *opp = rops + pd->op_begin;
+  LayoutState<NR> st = make_state<R, TB>(opp->u.lay, tid);
+  const uint32_t nslot = opp->a;
+  const cx<double> *dlane = pool + opp->b;
+  uint2 drec = make_uint2(0u, 0u);
+  uint32_t sb[256 / NT] = {};
+  if (nslot) {
+    drec = reinterpret_cast<const uint2 *>(dlane)[tid & 63u];
+    const uint32_t *stage_back = reinterpret_cast<const uint32_t *>(dlane + 32);
+#pragma unroll
+    for (int j = 0; j < 256 / NT; ++j) sb[j] = stage_back[j * NT + tid];
+  }
+  Amps<T, NR> a;
+  {
+    const RegOff<NR> ro = reg_offset<R>(opp->u.lay);
+    const cx<T> *p = sv + base + thread_offset<TB>(opp->u.lay, tid);
+#pragma unroll
+    for (int j = 0; j < NR; ++j) a.v[j] = ld_stream(p + ro.gr[j]);
+  }
+  if (nslot) {
+    stage_diag_tables<NT>(drec, dlane, nslot, base, tid, sb, dlt);
+    __syncthreads();
+  }
+  const uint32_t cnt = opp->extra;
+  for (uint32_t i = 0; i < cnt; ++i) {
+    ++opp;
+    const ROp<T> &op = *opp;
+    const uint32_t code = op.code;
+    const bool tile_ok = (base & op.cg) == op.cvg;
+    if ((code & 0xF0u) == C_U1) {
+      cx<T> m[4];
+      g_load_u1(op, tile_ok && (op.kind & ~F_ALL) == Q_U1X, m);
+      switch (code) {
+        case C_U1 + 0: g_u1b<T, NR, 0>(a, m); break;
+        case C_U1 + 1: g_u1b<T, NR, 1>(a, m); break;
+        case C_U1 + 2: g_u1b<T, NR, 2>(a, m); break;
+        case C_U1 + 3: if constexpr (R > 3) g_u1b<T, NR, R - 1>(a, m); break;
+      }
+      continue;
+    }
+    const uint32_t cl = op.cl, cvl = op.cvl;
+    if ((code & 0xF0u) == C_U2) {
+      if (cl == 0 && !tile_ok) continue;
+      cx<T> m[16];
+      const cx<T> *mp = reinterpret_cast<const cx<T> *>(pool + op.extra);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) m[e] = mp[e];
+      switch (code) {
+        case C_U2 + pair_index(0, 1): g_u2<T, NR, 0, 1>(a, m); break;
+        case C_U2 + pair_index(0, 2): g_u2<T, NR, 0, 2>(a, m); break;
+        case C_U2 + pair_index(1, 2): g_u2<T, NR, 1, 2>(a, m); break;
+        case C_U2 + pair_index(0, 3): if constexpr (R > 3) g_u2<T, NR, 0, R - 1>(a, m); break;
+        case C_U2 + pair_index(1, 3): if constexpr (R > 3) g_u2<T, NR, 1, R - 1>(a, m); break;
+        case C_U2 + pair_index(2, 3): if constexpr (R > 3) g_u2<T, NR, 2, R - 1>(a, m); break;
+      }
+      continue;
+    }
+    if (code == C_RELAYOUT) {
+      // Slot x of a component at x ^ ((x >> 4) & 15): consecutive lanes reach
+      // distinct banks also where the register bits are the low tile bits.
+      // Linear, so it splits into a per-lane and a per-register term.
+      auto swz = [](uint32_t x) { return x ^ ((x >> 4) & 15u); };
+      uint32_t w[NR], r[NR];
+      const uint32_t tw = swz(st.tl);
+#pragma unroll
+      for (int j = 0; j < NR; ++j) w[j] = tw ^ swz(st.ri.at(j));
+      st = make_state<R, TB>(op.u.lay, tid);
+      const uint32_t tr = swz(st.tl);
+#pragma unroll
+      for (int j = 0; j < NR; ++j) r[j] = tr ^ swz(st.ri.at(j));
+      __syncthreads();
+      g_exchange<T, NR, false>(a, xch, w, r);
+      __syncthreads();
+      g_exchange<T, NR, true>(a, xch, w, r);
+      continue;
+    }
+    if ((code & 0xF0u) == C_CXR) {
+      switch (code) {
+#define G_CASE(c, t)     \
+  case C_CXR + 4 * c + t: \
+    if constexpr (c < R && t < R) g_cxr<T, NR, c < R ? c : 0, t < R ? t : 1>(a); \
+    break;
+        G_CASE(0, 1) G_CASE(0, 2) G_CASE(0, 3) G_CASE(1, 0) G_CASE(1, 2) G_CASE(1, 3)
+        G_CASE(2, 0) G_CASE(2, 1) G_CASE(2, 3) G_CASE(3, 0) G_CASE(3, 1) G_CASE(3, 2)
+#undef G_CASE
+      }
+      continue;
+    }
+    if (!tile_ok) continue;  // controls fixed by the tile that do not hold
+    const uint32_t tlc = st.tl & cl;
+    const uint32_t rb = op.b;
+    uint32_t rbits = 0;
+#pragma unroll
+    for (int s = 0; s < R; ++s) rbits |= st.ri.bm[s];
+    const uint32_t clt = cl & ~rbits;
+    const bool lane_ok = (st.tl & clt) == (cvl & clt);
+    const cx<T> one = mk<T>(1, 0);
+    switch (code) {
+      case C_X + 0: g_x<T, NR, 0>(a); break;
+      case C_X + 1: g_x<T, NR, 1>(a); break;
+      case C_X + 2: g_x<T, NR, 2>(a); break;
+      case C_X + 3: g_x<T, NR, R - 1>(a); break;
+#define G_CASE(b) \
+  case C_XC + b: if constexpr (b < R) g_xc<T, NR, b < R ? b : 0, false>(a, tlc, st.ri, cl, cvl); break;       \
+  case C_Y + b: if constexpr (b < R) g_xc<T, NR, b < R ? b : 0, true>(a, tlc, st.ri, cl, cvl); break;         \
+  case C_U1C + b:                                                                                              \
+    if constexpr (b < R) {                                                                                     \
+      cx<T> m[4];                                                                                              \
+      g_load_u1(op, false, m);                                                                                 \
+      g_u1c<T, NR, b < R ? b : 0>(a, tlc, st.ri, cl, cvl, m);                                                  \
+    }                                                                                                          \
+    break;
+      G_CASE(0) G_CASE(1) G_CASE(2) G_CASE(3)
+#undef G_CASE
+      case C_PHASE: {
+        const cx<T> f = csel(lane_ok, mk<T>(op.u.m[0], op.u.m[1]), one);
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+          if ((rb >> j) & 1u) {
+            asm volatile("");  // keeps the branch (no if-conversion into selects)
+            g_mul(a.v[j], f);
+          }
+        break;
+      }
+      case C_D1: {
+        const cx<T> d0 = mk<T>(op.u.m[0], op.u.m[1]), d1 = mk<T>(op.u.m[2], op.u.m[3]);
+        const uint32_t t = op.a;
+        if ((rbits >> t) & 1u) {
+          // target on a register bit: bit j of rb is the target's value in register j
+#pragma unroll
+          for (int j = 0; j < NR; ++j) {
+            if ((rb >> j) & 1u) {
+              asm volatile("");  // keeps the branch (no if-conversion into selects)
+              g_mul(a.v[j], d1);
+            } else {
+              g_mul(a.v[j], d0);
+            }
+          }
+        } else {
+          const cx<T> d = csel(((st.tl >> t) & 1u) != 0, d1, d0);
+#pragma unroll
+          for (int j = 0; j < NR; ++j) g_mul(a.v[j], d);
+        }
+        break;
+      }
+      case C_DIAGF: {
+        // the fused diagonal of Q_DIAGF: factor G L R_j, G L per lane
+        const cx<double> *blk = pool + op.extra;
+        uint32_t t = tid;
+        asm volatile("" : "+v"(t));  // lane indices derived here, not held for the whole pass
+        cx<double> g;
+        const uint32_t ra = op.a;
+        if (const uint32_t slot = ra >> 16) {
+          const cx<double> *row = dlt + 32u * (slot - 1u);
+          g = cmul(row[t & 15u], row[16u + ((t >> 4) & 15u)]);
+        } else {
+          g = cmul(blk[NR + (t & 15u)], blk[NR + 16 + ((t >> 4) & 15u)]);
+          const cx<double> *tab = blk + NR + 32;
+          for (uint32_t c = 0; c < (ra & 0xFFu); ++c, tab += 16) {
+            uint32_t idx = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t q = op.u.fq[4 * c + k];
+              if (q < 64) idx |= static_cast<uint32_t>((base >> q) & 1ull) << k;
+            }
+            g = cmul(g, tab[idx]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+          if ((rb >> j) & 1u) {
+            asm volatile("");  // keeps the branch (no if-conversion into selects)
+            g_mul(a.v[j], csel(lane_ok, to_t<T>(cmul(g, blk[j])), one));
+          }
+        break;
+      }
+      default: break;
+    }
+  }
+  ++opp;
+  const RegOff<NR> ro = reg_offset<R>(opp->u.lay);
+  cx<T> *p = sv + base + thread_offset<TB>(opp->u.lay, tid);
+#pragma unroll
+  for (int j = 0; j < NR; ++j) st_stream(p + ro.gr[j], a.v[j]);
+}
+
+template <typename T, int B, int R>
+__global__ __launch_bounds__(1 << (B - R)) __attribute__((amdgpu_waves_per_eu(4))) void k_gate_pass(
+    cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd, const ROp<T> *__restrict__ rops,
+    const TileOp *__restrict__ tops, const cx<double> *__restrict__ pool, uint64_t state_stride, uint32_t pd_stride,
+    uint32_t tile_log) {
+  __shared__ T xch[1 << B];
+  const StateTile st = state_tile(tile_log);
+  gate_tile<T, B, R>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool, st.t, xch,
+                     reinterpret_cast<cx<double> *>(aerhip_dyn_lds));
+}
+
+}  // namespace aerhip

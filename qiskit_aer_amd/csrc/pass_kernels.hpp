@@ -3,6 +3,7 @@
 #pragma once
 
 #include "batch.hpp"
+#include "gate_pass.hpp"
 #include "reg_pass.hpp"
 #include "tile_pass.hpp"
 
@@ -10,6 +11,9 @@ namespace aerhip {
 
 constexpr uint32_t kTileBitsC128 = 11;  // 2^11 x 16 B = 32 KiB of LDS
 constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
+
+constexpr uint32_t kGateTileC128 = 12;  // 2^12 x 8 B = 32 KiB of LDS per component
+constexpr uint32_t kGateRegBits = 4;
 
 #define AERHIP_REG_PASS(EXT, T, B, R, V, WIDE)                                                        \
   EXT template __global__ void k_reg_pass<T, B, R, V, WIDE>(                                          \
@@ -22,6 +26,12 @@ constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
       const PassDesc *__restrict__, const ROp<T> *__restrict__, const TileOp *__restrict__,              \
       const cx<double> *__restrict__, double *__restrict__);
 
+#define AERHIP_GATE_PASS(EXT, T, B, R)                                                                   \
+  EXT template __global__ void k_gate_pass<T, B, R>(                                                     \
+      cx<T> *__restrict__, const PassDesc *__restrict__, const ROp<T> *__restrict__,                     \
+      const TileOp *__restrict__, const cx<double> *__restrict__, uint64_t, uint32_t, uint32_t);
+
+AERHIP_GATE_PASS(extern, double, kGateTileC128, kGateRegBits)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, false)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, true)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_GATES, false)

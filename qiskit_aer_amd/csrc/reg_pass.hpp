@@ -60,6 +60,7 @@ enum RegPassOpKind : uint32_t {
                     // 0-3, 4-7), then a & 0xFF = number of 16-entry tables over fixed
                     // qubits u.fq[4c .. 4c+3] (0xFF: unused); a >> 16 = slot + 1 of the
                     // phase's lane tables staged in LDS (0: none, read the tables)
+  Q_CXR = 61,       // moves registers: those with bit a set change places across bit b
 };
 
 // Fused diagonals of a register phase: the factor over the qubits fixed by
@@ -106,7 +107,7 @@ constexpr bool head_payload(int v) { return v == V_LEAN || v == V_PROBES; }
 constexpr int variant_of(uint32_t kind) {
   switch (kind & ~F_ALL) {
     case Q_LOAD: case Q_STORE: case Q_RELAYOUT: case Q_U1: case Q_U1X: case Q_U1M: case Q_U1MX:
-    case Q_X: case Q_D1: case Q_PHASE: case Q_NOP: case Q_DIAGF:
+    case Q_X: case Q_D1: case Q_PHASE: case Q_NOP: case Q_DIAGF: case Q_CXR:
       return V_LEAN;
     case Q_U2: case Q_U1C: case Q_Y: case Q_DIAG:
       return V_GATES;
@@ -164,7 +165,8 @@ struct alignas(128) ROp {
   uint64_t cg, cvg;  // controls on qubits fixed by the tile
   uint16_t map_bm[5];  // with F_MAP in kind: the relabelling in force from this op on
   uint16_t map_t0;
-  uint32_t pad[3];
+  uint32_t code;     // gate passes: the op with its register bits (gate_pass.hpp)
+  uint32_t pad[2];
   union {
     T m[8];          // 2x2 complex matrix (column major), diagonal, phase
     float mr[16];    // complex64 Q_U1 / Q_U1X / Q_U1M: the matrix as a real 4x4, rows over
@@ -544,6 +546,21 @@ __device__ __forceinline__ Amps<T, NR> q_xy(const Amps<T, NR> &a, uint32_t tlc,
   return o;
 }
 
+// CX between register bits as register moves: ends a relabelling where an op
+// needs the layout's own pairs.  A layout change does the same through LDS at
+// three times the cost and two barriers (30-qubit brickwork, fusion width 2: 94
+// of its 277 layout changes had no other purpose: 412 ms a step with them, 403
+// without).
+template <typename T, int NR, int c, int t>
+__device__ __forceinline__ Amps<T, NR> q_cxr(const Amps<T, NR> &a) {
+  Amps<T, NR> o;
+#pragma unroll
+  for (int j = 0; j < NR; ++j) o.v[j] = a.v[(j >> c) & 1 ? j ^ (1 << t) : j];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) asm volatile("" : "+v"(o.v[j].x), "+v"(o.v[j].y));
+  return o;
+}
+
 // 4x4 matrix on register bits b0 (matrix bit 0) and b1 (matrix bit 1).
 template <typename T, int NR, int b0, int b1>
 __device__ __forceinline__ Amps<T, NR> q_u2(const Amps<T, NR> &a, uint32_t tlc,
@@ -655,6 +672,20 @@ __device__ __forceinline__ Amps<T, NR> d_u2(uint32_t p, const Amps<T, NR> &a, ui
   } else {
     if (p == static_cast<uint32_t>(P)) return q_u2<T, NR, b0, b1>(a, tlc, ri, cl, cvl, mp);
     return d_u2<T, NR, P + 1>(p, a, tlc, ri, cl, cvl, mp);
+  }
+}
+
+template <typename T, int NR, int P = 1>
+__device__ __forceinline__ Amps<T, NR> d_cxr(uint32_t p, const Amps<T, NR> &a) {
+  constexpr int R = reg_bits_of<NR>();
+  constexpr int c = P / R, t = P % R;
+  if constexpr (P >= (R - 1) * R + (R - 2)) {
+    return q_cxr<T, NR, R - 1, R - 2>(a);
+  } else if constexpr (c == t) {
+    return d_cxr<T, NR, P + 1>(p, a);
+  } else {
+    if (p == static_cast<uint32_t>(P)) return q_cxr<T, NR, c, t>(a);
+    return d_cxr<T, NR, P + 1>(p, a);
   }
 }
 
@@ -1030,6 +1061,7 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     }
     return pass_through(a);
   }
+  if (kind == Q_CXR) return d_cxr<T, NR>(ra * reg_bits_of<NR>() + rb, a);
   if (kind == Q_RELAYOUT) {
     // complex64: the tile passes through LDS in a swizzled order, slot x at
     // x ^ ((x >> 4) & 15), so that consecutive lanes reach distinct banks also

@@ -1,0 +1,96 @@
+"""Gate passes (tiles of 2^12 complex128 amplitudes, from 21 qubits on): every
+op they run, on qubits inside and outside the tile, next to ops they leave to
+the other passes, against the oracle; and the same gates just below 21 qubits."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as O
+from qiskit_aer_amd import QubitVector, circuits
+from tests import dense as D
+
+pytestmark = pytest.mark.gpu
+
+
+def run_both(c, n, width=0, state=None):
+    e = QubitVector(n)
+    e.set_block_fusion(width)
+    e.initialize()
+    e.apply_ops(c)
+    _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+    return float(np.max(np.abs(e.copy_to_vector() - want)))
+
+
+def mixture(n, seed, count):
+    """Gates of every kind, most of them on a window of nearby qubits so that a
+    pass holds many."""
+    rng = np.random.default_rng(seed)
+    c = circuits.Circuit(n)
+    for q in range(n):
+        c.gate("h", [q])
+    for _ in range(count):
+        lo = int(rng.integers(0, n - 5)) if rng.random() < 0.8 else 0
+        hi = lo + 6 if lo or rng.random() < 0.5 else n
+        q = [int(x) for x in rng.choice(np.arange(lo, min(hi, n)), 3, replace=False)]
+        t = list(rng.uniform(-3, 3, 3))
+        k = int(rng.integers(16))
+        if k < 4:
+            c.gate("u3", q[:1], t)
+        elif k < 7:
+            c.gate("cx", q[:2])
+        elif k == 7:
+            c.unitary(D.random_unitary(4, rng), q[:2])
+        elif k == 8:
+            c.gate("rz", q[:1], t[:1])
+        elif k == 9:
+            c.gate("cp", q[:2], t[:1])
+        elif k == 10:
+            c.gate("ccx", q)
+        elif k == 11:
+            c.gate("cu3", q[:2], t)
+        elif k == 12:
+            c.gate("cy", q[:2])
+        elif k == 13:
+            c.gate("x", q[:1])
+        elif k == 14:
+            c.gate("mcp", q, t[:1])
+        else:
+            c.gate("swap", q[:2]) if rng.random() < 0.3 else c.gate("y", q[:1])
+    return c
+
+
+@pytest.mark.parametrize("n,seed", [(20, 1), (21, 2), (21, 3), (22, 4)])
+def test_mixture_matches_oracle(n, seed):
+    print(f"case: gate pass mixture n={n} seed={seed}", flush=True)
+    # 300 gates, each rounding amplitudes of at most 1 to a few 2^-53
+    assert run_both(mixture(n, seed, 300), n) < 1e-12
+
+
+@pytest.mark.parametrize("width", [0, 2, 3])
+def test_brickwork_fused_and_not(width):
+    n = 21
+    print(f"case: gate pass brickwork n={n} width={width}", flush=True)
+    assert run_both(circuits.brickwork_u3_cx(n, 12, 5, measure=False), n, width) < 1e-12
+
+
+def test_qft_ladders():
+    """Fused diagonals: lane tables staged in LDS, and beyond eight of them read
+    from memory."""
+    n = 22
+    print(f"case: gate pass qft n={n}", flush=True)
+    c = circuits.qft(n)
+    assert run_both(c, n) < 1e-12
+
+
+def test_gradients_use_them():
+    """The forward sweep of the adjoint method holds no probes."""
+    from qiskit_aer_amd.adjoint import AdjointEstimator
+    from bench import ry_rz_cz_ansatz, tfim
+    n = 20  # 21 with the flag qubit
+    print(f"case: gate pass gradients n={n}", flush=True)
+    c, idx, npar = ry_rz_cz_ansatz(n, 3)
+    est = AdjointEstimator(c, idx, npar, tfim(n))
+    rows = np.random.default_rng(2).uniform(-3, 3, size=(2, npar))
+    e, g = est.energy_and_gradient(rows)
+    assert np.max(np.abs(e - est.energy_one_by_one(rows))) < 1e-11
+    which = [0, npar // 2, npar - 1]
+    assert np.max(np.abs(est.parameter_shift(rows[:1], which)[0] - g[0, which])) < 1e-9
