@@ -7,6 +7,7 @@ them into the ``aerhip_op`` wire format of include/aerhip.h.
 """
 from __future__ import annotations
 
+import array
 import ctypes as C
 import itertools
 from dataclasses import dataclass, field
@@ -128,53 +129,50 @@ class Circuit:
         keep = []
         if nops == 0:
             return arr, keep
+        # One list per attribute, into arrays of machine words (several times
+        # faster than numpy reading the objects), and numpy for the rest.
         rec = np.frombuffer(arr, dtype=_OP_DTYPE)
-        types = np.fromiter((o.type for o in ops), dtype=np.int32, count=nops)
-        rec["type"] = types
+        chain = itertools.chain.from_iterable
+        types = [o.type for o in ops]
+        rec["type"] = _words("i", types)
+        only_gates = types.count(L.OP_GATE) == nops
         # qubits
-        nq = np.fromiter((len(o.qubits) for o in ops), dtype=np.int64, count=nops)
-        qflat = np.fromiter(itertools.chain.from_iterable(o.qubits for o in ops), dtype=np.uint64,
-                            count=int(nq.sum()))
-        qflat = np.concatenate([qflat, np.zeros(1, dtype=np.uint64)])
+        qubits = [o.qubits for o in ops]
+        nq = _words("q", list(map(len, qubits)))
+        qflat = array.array("Q", list(chain(qubits)) + [0])
         keep.append(qflat)
-        qoff = np.concatenate([[0], np.cumsum(nq)[:-1]])
         rec["num_qubits"] = nq
-        rec["qubits"] = np.uint64(qflat.ctypes.data) + (qoff * 8).astype(np.uint64)
-        # real parameters: gate angles, or complex matrices as (re, im) pairs
-        is_gate = types == L.OP_GATE
-        mats = [i for i in range(nops) if not is_gate[i] and ops[i].matrix is not None]
-        npar = np.fromiter((len(o.params) if o.type == L.OP_GATE else 0 for o in ops), dtype=np.int64,
-                           count=nops)
-        for i in mats:
-            npar[i] = 2 * ops[i].matrix.size
-        poff = np.concatenate([[0], np.cumsum(npar)[:-1]])
-        pflat = np.zeros(int(npar.sum()) + 1, dtype=np.float64)
-        gate_idx = np.nonzero(is_gate & (npar > 0))[0]
-        if gate_idx.size:
-            vals = np.fromiter(itertools.chain.from_iterable(ops[i].params for i in gate_idx),
-                               dtype=np.float64, count=int(npar[gate_idx].sum()))
-            starts = poff[gate_idx]
-            lens = npar[gate_idx]
-            pos = np.repeat(starts - np.concatenate([[0], np.cumsum(lens)[:-1]]), lens) + np.arange(vals.size)
-            pflat[pos] = vals
-        for i in mats:
-            pflat[poff[i]:poff[i] + npar[i]] = np.ascontiguousarray(
-                ops[i].matrix.astype(np.complex128)).view(np.float64)
+        rec["qubits"] = qflat.buffer_info()[0] + 8 * (np.cumsum(nq) - nq)
+        # real parameters: gate angles, then complex matrices as (re, im) pairs
+        params = [o.params for o in ops]
+        mats = []
+        if not only_gates:
+            params = [p if t == L.OP_GATE else () for p, t in zip(params, types)]
+            mats = [i for i, t in enumerate(types) if t != L.OP_GATE and ops[i].matrix is not None]
+        npar = _words("q", list(map(len, params)))
+        pflat = array.array("d", list(chain(params)) + [0.0])
         keep.append(pflat)
-        rec["num_params"] = np.where(is_gate, npar, npar // 2)
-        rec["params"] = np.uint64(pflat.ctypes.data) + (poff * 8).astype(np.uint64)
+        rec["num_params"] = npar
+        rec["params"] = pflat.buffer_info()[0] + 8 * (np.cumsum(npar) - npar)
+        for i in mats:
+            m = np.array(ops[i].matrix, dtype=np.complex128)  # packed ops do not follow later changes
+            keep.append(m)
+            rec["num_params"][i] = m.size
+            rec["params"][i] = m.ctypes.data
         # names: one NUL-terminated copy of each distinct name
-        names = sorted({o.name for o in ops})
-        blob = b"".join(nm.encode() + b"\0" for nm in names)
-        nbuf = np.frombuffer(blob + b"\0", dtype=np.uint8)
+        names = [o.name for o in ops]
+        distinct = sorted(set(names))
+        blob = b"".join(nm.encode() + b"\0" for nm in distinct)
+        nbuf = array.array("B", blob + b"\0")
         keep.append(nbuf)
-        addr, at = {}, 0
-        for nm in names:
-            addr[nm] = nbuf.ctypes.data + at
+        addr, at = {}, nbuf.buffer_info()[0]
+        for nm in distinct:
+            addr[nm] = at
             at += len(nm.encode()) + 1
-        rec["name"] = np.fromiter((addr[o.name] for o in ops), dtype=np.uint64, count=nops)
+        rec["name"] = _words("Q", list(map(addr.__getitem__, names)))
         # Pauli labels and measure clbits (rare)
-        for i, op in enumerate(ops):
+        for i in [i for i, o in enumerate(ops) if o.label is not None or o.memory]:
+            op = ops[i]
             if op.label is not None:
                 lab = op.label.encode()
                 keep.append(lab)
@@ -184,6 +182,10 @@ class Circuit:
                 keep.append(m)
                 arr[i].memory = m.ctypes.data_as(C.POINTER(C.c_uint64))
         return arr, keep
+
+
+def _words(code: str, values: list) -> np.ndarray:
+    return np.frombuffer(array.array(code, values), dtype=code)
 
 
 # Field layout of AerhipOp (include/aerhip.h) for filling packed records.

@@ -50,11 +50,11 @@ Engine::Engine(uint32_t num_qubits, int precision, int device)
   if (const char *e = std::getenv("AERHIP_REG_BITS")) set_reg_bits(std::atoi(e));
   if (const char *e = std::getenv("AERHIP_LOW_BITS")) set_low_bits(std::atoi(e));
   AERHIP_CHECK(hipSetDevice(device_));
-  const size_t bytes = size_ * (prec_ == AERHIP_PRECISION_DOUBLE ? 16 : 8);
-  AERHIP_CHECK(hipMalloc(&sv_, bytes));
-  AERHIP_CHECK(hipStreamCreate(&stream_));
-  AERHIP_CHECK(hipEventCreateWithFlags(&prog_ev_, hipEventDisableTiming));
-  AERHIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&h_scalar_), 64 * sizeof(double)));
+  ws_ = WorkspacePool::get().take(device_, size_ * (prec_ == AERHIP_PRECISION_DOUBLE ? 16 : 8));
+  sv_ = ws_.state.p;
+  stream_ = ws_.stream;
+  prog_ev_ = ws_.event;
+  h_scalar_ = ws_.scalars;
 }
 
 Engine::Engine(uint32_t num_qubits, int precision, int device, PlanOnly)
@@ -71,20 +71,17 @@ Engine::Engine(uint32_t num_qubits, int precision, int device, PlanOnly)
 
 Engine::~Engine() {
   if (plan_only_) return;
+  if (!stream_) return;
   (void)hipSetDevice(device_);
-  if (stream_) (void)hipStreamSynchronize(stream_);
+  // Work of other streams may still read a state whose address was handed out.
+  const hipError_t e = exposed_ ? hipDeviceSynchronize() : hipStreamSynchronize(stream_);
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
-  if (sv_) (void)hipFree(sv_);
-  if (d_prog_) (void)hipFree(d_prog_);
-  if (d_partial_) (void)hipFree(d_partial_);
-  if (d_scratch_) (void)hipFree(d_scratch_);
-  if (d_probes_) (void)hipFree(d_probes_);
-  if (h_prog_) (void)hipHostFree(h_prog_);
-  if (h_scalar_) (void)hipHostFree(h_scalar_);
-  if (prog_ev_) (void)hipEventDestroy(prog_ev_);
   if (t0_ev_) (void)hipEventDestroy(t0_ev_);
   if (t1_ev_) (void)hipEventDestroy(t1_ev_);
-  if (stream_) (void)hipStreamDestroy(stream_);
+  if (e == hipSuccess)
+    WorkspacePool::get().give(ws_);
+  else
+    ws_.release();
 }
 
 void Engine::set_tile_bits(uint32_t nb) {
@@ -737,23 +734,36 @@ RItem classify_item(const TileOp &op, uint32_t R) {
   return it;
 }
 
-// Scans `rem` in order; an item is taken if it conflicts with no earlier item
-// left behind and `ok(item)` holds.  Returns the taken indices.
-template <typename F>
-std::vector<size_t> scan_items(const std::vector<RItem> &rem, F ok) {
+// The masks of an item, apart from its op: what the scans below read, over and
+// over, for every register set they try.
+struct RMask {
+  uint32_t need, touch;
+  int8_t cls, cat;
+};
+
+// Scans `rem` in order; an item is taken (f(index)) if it conflicts with no
+// earlier item left behind and `ok(mask)` holds.
+template <typename F, typename G>
+void scan_items(const std::vector<RMask> &rem, F ok, G take) {
   uint32_t blocked[3] = {0, 0, 0};
-  std::vector<size_t> taken;
   for (size_t i = 0; i < rem.size(); ++i) {
-    const RItem &it = rem[i];
+    const RMask &it = rem[i];
     uint32_t conflict = blocked[0];
     for (int c = 1; c < 3; ++c)
       if (c != it.cat) conflict |= blocked[c];
     if (!(it.touch & conflict) && ok(it)) {
-      taken.push_back(i);
+      take(i);
     } else {
-      blocked[it.cat] |= it.touch;
+      blocked[static_cast<int>(it.cat)] |= it.touch;
+      if (blocked[0] == ~0u) return;  // nothing later can be taken
     }
   }
+}
+
+template <typename F>
+std::vector<size_t> scan_items(const std::vector<RMask> &rem, F ok) {
+  std::vector<size_t> taken;
+  scan_items(rem, ok, [&](size_t i) { taken.push_back(i); });
   return taken;
 }
 
@@ -1042,15 +1052,34 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
                       std::vector<ROp<double>> &rops, std::vector<TileOp> &tops,
                       uint64_t *relayouts) {
   const size_t first_rop = rops.size();
-  std::vector<RItem> rem;
+  std::vector<RMask> rem;          // the pending items ...
+  std::vector<uint32_t> rem_op;    // ... and which op of `in` each is
   rem.reserve(in.size());
-  for (const TileOp &op : in) rem.push_back(classify_item(op, R));
+  for (size_t i = 0; i < in.size(); ++i) {
+    const RItem it = classify_item(in[i], R);
+    rem.push_back(RMask{it.need, it.touch, static_cast<int8_t>(it.cls), static_cast<int8_t>(it.cat)});
+    rem_op.push_back(static_cast<uint32_t>(i));
+  }
+  uint32_t all_touch = 0;
+  for (const RMask &it : rem) all_touch |= it.touch;
   const uint32_t lowmask = (1u << lowb) - 1u;
-  auto fits = [](const RItem &it, uint32_t rs) { return it.cls == 1 || (it.cls == 0 && (it.need & ~rs) == 0); };
+  auto fits = [](const RMask &it, uint32_t rs) { return it.cls == 1 || (it.cls == 0 && (it.need & ~rs) == 0); };
   auto score = [&](uint32_t rs) {
+    // Counts the register gates the set rs lets run; stops once every tile bit
+    // the pending items touch is blocked for gates.
     size_t n = 0;
-    for (size_t i : scan_items(rem, [&](const RItem &it) { return fits(it, rs); }))
-      if (rem[i].cls == 0) ++n;
+    uint32_t blocked[3] = {0, 0, 0};
+    for (const RMask &it : rem) {
+      uint32_t conflict = blocked[0];
+      for (int c = 1; c < 3; ++c)
+        if (c != it.cat) conflict |= blocked[c];
+      if (!(it.touch & conflict) && fits(it, rs)) {
+        n += it.cls == 0;
+      } else {
+        blocked[static_cast<int>(it.cat)] |= it.touch;
+        if ((blocked[0] & all_touch) == all_touch) break;
+      }
+    }
     return n;
   };
   // Fills rs up to R bits: bits that keep the low bits on lanes first, highest first.
@@ -1066,7 +1095,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   auto best_set = [&](bool compat) {
     uint32_t cand_bits = 0;
     size_t seen = 0;
-    for (size_t i : scan_items(rem, [&](const RItem &it) { return it.cls != 2; })) {
+    for (size_t i : scan_items(rem, [&](const RMask &it) { return it.cls != 2; })) {
       if (rem[i].cls != 0) continue;
       const uint32_t nb = cand_bits | rem[i].need;
       if (static_cast<uint32_t>(__builtin_popcount(nb)) > R + 4) break;
@@ -1561,20 +1590,20 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   };
   auto take = [&](const std::vector<size_t> &idx, uint32_t rs, bool lds_mode) {
     for (size_t i : idx) {
-      if (lds_mode) emit_lds(rem[i].op);
-      else emit_gate(rem[i].op, rs);
+      if (lds_mode) emit_lds(in[rem_op[i]]);
+      else emit_gate(in[rem_op[i]], rs);
     }
-    std::vector<RItem> keep;
-    keep.reserve(rem.size() - idx.size());
-    size_t k = 0;
+    size_t k = 0, to = 0;
     for (size_t i = 0; i < rem.size(); ++i) {
       if (k < idx.size() && idx[k] == i) {
         ++k;
         continue;
       }
-      keep.push_back(rem[i]);
+      rem[to] = rem[i];
+      rem_op[to++] = rem_op[i];
     }
-    rem.swap(keep);
+    rem.resize(to);
+    rem_op.resize(to);
   };
 
   // Load in the best set that keeps the low bits on lanes.
@@ -1583,7 +1612,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   bool lds_mode = false;
   while (!rem.empty()) {
     if (!lds_mode) {
-      const auto idx = scan_items(rem, [&](const RItem &it) { return fits(it, rs); });
+      const auto idx = scan_items(rem, [&](const RMask &it) { return fits(it, rs); });
       if (!idx.empty()) {
         take(idx, rs, false);
         continue;
@@ -1601,8 +1630,8 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     // LDS mode: run every ready op that cannot run in registers (and ready
     // diagonals; fused diagonals run only in registers), then return to
     // registers if register gates are pending.
-    const auto idx = scan_items(rem, [&](const RItem &it) {
-      return it.cls == 2 || (it.cls == 1 && it.op.kind != K_PHASES);
+    const auto idx = scan_items(rem, [&](const RMask &it) {
+      return it.cls == 2 || (it.cls == 1 && in[rem_op[static_cast<size_t>(&it - rem.data())]].kind != K_PHASES);
     });
     if (!idx.empty()) {
       take(idx, rs, true);
@@ -1704,26 +1733,33 @@ std::vector<PassPlan> Engine::plan() const {
   while (seg_begin < queue_.size()) {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
-    std::vector<uint32_t> remaining;
-    for (size_t i = seg_begin; i < seg_end; ++i) remaining.push_back(static_cast<uint32_t>(i));
+    // What the scans read of the primitives, kept together.
+    struct Pending {
+      uint64_t tmask, touch;
+      uint32_t idx;
+      bool probe, unitary, gate;
+    };
+    std::vector<Pending> remaining;
+    for (size_t i = seg_begin; i < seg_end; ++i) {
+      const Prim &p = queue_[i];
+      remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
+                                  gates && gate_prim(p)});
+    }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
       // primitives in program order while their mixed qubits fit.  With
       // `take` null it only counts, and stops once every qubit the remaining
       // primitives touch is blocked.
       uint64_t active = 0;
-      for (uint32_t idx : remaining) active |= queue_[idx].touch;
+      for (const Pending &p : remaining) active |= p.touch;
       // A gate pass (`cap` qubits) takes only what its kernel runs.
-      auto scan = [&](uint32_t cap, uint64_t s0, PassPlan *take, std::vector<uint32_t> *rest) {
+      auto scan = [&](uint32_t cap, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
         size_t count = 0;
-        for (size_t r = 0; r < remaining.size(); ++r) {
-          const uint32_t idx = remaining[r];
-          const Prim &p = queue_[idx];
-          bool fits = !(p.touch & blocked) && !(p.kind == K_PROBE && nonunitary_blocked) &&
-                      (cap == nb || gate_prim(p));
+        for (const Pending &p : remaining) {
+          bool fits = !(p.touch & blocked) && !(p.probe && nonunitary_blocked) && (cap == nb || p.gate);
           if (fits) {
             const uint64_t ns = s | p.tmask;
             fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
@@ -1731,10 +1767,10 @@ std::vector<PassPlan> Engine::plan() const {
           }
           if (fits) {
             ++count;
-            if (take) take->prims.push_back(idx);
+            if (take) take->prims.push_back(p.idx);
             continue;
           }
-          if (rest) rest->push_back(idx);
+          if (rest) rest->push_back(p);
           blocked |= p.touch;
           nonunitary_blocked |= !p.unitary;
           if (!take && (blocked & active) == active) break;
@@ -1773,7 +1809,7 @@ std::vector<PassPlan> Engine::plan() const {
       PassPlan pp;
       pp.solo = false;
       pp.gate = cap != nb;
-      std::vector<uint32_t> rest;
+      std::vector<Pending> rest;
       scan(cap, seed, &pp, &rest);
       uint64_t s = pp.smask;
       // Complete the tile with the lowest free qubits (longer contiguous runs).
@@ -2456,18 +2492,20 @@ void Engine::flush() {
   const size_t pool_off = align_up(rops_off + rops_bytes, 256);
   const size_t total = pool_off + pool.size() * sizeof(cd) + 16;
   AERHIP_CHECK(hipEventSynchronize(prog_ev_));  // previous upload finished with staging
-  if (total > h_prog_cap_) {
-    if (h_prog_) AERHIP_CHECK(hipHostFree(h_prog_));
-    h_prog_cap_ = align_up(total * 2, 1 << 16);
-    AERHIP_CHECK(hipHostMalloc(&h_prog_, h_prog_cap_));
+  if (total > ws_.staging.bytes) {
+    void *old = ws_.staging.p;
+    ws_.staging = Workspace::Buffer{};
+    if (old) AERHIP_CHECK(hipHostFree(old));
+    const size_t bytes = align_up(total * 2, 1 << 16);
+    AERHIP_CHECK(hipHostMalloc(&ws_.staging.p, bytes));
+    ws_.staging.bytes = bytes;
   }
-  if (total > d_prog_cap_) {
+  if (total > ws_.program.bytes) {
     AERHIP_CHECK(hipStreamSynchronize(stream_));
-    if (d_prog_) AERHIP_CHECK(hipFree(d_prog_));
-    d_prog_cap_ = align_up(total * 2, 1 << 16);
-    AERHIP_CHECK(hipMalloc(&d_prog_, d_prog_cap_));
+    WorkspacePool::grow(ws_.program, align_up(total * 2, 1 << 16));
   }
-  char *h = static_cast<char *>(h_prog_);
+  void *const h_prog = ws_.staging.p, *const d_prog = ws_.program.p;
+  char *h = static_cast<char *>(h_prog);
   std::memcpy(h, passes.data(), pass_bytes);
   std::memcpy(h + ops_off, ops.data(), ops_bytes);
   if (prec_ == AERHIP_PRECISION_DOUBLE) {
@@ -2477,10 +2515,10 @@ void Engine::flush() {
     rops_to_float(rops.data(), rops.size(), reinterpret_cast<ROp<float> *>(h + rops_off));
   }
   if (!pool.empty()) std::memcpy(h + pool_off, pool.data(), pool.size() * sizeof(cd));
-  AERHIP_CHECK(hipMemcpyAsync(d_prog_, h_prog_, total, hipMemcpyHostToDevice, stream_));
+  AERHIP_CHECK(hipMemcpyAsync(d_prog, h_prog, total, hipMemcpyHostToDevice, stream_));
   AERHIP_CHECK(hipEventRecord(prog_ev_, stream_));
 
-  char *d = static_cast<char *>(d_prog_);
+  char *d = static_cast<char *>(d_prog);
   const PassDesc *dpass = reinterpret_cast<const PassDesc *>(d);
   const TileOp *dops = reinterpret_cast<const TileOp *>(d + ops_off);
   const void *drops = d + rops_off;
@@ -2491,13 +2529,11 @@ void Engine::flush() {
   const uint64_t ntiles = 1ull << (n_ - tile_bits_);
   if (nprobes) {
     const size_t need = (nprobes * ntiles + nprobes) * sizeof(double);
-    if (need > probes_cap_) {
+    if (need > ws_.probes.bytes) {
       AERHIP_CHECK(hipStreamSynchronize(stream_));
-      if (d_probes_) AERHIP_CHECK(hipFree(d_probes_));
-      probes_cap_ = align_up(need, 1 << 20);
-      AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_probes_), probes_cap_));
+      WorkspacePool::grow(ws_.probes, align_up(need, 1 << 20));
     }
-    dprobes = d_probes_;
+    dprobes = static_cast<double *>(ws_.probes.p);
   }
   if (event_timing_) AERHIP_CHECK(hipEventRecord(t0_ev_, stream_));
   const DeviceProgram dp{dpass, dops, drops, dpool, dprobes, 0};
@@ -2507,7 +2543,7 @@ void Engine::flush() {
   // circuit again, or the same shape with other angles: the new program was
   // uploaded to the same buffer above) replays the sequence as a HIP graph:
   // captured on the second occurrence, replayed from the third on.
-  std::vector<uint64_t> sig = {reinterpret_cast<uint64_t>(d_prog_), reinterpret_cast<uint64_t>(sv_),
+  std::vector<uint64_t> sig = {reinterpret_cast<uint64_t>(d_prog), reinterpret_cast<uint64_t>(sv_),
                                reinterpret_cast<uint64_t>(dprobes), static_cast<uint64_t>(prec_),
                                reg_bits_, n_, tile_bits_, passes.size(), ops_off, rops_off, pool_off};
   std::vector<PassKernel> kernels(passes.size());
@@ -2552,8 +2588,8 @@ void Engine::flush() {
   stats_.passes += passes.size();
   if (nprobes) {
     // Sum each probe's tile partials in tile order and fetch the values.
-    double *sums = d_probes_ + nprobes * ntiles;
-    sum_rows(d_probes_, nprobes, static_cast<uint32_t>(ntiles), sums, stream_);
+    double *sums = dprobes + nprobes * ntiles;
+    sum_rows(dprobes, nprobes, static_cast<uint32_t>(ntiles), sums, stream_);
     AERHIP_CHECK(hipGetLastError());
     const size_t base = saved_expvals_.size();
     saved_expvals_.resize(base + nprobes);
@@ -2601,21 +2637,19 @@ void Engine::set_event_timing(bool on) {
 // ---------------------------------------------------------------------------
 
 void Engine::ensure_partial(size_t n) {
-  if (n <= partial_cap_) return;
-  AERHIP_CHECK(hipStreamSynchronize(stream_));
-  if (d_partial_) AERHIP_CHECK(hipFree(d_partial_));
-  partial_cap_ = std::max<size_t>(n, 1 << 16);
-  AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_partial_), partial_cap_ * sizeof(double)));
+  if (n * sizeof(double) > ws_.partial.bytes) {
+    AERHIP_CHECK(hipStreamSynchronize(stream_));
+    WorkspacePool::grow(ws_.partial, std::max<size_t>(n, 1 << 16) * sizeof(double));
+  }
+  d_partial_ = static_cast<double *>(ws_.partial.p);
 }
 
 void *Engine::scratch(size_t bytes) {
-  if (bytes > scratch_cap_) {
+  if (bytes > ws_.scratch.bytes) {
     AERHIP_CHECK(hipStreamSynchronize(stream_));
-    if (d_scratch_) AERHIP_CHECK(hipFree(d_scratch_));
-    scratch_cap_ = std::max<size_t>(align_up(bytes, 1 << 16), 1 << 20);
-    AERHIP_CHECK(hipMalloc(&d_scratch_, scratch_cap_));
+    WorkspacePool::grow(ws_.scratch, std::max<size_t>(align_up(bytes, 1 << 16), 1 << 20));
   }
-  return d_scratch_;
+  return ws_.scratch.p;
 }
 
 double Engine::fetch_scalar(const double *dptr) {
@@ -3098,26 +3132,26 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   });
 
   AERHIP_CHECK(hipSetDevice(device));
-  void *d_states = nullptr, *d_prog = nullptr;
-  double *d_probes = nullptr;
-  hipStream_t st = nullptr;
+  Workspace ws = WorkspacePool::get().take(device, sv_off * amp);
+  const hipStream_t st = ws.stream;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  auto release = [&] {
-    if (st) (void)hipStreamSynchronize(st);
-    if (d_states) (void)hipFree(d_states);
-    if (d_prog) (void)hipFree(d_prog);
-    if (d_probes) (void)hipFree(d_probes);
+  auto release = [&](bool ok) {
+    ok = hipStreamSynchronize(st) == hipSuccess && ok;
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
-    if (st) (void)hipStreamDestroy(st);
+    if (ok)
+      WorkspacePool::get().give(ws);
+    else
+      ws.release();
   };
   try {
-    AERHIP_CHECK(hipStreamCreate(&st));
     AERHIP_CHECK(hipEventCreate(&e0));
     AERHIP_CHECK(hipEventCreate(&e1));
-    AERHIP_CHECK(hipMalloc(&d_states, sv_off * amp));
-    AERHIP_CHECK(hipMalloc(&d_prog, total));
-    AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_probes), (probe_off + part_off + 1) * sizeof(double)));
+    if (total > ws.program.bytes) WorkspacePool::grow(ws.program, total);
+    const size_t probe_bytes = (probe_off + part_off + 1) * sizeof(double);
+    if (probe_bytes > ws.probes.bytes) WorkspacePool::grow(ws.probes, probe_bytes);
+    void *const d_states = ws.state.p, *const d_prog = ws.program.p;
+    double *const d_probes = static_cast<double *>(ws.probes.p);
     AERHIP_CHECK(hipMemcpyAsync(d_prog, h.get(), total, hipMemcpyHostToDevice, st));
     char *d = static_cast<char *>(d_prog);
     const auto *dc = reinterpret_cast<const BatchCircuit *>(d);
@@ -3168,10 +3202,10 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     AERHIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
     if (kernel_ms) *kernel_ms = ms;
   } catch (...) {
-    release();
+    release(false);
     throw;
   }
-  release();
+  release(true);
 }
 
 // ---------------------------------------------------------------------------
@@ -3193,21 +3227,22 @@ class MultiState {
         throw std::invalid_argument("aerhip: states need planning handles of one size and precision");
     for (Engine *e : planners_) e->use_gate_passes();
     AERHIP_CHECK(hipSetDevice(device_));
-    AERHIP_CHECK(hipStreamCreate(&st_));
+    ws_ = WorkspacePool::get().take(device_, planners_.size() * (1ull << n_) * amp_bytes());
+    states_ = ws_.state.p;
+    st_ = ws_.stream;
     AERHIP_CHECK(hipEventCreate(&e0_));
     AERHIP_CHECK(hipEventCreate(&e1_));
-    AERHIP_CHECK(hipMalloc(&states_, planners_.size() * (1ull << n_) * amp_bytes()));
   }
   ~MultiState() {
     (void)hipSetDevice(device_);
-    if (st_) (void)hipStreamSynchronize(st_);
-    if (states_) (void)hipFree(states_);
-    if (d_prog_) (void)hipFree(d_prog_);
-    if (d_probes_) (void)hipFree(d_probes_);
+    const hipError_t e = hipStreamSynchronize(st_);
     if (d_terms_) (void)hipFree(d_terms_);
     if (e0_) (void)hipEventDestroy(e0_);
     if (e1_) (void)hipEventDestroy(e1_);
-    if (st_) (void)hipStreamDestroy(st_);
+    if (e == hipSuccess)
+      WorkspacePool::get().give(ws_);
+    else
+      ws_.release();
   }
   MultiState(const MultiState &) = delete;
   MultiState &operator=(const MultiState &) = delete;
@@ -3235,7 +3270,7 @@ class MultiState {
     AERHIP_CHECK(hipStreamSynchronize(st_));
     if (d_terms_) AERHIP_CHECK(hipFree(d_terms_));
     d_terms_ = nullptr;
-    AERHIP_CHECK(hipMalloc(&d_terms_, std::max<size_t>(1, terms.size()) * sizeof(PauliTerm)));
+    d_terms_ = WorkspacePool::allocate(std::max<size_t>(1, terms.size()) * sizeof(PauliTerm));
     AERHIP_CHECK(hipMemcpy(d_terms_, terms.data(), terms.size() * sizeof(PauliTerm), hipMemcpyHostToDevice));
     const uint64_t half = 1ull << (n_ - 1);
     const auto *dt = static_cast<const PauliTerm *>(d_terms_);
@@ -3344,39 +3379,33 @@ class MultiState {
     else
       rops_to_float(rops.data(), rops.size(), reinterpret_cast<ROp<float> *>(h.data() + rops_off));
     if (!pool.empty()) std::memcpy(h.data() + pool_off, pool.data(), pool.size() * sizeof(cd));
-    if (total > prog_cap_) {
+    if (total > ws_.program.bytes) {
       AERHIP_CHECK(hipStreamSynchronize(st_));
-      if (d_prog_) AERHIP_CHECK(hipFree(d_prog_));
-      d_prog_ = nullptr;
-      prog_cap_ = align_up(total, 1 << 16);
-      AERHIP_CHECK(hipMalloc(&d_prog_, prog_cap_));
+      WorkspacePool::grow(ws_.program, align_up(total, 1 << 16));
     }
+    void *const d_prog = ws_.program.p;
     // pageable source: the copy is complete when hipMemcpyAsync returns
-    AERHIP_CHECK(hipMemcpyAsync(d_prog_, h.data(), total, hipMemcpyHostToDevice, st_));
+    AERHIP_CHECK(hipMemcpyAsync(d_prog, h.data(), total, hipMemcpyHostToDevice, st_));
     AERHIP_CHECK(hipStreamSynchronize(st_));
     const uint32_t tb = planners_[first]->tile_bits();
     const uint64_t ntiles = 1ull << (n_ - tb);
     if (pps) {
       const size_t need = (cnt * pps * ntiles + cnt * pps) * sizeof(double);
-      if (need > probes_cap_) {
-        if (d_probes_) AERHIP_CHECK(hipFree(d_probes_));
-        d_probes_ = nullptr;
-        probes_cap_ = align_up(need, 1 << 20);
-        AERHIP_CHECK(hipMalloc(reinterpret_cast<void **>(&d_probes_), probes_cap_));
-      }
+      if (need > ws_.probes.bytes) WorkspacePool::grow(ws_.probes, align_up(need, 1 << 20));
     }
-    char *d = static_cast<char *>(d_prog_);
+    double *const d_probes = static_cast<double *>(ws_.probes.p);
+    char *d = static_cast<char *>(d_prog);
     const DeviceProgram dp{reinterpret_cast<const PassDesc *>(d), reinterpret_cast<const TileOp *>(d + ops_off),
                            d + rops_off, reinterpret_cast<const cx<double> *>(d + pool_off),
-                           pps ? d_probes_ : nullptr, static_cast<uint32_t>(pps)};
+                           pps ? d_probes : nullptr, static_cast<uint32_t>(pps)};
     void *sv = static_cast<char *>(states_) + first * (1ull << n_) * amp_bytes();
     for (size_t k = 0; k < P; ++k)
       launch_pass(prec_, planners_[first]->reg_bits(), n_, tb, parts[first].passes[k],
                   static_cast<uint32_t>(k), kernels[k], dp, sv, cnt,
                   static_cast<uint32_t>(P), st_);
     if (pps) {
-      double *sums = d_probes_ + cnt * pps * ntiles;
-      sum_rows(d_probes_, cnt * pps, static_cast<uint32_t>(ntiles), sums, st_);
+      double *sums = d_probes + cnt * pps * ntiles;
+      sum_rows(d_probes, cnt * pps, static_cast<uint32_t>(ntiles), sums, st_);
       AERHIP_CHECK(hipGetLastError());
       AERHIP_CHECK(hipMemcpyAsync(values, sums, cnt * pps * sizeof(double), hipMemcpyDeviceToHost, st_));
     }
@@ -3390,10 +3419,7 @@ class MultiState {
   void *states_ = nullptr;
   hipStream_t st_ = nullptr;
   hipEvent_t e0_ = nullptr, e1_ = nullptr;
-  void *d_prog_ = nullptr;
-  size_t prog_cap_ = 0;
-  double *d_probes_ = nullptr;
-  size_t probes_cap_ = 0;
+  Workspace ws_;
   void *d_terms_ = nullptr;
   double kernel_ms_ = 0;
 };
@@ -3632,7 +3658,7 @@ int aerhip_qv_device_pointer(aerhip_qv *qv, void **out) {
   return guard([&] {
     if (!out) throw std::invalid_argument("aerhip: null argument");
     E(qv).synchronize();
-    *out = E(qv).device_data();
+    *out = E(qv).hand_out();
   });
 }
 

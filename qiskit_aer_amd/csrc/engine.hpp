@@ -10,6 +10,7 @@
 
 #include "common.hpp"
 #include "reg_pass.hpp"
+#include "workspace.hpp"
 
 namespace aerhip {
 
@@ -73,6 +74,11 @@ class Engine {
   int precision() const { return prec_; }
   uint64_t size() const { return size_; }
   void *device_data() { return sv_; }
+  // The state's address for work on other streams.
+  void *hand_out() {
+    exposed_ = true;
+    return sv_;
+  }
   hipStream_t stream() const { return stream_; }
   EngineStats &stats() { return stats_; }
 
@@ -202,23 +208,16 @@ class Engine {
   std::vector<Prim> queue_;
   std::vector<cd> pool_;
 
-  // device program of a flush: [passes | ops | pool]
-  void *d_prog_ = nullptr;
-  size_t d_prog_cap_ = 0;
-  void *h_prog_ = nullptr;  // pinned staging
-  size_t h_prog_cap_ = 0;
+  // Stream, staging and device buffers, shared with later handles; sv_,
+  // stream_, prog_ev_, h_scalar_ and d_partial_ are its members.
+  Workspace ws_;
+  bool exposed_ = false;  // the state's address left the handle
   hipEvent_t prog_ev_ = nullptr;
-
   double *d_partial_ = nullptr;
-  size_t partial_cap_ = 0;
   double *h_scalar_ = nullptr;  // pinned
-  void *d_scratch_ = nullptr;   // descriptors, draws and samples of readouts
-  size_t scratch_cap_ = 0;
 
   uint64_t probes_queued_ = 0;        // probes in the current queue
   std::vector<double> saved_expvals_; // values of flushed probes, slot order
-  double *d_probes_ = nullptr;        // per-tile probe partials
-  size_t probes_cap_ = 0;
 
   EngineStats stats_;
   // HIP graph of the last repeated flush (its launch signature and the

@@ -104,7 +104,7 @@ class AerSimulator:
             del keep
             mem = mem[:shots]
             vals, cnt = np.unique(mem, return_counts=True)
-            counts = {hex(int(v)): int(c) for v, c in zip(vals, cnt)} if circ.num_clbits else {}
+            counts = dict(zip(map(hex, vals.tolist()), cnt.tolist())) if circ.num_clbits else {}
             out.append(ExperimentResult(counts, mem, sv, int(cfg.seed), float(timing[0]),
                                         float(timing[1]), int(timing[2]), int(timing[3]),
                                         {"method": "statevector", "device": "GPU",
