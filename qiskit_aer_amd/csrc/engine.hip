@@ -1454,14 +1454,30 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         }
         if (single) {
           // rounded here: the kernel reads the entries as scalars, where
-          // rounding them would cost it a conversion and a register each
+          // rounding them would cost it a conversion and a register each; a
+          // gate pass reads rows of the real 8x8 form, for MFMA
           cx<float> m[16];
           for (int e = 0; e < 16; ++e)
-            m[e] = to_t<float>(mk<double>(pool[op.off + e].real(), pool[op.off + e].imag()));
-          cd rec[8];
-          std::memcpy(rec, m, sizeof(rec));
+            m[e] = to_t<float>(mk<double>(pool[r.extra + e].real(), pool[r.extra + e].imag()));
           r.extra = static_cast<uint32_t>(pool.size());
-          pool.insert(pool.end(), rec, rec + 8);
+          if (gate) {
+            float rows[64];
+            for (int i = 0; i < 4; ++i)
+              for (int k = 0; k < 4; ++k) {
+                const cx<float> v = m[i + 4 * k];
+                rows[16 * i + 2 * k] = v.x;
+                rows[16 * i + 2 * k + 1] = -v.y;
+                rows[16 * i + 8 + 2 * k] = v.y;
+                rows[16 * i + 8 + 2 * k + 1] = v.x;
+              }
+            cd rec[16];
+            std::memcpy(rec, rows, sizeof(rec));
+            pool.insert(pool.end(), rec, rec + 16);
+          } else {
+            cd rec[8];
+            std::memcpy(rec, m, sizeof(rec));
+            pool.insert(pool.end(), rec, rec + 8);
+          }
         }
         break;
       }
@@ -1703,12 +1719,15 @@ std::vector<PassPlan> Engine::gather_sweeps(std::vector<PassPlan> plans) const {
   return out;
 }
 
-// Whether the handle's passes may use the gate pass's larger tiles: complex128
-// under the engine's own tile settings, with diagonal fusion (single diagonals
-// on fixed qubits run fused), and enough tiles to fill the device.
-bool Engine::gate_tiles() const {
-  return gate_passes_ && prec_ == AERHIP_PRECISION_DOUBLE && tile_bits_ == kTileBitsC128 && low_bits_ == 3 &&
-         reg_bits_ == 3 && fusion_enable_ && n_ > fusion_threshold_ && n_ >= kGateMinQubits;
+// Tile bits of the handle's gate passes; 0: it has none.  They run under the
+// engine's own tile settings, with diagonal fusion (single diagonals on fixed
+// qubits run fused).  complex128 tiles are twice the other passes', so they need
+// enough of them to fill the device; complex64 ones are as large.
+uint32_t Engine::gate_tile_bits() const {
+  if (!gate_passes_ || !fusion_enable_ || n_ <= fusion_threshold_) return 0;
+  if (prec_ == AERHIP_PRECISION_DOUBLE)
+    return tile_bits_ == kTileBitsC128 && low_bits_ == 3 && reg_bits_ == 3 && n_ >= kGateMinQubits ? kGateTileC128 : 0;
+  return tile_bits_ == kTileBitsC64 && low_bits_ == 4 && reg_bits_ == 4 ? kTileBitsC64 : 0;
 }
 
 // Whether the gate pass runs a primitive.
@@ -1729,7 +1748,7 @@ std::vector<PassPlan> Engine::plan() const {
   for (const Prim &p : queue_)
     if (!p.solo && static_cast<uint32_t>(__builtin_popcountll(p.tmask | lowmask)) > nb)
       throw std::logic_error("aerhip: a primitive mixes more qubits than a tile holds");
-  const bool gates = gate_tiles();
+  const uint32_t gate_bits = gate_tile_bits();
   while (seg_begin < queue_.size()) {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
@@ -1743,7 +1762,7 @@ std::vector<PassPlan> Engine::plan() const {
     for (size_t i = seg_begin; i < seg_end; ++i) {
       const Prim &p = queue_[i];
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
-                                  gates && gate_prim(p)});
+                                  gate_bits && gate_prim(p)});
     }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
@@ -1752,14 +1771,14 @@ std::vector<PassPlan> Engine::plan() const {
       // primitives touch is blocked.
       uint64_t active = 0;
       for (const Pending &p : remaining) active |= p.touch;
-      // A gate pass (`cap` qubits) takes only what its kernel runs.
-      auto scan = [&](uint32_t cap, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
+      // A gate pass takes only what its kernel runs.
+      auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
         size_t count = 0;
         for (const Pending &p : remaining) {
-          bool fits = !(p.touch & blocked) && !(p.probe && nonunitary_blocked) && (cap == nb || p.gate);
+          bool fits = !(p.touch & blocked) && !(p.probe && nonunitary_blocked) && (!gate || p.gate);
           if (fits) {
             const uint64_t ns = s | p.tmask;
             fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
@@ -1784,19 +1803,21 @@ std::vector<PassPlan> Engine::plan() const {
       // (the 30-qubit U3+CX brickwork takes 29 passes instead of 66); the
       // pass keeps the candidate that takes the most primitives, the first
       // on ties.
-      // A pass on the small tile runs every primitive; a gate pass is taken
-      // where it holds more of them, or as many but more than a few: a pass of
-      // one gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.
+      // The other tile passes run every primitive; a gate pass is taken where
+      // it holds more of them, or as many but more than a few: a pass of one
+      // gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.
       uint64_t seed = lowmask;
       uint32_t cap = nb;
+      bool gate = false;
       size_t best = 0;
-      auto try_tile = [&](uint32_t c) {
+      auto try_tile = [&](uint32_t c, bool g) {
         auto candidate = [&](uint64_t s0) {
-          const size_t k = scan(c, s0, nullptr, nullptr);
-          if (k > best || (k == best && k > 4 && c > cap)) {
+          const size_t k = scan(c, g, s0, nullptr, nullptr);
+          if (k > best || (k == best && k > 4 && g && !gate)) {
             best = k;
             seed = s0;
             cap = c;
+            gate = g;
           }
         };
         candidate(lowmask);
@@ -1804,13 +1825,12 @@ std::vector<PassPlan> Engine::plan() const {
         if (n_ > c && w > 0)
           for (uint32_t a = 0; a + w <= n_; ++a) candidate(lowmask | (((1ull << w) - 1ull) << a));
       };
-      try_tile(nb);
-      if (gates) try_tile(kGateTileC128);
+      try_tile(nb, false);
+      if (gate_bits) try_tile(gate_bits, true);
       PassPlan pp;
-      pp.solo = false;
-      pp.gate = cap != nb;
+      pp.gate = gate;
       std::vector<Pending> rest;
-      scan(cap, seed, &pp, &rest);
+      scan(cap, gate, seed, &pp, &rest);
       uint64_t s = pp.smask;
       // Complete the tile with the lowest free qubits (longer contiguous runs).
       for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < cap; ++q)
@@ -2288,7 +2308,9 @@ void Engine::emit_program(Program &prog) {
       }
       pops.push_back(op);
     }
-    const uint32_t full_bits = pp.gate ? kGateTileC128 : prec_ == AERHIP_PRECISION_DOUBLE ? kTileBitsC128 : kTileBitsC64;
+    const uint32_t full_bits = pp.gate                             ? gate_tile_bits()
+                               : prec_ == AERHIP_PRECISION_DOUBLE ? kTileBitsC128
+                                                                  : kTileBitsC64;
     const uint32_t R = pp.gate ? kGateRegBits : reg_bits_;
     if (!pp.solo && reg_bits_ > 0 && ns == full_bits) {
       if (fusion_enable_ && n_ > fusion_threshold_)
@@ -2397,10 +2419,17 @@ void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, co
     }
   } else if (pd.kind == 5) {
     const uint32_t tl = pd.ncomp;
-    k_gate_pass<double, kGateTileC128, kGateRegBits>
-        <<<grid_of(tl), 1 << (kGateTileC128 - kGateRegBits), pk.diag ? kDiagLdsBytes : 0, stream>>>(
-            static_cast<cx<double> *>(sv), dpd, static_cast<const ROp<double> *>(dp.rops), dp.ops, dp.pool,
-            state_stride, pd_stride, tl);
+    const size_t dyn = pk.diag ? kDiagLdsBytes : 0;
+    if (prec == AERHIP_PRECISION_DOUBLE)
+      k_gate_pass<double, kGateTileC128, kGateRegBits>
+          <<<grid_of(tl), 1 << (kGateTileC128 - kGateRegBits), dyn, stream>>>(
+              static_cast<cx<double> *>(sv), dpd, static_cast<const ROp<double> *>(dp.rops), dp.ops, dp.pool,
+              state_stride, pd_stride, tl);
+    else
+      k_gate_pass<float, kTileBitsC64, kGateRegBits>
+          <<<grid_of(tl), 1 << (kTileBitsC64 - kGateRegBits), dyn, stream>>>(
+              static_cast<cx<float> *>(sv), dpd, static_cast<const ROp<float> *>(dp.rops), dp.ops, dp.pool,
+              state_stride, pd_stride, tl);
   } else if (pd.kind == 3) {
     // probes over the whole state, one workgroup per tile-sized slice
     const uint32_t tl = n - tile_bits;

@@ -172,7 +172,7 @@ class Engine {
   void apply_matrix_1(uint32_t q, const std::vector<cd> &mat);
   void apply_diagonal_1(uint32_t q, const cd *diag);
   std::vector<PassPlan> plan() const;
-  bool gate_tiles() const;
+  uint32_t gate_tile_bits() const;
   bool gate_prim(const Prim &p) const;
   std::vector<PassPlan> gather_sweeps(std::vector<PassPlan> plans) const;
   std::vector<Prim> fuse_blocks(const std::vector<Prim> &in);

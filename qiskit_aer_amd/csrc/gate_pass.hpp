@@ -91,6 +91,60 @@ __device__ __forceinline__ void g_u1b(Amps<T, NR> &a, const cx<T> (&u)[4]) {
   for (int k = 0; k < NR / 2; ++k) g_u1(a.v[pair_lo<b>(k)], a.v[pair_lo<b>(k) | (1 << b)], u);
 }
 
+// complex64 2x2 gate with MFMA (see q_u1_mfma): `A` is row lane % 4 of the real
+// 4x4 form.
+template <int NR, int b>
+__device__ __forceinline__ void g_u1b_mfma(Amps<float, NR> &a, f32x4 A) {
+  constexpr int G = 4;  // pairs whose accumulation chains interleave
+#pragma unroll
+  for (int g = 0; g < NR / 2; g += G) {
+    f32x4 acc[G];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int p = 0; p < G; ++p) {
+        const cx<float> v = a.v[pair_lo<b>(g + p) | (k < 2 ? 0 : 1 << b)];
+        acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[k], k & 1 ? v.y : v.x, k ? acc[p] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      a.v[pair_lo<b>(g + p)] = mk<float>(acc[p][0], acc[p][1]);
+      a.v[pair_lo<b>(g + p) | (1 << b)] = mk<float>(acc[p][2], acc[p][3]);
+    }
+  }
+}
+
+// complex64 4x4 gate with MFMA: the real 8x8 form in two halves of four rows,
+// each a chain of eight v_mfma_f32_4x4x1f32 per group of four amplitudes, at
+// twice the rate of FMAs on the vector ALU.  A[0..1]: row lane % 4 of the first
+// half (amplitudes 0 and 1 of the group), A[2..3]: of the second.
+template <int NR, int b0, int b1>
+__device__ __forceinline__ void g_u2_mfma(Amps<float, NR> &a, const f32x4 (&A)[4]) {
+#pragma unroll
+  for (int g = 0; g < NR / 4; g += 2) {  // two groups: four chains interleave
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int j = pair_lo<b1>(pair_lo<b0>(g + q)) | (k & 2 ? 1 << b0 : 0) | (k & 4 ? 1 << b1 : 0);
+        const float v = k & 1 ? a.v[j].y : a.v[j].x;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc[q][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[2 * h + (k >> 2)][k & 3], v,
+                                                         k ? acc[q][h] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int j = pair_lo<b1>(pair_lo<b0>(g + q));
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        a.v[j | (r & 1 ? 1 << b0 : 0) | (r & 2 ? 1 << b1 : 0)] =
+            mk<float>(acc[q][r >> 1][2 * (r & 1)], acc[q][r >> 1][2 * (r & 1) + 1]);
+    }
+  }
+}
+
 // 4x4 gate on register bits b0 (matrix bit 0) < b1, column major.
 template <typename T, int NR, int b0, int b1>
 __device__ __forceinline__ void g_u2(Amps<T, NR> &a, const cx<T> (&m)[16]) {
@@ -202,21 +256,55 @@ __device__ __forceinline__ void g_load_u1(const ROp<T> &op, bool fx, cx<T> (&m)[
   m[3] = mk<T>(c1[2], c1[3]);
 }
 
-// One component of every amplitude moves from slots ws ^ rw(j) to rs ^ rr(j).
-template <typename T, int NR, bool im>
-__device__ __forceinline__ void g_exchange(Amps<T, NR> &a, T *xch, const uint32_t (&w)[NR], const uint32_t (&r)[NR]) {
+// Slot x of the exchange buffer, as a byte offset: x ^ ((x >> 4) & 15), so that
+// consecutive lanes reach distinct banks also where the register bits are the
+// low tile bits.  Linear, so it splits into a per-lane and a per-register term.
+__device__ __forceinline__ uint32_t g_slot(uint32_t x) { return (x ^ ((x >> 4) & 15u)) << 3; }
+
+// Tile index of thread `t`'s part of the layout with register tile bits rp
+// (ascending): t with a zero inserted at each of them.
+template <int R>
+__device__ __forceinline__ uint32_t g_thread(const RLayout &lay, uint32_t t) {
 #pragma unroll
-  for (int j = 0; j < NR; ++j) xch[w[j]] = im ? a.v[j].y : a.v[j].x;
+  for (int r = 0; r < R; ++r) t += t & (~0u << byte_at(lay.rp, r));
+  return t;
+}
+
+// The tile moves from the layout of byte offsets w0 ^ w(j) to that of r0 ^ r(j),
+// w and r uniform.  complex128: one component at a time, so that the buffer
+// holds half a tile.
+template <typename T, int NR>
+__device__ __forceinline__ void g_exchange(Amps<T, NR> &a, char *xch, uint32_t w0, const uint32_t (&w)[NR],
+                                           uint32_t r0, const uint32_t (&r)[NR]) {
+  asm volatile("" : "+v"(w0), "+v"(r0));  // shifted already: one XOR per address
   __syncthreads();
+  if constexpr (sizeof(T) == 4) {
 #pragma unroll
-  for (int j = 0; j < NR; ++j) (im ? a.v[j].y : a.v[j].x) = xch[r[j]];
+    for (int j = 0; j < NR; ++j) *reinterpret_cast<cx<T> *>(xch + (w0 ^ w[j])) = a.v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; ++j) a.v[j] = *reinterpret_cast<const cx<T> *>(xch + (r0 ^ r[j]));
+  } else {
+#pragma unroll
+    for (int j = 0; j < NR; ++j) *reinterpret_cast<T *>(xch + (w0 ^ w[j])) = a.v[j].x;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; ++j) a.v[j].x = *reinterpret_cast<const T *>(xch + (r0 ^ r[j]));
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; ++j) *reinterpret_cast<T *>(xch + (w0 ^ w[j])) = a.v[j].y;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; ++j) a.v[j].y = *reinterpret_cast<const T *>(xch + (r0 ^ r[j]));
+  }
 }
 
 template <typename T, int B, int R>
 __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd,
                                           const ROp<T> *__restrict__ rops, const TileOp *__restrict__ tops,
-                                          const cx<double> *__restrict__ pool, uint64_t tile_id, T *xch,
+                                          const cx<double> *__restrict__ pool, uint64_t tile_id, char *xch,
                                           cx<double> *dlt) {
+  static_assert(R == 4, "the op codes name four register bits");
   constexpr int TB = B - R, NT = 1 << TB, NR = 1 << R;
   const uint32_t tid = threadIdx.x;
   uint64_t base = tile_id;
@@ -227,7 +315,9 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
   }
   base = uniform64(base);
   const ROp<T> *opp = rops + pd->op_begin;
-  LayoutState<NR> st = make_state<R, TB>(opp->u.lay, tid);
+  LayoutState<NR> st;
+  st.tl = g_thread<R>(opp->u.lay, tid);
+  st.ri = reg_index<R>(opp->u.lay);
   const uint32_t nslot = opp->a;
   const cx<double> *dlane = pool + opp->b;
   uint2 drec = make_uint2(0u, 0u);
@@ -256,58 +346,74 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
     const uint32_t code = op.code;
     const bool tile_ok = (base & op.cg) == op.cvg;
     if ((code & 0xF0u) == C_U1) {
-      cx<T> m[4];
-      g_load_u1(op, tile_ok && (op.kind & ~F_ALL) == Q_U1X, m);
-      switch (code) {
-        case C_U1 + 0: g_u1b<T, NR, 0>(a, m); break;
-        case C_U1 + 1: g_u1b<T, NR, 1>(a, m); break;
-        case C_U1 + 2: g_u1b<T, NR, 2>(a, m); break;
-        case C_U1 + 3: if constexpr (R > 3) g_u1b<T, NR, R - 1>(a, m); break;
+      const bool fx = tile_ok && (op.kind & ~F_ALL) == Q_U1X;
+      if constexpr (sizeof(T) == 4) {
+        const f32x4 row = *reinterpret_cast<const f32x4 *>(op.u.mr + 4 * (tid & 3u));
+        const f32x4 A = fx ? f32x4{row.z, row.w, row.x, row.y} : row;  // U X: the columns change places
+        switch (code) {
+          case C_U1 + 0: g_u1b_mfma<NR, 0>(a, A); break;
+          case C_U1 + 1: g_u1b_mfma<NR, 1>(a, A); break;
+          case C_U1 + 2: g_u1b_mfma<NR, 2>(a, A); break;
+          case C_U1 + 3: g_u1b_mfma<NR, 3>(a, A); break;
+        }
+      } else {
+        cx<T> m[4];
+        g_load_u1(op, fx, m);
+        switch (code) {
+          case C_U1 + 0: g_u1b<T, NR, 0>(a, m); break;
+          case C_U1 + 1: g_u1b<T, NR, 1>(a, m); break;
+          case C_U1 + 2: g_u1b<T, NR, 2>(a, m); break;
+          case C_U1 + 3: g_u1b<T, NR, 3>(a, m); break;
+        }
       }
       continue;
     }
     const uint32_t cl = op.cl, cvl = op.cvl;
     if ((code & 0xF0u) == C_U2) {
-      if (cl == 0 && !tile_ok) continue;
-      cx<T> m[16];
-      const cx<T> *mp = reinterpret_cast<const cx<T> *>(pool + op.extra);
+      if constexpr (sizeof(T) == 4) {
+        const f32x4 *rows = reinterpret_cast<const f32x4 *>(pool + op.extra) + 2 * (tid & 3u);
+        const f32x4 A[4] = {rows[0], rows[1], rows[8], rows[9]};
+        switch (code) {
+          case C_U2 + pair_index(0, 1): g_u2_mfma<NR, 0, 1>(a, A); break;
+          case C_U2 + pair_index(0, 2): g_u2_mfma<NR, 0, 2>(a, A); break;
+          case C_U2 + pair_index(1, 2): g_u2_mfma<NR, 1, 2>(a, A); break;
+          case C_U2 + pair_index(0, 3): g_u2_mfma<NR, 0, 3>(a, A); break;
+          case C_U2 + pair_index(1, 3): g_u2_mfma<NR, 1, 3>(a, A); break;
+          case C_U2 + pair_index(2, 3): g_u2_mfma<NR, 2, 3>(a, A); break;
+        }
+      } else {
+        cx<T> m[16];
+        const cx<T> *mp = reinterpret_cast<const cx<T> *>(pool + op.extra);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) m[e] = mp[e];
-      switch (code) {
-        case C_U2 + pair_index(0, 1): g_u2<T, NR, 0, 1>(a, m); break;
-        case C_U2 + pair_index(0, 2): g_u2<T, NR, 0, 2>(a, m); break;
-        case C_U2 + pair_index(1, 2): g_u2<T, NR, 1, 2>(a, m); break;
-        case C_U2 + pair_index(0, 3): if constexpr (R > 3) g_u2<T, NR, 0, R - 1>(a, m); break;
-        case C_U2 + pair_index(1, 3): if constexpr (R > 3) g_u2<T, NR, 1, R - 1>(a, m); break;
-        case C_U2 + pair_index(2, 3): if constexpr (R > 3) g_u2<T, NR, 2, R - 1>(a, m); break;
+        for (int e = 0; e < 16; ++e) m[e] = mp[e];
+        switch (code) {
+          case C_U2 + pair_index(0, 1): g_u2<T, NR, 0, 1>(a, m); break;
+          case C_U2 + pair_index(0, 2): g_u2<T, NR, 0, 2>(a, m); break;
+          case C_U2 + pair_index(1, 2): g_u2<T, NR, 1, 2>(a, m); break;
+          case C_U2 + pair_index(0, 3): g_u2<T, NR, 0, 3>(a, m); break;
+          case C_U2 + pair_index(1, 3): g_u2<T, NR, 1, 3>(a, m); break;
+          case C_U2 + pair_index(2, 3): g_u2<T, NR, 2, 3>(a, m); break;
+        }
       }
       continue;
     }
     if (code == C_RELAYOUT) {
-      // Slot x of a component at x ^ ((x >> 4) & 15): consecutive lanes reach
-      // distinct banks also where the register bits are the low tile bits.
-      // Linear, so it splits into a per-lane and a per-register term.
-      auto swz = [](uint32_t x) { return x ^ ((x >> 4) & 15u); };
       uint32_t w[NR], r[NR];
-      const uint32_t tw = swz(st.tl);
+      const uint32_t w0 = g_slot(st.tl);
 #pragma unroll
-      for (int j = 0; j < NR; ++j) w[j] = tw ^ swz(st.ri.at(j));
-      st = make_state<R, TB>(op.u.lay, tid);
-      const uint32_t tr = swz(st.tl);
+      for (int j = 0; j < NR; ++j) w[j] = g_slot(st.ri.at(j));
+      st.tl = g_thread<R>(op.u.lay, tid);
+      st.ri = reg_index<R>(op.u.lay);
+      const uint32_t r0 = g_slot(st.tl);
 #pragma unroll
-      for (int j = 0; j < NR; ++j) r[j] = tr ^ swz(st.ri.at(j));
-      __syncthreads();
-      g_exchange<T, NR, false>(a, xch, w, r);
-      __syncthreads();
-      g_exchange<T, NR, true>(a, xch, w, r);
+      for (int j = 0; j < NR; ++j) r[j] = g_slot(st.ri.at(j));
+      g_exchange<T, NR>(a, xch, w0, w, r0, r);
       continue;
     }
     if ((code & 0xF0u) == C_CXR) {
       switch (code) {
-#define G_CASE(c, t)     \
-  case C_CXR + 4 * c + t: \
-    if constexpr (c < R && t < R) g_cxr<T, NR, c < R ? c : 0, t < R ? t : 1>(a); \
-    break;
+#define G_CASE(c, t) \
+  case C_CXR + 4 * c + t: g_cxr<T, NR, c, t>(a); break;
         G_CASE(0, 1) G_CASE(0, 2) G_CASE(0, 3) G_CASE(1, 0) G_CASE(1, 2) G_CASE(1, 3)
         G_CASE(2, 0) G_CASE(2, 1) G_CASE(2, 3) G_CASE(3, 0) G_CASE(3, 1) G_CASE(3, 2)
 #undef G_CASE
@@ -327,17 +433,16 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
       case C_X + 0: g_x<T, NR, 0>(a); break;
       case C_X + 1: g_x<T, NR, 1>(a); break;
       case C_X + 2: g_x<T, NR, 2>(a); break;
-      case C_X + 3: g_x<T, NR, R - 1>(a); break;
-#define G_CASE(b) \
-  case C_XC + b: if constexpr (b < R) g_xc<T, NR, b < R ? b : 0, false>(a, tlc, st.ri, cl, cvl); break;       \
-  case C_Y + b: if constexpr (b < R) g_xc<T, NR, b < R ? b : 0, true>(a, tlc, st.ri, cl, cvl); break;         \
-  case C_U1C + b:                                                                                              \
-    if constexpr (b < R) {                                                                                     \
-      cx<T> m[4];                                                                                              \
-      g_load_u1(op, false, m);                                                                                 \
-      g_u1c<T, NR, b < R ? b : 0>(a, tlc, st.ri, cl, cvl, m);                                                  \
-    }                                                                                                          \
-    break;
+      case C_X + 3: g_x<T, NR, 3>(a); break;
+#define G_CASE(b)                                                                        \
+  case C_XC + b: g_xc<T, NR, b, false>(a, tlc, st.ri, cl, cvl); break;                   \
+  case C_Y + b: g_xc<T, NR, b, true>(a, tlc, st.ri, cl, cvl); break;                     \
+  case C_U1C + b: {                                                                      \
+    cx<T> m[4];                                                                          \
+    g_load_u1(op, false, m);                                                             \
+    g_u1c<T, NR, b>(a, tlc, st.ri, cl, cvl, m);                                          \
+    break;                                                                               \
+  }
       G_CASE(0) G_CASE(1) G_CASE(2) G_CASE(3)
 #undef G_CASE
       case C_PHASE: {
@@ -413,11 +518,12 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
 }
 
 template <typename T, int B, int R>
-__global__ __launch_bounds__(1 << (B - R)) __attribute__((amdgpu_waves_per_eu(4))) void k_gate_pass(
+__global__ __launch_bounds__(1 << (B - R))
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 5))) void k_gate_pass(
     cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd, const ROp<T> *__restrict__ rops,
     const TileOp *__restrict__ tops, const cx<double> *__restrict__ pool, uint64_t state_stride, uint32_t pd_stride,
     uint32_t tile_log) {
-  __shared__ T xch[1 << B];
+  __shared__ __align__(16) char xch[8 << B];
   const StateTile st = state_tile(tile_log);
   gate_tile<T, B, R>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool, st.t, xch,
                      reinterpret_cast<cx<double> *>(aerhip_dyn_lds));

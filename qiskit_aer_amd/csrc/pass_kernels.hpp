@@ -32,6 +32,7 @@ constexpr uint32_t kGateRegBits = 4;
       const TileOp *__restrict__, const cx<double> *__restrict__, uint64_t, uint32_t, uint32_t);
 
 AERHIP_GATE_PASS(extern, double, kGateTileC128, kGateRegBits)
+AERHIP_GATE_PASS(extern, float, kTileBitsC64, kGateRegBits)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, false)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, true)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_GATES, false)
