@@ -1455,20 +1455,18 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         if (single) {
           // rounded here: the kernel reads the entries as scalars, where
           // rounding them would cost it a conversion and a register each; a
-          // gate pass reads rows of the real 8x8 form, for MFMA
+          // gate pass reads the real 8x8 form, for MFMA
           cx<float> m[16];
           for (int e = 0; e < 16; ++e)
             m[e] = to_t<float>(mk<double>(pool[r.extra + e].real(), pool[r.extra + e].imag()));
           r.extra = static_cast<uint32_t>(pool.size());
           if (gate) {
-            float rows[64];
-            for (int i = 0; i < 4; ++i)
-              for (int k = 0; k < 4; ++k) {
-                const cx<float> v = m[i + 4 * k];
-                rows[16 * i + 2 * k] = v.x;
-                rows[16 * i + 2 * k + 1] = -v.y;
-                rows[16 * i + 8 + 2 * k] = v.y;
-                rows[16 * i + 8 + 2 * k + 1] = v.x;
+            float rows[64];  // entry (4h + i, k) of the real form at 4 (8h + k) + i
+            for (int i = 0; i < 8; ++i)
+              for (int k = 0; k < 8; ++k) {
+                const cx<float> v = m[i / 2 + 4 * (k / 2)];
+                const float e = (i ^ k) & 1 ? (i & 1 ? v.y : -v.y) : v.x;
+                rows[4 * (8 * (i / 4) + k) + i % 4] = e;
               }
             cd rec[16];
             std::memcpy(rec, rows, sizeof(rec));

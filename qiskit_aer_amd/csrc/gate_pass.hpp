@@ -91,21 +91,28 @@ __device__ __forceinline__ void g_u1b(Amps<T, NR> &a, const cx<T> (&u)[4]) {
   for (int k = 0; k < NR / 2; ++k) g_u1(a.v[pair_lo<b>(k)], a.v[pair_lo<b>(k) | (1 << b)], u);
 }
 
-// complex64 2x2 gate with MFMA (see q_u1_mfma): `A` is row lane % 4 of the real
-// 4x4 form.
+// complex64 2x2 gate with MFMA: v_mfma_f32_4x4x1 runs 16 blocks of 4 x 4 (lanes
+// 4k .. 4k + 3 form block k), of which the broadcast controls (16 blocks, block
+// k) let all take column k of the matrix: lane 4k + i of the one register `A`
+// holds entry (i, k) of the real 4x4 form.  Four accumulating issues leave the
+// pair's four output components in the lane's accumulator.
 template <int NR, int b>
-__device__ __forceinline__ void g_u1b_mfma(Amps<float, NR> &a, f32x4 A) {
+__device__ __forceinline__ void g_u1b_mfma(Amps<float, NR> &a, float A) {
+  constexpr f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   constexpr int G = 4;  // pairs whose accumulation chains interleave
 #pragma unroll
   for (int g = 0; g < NR / 2; g += G) {
     f32x4 acc[G];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].x, zero, 4, 0, 0);
 #pragma unroll
-      for (int p = 0; p < G; ++p) {
-        const cx<float> v = a.v[pair_lo<b>(g + p) | (k < 2 ? 0 : 1 << b)];
-        acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[k], k & 1 ? v.y : v.x, k ? acc[p] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-      }
+    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].y, acc[p], 4, 1, 0);
+#pragma unroll
+    for (int p = 0; p < G; ++p)
+      acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p) | (1 << b)].x, acc[p], 4, 2, 0);
+#pragma unroll
+    for (int p = 0; p < G; ++p)
+      acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p) | (1 << b)].y, acc[p], 4, 3, 0);
 #pragma unroll
     for (int p = 0; p < G; ++p) {
       a.v[pair_lo<b>(g + p)] = mk<float>(acc[p][0], acc[p][1]);
@@ -115,25 +122,27 @@ __device__ __forceinline__ void g_u1b_mfma(Amps<float, NR> &a, f32x4 A) {
 }
 
 // complex64 4x4 gate with MFMA: the real 8x8 form in two halves of four rows,
-// each a chain of eight v_mfma_f32_4x4x1f32 per group of four amplitudes, at
-// twice the rate of FMAs on the vector ALU.  A[0..1]: row lane % 4 of the first
-// half (amplitudes 0 and 1 of the group), A[2..3]: of the second.
+// each a chain of eight issues per group of four amplitudes, at twice the rate
+// of FMAs on the vector ALU.  Lane 4 (8h + k) + i of `A` holds entry (4h + i, k).
+template <int b0, int b1, int NR, int k = 0>
+__device__ __forceinline__ void g_u2_chain(const Amps<float, NR> &a, int g, float A, f32x4 (&acc)[2][2]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int j = pair_lo<b1>(pair_lo<b0>(g + q)) | (k & 2 ? 1 << b0 : 0) | (k & 4 ? 1 << b1 : 0);
+    const float v = k & 1 ? a.v[j].y : a.v[j].x;
+    acc[q][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, v, acc[q][0], 4, k, 0);
+    acc[q][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, v, acc[q][1], 4, 8 + k, 0);
+  }
+  if constexpr (k < 7) g_u2_chain<b0, b1, NR, k + 1>(a, g, A, acc);
+}
+
 template <int NR, int b0, int b1>
-__device__ __forceinline__ void g_u2_mfma(Amps<float, NR> &a, const f32x4 (&A)[4]) {
+__device__ __forceinline__ void g_u2_mfma(Amps<float, NR> &a, float A) {
+  constexpr f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int g = 0; g < NR / 4; g += 2) {  // two groups: four chains interleave
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int j = pair_lo<b1>(pair_lo<b0>(g + q)) | (k & 2 ? 1 << b0 : 0) | (k & 4 ? 1 << b1 : 0);
-        const float v = k & 1 ? a.v[j].y : a.v[j].x;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          acc[q][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[2 * h + (k >> 2)][k & 3], v,
-                                                         k ? acc[q][h] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-      }
+    f32x4 acc[2][2] = {{zero, zero}, {zero, zero}};
+    g_u2_chain<b0, b1, NR>(a, g, A, acc);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const int j = pair_lo<b1>(pair_lo<b0>(g + q));
@@ -348,8 +357,8 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
     if ((code & 0xF0u) == C_U1) {
       const bool fx = tile_ok && (op.kind & ~F_ALL) == Q_U1X;
       if constexpr (sizeof(T) == 4) {
-        const f32x4 row = *reinterpret_cast<const f32x4 *>(op.u.mr + 4 * (tid & 3u));
-        const f32x4 A = fx ? f32x4{row.z, row.w, row.x, row.y} : row;  // U X: the columns change places
+        // U X: the columns of the pair's two amplitudes change places
+        const float A = op.u.mr[4 * (tid & 3u) + (((tid >> 2) & 3u) ^ (fx ? 2u : 0u))];
         switch (code) {
           case C_U1 + 0: g_u1b_mfma<NR, 0>(a, A); break;
           case C_U1 + 1: g_u1b_mfma<NR, 1>(a, A); break;
@@ -371,8 +380,7 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
     const uint32_t cl = op.cl, cvl = op.cvl;
     if ((code & 0xF0u) == C_U2) {
       if constexpr (sizeof(T) == 4) {
-        const f32x4 *rows = reinterpret_cast<const f32x4 *>(pool + op.extra) + 2 * (tid & 3u);
-        const f32x4 A[4] = {rows[0], rows[1], rows[8], rows[9]};
+        const float A = reinterpret_cast<const float *>(pool + op.extra)[tid & 63u];
         switch (code) {
           case C_U2 + pair_index(0, 1): g_u2_mfma<NR, 0, 1>(a, A); break;
           case C_U2 + pair_index(0, 2): g_u2_mfma<NR, 0, 2>(a, A); break;

@@ -1,4 +1,4 @@
-"""Gate passes (tiles of 2^12 complex128 amplitudes, from 21 qubits on): every
+"""Gate passes (tiles of 2^12 amplitudes; complex128 from 21 qubits on): every
 op they run, on qubits inside and outside the tile, next to ops they leave to
 the other passes, against the oracle; and the same gates just below 21 qubits."""
 import numpy as np
@@ -94,3 +94,36 @@ def test_gradients_use_them():
     assert np.max(np.abs(e - est.energy_one_by_one(rows))) < 1e-11
     which = [0, npar // 2, npar - 1]
     assert np.max(np.abs(est.parameter_shift(rows[:1], which)[0] - g[0, which])) < 1e-9
+
+
+@pytest.mark.parametrize("width", [0, 2, 3])
+@pytest.mark.parametrize("n,seed", [(12, 5), (13, 6), (17, 7), (20, 8)])
+def test_complex64(n, seed, width):
+    """2x2 and 4x4 gates on the matrix cores, from one tile (12 qubits) on."""
+    print(f"case: complex64 gate pass n={n} seed={seed} width={width}", flush=True)
+    c = mixture(n, seed, 200)
+    e = QubitVector(n, "single")
+    e.set_block_fusion(width)
+    e.initialize()
+    e.apply_ops(c)
+    _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+    # a gate is unitary and rounds each amplitude to a few 2^-24 of its group's
+    # norm: at most 4 * 2^-24 a gate in the norm of the state
+    assert np.linalg.norm(e.copy_to_vector() - want) < (200 + n) * 4 * 2.0**-24
+
+
+def test_complex64_pairs():
+    """A 4x4 gate on every ordered pair of a tile's qubits, then all of a register."""
+    n = 13
+    rng = np.random.default_rng(9)
+    print("case: complex64 4x4 gates on every pair", flush=True)
+    c = circuits.Circuit(n)
+    for a in range(n):
+        for b in range(n):
+            if a != b:
+                c.unitary(D.random_unitary(4, rng), [a, b])
+    e = QubitVector(n, "single")
+    e.initialize()
+    e.apply_ops(c)
+    _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+    assert np.linalg.norm(e.copy_to_vector() - want) < n * (n - 1) * 8 * 2.0**-24
