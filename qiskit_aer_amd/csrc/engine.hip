@@ -672,7 +672,7 @@ struct RItem {
 constexpr uint32_t kProbeSentinel = 1u << 31;
 constexpr size_t kMaxMoves = 4;  // register moves that still cost less than a layout change
 
-RItem classify_item(const TileOp &op, uint32_t R) {
+RItem classify_item(const TileOp &op, uint32_t R, bool gate) {
   RItem it;
   it.op = op;
   it.cls = 2;
@@ -692,7 +692,14 @@ RItem classify_item(const TileOp &op, uint32_t R) {
       break;
     case K_DENSE:
       it.touch |= pos;
-      if (op.k == 2 && R >= 2) {
+      if ((op.k == 2 && R >= 2) || (op.k == 3 && gate)) {
+        it.cls = 0;
+        it.need = pos;
+      }
+      break;
+    case K_MCSWAP:
+      it.touch |= pos;
+      if (gate) {
         it.cls = 0;
         it.need = pos;
       }
@@ -947,7 +954,7 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
 // program inside a concatenated one.
 void rebase_rop(ROp<double> &r, uint32_t pool_base, uint32_t op_base) {
   const uint32_t kk = r.kind & ~F_ALL;
-  if (kk == Q_U2 || kk == Q_DIAGF || kk == Q_PROBE) r.extra += pool_base;
+  if (kk == Q_U2 || kk == Q_U3 || kk == Q_DIAGF || kk == Q_DIAGK || kk == Q_PROBE) r.extra += pool_base;
   else if (kk == Q_DIAG || kk == Q_LDS) r.extra += op_base;
   else if ((kk == Q_LOAD || kk == Q_FILL) && r.a) r.b += pool_base;
 }
@@ -1009,6 +1016,26 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
         case Q_U2: case Q_CXR:
           if (r.a >= R || r.b >= R || r.a == r.b) fail("register bits of a 2-qubit gate");
           break;
+        case Q_SWAP:
+          if (r.a >= r.b || r.b >= R) fail("register bits of a swap");
+          break;
+        case Q_U3:
+          if (R != 4 || r.a >= R || r.extra + 64ull > pool.size()) fail("8x8 gate");
+          break;
+        case Q_DIAGK: {
+          const uint32_t k = r.a & 0xFFu, ng = r.a >> 8;
+          if (k < 1 || k > 8 || ng > 16 || r.extra + (1ull << k) + 4 > pool.size()) fail("diagonal table");
+          for (uint32_t d = 0; d < 8; ++d) {
+            const uint32_t tb = r.u.fq[d], q = r.u.fq[8 + d];
+            if (tb != 0xFF && (d >= k || tb >= B || (regmask >> tb) & 1u)) fail("lane bit of a diagonal");
+            if (q != 0xFF && (d >= k || q >= 64 || tb != 0xFF)) fail("fixed qubit of a diagonal");
+          }
+          uint32_t words[16];
+          std::memcpy(words, pool.data() + r.extra + (1ull << k), sizeof(words));
+          for (uint32_t g = 0; g < ng; ++g)
+            if (words[g] >> (16 + k)) fail("register part of a diagonal");
+          break;
+        }
         case Q_D1: if (r.a >= B) fail("diagonal bit"); break;
         case Q_DIAG: if (r.extra >= ntops) fail("diagonal index"); break;
         case Q_PROBE:
@@ -1056,7 +1083,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   std::vector<uint32_t> rem_op;    // ... and which op of `in` each is
   rem.reserve(in.size());
   for (size_t i = 0; i < in.size(); ++i) {
-    const RItem it = classify_item(in[i], R);
+    const RItem it = classify_item(in[i], R, gate);
     rem.push_back(RMask{it.need, it.touch, static_cast<int8_t>(it.cls), static_cast<int8_t>(it.cat)});
     rem_op.push_back(static_cast<uint32_t>(i));
   }
@@ -1435,7 +1462,41 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         r.a = t;
         break;
       }
+      case K_MCSWAP: {
+        const uint32_t b0 = regidx(rs, op.pos[0]), b1 = regidx(rs, op.pos[1]);
+        materialize((1u << b0) | (1u << b1) | reg_bits(op.cl));
+        r.kind = Q_SWAP;
+        r.a = std::min(b0, b1);
+        r.b = std::max(b0, b1);
+        break;
+      }
       case K_DENSE: {
+        if (op.k == 3) {
+          // rows of the matrix with ascending register bits; complex64: of its
+          // real 16x16 form, the four MFMA operands of g_u3_mfma
+          uint32_t bits = 0, at[3];
+          for (uint32_t j = 0; j < 3; ++j) bits |= 1u << regidx(rs, op.pos[j]);
+          for (uint32_t j = 0; j < 3; ++j)
+            at[j] = static_cast<uint32_t>(__builtin_popcount(bits & ((1u << regidx(rs, op.pos[j])) - 1u)));
+          auto perm = [&](uint32_t i) { return (i & 1u) << at[0] | (i >> 1 & 1u) << at[1] | (i >> 2) << at[2]; };
+          materialize(bits);
+          r.kind = Q_U3;
+          r.a = static_cast<uint32_t>(__builtin_ctz(~bits));
+          r.extra = static_cast<uint32_t>(pool.size());
+          cd m[64];
+          for (uint32_t e = 0; e < 64; ++e) m[8 * perm(e & 7u) + perm(e >> 3)] = pool[op.off + e];
+          if (single) {
+            float rec[256];
+            for (uint32_t i = 0; i < 16; ++i)
+              for (uint32_t k = 0; k < 16; ++k) {
+                const cx<float> v = to_t<float>(mk<double>(m[8 * (i / 2) + k / 2].real(), m[8 * (i / 2) + k / 2].imag()));
+                rec[64 * (i / 4) + 4 * k + i % 4] = (i ^ k) & 1u ? (i & 1u ? v.y : -v.y) : v.x;
+              }
+            std::memcpy(m, rec, sizeof(m));
+          }
+          pool.insert(pool.end(), m, m + 64);
+          break;
+        }
         const uint32_t b0 = regidx(rs, op.pos[0]), b1 = regidx(rs, op.pos[1]);
         materialize((1u << b0) | (1u << b1) | reg_bits(op.cl));
         need_identity(rs, {b0, b1});
@@ -1481,7 +1542,33 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       }
       case K_DIAG:
         materialize(pend);
-        if (op.k == 1 && op.pos[0] != kNotLocal) {
+        if (gate && (op.k > 1 || op.pos[0] == kNotLocal || op.cl || op.cg)) {
+          r.kind = Q_DIAGK;
+          std::memset(r.u.fq, 0xFF, sizeof(r.u.fq));
+          for (uint32_t d = 0; d < op.k; ++d) {
+            if (op.pos[d] == kNotLocal) r.u.fq[8 + d] = static_cast<uint8_t>(op.gpos[d]);
+            else if (!((cur_rs >> op.pos[d]) & 1u)) r.u.fq[d] = static_cast<uint8_t>(op.pos[d]);
+          }
+          uint32_t groups[16] = {}, ng = 0;
+          for (uint32_t j = 0; j < (1u << R); ++j) {
+            const uint32_t tb = reg_tile_bits(j);
+            if ((tb & op.cl & cur_rs) != (op.cvl & op.cl & cur_rs)) continue;
+            uint32_t part = 0;
+            for (uint32_t d = 0; d < op.k; ++d)
+              if (op.pos[d] != kNotLocal) part |= ((tb >> op.pos[d]) & 1u) << d;
+            uint32_t g = 0;
+            while (g < ng && groups[g] >> 16 != part) ++g;
+            if (g == ng) groups[ng++] = part << 16;
+            groups[g] |= 1u << j;
+          }
+          r.a = op.k | ng << 8;
+          std::vector<cd> tab(pool.begin() + op.off, pool.begin() + op.off + (1u << op.k));
+          r.extra = static_cast<uint32_t>(pool.size());
+          pool.insert(pool.end(), tab.begin(), tab.end());
+          cd rec[4];
+          std::memcpy(rec, groups, sizeof(rec));
+          pool.insert(pool.end(), rec, rec + 4);
+        } else if (op.k == 1 && op.pos[0] != kNotLocal) {
           r.kind = Q_D1;
           r.a = op.pos[0];
           r.b = 0;  // registers whose target bit is 1 (a register target)
@@ -1731,9 +1818,9 @@ uint32_t Engine::gate_tile_bits() const {
 // Whether the gate pass runs a primitive.
 bool Engine::gate_prim(const Prim &p) const {
   switch (p.kind) {
-    case K_DENSE1: case K_MCX: case K_MCY: case K_MCPHASE: return true;
-    case K_DENSE: return p.q.size() == 2 && p.ctrl.empty();
-    case K_DIAG: return p.q.size() == 1 && p.ctrl.empty();
+    case K_DENSE1: case K_MCX: case K_MCY: case K_MCSWAP: case K_MCPHASE: return true;
+    case K_DENSE: return (p.q.size() == 2 || p.q.size() == 3) && p.ctrl.empty();
+    case K_DIAG: return p.q.size() <= 8;
     default: return false;
   }
 }

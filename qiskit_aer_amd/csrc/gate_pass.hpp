@@ -37,16 +37,13 @@ enum GateCode : uint32_t {
   C_D1 = 0x61,
   C_DIAGF = 0x62,
   C_RELAYOUT = 0x63,
+  C_DIAGK = 0x64,
+  C_SWAP = 0x70,     // + index of the register bits b0 < b1
+  C_U3 = 0x78,       // + b: 8x8 gate on the register bits but b
 };
 
 // Index of a pair of register bits b0 < b1.
 constexpr uint32_t pair_index(uint32_t b0, uint32_t b1) { return b1 * (b1 - 1) / 2 + b0; }
-
-// Whether a gate pass runs this op.
-constexpr bool gate_kind(uint32_t kind) {
-  const int v = variant_of(kind);
-  return v == V_LEAN || v == V_GATES;
-}
 
 // The code of a register op; U2 ops come with a < b.
 inline uint32_t gate_code(const ROp<double> &r) {
@@ -60,6 +57,9 @@ inline uint32_t gate_code(const ROp<double> &r) {
     case Q_PHASE: return C_PHASE;
     case Q_D1: return C_D1;
     case Q_DIAGF: return C_DIAGF;
+    case Q_DIAGK: return C_DIAGK;
+    case Q_SWAP: return C_SWAP + pair_index(r.a, r.b);
+    case Q_U3: return C_U3 + r.a;
     case Q_RELAYOUT: return C_RELAYOUT;
     default: return C_NOP;
   }
@@ -189,6 +189,78 @@ __device__ __forceinline__ void g_u2(Amps<T, NR> &a, const cx<T> (&m)[16]) {
   }
 }
 
+// Register p (0 or 1) of those with the bits other than `omit` clear, and the
+// offset of the group's amplitude i from it.
+template <int omit>
+constexpr int u3_base(int p) { return p << omit; }
+template <int omit>
+constexpr int u3_off(int i) { return (i & ((1 << omit) - 1)) | (i >> omit) << (omit + 1); }
+
+// 8x8 gate on the register bits but `omit`, rows of m: as g_u2, a row of the
+// matrix in scalar registers at a time.
+template <typename T, int NR, int omit>
+__device__ __forceinline__ void g_u3(Amps<T, NR> &a, const cx<T> *__restrict__ m) {
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    T tx[8], ty[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      uint64_t at = 8 * r;
+      asm volatile("" : "+s"(at));  // keeps the loads of the rows apart
+      const cx<T> *mr = m + at;
+      cx<T> row[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) row[c] = mr[c];
+      const cx<T> v = a.v[u3_base<omit>(p) | u3_off<omit>(r)];
+      tx[r] = row[r].y * v.y;
+      ty[r] = -row[r].y * v.x;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        if (c == r) continue;
+        const cx<T> w = a.v[u3_base<omit>(p) | u3_off<omit>(c)];
+        tx[r] = fma_t(-row[c].x, w.x, tx[r]);
+        ty[r] = fma_t(-row[c].x, w.y, ty[r]);
+        tx[r] = fma_t(row[c].y, w.y, tx[r]);
+        ty[r] = fma_t(-row[c].y, w.x, ty[r]);
+      }
+    }
+    uint64_t at = 0;
+    asm volatile("" : "+s"(at));
+    const cx<T> *md = m + at;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      cx<T> &v = a.v[u3_base<omit>(p) | u3_off<omit>(r)];
+      const T d = md[9 * r].x;
+      v.x = fma_t(d, v.x, -tx[r]);
+      v.y = fma_t(d, v.y, -ty[r]);
+    }
+  }
+}
+
+// complex64 8x8 gate with MFMA: the real 16x16 form in four quarters of four
+// rows, quarter h from lane 4k + i of A[h] = entry (4h + i, k).
+template <int omit, int NR, int k = 0>
+__device__ __forceinline__ void g_u3_chain(const Amps<float, NR> &a, int p, const float (&A)[4], f32x4 (&acc)[4]) {
+  const cx<float> w = a.v[u3_base<omit>(p) | u3_off<omit>(k >> 1)];
+  const float v = k & 1 ? w.y : w.x;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) acc[h] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[h], v, acc[h], 4, k, 0);
+  if constexpr (k < 15) g_u3_chain<omit, NR, k + 1>(a, p, A, acc);
+}
+
+template <int NR, int omit>
+__device__ __forceinline__ void g_u3_mfma(Amps<float, NR> &a, const float (&A)[4]) {
+  constexpr f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    f32x4 acc[4] = {zero, zero, zero, zero};
+    g_u3_chain<omit, NR>(a, p, A, acc);
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      a.v[u3_base<omit>(p) | u3_off<omit>(r)] = mk<float>(acc[r >> 1][2 * (r & 1)], acc[r >> 1][2 * (r & 1) + 1]);
+  }
+}
+
 // Exchanges two components.  Written out, because as a permutation of values it
 // would tie the registers of the op loop's paths in knots: the compiler then
 // keeps a second copy of the amplitudes and moves between the two at every op.
@@ -230,6 +302,18 @@ __device__ __forceinline__ void g_xc(Amps<T, NR> &a, uint32_t tlc, const RegIdx<
     const cx<T> p = a.v[j], q = a.v[jj];
     a.v[j] = csel(on, isy ? mk<T>(q.y, -q.x) : q, p);
     a.v[jj] = csel(on, isy ? mk<T>(-p.y, p.x) : p, q);
+  }
+}
+
+template <typename T, int NR, int b0, int b1>
+__device__ __forceinline__ void g_swapc(Amps<T, NR> &a, uint32_t tlc, const RegIdx<NR> &ri, uint32_t cl, uint32_t cvl) {
+#pragma unroll
+  for (int k = 0; k < NR / 4; ++k) {
+    const int j = pair_lo<b1>(pair_lo<b0>(k)), lo = j | (1 << b0), hi = j | (1 << b1);
+    const bool on = (tlc | (ri.at(j) & cl)) == cvl;
+    const cx<T> p = a.v[lo], q = a.v[hi];
+    a.v[lo] = csel(on, q, p);
+    a.v[hi] = csel(on, p, q);
   }
 }
 
@@ -428,6 +512,27 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
       }
       continue;
     }
+    if ((code & 0xF8u) == C_U3) {
+      if constexpr (sizeof(T) == 4) {
+        const float *mp = reinterpret_cast<const float *>(pool + op.extra) + (tid & 63u);
+        const float A[4] = {mp[0], mp[64], mp[128], mp[192]};
+        switch (code) {
+          case C_U3 + 0: g_u3_mfma<NR, 0>(a, A); break;
+          case C_U3 + 1: g_u3_mfma<NR, 1>(a, A); break;
+          case C_U3 + 2: g_u3_mfma<NR, 2>(a, A); break;
+          case C_U3 + 3: g_u3_mfma<NR, 3>(a, A); break;
+        }
+      } else {
+        const cx<T> *mp = reinterpret_cast<const cx<T> *>(pool + op.extra);
+        switch (code) {
+          case C_U3 + 0: g_u3<T, NR, 0>(a, mp); break;
+          case C_U3 + 1: g_u3<T, NR, 1>(a, mp); break;
+          case C_U3 + 2: g_u3<T, NR, 2>(a, mp); break;
+          case C_U3 + 3: g_u3<T, NR, 3>(a, mp); break;
+        }
+      }
+      continue;
+    }
     if (!tile_ok) continue;  // controls fixed by the tile that do not hold
     const uint32_t tlc = st.tl & cl;
     const uint32_t rb = op.b;
@@ -481,6 +586,35 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
           const cx<T> d = csel(((st.tl >> t) & 1u) != 0, d1, d0);
 #pragma unroll
           for (int j = 0; j < NR; ++j) g_mul(a.v[j], d);
+        }
+        break;
+      }
+#define G_CASE(b0, b1) \
+  case C_SWAP + pair_index(b0, b1): g_swapc<T, NR, b0, b1>(a, tlc, st.ri, cl, cvl); break;
+      G_CASE(0, 1) G_CASE(0, 2) G_CASE(1, 2) G_CASE(0, 3) G_CASE(1, 3) G_CASE(2, 3)
+#undef G_CASE
+      case C_DIAGK: {
+        // one entry per lane and group of registers that share their part of the index
+        const cx<double> *tab = pool + op.extra;
+        const uint32_t *w = reinterpret_cast<const uint32_t *>(op.u.fq);
+        uint32_t idx = 0;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+          const uint32_t tb = byte_at(w, d), q = byte_at(w, 8 + d);
+          if (tb < 32) idx |= ((st.tl >> tb) & 1u) << d;
+          if (q < 64) idx |= static_cast<uint32_t>((base >> q) & 1ull) << d;
+        }
+        const uint32_t ka = op.a;
+        const uint32_t *grp = reinterpret_cast<const uint32_t *>(tab + (1u << (ka & 0xFFu)));
+        for (uint32_t g = 0; g < ka >> 8; ++g) {
+          const uint32_t gr = grp[g];
+          const cx<T> f = csel(lane_ok, to_t<T>(tab[idx | (gr >> 16)]), one);
+#pragma unroll
+          for (int j = 0; j < NR; ++j)
+            if ((gr >> j) & 1u) {
+              asm volatile("");  // keeps the branch (no if-conversion into selects)
+              g_mul(a.v[j], f);
+            }
         }
         break;
       }

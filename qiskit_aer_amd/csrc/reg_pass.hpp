@@ -61,6 +61,14 @@ enum RegPassOpKind : uint32_t {
                     // qubits u.fq[4c .. 4c+3] (0xFF: unused); a >> 16 = slot + 1 of the
                     // phase's lane tables staged in LDS (0: none, read the tables)
   Q_CXR = 61,       // moves registers: those with bit a set change places across bit b
+  // gate passes only
+  Q_SWAP = 62,      // register bits a < b change places where (l & cl) == cvl
+  Q_U3 = 63,        // 8x8 matrix pool[extra..] on the register bits but a, the lowest as
+                    // matrix bit 0: rows of complex128, or (complex64) four MFMA operands
+  Q_DIAGK = 64,     // where (l & cl) == cvl: diagonal of a & 0xFF qubits, entries pool[extra..],
+                    // then per group of registers that share their part of the index a word
+                    // (index << 16 | registers), a >> 8 of them; u.fq[d] is the tile bit of
+                    // index bit d on lanes, u.fq[8 + d] its qubit where the tile fixes it
 };
 
 // Fused diagonals of a register phase: the factor over the qubits fixed by

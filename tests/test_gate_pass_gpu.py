@@ -127,3 +127,53 @@ def test_complex64_pairs():
     e.apply_ops(c)
     _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
     assert np.linalg.norm(e.copy_to_vector() - want) < n * (n - 1) * 8 * 2.0**-24
+
+
+def wide_mixture(n, seed, count):
+    """What needs three register bits, or none: 8x8 gates on every order of their
+    qubits, (controlled) swaps, diagonals of one to nine qubits with and without
+    controls, between 2x2 gates."""
+    rng = np.random.default_rng(seed)
+    c = circuits.Circuit(n)
+    for q in range(n):
+        c.gate("h", [q])
+    for _ in range(count):
+        lo = int(rng.integers(0, n - 8)) if rng.random() < 0.7 else 0
+        q = [int(x) for x in rng.choice(np.arange(lo, n if lo == 0 else lo + 9), 9, replace=False)]
+        k = int(rng.integers(9))
+        if k < 2:
+            c.unitary(D.random_unitary(8, rng), q[:3])
+        elif k == 2:
+            c.gate("swap", q[:2])
+        elif k == 3:
+            c.gate("cswap", q[:3])
+        elif k == 4:
+            w = int(rng.integers(1, 10))
+            c.diagonal(np.exp(1j * rng.uniform(-3, 3, 1 << w)), q[:w])
+        elif k == 5:
+            c.gate("rzz", q[:2], [float(rng.uniform(-3, 3))])
+        elif k == 6:
+            c.gate("crz", q[:2], [float(rng.uniform(-3, 3))])
+        elif k == 7:
+            c.gate("cx", q[:2])
+        else:
+            c.gate("u3", q[:1], list(rng.uniform(-3, 3, 3)))
+    return c
+
+
+@pytest.mark.parametrize("n,seed", [(21, 11), (22, 12)])
+def test_wide_ops(n, seed):
+    print(f"case: gate pass wide ops n={n} seed={seed}", flush=True)
+    assert run_both(wide_mixture(n, seed, 120), n) < 1e-12
+
+
+@pytest.mark.parametrize("n,seed", [(12, 13), (13, 14), (18, 15)])
+def test_wide_ops_complex64(n, seed):
+    print(f"case: complex64 gate pass wide ops n={n} seed={seed}", flush=True)
+    c = wide_mixture(n, seed, 120)
+    e = QubitVector(n, "single")
+    e.initialize()
+    e.apply_ops(c)
+    _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+    # as above; a component of an 8x8 gate is a sum of 16 rounded products
+    assert np.linalg.norm(e.copy_to_vector() - want) < (120 + n) * 16 * 2.0**-24
