@@ -1842,12 +1842,13 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t tmask, touch;
       uint32_t idx;
       bool probe, unitary, gate;
+      bool lds;  // a register pass spills the tile for it, a gate pass does not
     };
     std::vector<Pending> remaining;
     for (size_t i = seg_begin; i < seg_end; ++i) {
       const Prim &p = queue_[i];
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
-                                  gate_bits && gate_prim(p)});
+                                  gate_bits && gate_prim(p), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2)});
     }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
@@ -1857,7 +1858,9 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t active = 0;
       for (const Pending &p : remaining) active |= p.touch;
       // A gate pass takes only what its kernel runs.
+      bool lds = false;  // whether the last scan took an `lds` primitive
       auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
+        lds = false;
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
@@ -1871,6 +1874,7 @@ std::vector<PassPlan> Engine::plan() const {
           }
           if (fits) {
             ++count;
+            lds |= p.lds;
             if (take) take->prims.push_back(p.idx);
             continue;
           }
@@ -1890,32 +1894,43 @@ std::vector<PassPlan> Engine::plan() const {
       // on ties.
       // The other tile passes run every primitive; a gate pass is taken where
       // it holds more of them, or as many but more than a few: a pass of one
-      // gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.
-      uint64_t seed = lowmask;
-      uint32_t cap = nb;
-      bool gate = false;
-      size_t best = 0;
-      auto try_tile = [&](uint32_t c, bool g) {
+      // gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.  Where a
+      // register pass would spill the tile to LDS (swaps, 3-qubit gates), it
+      // has to hold twice as many: on 25 qubits it takes 0.73 ms, a gate pass
+      // 0.21 to 0.45.
+      struct Tile {
+        size_t count = 0;
+        uint64_t seed = 0;
+        bool lds = false;
+      };
+      auto best_tile = [&](uint32_t c, bool g) {
+        Tile t;
+        t.seed = lowmask;
         auto candidate = [&](uint64_t s0) {
           const size_t k = scan(c, g, s0, nullptr, nullptr);
-          if (k > best || (k == best && k > 4 && g && !gate)) {
-            best = k;
-            seed = s0;
-            cap = c;
-            gate = g;
-          }
+          if (k > t.count) t = Tile{k, s0, lds};
         };
         candidate(lowmask);
         const uint32_t w = c - low_bits_;
         if (n_ > c && w > 0)
           for (uint32_t a = 0; a + w <= n_; ++a) candidate(lowmask | (((1ull << w) - 1ull) << a));
+        return t;
       };
-      try_tile(nb, false);
-      if (gate_bits) try_tile(gate_bits, true);
+      Tile best = best_tile(nb, false);
+      uint32_t cap = nb;
+      bool gate = false;
+      if (gate_bits) {
+        const Tile t = best_tile(gate_bits, true);
+        gate = best.lds ? 2 * t.count >= best.count : t.count > best.count || (t.count == best.count && t.count > 4);
+        if (gate) {
+          best = t;
+          cap = gate_bits;
+        }
+      }
       PassPlan pp;
       pp.gate = gate;
       std::vector<Pending> rest;
-      scan(cap, gate, seed, &pp, &rest);
+      scan(cap, gate, best.seed, &pp, &rest);
       uint64_t s = pp.smask;
       // Complete the tile with the lowest free qubits (longer contiguous runs).
       for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < cap; ++q)
