@@ -1658,6 +1658,8 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         pr.pr = op.pr;
         pr.pi = op.pi;
         pr.slot = op.npairs;
+        for (uint32_t j = 0; j < (1u << R); ++j)
+          pr.neg |= (static_cast<uint32_t>(__builtin_popcount(reg_tile_bits(j) & op.zl)) & 1u) << j;
         pr.idx = nprobes++ % kProbeBatch;
         if (pr.idx == kProbeBatch - 1) pr.flush = kProbeBatch;
         cd rec[3];
@@ -1815,12 +1817,14 @@ uint32_t Engine::gate_tile_bits() const {
   return tile_bits_ == kTileBitsC64 && low_bits_ == 4 && reg_bits_ == 4 ? kTileBitsC64 : 0;
 }
 
-// Whether the gate pass runs a primitive.
-bool Engine::gate_prim(const Prim &p) const {
+// Whether the gate pass runs a primitive; `probes`: one of a segment with probes,
+// whose kernel has no scalar registers to spare for the rows of 8x8 gates.
+bool Engine::gate_prim(const Prim &p, bool probes) const {
   switch (p.kind) {
     case K_DENSE1: case K_MCX: case K_MCY: case K_MCSWAP: case K_MCPHASE: return true;
-    case K_DENSE: return (p.q.size() == 2 || p.q.size() == 3) && p.ctrl.empty();
+    case K_DENSE: return (p.q.size() == 2 || (p.q.size() == 3 && !probes)) && p.ctrl.empty();
     case K_DIAG: return p.q.size() <= 8;
+    case K_PROBE: return !p.solo && __builtin_popcountll(p.xmask) <= static_cast<int>(kGateRegBits);
     default: return false;
   }
 }
@@ -1845,10 +1849,12 @@ std::vector<PassPlan> Engine::plan() const {
       bool lds;  // a register pass spills the tile for it, a gate pass does not
     };
     std::vector<Pending> remaining;
+    bool probes = false;
+    for (size_t i = seg_begin; i < seg_end; ++i) probes |= queue_[i].kind == K_PROBE;
     for (size_t i = seg_begin; i < seg_end; ++i) {
       const Prim &p = queue_[i];
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
-                                  gate_bits && gate_prim(p), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2)});
+                                  gate_bits && gate_prim(p, probes), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2)});
     }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
@@ -2457,10 +2463,12 @@ struct DeviceProgram {
 struct PassKernel {
   int variant = V_LEAN;
   bool wide = true, diag = false;
+  bool probes = false;  // a gate pass with probes
   void add(const PassKernel &o) {  // one kernel for several states' programs
     variant |= o.variant;
     wide = wide && o.wide;
     diag = diag || o.diag;
+    probes = probes || o.probes;
   }
 };
 
@@ -2519,17 +2527,18 @@ void launch_pass(int prec, uint32_t reg_bits, uint32_t n, uint32_t tile_bits, co
     }
   } else if (pd.kind == 5) {
     const uint32_t tl = pd.ncomp;
-    const size_t dyn = pk.diag ? kDiagLdsBytes : 0;
+    auto go = [&](auto kernel, auto *s, auto *ro) {
+      kernel<<<grid_of(tl), 1 << (kGateTileC128 - kGateRegBits), pk.diag ? kDiagLdsBytes : 0, stream>>>(
+          s, dpd, ro, dp.pool, dp.probes, state_stride, pd_stride, tl, pps);
+    };
     if (prec == AERHIP_PRECISION_DOUBLE)
-      k_gate_pass<double, kGateTileC128, kGateRegBits>
-          <<<grid_of(tl), 1 << (kGateTileC128 - kGateRegBits), dyn, stream>>>(
-              static_cast<cx<double> *>(sv), dpd, static_cast<const ROp<double> *>(dp.rops), dp.ops, dp.pool,
-              state_stride, pd_stride, tl);
+      go(pk.probes ? k_gate_pass<double, kGateTileC128, kGateRegBits, true>
+                   : k_gate_pass<double, kGateTileC128, kGateRegBits, false>,
+         static_cast<cx<double> *>(sv), static_cast<const ROp<double> *>(dp.rops));
     else
-      k_gate_pass<float, kTileBitsC64, kGateRegBits>
-          <<<grid_of(tl), 1 << (kTileBitsC64 - kGateRegBits), dyn, stream>>>(
-              static_cast<cx<float> *>(sv), dpd, static_cast<const ROp<float> *>(dp.rops), dp.ops, dp.pool,
-              state_stride, pd_stride, tl);
+      go(pk.probes ? k_gate_pass<float, kTileBitsC64, kGateRegBits, true>
+                   : k_gate_pass<float, kTileBitsC64, kGateRegBits, false>,
+         static_cast<cx<float> *>(sv), static_cast<const ROp<float> *>(dp.rops));
   } else if (pd.kind == 3) {
     // probes over the whole state, one workgroup per tile-sized slice
     const uint32_t tl = n - tile_bits;
@@ -2594,6 +2603,7 @@ PassKernel pass_kernel(const PassDesc &pd, const std::vector<ROp<double>> &rops)
     const ROp<double> &r = rops[pd.op_begin + i];
     k.variant |= variant_of(r.kind);
     const uint32_t kk = r.kind & ~F_ALL;
+    k.probes = k.probes || kk == Q_PROBE;
     k.diag = k.diag || ((kk == Q_LOAD || kk == Q_FILL) && r.a != 0);
   }
   return k;
@@ -2652,8 +2662,8 @@ void Engine::flush() {
   const TileOp *dops = reinterpret_cast<const TileOp *>(d + ops_off);
   const void *drops = d + rops_off;
   const cx<double> *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
-  // Probe partials: one double per (probe, tile); every tile pass has
-  // 2^(n - tile_bits) tiles.
+  // Probe partials: one double per (probe, tile); tile passes have
+  // 2^(n - tile_bits) tiles, and gate passes on larger ones fill as many.
   double *dprobes = nullptr;
   const uint64_t ntiles = 1ull << (n_ - tile_bits_);
   if (nprobes) {

@@ -173,7 +173,7 @@ class Engine {
   void apply_diagonal_1(uint32_t q, const cd *diag);
   std::vector<PassPlan> plan() const;
   uint32_t gate_tile_bits() const;
-  bool gate_prim(const Prim &p) const;
+  bool gate_prim(const Prim &p, bool probes) const;
   std::vector<PassPlan> gather_sweeps(std::vector<PassPlan> plans) const;
   std::vector<Prim> fuse_blocks(const std::vector<Prim> &in);
   std::vector<Prim> merge_swap_layers(const std::vector<Prim> &in) const;

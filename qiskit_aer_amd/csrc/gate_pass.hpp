@@ -38,6 +38,7 @@ enum GateCode : uint32_t {
   C_DIAGF = 0x62,
   C_RELAYOUT = 0x63,
   C_DIAGK = 0x64,
+  C_PROBE = 0x65,    // a run of probes
   C_SWAP = 0x70,     // + index of the register bits b0 < b1
   C_U3 = 0x78,       // + b: 8x8 gate on the register bits but b
 };
@@ -58,6 +59,7 @@ inline uint32_t gate_code(const ROp<double> &r) {
     case Q_D1: return C_D1;
     case Q_DIAGF: return C_DIAGF;
     case Q_DIAGK: return C_DIAGK;
+    case Q_PROBE: return C_PROBE;
     case Q_SWAP: return C_SWAP + pair_index(r.a, r.b);
     case Q_U3: return C_U3 + r.a;
     case Q_RELAYOUT: return C_RELAYOUT;
@@ -392,11 +394,25 @@ __device__ __forceinline__ void g_exchange(Amps<T, NR> &a, char *xch, uint32_t w
   }
 }
 
-template <typename T, int B, int R>
+// Where a gate tile's share of a probe goes: the partials hold one entry per
+// 2^(B - SPLIT) amplitudes, as the other passes write them; the tile's first
+// takes its sum and the others zero.
+template <int SPLIT>
+struct GateSink {
+  double *p;
+  uint64_t tile, ntiles;
+  __device__ __forceinline__ void put(uint32_t slot, double v) const {
+    double *e = p + ((static_cast<uint64_t>(slot) * ntiles + tile) << SPLIT);
+    e[0] = v;
+    if constexpr (SPLIT) e[1] = 0.0;
+  }
+};
+
+template <typename T, int B, int R, bool PROBES, typename Sink>
 __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd,
-                                          const ROp<T> *__restrict__ rops, const TileOp *__restrict__ tops,
-                                          const cx<double> *__restrict__ pool, uint64_t tile_id, char *xch,
-                                          cx<double> *dlt) {
+                                          const ROp<T> *__restrict__ rops, const cx<double> *__restrict__ pool,
+                                          uint64_t tile_id, char *xch, cx<double> *dlt, double *red,
+                                          const Sink &sink) {
   static_assert(R == 4, "the op codes name four register bits");
   constexpr int TB = B - R, NT = 1 << TB, NR = 1 << R;
   const uint32_t tid = threadIdx.x;
@@ -512,7 +528,7 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
       }
       continue;
     }
-    if ((code & 0xF8u) == C_U3) {
+    if (!PROBES && (code & 0xF8u) == C_U3) {
       if constexpr (sizeof(T) == 4) {
         const float *mp = reinterpret_cast<const float *>(pool + op.extra) + (tid & 63u);
         const float A[4] = {mp[0], mp[64], mp[128], mp[192]};
@@ -533,6 +549,12 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
       }
       continue;
     }
+    if constexpr (PROBES)
+      if (code == C_PROBE) {
+        q_probes<T, NR, NT>(reinterpret_cast<const RProbe *>(pool + op.extra), op.a, a, st.tl, base, tid, red,
+                            sink);
+        continue;
+      }
     if (!tile_ok) continue;  // controls fixed by the tile that do not hold
     const uint32_t tlc = st.tl & cl;
     const uint32_t rb = op.b;
@@ -653,22 +675,27 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
     }
   }
   ++opp;
+  if constexpr (PROBES)
+    if (opp->extra) return;  // a read-only pass
   const RegOff<NR> ro = reg_offset<R>(opp->u.lay);
   cx<T> *p = sv + base + thread_offset<TB>(opp->u.lay, tid);
 #pragma unroll
   for (int j = 0; j < NR; ++j) st_stream(p + ro.gr[j], a.v[j]);
 }
 
-template <typename T, int B, int R>
+template <typename T, int B, int R, bool PROBES>
 __global__ __launch_bounds__(1 << (B - R))
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 5))) void k_gate_pass(
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 || PROBES ? 4 : 5))) void k_gate_pass(
     cx<T> *__restrict__ sv, const PassDesc *__restrict__ pd, const ROp<T> *__restrict__ rops,
-    const TileOp *__restrict__ tops, const cx<double> *__restrict__ pool, uint64_t state_stride, uint32_t pd_stride,
-    uint32_t tile_log) {
+    const cx<double> *__restrict__ pool, double *__restrict__ probes, uint64_t state_stride, uint32_t pd_stride,
+    uint32_t tile_log, uint32_t probes_per_state) {
   __shared__ __align__(16) char xch[8 << B];
+  __shared__ double red[PROBES ? red_doubles((1 << (B - R)) / 64) : 1];
+  constexpr int SPLIT = sizeof(T) == 8 ? 1 : 0;
   const StateTile st = state_tile(tile_log);
-  gate_tile<T, B, R>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, tops, pool, st.t, xch,
-                     reinterpret_cast<cx<double> *>(aerhip_dyn_lds));
+  const GateSink<SPLIT> sink{probes + ((st.b * probes_per_state * st.ntiles) << SPLIT), st.t, st.ntiles};
+  gate_tile<T, B, R, PROBES>(sv + st.b * state_stride, pd + st.b * pd_stride, rops, pool, st.t, xch,
+                             reinterpret_cast<cx<double> *>(aerhip_dyn_lds), red, sink);
 }
 
 }  // namespace aerhip

@@ -2,5 +2,5 @@
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_GATE_PASS(, double, kGateTileC128, kGateRegBits)
+AERHIP_GATE_PASS(, double, kGateTileC128, kGateRegBits, false)
 }  // namespace aerhip

@@ -1,0 +1,6 @@
+// complex128 gate pass on tiles of 2^12 amplitudes, with probes.
+#include "pass_kernels.hpp"
+
+namespace aerhip {
+AERHIP_GATE_PASS(, double, kGateTileC128, kGateRegBits, true)
+}  // namespace aerhip

@@ -2,5 +2,5 @@
 #include "pass_kernels.hpp"
 
 namespace aerhip {
-AERHIP_GATE_PASS(, float, kTileBitsC64, kGateRegBits)
+AERHIP_GATE_PASS(, float, kTileBitsC64, kGateRegBits, false)
 }  // namespace aerhip

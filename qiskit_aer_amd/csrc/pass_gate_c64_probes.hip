@@ -1,0 +1,6 @@
+// complex64 gate pass on tiles of 2^12 amplitudes, with probes.
+#include "pass_kernels.hpp"
+
+namespace aerhip {
+AERHIP_GATE_PASS(, float, kTileBitsC64, kGateRegBits, true)
+}  // namespace aerhip

@@ -14,6 +14,8 @@ constexpr uint32_t kTileBitsC64 = 12;   // 2^12 x 8 B  = 32 KiB of LDS
 
 constexpr uint32_t kGateTileC128 = 12;  // 2^12 x 8 B = 32 KiB of LDS per component
 constexpr uint32_t kGateRegBits = 4;
+static_assert(kGateTileC128 == kTileBitsC64, "gate passes of both types launch workgroups of one size");
+static_assert(kGateTileC128 == kTileBitsC128 + 1, "a complex128 gate tile fills two probe partials");
 
 #define AERHIP_REG_PASS(EXT, T, B, R, V, WIDE)                                                        \
   EXT template __global__ void k_reg_pass<T, B, R, V, WIDE>(                                          \
@@ -26,13 +28,15 @@ constexpr uint32_t kGateRegBits = 4;
       const PassDesc *__restrict__, const ROp<T> *__restrict__, const TileOp *__restrict__,              \
       const cx<double> *__restrict__, double *__restrict__);
 
-#define AERHIP_GATE_PASS(EXT, T, B, R)                                                                   \
-  EXT template __global__ void k_gate_pass<T, B, R>(                                                     \
+#define AERHIP_GATE_PASS(EXT, T, B, R, PROBES)                                                           \
+  EXT template __global__ void k_gate_pass<T, B, R, PROBES>(                                             \
       cx<T> *__restrict__, const PassDesc *__restrict__, const ROp<T> *__restrict__,                     \
-      const TileOp *__restrict__, const cx<double> *__restrict__, uint64_t, uint32_t, uint32_t);
+      const cx<double> *__restrict__, double *__restrict__, uint64_t, uint32_t, uint32_t, uint32_t);
 
-AERHIP_GATE_PASS(extern, double, kGateTileC128, kGateRegBits)
-AERHIP_GATE_PASS(extern, float, kTileBitsC64, kGateRegBits)
+AERHIP_GATE_PASS(extern, double, kGateTileC128, kGateRegBits, false)
+AERHIP_GATE_PASS(extern, double, kGateTileC128, kGateRegBits, true)
+AERHIP_GATE_PASS(extern, float, kTileBitsC64, kGateRegBits, false)
+AERHIP_GATE_PASS(extern, float, kTileBitsC64, kGateRegBits, true)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, false)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_LEAN, true)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 3, V_GATES, false)

@@ -155,7 +155,7 @@ struct RProbe {
   uint32_t slot;   // index of the saved value
   uint32_t idx;    // entry of the batch
   uint32_t flush;
-  uint32_t pad;
+  uint32_t neg;    // bit j: register j's tile bits have odd parity with zl
 };
 static_assert(sizeof(RProbe) == 3 * sizeof(cx<double>), "a probe record is three pool entries");
 // LDS doubles of a workgroup of nw waves: one per wave for the probes that run
@@ -733,8 +733,14 @@ __device__ __forceinline__ double wide(float v) {
 // products c, conj(c): equal signs add up to 2 Re(phase) Re(c), opposite ones
 // to -2 Im(phase) Im(c), so a pair costs three FMAs.
 template <typename T, int NR, int xr>
-__device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RegIdx<NR> &ri, const RProbe &pr) {
-  auto sign = [&](int j) { return (__popc(ri.at(j) & pr.zl) & 1u) ? -1.0 : 1.0; };
+__device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RProbe &pr) {
+  // the signs are made from one word here: as values shared by all shapes they
+  // would take two scalar registers each, ahead of the dispatch
+  uint32_t neg = pr.neg;
+  asm volatile("" : "+s"(neg));
+  auto sign = [&](int j) {
+    return __builtin_bit_cast(double, static_cast<uint64_t>(0x3FF00000u | (neg << (31 - j) & 0x80000000u)) << 32);
+  };
   double acc = 0;
   if constexpr (xr == 0) {
 #pragma unroll
@@ -745,7 +751,7 @@ __device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RegIdx<NR>
     return pr.pr * acc;
   } else {
     constexpr int hb = top_bit<xr>();
-    const bool odd = (__popc((ri.at(xr) ^ ri.t0) & pr.zl) & 1u) != 0;
+    const bool odd = ((neg >> xr ^ neg) & 1u) != 0;
     if (odd) {
 #pragma unroll
       for (int j = 0; j < NR; ++j) {
@@ -766,10 +772,10 @@ __device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RegIdx<NR>
 }
 
 template <typename T, int NR, int X>
-__device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const RegIdx<NR> &ri, const RProbe &pr) {
+__device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const RProbe &pr) {
   if constexpr (X < NR) {
-    if (pr.xr == X) return q_probe<T, NR, X>(a, ri, pr);
-    return q_probe_dispatch<T, NR, X + 1>(a, ri, pr);
+    if (pr.xr == X) return q_probe<T, NR, X>(a, pr);
+    return q_probe_dispatch<T, NR, X + 1>(a, pr);
   } else {
     return 0.0;
   }
@@ -777,13 +783,14 @@ __device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const R
 
 // A run of probes on the amplitudes in registers.  What a probe needs is FMAs
 // and one sum over the workgroup; barriers per probe are what cost most, so the
-// waves leave their sums in LDS and one barrier serves a batch.  33 probes per
-// pass on 2^28 complex128 amplitudes: 7.6 ms with two barriers, shuffles and
-// both orders of every pair per probe, TIME here.
-template <typename T, int NR, int NT>
-__device__ __forceinline__ Amps<T, NR> q_probes(const RProbe *recs, uint32_t count, Amps<T, NR> a, uint32_t tl,
-                                                const RegIdx<NR> &ri, uint64_t base, uint32_t tid, double *red,
-                                                const ProbeSink &sink) {
+// waves leave their sums in LDS and one barrier serves a batch.  The 55 terms of
+// a spin chain on 2^28 complex128 amplitudes: four passes of 3.1 ms with two
+// barriers, shuffles and both orders of every pair per probe, of 1.6 ms so;
+// three gate passes, with half as many wave sums per amplitude, of 1.2 ms.
+template <typename T, int NR, int NT, typename Sink>
+__device__ __forceinline__ void q_probes(const RProbe *recs, uint32_t count, Amps<T, NR> &a, uint32_t tl,
+                                         uint64_t base, uint32_t tid, double *red,
+                                         const Sink &sink) {
   constexpr uint32_t NW = NT / 64;
   double *sums = red + NW;
   uint32_t *slots = reinterpret_cast<uint32_t *>(sums + kProbeBatch * NW);
@@ -795,7 +802,7 @@ __device__ __forceinline__ Amps<T, NR> q_probes(const RProbe *recs, uint32_t cou
       for (int j = 0; j < NR; ++j) asm volatile("" : "+v"(a.v[j].x), "+v"(a.v[j].y));
     }
     const RProbe pr = recs[k];
-    double v = q_probe_dispatch<T, NR, 0>(a, ri, pr);
+    double v = q_probe_dispatch<T, NR, 0>(a, pr);
     if ((__popc(tl & pr.zl) ^ __popcll(base & pr.zg)) & 1u) v = -v;
     v = wave_sum_dpp(v);
     if ((tid & 63u) == 63u) {
@@ -812,7 +819,6 @@ __device__ __forceinline__ Amps<T, NR> q_probes(const RProbe *recs, uint32_t cou
       __syncthreads();  // the entries are free for the next batch
     }
   }
-  return a;
 }
 
 // Layout state of a thread: tile index of its thread part and of each register.
@@ -1063,9 +1069,12 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
   }
   if (kind == Q_PROBE || kind == Q_NOP) {
     if constexpr (has_probes(V)) {
-      if (kind == Q_PROBE)
-        return q_probes<T, NR, 1 << TB>(reinterpret_cast<const RProbe *>(pool + extra), ra, a, st.tl, st.ri, base,
-                                        tid, red, sink);
+      if (kind == Q_PROBE) {
+        Amps<T, NR> o = a;
+        q_probes<T, NR, 1 << TB>(reinterpret_cast<const RProbe *>(pool + extra), ra, o, st.tl, base, tid, red,
+                                 sink);
+        return o;
+      }
     }
     return pass_through(a);
   }

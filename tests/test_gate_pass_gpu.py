@@ -177,3 +177,55 @@ def test_wide_ops_complex64(n, seed):
     _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
     # as above; a component of an 8x8 gate is a sum of 16 rounded products
     assert np.linalg.norm(e.copy_to_vector() - want) < (120 + n) * 16 * 2.0**-24
+
+
+def pauli_value(psi, label):
+    n = len(label)
+    x = sum(1 << (n - 1 - i) for i, p in enumerate(label) if p in "XY")
+    i = np.arange(psi.size)
+    parity = np.zeros_like(i)
+    for k, p in enumerate(label):
+        if p in "YZ":
+            parity ^= i >> (n - 1 - k)
+    return float(np.real(1j ** label.count("Y") * np.sum(np.conj(psi[i ^ x]) * psi * (1 - 2.0 * (parity & 1)))))
+
+
+@pytest.mark.parametrize("precision,n,seed", [("double", 21, 21), ("double", 22, 22), ("single", 12, 23),
+                                              ("single", 13, 24), ("single", 16, 25)])
+def test_probes_between_gates(precision, n, seed):
+    """Saved Pauli values between gates of one queue: X and Y on none to seven
+    qubits inside and outside a tile, more of them than a batch holds, 3-qubit
+    gates and swaps next to them, and a read-only end."""
+    print(f"case: gate pass probes {precision} n={n} seed={seed}", flush=True)
+    rng = np.random.default_rng(seed)
+    e = QubitVector(n, precision)
+    e.initialize()
+    want, slots, psi = [], [], None
+    prefix = circuits.Circuit(n)
+    blocks = [mixture(n, seed, 30), wide_mixture(n, seed + 1, 12), mixture(n, seed + 2, 20)]
+    for k, c in enumerate(blocks):
+        e.apply_ops(c)
+        for op in c.ops:
+            prefix.ops.append(op)
+        _, psi, _ = O.run_circuit(prefix, shots=0, seed=0, fusion=False)
+        for i in range(70 if k == 2 else 8):
+            lab = ["I"] * n
+            at = rng.permutation(n)
+            for q in at[: int(rng.integers(0, 8))]:
+                lab[q] = "XY"[int(rng.integers(2))]
+            for q in at[8: 8 + int(rng.integers(0, 4))]:
+                lab[q] = "Z"
+            if i % 2:  # local strings, which share tiles
+                q = int(rng.integers(0, n - 1))
+                lab = ["I"] * n
+                lab[q], lab[q + 1] = "XYZ"[int(rng.integers(3))], "IXYZ"[int(rng.integers(4))]
+            lab = "".join(lab)
+            slots.append(e.save_expval_pauli(list(range(n)), lab, 1.0))
+            want.append(pauli_value(psi, lab))
+    got = e.saved_expvals()[slots]
+    # FP64 sums; the state before them within 4 (16 for 8x8 gates) roundings of
+    # its norm per gate, which a value of a Pauli string doubles
+    gates = sum(len(c.ops) for c in blocks)
+    bound = 1e-12 if precision == "double" else 2 * gates * 16 * 2.0**-24
+    assert np.max(np.abs(got - np.array(want))) < bound
+    assert np.linalg.norm(e.copy_to_vector() - psi) < bound
