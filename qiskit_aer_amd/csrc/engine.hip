@@ -1760,7 +1760,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   if (gate)
     for (size_t i = first_rop; i < rops.size(); ++i) {
       const uint32_t k = rops[i].kind;
-      rops[i].code = gate_code(rops[i]);
+      rops[i].code = gate_code(rops[i], single);
       if (rops[i].code == C_NOP && k != Q_NOP && k != Q_LOAD && k != Q_STORE)
         throw std::logic_error("aerhip: op outside the gate pass");
     }
