@@ -1368,8 +1368,6 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     emit(Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
   };
-  uint32_t nprobes = 0;   // register probes of the pass so far
-  size_t last_probe = 0;  // pool offset of the last one's record
   auto emit_gate = [&](const TileOp &op, uint32_t rs) {
     ROp<double> r;
     std::memset(&r, 0, sizeof(r));
@@ -1660,21 +1658,19 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         pr.slot = op.npairs;
         for (uint32_t j = 0; j < (1u << R); ++j)
           pr.neg |= (static_cast<uint32_t>(__builtin_popcount(reg_tile_bits(j) & op.zl)) & 1u) << j;
-        pr.idx = nprobes++ % kProbeBatch;
-        if (pr.idx == kProbeBatch - 1) pr.flush = kProbeBatch;
         cd rec[3];
         std::memcpy(rec, &pr, sizeof(rec));
-        last_probe = pool.size();
+        const size_t at = pool.size();
         pool.insert(pool.end(), rec, rec + 3);
         // the next record of the run that the last op holds, or a new run
         if (!map_dirty && (rops.back().kind & ~F_ALL) == Q_PROBE && rops.size() - 1 > enter_at &&
-            rops.back().extra + 3ull * rops.back().a == last_probe) {
+            rops.back().extra + 3ull * rops.back().a == at) {
           ++rops.back().a;
           return;
         }
         r.kind = Q_PROBE;
         r.a = 1;
-        r.extra = static_cast<uint32_t>(last_probe);
+        r.extra = static_cast<uint32_t>(at);
         break;
       }
       default:
@@ -1750,12 +1746,22 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     emit(lds_mode ? Q_FILL : Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
   }
-  if (nprobes % kProbeBatch) {  // the last batch's entries go out with its last probe
-    RProbe pr;
-    std::memcpy(&pr, pool.data() + last_probe, sizeof(pr));
-    pr.flush = nprobes % kProbeBatch;
-    std::memcpy(pool.data() + last_probe, &pr, sizeof(pr));
+  // The probes of a run commute: those without X come first.  Entries of the
+  // batches are handed out in the final order.
+  uint32_t nprobes = 0;
+  RProbe *last = nullptr;
+  for (size_t i = first_rop; i < rops.size(); ++i) {
+    ROp<double> &r = rops[i];
+    if ((r.kind & ~F_ALL) != Q_PROBE) continue;
+    RProbe *p = reinterpret_cast<RProbe *>(pool.data() + r.extra);
+    r.b = static_cast<uint32_t>(std::stable_partition(p, p + r.a, [](const RProbe &q) { return q.xr == 0; }) - p);
+    for (uint32_t k = 0; k < r.a; ++k) {
+      p[k].idx = nprobes++ % kProbeBatch;
+      if (p[k].idx == kProbeBatch - 1) p[k].flush = kProbeBatch;
+    }
+    last = p + r.a - 1;
   }
+  if (nprobes % kProbeBatch) last->flush = nprobes % kProbeBatch;  // with the last probe, what is left
   emit(Q_STORE, rs);
   if (gate)
     for (size_t i = first_rop; i < rops.size(); ++i) {

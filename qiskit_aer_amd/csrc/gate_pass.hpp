@@ -584,7 +584,7 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
     }
     if constexpr (PROBES)
       if (code == C_PROBE) {
-        q_probes<T, NR, NT>(reinterpret_cast<const RProbe *>(pool + op.extra), op.a, a, st.tl, base, tid, red,
+        q_probes<T, NR, NT>(reinterpret_cast<const RProbe *>(pool + op.extra), op.a, op.b, a, st.tl, base, tid, red,
                             sink);
         continue;
       }

@@ -48,7 +48,7 @@ enum RegPassOpKind : uint32_t {
                     // meets the register part of the predicate
   Q_DIAG = 53,      // diagonal of TileOp extra (local and fixed bits)
   Q_PROBE = 54,     // a run of a Pauli probes whose X/Y bits are register bits: RProbe
-                    // records at pool[extra..]
+                    // records at pool[extra..], the first b of them without X
   Q_NOP = 55,       // keeps the amplitudes (pads a register phase to an even length)
   Q_U1M = 57,       // 2x2 matrix on the register pairs {j, j ^ a}; bit k of extra set:
                     // the k-th pair's lower register holds the |1> amplitude
@@ -142,11 +142,12 @@ __host__ __device__ __forceinline__ void set_byte(uint32_t *w, int i, uint32_t v
   w[i >> 2] = (w[i >> 2] & ~(0xFFu << (8 * (i & 3)))) | ((v & 0xFFu) << (8 * (i & 3)));
 }
 
-// One Pauli probe of a run (three pool entries).  A probe's sum over each wave
-// goes to LDS entry idx; a record with flush = k hands the first k entries of
-// the pass on, after one barrier for all of them (the host sets it on every
-// kProbeBatch-th probe of the pass and on its last).
-constexpr uint32_t kProbeBatch = 64;
+// One Pauli probe of a run (three pool entries).  A probe's four sums over
+// each wave (wave_sums) go to LDS entry idx; a record with flush = k hands the
+// first k entries of the pass on, after one barrier for all of them (the host
+// sets it on every kProbeBatch-th probe of the pass and on its last).  A batch
+// is as large as four workgroups per CU leave LDS for.
+constexpr uint32_t kProbeBatch = 16;
 struct RProbe {
   uint32_t xr;     // X/Y mask in register-index space
   uint32_t zl;     // Z mask over tile bits
@@ -160,7 +161,7 @@ struct RProbe {
 static_assert(sizeof(RProbe) == 3 * sizeof(cx<double>), "a probe record is three pool entries");
 // LDS doubles of a workgroup of nw waves: one per wave for the probes that run
 // on the LDS tile, then the batch's sums and its slots.
-constexpr uint32_t red_doubles(uint32_t nw) { return nw + kProbeBatch * nw + kProbeBatch / 2; }
+constexpr uint32_t red_doubles(uint32_t nw) { return nw + 4 * kProbeBatch * nw + kProbeBatch / 2; }
 
 // 128-byte op record: a 64-byte header and a 64-byte payload, each read with
 // one scalar load (both issued together, so an op costs one load latency).
@@ -697,23 +698,29 @@ __device__ __forceinline__ Amps<T, NR> d_cxr(uint32_t p, const Amps<T, NR> &a) {
   }
 }
 
-// The wave's sum of v, valid in lane 63: DPP moves within rows of 16 lanes and
-// two row broadcasts, so that no step waits for LDS as a shuffle does.
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-  auto step = [](double x, auto ctrl, auto rows) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, x);
-    const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), decltype(ctrl)::value, decltype(rows)::value, 0xF, true);
-    const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, true);
-    return x + __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
-  };
-  using std::integral_constant;
-  v = step(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});  // row_shr 1
-  v = step(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});  // row_shr 2
-  v = step(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});  // row_shr 4
-  v = step(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});  // row_shr 8
-  v = step(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});  // row_bcast 15
-  v = step(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});  // row_bcast 31
-  return v;
+// The wave's sum of v in four parts: lane l receives the sum over the lanes with
+// its bits 2 and 3.  Two 4x4x4 products with ones add up first the lanes that
+// differ in bits 4 and 5 or 0 and 1, then the rest of the block, on the matrix
+// cores, which the probes leave idle: two issues where moving and adding across
+// lanes takes eighteen on the vector ALU.
+__device__ __forceinline__ double wave_sums(double v) {
+  const double s = __builtin_amdgcn_mfma_f64_4x4x4f64(v, 1.0, 0.0, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, s, 0.0, 0, 0, 0);
+}
+
+// Leaves the four parts of the wave's sum in entry `idx` of a batch.
+template <uint32_t NW>
+__device__ __forceinline__ void put_wave_sums(double *sums, uint32_t idx, uint32_t tid, double v) {
+  v = wave_sums(v);
+  if (!(tid & 0x33u)) sums[4 * (idx * NW + (tid >> 6)) + ((tid >> 2) & 3u)] = v;
+}
+
+// The workgroup's sum of entry `idx`.
+template <uint32_t NW>
+__device__ __forceinline__ double batch_entry(const double *sums, uint32_t idx) {
+  double s = 0;
+  for (uint32_t w = 0; w < 4 * NW; ++w) s += sums[4 * idx * NW + w];
+  return s;
 }
 
 // An amplitude's component in FP64.  The complex64 conversion is written out so
@@ -771,6 +778,19 @@ __device__ __forceinline__ double q_probe(const Amps<T, NR> &a, const RProbe &pr
   }
 }
 
+// Entry m of w, m uniform: a branch per bit.
+template <int NR, int BIT = NR / 2, int X = 0>
+__device__ __forceinline__ double pick(const double (&w)[NR], uint32_t m) {
+  if constexpr (BIT == 0) {
+    double v = w[X];
+    asm volatile("" : "+v"(v));  // keeps the branches
+    return v;
+  } else {
+    if (m & BIT) return pick<NR, BIT / 2, X | BIT>(w, m);
+    return pick<NR, BIT / 2, X>(w, m);
+  }
+}
+
 template <typename T, int NR, int X>
 __device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const RProbe &pr) {
   if constexpr (X < NR) {
@@ -787,14 +807,58 @@ __device__ __forceinline__ double q_probe_dispatch(const Amps<T, NR> &a, const R
 // a spin chain on 2^28 complex128 amplitudes: four passes of 3.1 ms with two
 // barriers, shuffles and both orders of every pair per probe, of 1.6 ms so;
 // three gate passes, with half as many wave sums per amplitude, of 1.2 ms.
+//
+// Probes without X (diagonal ones) come first; from three on (kDiagProbes) they
+// share the norms |a_j|^2 and a Walsh-Hadamard transform of them over the
+// register bits, which holds the sum for every Z mask.  The pass of the spin
+// chain above that holds all 27 ZZ and 12 X: 2.18 -> 1.70 ms.
+constexpr uint32_t kDiagProbes = 3;
 template <typename T, int NR, int NT, typename Sink>
-__device__ __forceinline__ void q_probes(const RProbe *recs, uint32_t count, Amps<T, NR> &a, uint32_t tl,
-                                         uint64_t base, uint32_t tid, double *red,
-                                         const Sink &sink) {
+__device__ __forceinline__ void q_probes(const RProbe *recs, uint32_t count, uint32_t ndiag, Amps<T, NR> &a,
+                                         uint32_t tl, uint64_t base, uint32_t tid, double *red, const Sink &sink) {
   constexpr uint32_t NW = NT / 64;
   double *sums = red + NW;
-  uint32_t *slots = reinterpret_cast<uint32_t *>(sums + kProbeBatch * NW);
-  for (uint32_t k = 0; k < count; ++k) {
+  uint32_t *slots = reinterpret_cast<uint32_t *>(sums + 4 * kProbeBatch * NW);
+  auto finish = [&](const RProbe &pr, double v) {
+    if ((__popc(tl & pr.zl) ^ __popcll(base & pr.zg)) & 1u) v = -v;
+    put_wave_sums<NW>(sums, pr.idx, tid, v);
+    if (tid == 0) slots[pr.idx] = pr.slot;
+    if (pr.flush) {
+      __syncthreads();
+      if (tid < pr.flush) sink.put(slots[tid], batch_entry<NW>(sums, tid));
+      __syncthreads();  // the entries are free for the next batch
+    }
+  };
+  uint32_t k = 0;
+  if constexpr (NR <= 16)
+    if (ndiag >= kDiagProbes) {
+      double w[NR];
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        const double x = wide(a.v[j].x), y = wide(a.v[j].y);
+        w[j] = fma_t(x, x, y * y);
+      }
+#pragma unroll
+      for (int h = 1; h < NR; h *= 2)
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+          if (!(j & h)) {
+            const double p = w[j], q = w[j | h];
+            w[j] = p + q;
+            w[j | h] = p - q;
+          }
+      for (; k < ndiag; ++k) {
+        const RProbe pr = recs[k];
+        // the sign of register j is linear in j but for that of register 0
+        const uint32_t neg = pr.neg & 1u ? ~pr.neg : pr.neg;
+        uint32_t m = 0;
+#pragma unroll
+        for (int r = 0; (1 << r) < NR; ++r) m |= ((neg >> (1 << r)) & 1u) << r;
+        const double v = pick<NR>(w, m);
+        finish(pr, (pr.neg & 1u ? -pr.pr : pr.pr) * v);
+      }
+    }
+  for (; k < count; ++k) {
     // complex128 amplitudes pass through the loop as values the compiler cannot
     // know: it would compute the products of every probe shape ahead of it
     if constexpr (sizeof(T) == 8) {
@@ -802,22 +866,7 @@ __device__ __forceinline__ void q_probes(const RProbe *recs, uint32_t count, Amp
       for (int j = 0; j < NR; ++j) asm volatile("" : "+v"(a.v[j].x), "+v"(a.v[j].y));
     }
     const RProbe pr = recs[k];
-    double v = q_probe_dispatch<T, NR, 0>(a, pr);
-    if ((__popc(tl & pr.zl) ^ __popcll(base & pr.zg)) & 1u) v = -v;
-    v = wave_sum_dpp(v);
-    if ((tid & 63u) == 63u) {
-      sums[pr.idx * NW + (tid >> 6)] = v;
-      if (tid == 63u) slots[pr.idx] = pr.slot;
-    }
-    if (pr.flush) {
-      __syncthreads();
-      if (tid < pr.flush) {
-        double s = 0;
-        for (uint32_t w = 0; w < NW; ++w) s += sums[tid * NW + w];
-        sink.put(slots[tid], s);
-      }
-      __syncthreads();  // the entries are free for the next batch
-    }
+    finish(pr, q_probe_dispatch<T, NR, 0>(a, pr));
   }
 }
 
@@ -1071,7 +1120,7 @@ __device__ __forceinline__ Amps<T, 1 << R> rw_op(const ROp<T> &op, const OpHead<
     if constexpr (has_probes(V)) {
       if (kind == Q_PROBE) {
         Amps<T, NR> o = a;
-        q_probes<T, NR, 1 << TB>(reinterpret_cast<const RProbe *>(pool + extra), ra, o, st.tl, base, tid, red,
+        q_probes<T, NR, 1 << TB>(reinterpret_cast<const RProbe *>(pool + extra), ra, rb, o, st.tl, base, tid, red,
                                  sink);
         return o;
       }
@@ -1483,16 +1532,11 @@ __device__ __forceinline__ void probe_sweep(const cx<T> *__restrict__ sv, const 
       acc *= (odd ? -op.pi : op.pr) * (xh ? 2.0 : 1.0);
       if (__popcll(z & (base | (tid & (NT - 1u)))) & 1u) acc = -acc;
     }
-    acc = wave_sum_dpp(acc);
     const uint32_t idx = k % kProbeBatch;
-    if ((tid & 63u) == 63u) sums[idx * NW + (tid >> 6)] = acc;
+    put_wave_sums<NW>(sums, idx, tid, acc);
     if (idx == kProbeBatch - 1 || k + 1 == nops) {
       __syncthreads();
-      if (tid <= idx) {
-        double t = 0;
-        for (uint32_t w = 0; w < NW; ++w) t += sums[tid * NW + w];
-        sink.put(ops[k - idx + tid].npairs, t);
-      }
+      if (tid <= idx) sink.put(ops[k - idx + tid].npairs, batch_entry<NW>(sums, tid));
       __syncthreads();
     }
   }
