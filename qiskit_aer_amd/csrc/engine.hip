@@ -1004,6 +1004,11 @@ void validate_register_program(const ROp<double> *p, size_t n, uint32_t B, uint3
       switch (r.kind & ~F_ALL) {
         case Q_RELAYOUT:
           check_layout(r.u.lay);
+          if (r.a > kMaxRelayoutCx) fail("CX of a layout change");
+          for (uint32_t k = 0; k < r.a; ++k) {
+            const uint32_t c = r.u.rel.cx[2 * k], t = r.u.rel.cx[2 * k + 1];
+            if (t >= B || c == t || (c >= B && c != kNoControl)) fail("CX of a layout change");
+          }
           regmask = 0;
           for (uint32_t q = 0; q < R; ++q) regmask |= 1u << byte_at(r.u.lay.rp, static_cast<int>(q));
           break;
@@ -1250,6 +1255,16 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     e.a = static_cast<uint32_t>(df.size());
     e.b = static_cast<uint32_t>(first);
   };
+  // Gate passes: the ops since the last layout change, by the tile bits they
+  // touch, and the CX that the next one takes along (see C_RELAYOUT).
+  struct Tail {
+    uint32_t touch;
+    uint8_t c, t;  // a CX or X (c = kNoControl) of tile bits
+    bool cx;
+  };
+  std::vector<Tail> tail;
+  size_t tail_at = 0;
+  std::vector<std::pair<uint8_t, uint8_t>> cxs;
   auto emit_raw = [&](uint32_t kind, uint32_t rs) {
     if (kind == Q_STORE || kind == Q_SPILL) {
       uint32_t cnt = static_cast<uint32_t>(rops.size() - enter_at - 1);
@@ -1269,7 +1284,17 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     r.kind = kind;
     r.u.lay = make_layout(rs, B, spos);
     if (kind == Q_STORE || kind == Q_SPILL || kind == Q_RELAYOUT) stamp(r);
+    if (kind == Q_RELAYOUT) {
+      r.a = static_cast<uint32_t>(cxs.size());
+      for (size_t k = 0; k < cxs.size(); ++k) {
+        r.u.rel.cx[2 * k] = cxs[k].first;
+        r.u.rel.cx[2 * k + 1] = cxs[k].second;
+      }
+      cxs.clear();
+    }
     rops.push_back(r);
+    tail.clear();
+    tail_at = rops.size();
     if (kind == Q_LOAD || kind == Q_FILL || kind == Q_RELAYOUT) {
       map_reset();
       cur_rs = rs;
@@ -1355,8 +1380,36 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     }
     pend &= ~bits;
   };
+  // Fills `tail` up to the ops emitted.
+  auto note = [&](const Tail &t) {
+    while (tail.size() < rops.size() - tail_at) tail.push_back(t);
+  };
+  // CX and X on tile bits, which a layout change can take along.
+  auto is_cx = [](const TileOp &op) {
+    return op.kind == K_MCX && !op.cg && __builtin_popcount(op.cl) <= 1 && op.cvl == op.cl;
+  };
+  auto cx_of = [](const TileOp &op) {
+    return std::make_pair(static_cast<uint8_t>(op.cl ? __builtin_ctz(op.cl) : kNoControl), static_cast<uint8_t>(op.t));
+  };
+  // Hands the CX of the layout in force that no later op of it touches to the
+  // layout change that comes.
+  auto sink_cxs = [&] {
+    note(Tail{~0u, 0, 0, false});
+    uint32_t blocked = 0;
+    std::vector<std::pair<uint8_t, uint8_t>> found;
+    for (size_t k = tail.size(); k-- > 0;) {
+      if (tail[k].cx && !(tail[k].touch & blocked) && cxs.size() + found.size() < kMaxRelayoutCx) {
+        found.push_back({tail[k].c, tail[k].t});
+        rops.erase(rops.begin() + static_cast<std::ptrdiff_t>(tail_at + k));
+      } else {
+        blocked |= tail[k].touch;
+      }
+    }
+    cxs.insert(cxs.begin(), found.rbegin(), found.rend());
+  };
   auto emit = [&](uint32_t kind, uint32_t rs) {
     if (kind == Q_RELAYOUT || kind == Q_STORE || kind == Q_SPILL) materialize(pend);
+    if (gate && kind == Q_RELAYOUT) sink_cxs();
     emit_raw(kind, rs);
   };
   // Ops that need the registers in the layout's own order (pair structure on
@@ -1687,11 +1740,8 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     tops.push_back(op);
     rops.push_back(r);
   };
-  auto take = [&](const std::vector<size_t> &idx, uint32_t rs, bool lds_mode) {
-    for (size_t i : idx) {
-      if (lds_mode) emit_lds(in[rem_op[i]]);
-      else emit_gate(in[rem_op[i]], rs);
-    }
+  // Takes items out of the pending ones.
+  auto drop = [&](const std::vector<size_t> &idx) {
     size_t k = 0, to = 0;
     for (size_t i = 0; i < rem.size(); ++i) {
       if (k < idx.size() && idx[k] == i) {
@@ -1704,6 +1754,26 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     rem.resize(to);
     rem_op.resize(to);
   };
+  auto take = [&](const std::vector<size_t> &idx, uint32_t rs, bool lds_mode) {
+    for (size_t i : idx) {
+      const TileOp &op = in[rem_op[i]];
+      if (lds_mode) {
+        emit_lds(op);
+        continue;
+      }
+      const size_t before = rops.size();
+      emit_gate(op, rs);
+      if (!gate) continue;
+      // with register moves of other ops made up before it, it touches what they do
+      Tail t{rops.size() == before + 1 ? rem[i].touch : rem[i].touch | rs, 0, 0, false};
+      if (is_cx(op) && rops.size() == before + 1) {
+        t.cx = true;
+        std::tie(t.c, t.t) = cx_of(op);
+      }
+      note(t);
+    }
+    drop(idx);
+  };
 
   // Load in the best set that keeps the low bits on lanes.
   uint32_t rs = best_set(true).first;
@@ -1715,6 +1785,28 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       if (!idx.empty()) {
         take(idx, rs, false);
         continue;
+      }
+      if (gate) {
+        // the CX that are ready, on whatever bits, go with the layout change
+        // if more gates come after it
+        const auto rem0 = rem;
+        const auto op0 = rem_op;
+        std::vector<size_t> ready;
+        scan_items(rem,
+                   [&](const RMask &it) {
+                     return ready.size() < kMaxRelayoutCx / 2 &&
+                            is_cx(in[rem_op[static_cast<size_t>(&it - rem.data())]]);
+                   },
+                   [&](size_t i) { ready.push_back(i); });
+        if (!ready.empty()) {
+          for (size_t i : ready) cxs.push_back(cx_of(in[rem_op[i]]));
+          drop(ready);
+          if (best_set(false).second == 0) {
+            cxs.clear();
+            rem = rem0;
+            rem_op = op0;
+          }
+        }
       }
       const auto b = best_set(false);
       if (b.second > 0) {

@@ -539,6 +539,23 @@ __device__ __forceinline__ void gate_tile(cx<T> *__restrict__ sv, const PassDesc
       continue;
     }
     if (code == C_RELAYOUT) {
+      // A CX between tile bits is a linear map of the tile index, so those that
+      // come just before (or just after) cost the write addresses a shift and an
+      // XOR, not the amplitudes a move.
+      const uint32_t ncx = op.a;
+      const uint32_t *cxw = reinterpret_cast<const uint32_t *>(op.u.rel.cx);
+      for (uint32_t k = 0; k < ncx; ++k) {
+        const uint32_t p = cxw[k >> 1] >> (16 * (k & 1u)), c = p & 0xFFu, t = (p >> 8) & 0xFFu;
+        if (c == kNoControl) {
+          st.ri.t0 ^= 1u << t;
+        } else {
+          auto map = [&](uint32_t x) { return x ^ (((x >> c) & 1u) << t); };
+          st.tl = map(st.tl);
+#pragma unroll
+          for (int s = 0; s < R; ++s) st.ri.bm[s] = map(st.ri.bm[s]);
+          st.ri.t0 = map(st.ri.t0);
+        }
+      }
       uint32_t w[NR], r[NR];
       const uint32_t w0 = g_slot(st.tl);
 #pragma unroll

@@ -32,7 +32,8 @@ enum RegPassOpKind : uint32_t {
                     // a: fused-diagonal slots of the phase, b: pool offset of their
                     // DiagLane records
   Q_STORE = 41,     // registers -> HBM in layout u.lay (extra = 1: read-only pass, no write)
-  Q_RELAYOUT = 42,  // registers -> LDS -> registers in layout u.lay
+  Q_RELAYOUT = 42,  // registers -> LDS -> registers in layout u.lay; gate passes: a CX
+                    // come first, of u.rel.cx[2k] (kNoControl: X) on tile bit u.rel.cx[2k + 1]
   Q_SPILL = 43,     // registers -> LDS (the tile is then in LDS)
   Q_FILL = 44,      // LDS -> registers in layout u.lay; extra, a, b: as Q_LOAD
   Q_LDS = 45,       // TileOp primitive extra on the LDS tile
@@ -163,6 +164,10 @@ static_assert(sizeof(RProbe) == 3 * sizeof(cx<double>), "a probe record is three
 // on the LDS tile, then the batch's sums and its slots.
 constexpr uint32_t red_doubles(uint32_t nw) { return nw + 4 * kProbeBatch * nw + kProbeBatch / 2; }
 
+// CX ops of a layout change (gate passes): at most, and the control of an X.
+constexpr uint32_t kMaxRelayoutCx = 16;
+constexpr uint32_t kNoControl = 0xFF;
+
 // 128-byte op record: a 64-byte header and a 64-byte payload, each read with
 // one scalar load (both issued together, so an op costs one load latency).
 template <typename T>
@@ -182,6 +187,10 @@ struct alignas(128) ROp {
                      // (re a0', im a0', re a1', im a1'), columns over (re a0, im a0, re a1, im a1)
     RLayout lay;
     uint8_t fq[32];  // Q_DIAGF: fixed qubits of the tables, four per table
+    struct {
+      RLayout lay;
+      uint8_t cx[32];
+    } rel;           // Q_RELAYOUT
   } u;
 };
 static_assert(sizeof(ROp<double>) == 128 && sizeof(ROp<float>) == 128, "ROp is one 128-byte record");

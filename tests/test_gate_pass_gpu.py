@@ -229,3 +229,32 @@ def test_probes_between_gates(precision, n, seed):
     bound = 1e-12 if precision == "double" else 2 * gates * 16 * 2.0**-24
     assert np.max(np.abs(got - np.array(want))) < bound
     assert np.linalg.norm(e.copy_to_vector() - psi) < bound
+
+
+@pytest.mark.parametrize("precision,n", [("double", 21), ("single", 13)])
+def test_cx_taken_by_layout_changes(precision, n):
+    """CX and X on every ordered pair of a tile's qubits between gates that force
+    layout changes: chains of them, more than one layout change takes, before,
+    between and after the gates."""
+    print(f"case: CX in layout changes {precision} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    c = circuits.Circuit(n)
+    for _ in range(3):
+        for q in range(12):
+            c.gate("u3", [q], list(rng.uniform(-3, 3, 3)))
+    pairs = [(a, b) for a in range(12) for b in range(12) if a != b]
+    for k, i in enumerate(rng.permutation(len(pairs))):
+        a, b = pairs[int(i)]
+        c.gate("cx", [a, b])
+        if k % 5 == 0:
+            c.gate("x", [int(rng.integers(12))])
+        if k % 7 == 0 or 40 < k < 60:
+            c.gate("u3", [int(rng.integers(12))], list(rng.uniform(-3, 3, 3)))
+        if k % 11 == 0:
+            c.gate("cp", [a, int((b + 1) % 12) if (b + 1) % 12 != a else b], [float(rng.uniform(-3, 3))])
+    e = QubitVector(n, precision)
+    e.initialize()
+    e.apply_ops(c)
+    _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+    bound = 1e-12 if precision == "double" else len(c.ops) * 4 * 2.0**-24
+    assert np.linalg.norm(e.copy_to_vector() - want) < bound
