@@ -2788,7 +2788,7 @@ void Engine::flush() {
     const PassDesc &pd = passes[i];
     const PassKernel &k = kernels[i] = pass_kernel(pd, rops);
     sig.push_back((uint64_t(pd.kind) << 48) | (uint64_t(pd.ncomp) << 32) | (uint64_t(pd.nb) << 16) |
-                  (uint64_t(k.variant) << 2) | (uint64_t(k.diag) << 1) | uint64_t(k.wide));
+                  (uint64_t(k.probes) << 8) | (uint64_t(k.variant) << 2) | (uint64_t(k.diag) << 1) | uint64_t(k.wide));
   }
   auto launch_all = [&] {
     for (size_t i = 0; i < passes.size(); ++i)

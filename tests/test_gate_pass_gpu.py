@@ -258,3 +258,32 @@ def test_cx_taken_by_layout_changes(precision, n):
     _, want, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
     bound = 1e-12 if precision == "double" else len(c.ops) * 4 * 2.0**-24
     assert np.linalg.norm(e.copy_to_vector() - want) < bound
+
+
+def test_replayed_launches_follow_the_probes():
+    """Two flushes of one size and pass count whose probes sit in different
+    passes: the second does not replay the launches captured for the first."""
+    n = 20
+    print("case: gate pass probes under replay", flush=True)
+    rng = np.random.default_rng(31)
+    c = circuits.Circuit(n)
+    for lo in (4, 12):  # two passes, a swap and more than a handful of gates in each
+        for layer in range(3):
+            for q in range(lo, lo + 8):
+                c.gate("u3", [q], list(rng.uniform(-3, 3, 3)))
+            for q in range(lo + layer % 2, lo + 7, 2):
+                c.gate("cx", [q, q + 1])
+        c.gate("swap", [lo, lo + 5])
+    _, psi, _ = O.run_circuit(c, shots=0, seed=0, fusion=False)
+
+    def label(q):
+        return "".join("X" if n - 1 - i == q else "I" for i in range(n))
+
+    e = QubitVector(n, "single")
+    for q in (13, 13, 13, 13, 5, 5, 13, 5):
+        e.initialize()
+        e.apply_ops(c)
+        slot = e.save_expval_pauli(list(range(n)), label(q), 1.0)
+        got = e.saved_expvals()[slot]
+        # 4 roundings of 2^-24 of the norm per gate, doubled by the value
+        assert abs(got - pauli_value(psi, label(q))) < 2 * len(c.ops) * 4 * 2.0**-24
