@@ -812,7 +812,7 @@ RLayout make_layout(uint32_t rs, uint32_t B, const uint8_t *spos) {
 // `pool` as (qubit, u, v) triples.
 std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t *spos, uint32_t ns,
                                     std::vector<cd> &pool, uint32_t max_qubits,
-                                    uint64_t *fused_ops) {
+                                    uint64_t *fused_ops, bool single) {
   struct Group {
     int pivot = -1;
     uint64_t qmask = 0;
@@ -837,8 +837,9 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
     // A single op stays as it is, but for a diagonal on a qubit that the tile
     // fixes: as a fused diagonal of one member it runs in every register
     // variant, as a general one (Q_DIAG) only in those with 4x4 gates.
+    // complex64 keeps the general one, which rounds differently.
     const TileOp &first = g.originals[0];
-    if (g.originals.size() == 1 && !(first.kind == K_DIAG && first.pos[0] == kNotLocal)) {
+    if (g.originals.size() == 1 && (single || !(first.kind == K_DIAG && first.pos[0] == kNotLocal))) {
       out.push_back(first);
       return;
     }
@@ -1316,6 +1317,9 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
   // false, with nothing done, where that takes more moves than a layout change
   // is worth.
   auto move_home = [&] {
+    // complex64 register passes: a 2x2 gate sums its products in another order on
+    // a relabelled bit, so ending the relabelling earlier would change results
+    if (single && !gate) return false;
     uint32_t col[8];
     std::vector<std::pair<uint32_t, uint32_t>> steps;
     for (uint32_t q = 0; q < R; ++q) col[q] = colinv[q];
@@ -2518,7 +2522,7 @@ void Engine::emit_program(Program &prog) {
     const uint32_t R = pp.gate ? kGateRegBits : reg_bits_;
     if (!pp.solo && reg_bits_ > 0 && ns == full_bits) {
       if (fusion_enable_ && n_ > fusion_threshold_)
-        pops = fuse_phase_runs(pops, pd.spos, ns, prog.pool, fusion_max_qubit_, &stats_.fused);
+        pops = fuse_phase_runs(pops, pd.spos, ns, prog.pool, fusion_max_qubit_, &stats_.fused, prec_ == AERHIP_PRECISION_SINGLE);
       pd.kind = pp.gate ? 5 : 2;  // register-layout tile pass: op_begin/nops index the ROps
       pd.op_begin = static_cast<uint32_t>(rops.size());
       register_program(pops, ns, R, low_bits_, prec_ == AERHIP_PRECISION_SINGLE, pp.gate, pd.spos, prog.pool, rops,
@@ -2583,7 +2587,8 @@ void launch_reg_pass(const PassKernel &k, uint32_t grid, hipStream_t stream, cx<
     if constexpr (sizeof(T) == 8)
       if (k.variant == V_LEAN && k.wide) return go(k_reg_pass<T, B, R, V_LEAN, true>);
     if (k.variant == V_GATES) return go(k_reg_pass<T, B, R, V_GATES, false>);
-    if (k.variant == V_PROBES) return go(k_reg_pass<T, B, R, V_PROBES, false>);
+    if constexpr (sizeof(T) == 8)
+      if (k.variant == V_PROBES) return go(k_reg_pass<T, B, R, V_PROBES, false>);
   }
   if (k.variant == V_LEAN) return go(k_reg_pass<T, B, R, V_LEAN, false>);
   go(k_reg_pass<T, B, R, V_FULL, false>);
@@ -2692,8 +2697,10 @@ bool graphs_enabled() {
   return on;
 }
 
-// The kernel of a pass, from its ops.
-PassKernel pass_kernel(const PassDesc &pd, const std::vector<ROp<double>> &rops) {
+// The kernel of a pass, from its ops.  A complex64 pass with probes runs the full
+// variant: the lean ops of the probe variant contract their products in another
+// order, and the values, FP64 sums over complex64 amplitudes, would move by 1e-8.
+PassKernel pass_kernel(int prec, const PassDesc &pd, const std::vector<ROp<double>> &rops) {
   PassKernel k;
   k.wide = pd.nops <= kWidePassOps;
   if (pd.kind != 2 && pd.kind != 5) return k;
@@ -2704,6 +2711,7 @@ PassKernel pass_kernel(const PassDesc &pd, const std::vector<ROp<double>> &rops)
     k.probes = k.probes || kk == Q_PROBE;
     k.diag = k.diag || ((kk == Q_LOAD || kk == Q_FILL) && r.a != 0);
   }
+  if (prec == AERHIP_PRECISION_SINGLE && has_probes(k.variant)) k.variant = V_FULL;
   return k;
 }
 }  // namespace
@@ -2786,7 +2794,7 @@ void Engine::flush() {
   std::vector<PassKernel> kernels(passes.size());
   for (size_t i = 0; i < passes.size(); ++i) {
     const PassDesc &pd = passes[i];
-    const PassKernel &k = kernels[i] = pass_kernel(pd, rops);
+    const PassKernel &k = kernels[i] = pass_kernel(prec_, pd, rops);
     sig.push_back((uint64_t(pd.kind) << 48) | (uint64_t(pd.ncomp) << 32) | (uint64_t(pd.nb) << 16) |
                   (uint64_t(k.probes) << 8) | (uint64_t(k.variant) << 2) | (uint64_t(k.diag) << 1) | uint64_t(k.wide));
   }
@@ -3316,12 +3324,12 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   uint32_t max_passes = 0;
   for (const BatchCircuit &c : sorted) max_passes = std::max(max_passes, c.pass_count);
   // Per pass index: which kernels its passes need (bit 0 k_batch<V_PROBES>,
-  // bit 1 k_batch<V_FULL>).
+  // complex128 only; bit 1 k_batch<V_FULL>).
   std::vector<uint32_t> classes(max_passes, 0);
   for (Program &p : parts)
     for (size_t k = 0; k < p.passes.size(); ++k) {
       PassDesc &d = p.passes[k];
-      d.batch_class = d.kind == 2 && !has_gates(pass_kernel(d, p.rops).variant) ? 0u : 1u;
+      d.batch_class = prec == AERHIP_PRECISION_DOUBLE && d.kind == 2 && !has_gates(pass_kernel(prec, d, p.rops).variant) ? 0u : 1u;
       classes[k] |= 1u << d.batch_class;
     }
 
@@ -3418,9 +3426,10 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
           i = end;
         }
         if (wgs > 0xFFFFFFFFull / kThreads) throw std::invalid_argument("aerhip: batch too large for one launch");
-        if (classes[p] & 1u)
-          k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops,
-                                                                                     dpool, d_probes + probe_off);
+        if constexpr (sizeof(T) == 8)
+          if (classes[p] & 1u)
+            k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(
+                sv, dc, gr, p, dp, dr, dops, dpool, d_probes + probe_off);
         if (classes[p] & 2u)
           k_batch<T, B, R, V_FULL><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops, dpool,
                                                                                    d_probes + probe_off);
@@ -3462,7 +3471,12 @@ class MultiState {
     for (Engine *e : planners_)
       if (!e->plan_only() || e->num_qubits() != n || e->precision() != prec)
         throw std::invalid_argument("aerhip: states need planning handles of one size and precision");
-    for (Engine *e : planners_) e->use_gate_passes();
+    // Energies and gradients are FP64 values of the states.  In complex128 they
+    // keep their digits under any order of the gates' FMAs; in complex64 they
+    // would move by 1e-7 with the order that gate passes use, as accurate, but
+    // not the values callers have had: those states keep register passes.
+    if (prec_ == AERHIP_PRECISION_DOUBLE)
+      for (Engine *e : planners_) e->use_gate_passes();
     AERHIP_CHECK(hipSetDevice(device_));
     ws_ = WorkspacePool::get().take(device_, planners_.size() * (1ull << n_) * amp_bytes());
     states_ = ws_.state.p;
@@ -3586,7 +3600,7 @@ class MultiState {
       const uint32_t ob = static_cast<uint32_t>(ops.size()), rb = static_cast<uint32_t>(rops.size()),
                      pb = static_cast<uint32_t>(pool.size());
       for (size_t k = 0; k < P; ++k) {
-        kernels[k].add(pass_kernel(p.passes[k], p.rops));
+        kernels[k].add(pass_kernel(prec_, p.passes[k], p.rops));
         PassDesc d = p.passes[k];
         d.op_begin += d.kind == 2 || d.kind == 5 ? rb : ob;
         passes.push_back(d);

@@ -46,13 +46,11 @@ AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, V_LEAN, false)
 AERHIP_REG_PASS(extern, double, kTileBitsC128, 4, V_FULL, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_LEAN, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_GATES, false)
-AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_PROBES, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 4, V_FULL, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_LEAN, false)
 AERHIP_REG_PASS(extern, float, kTileBitsC64, 5, V_FULL, false)
 AERHIP_BATCH(extern, double, kTileBitsC128, 3, V_PROBES)
 AERHIP_BATCH(extern, double, kTileBitsC128, 3, V_FULL)
-AERHIP_BATCH(extern, float, kTileBitsC64, 4, V_PROBES)
 AERHIP_BATCH(extern, float, kTileBitsC64, 4, V_FULL)
 
 }  // namespace aerhip
