@@ -1425,6 +1425,13 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
     emit(Q_RELAYOUT, rs);
     if (relayouts) ++*relayouts;
   };
+  // Registers that meet the register part of an op's predicate.
+  auto regs_of = [&](const TileOp &op) {
+    uint32_t m = 0;
+    for (uint32_t j = 0; j < (1u << R); ++j)
+      if ((reg_tile_bits(j) & op.cl & cur_rs) == (op.cvl & op.cl & cur_rs)) m |= 1u << j;
+    return m;
+  };
   auto emit_gate = [&](const TileOp &op, uint32_t rs) {
     ROp<double> r;
     std::memset(&r, 0, sizeof(r));
@@ -1515,6 +1522,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         need_identity(rs, {t});
         r.kind = op.kind == K_MCX ? Q_X : Q_Y;
         r.a = t;
+        if (gate) r.b = regs_of(op);
         break;
       }
       case K_MCSWAP: {
@@ -1523,6 +1531,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         r.kind = Q_SWAP;
         r.a = std::min(b0, b1);
         r.b = std::max(b0, b1);
+        r.extra = regs_of(op);
         break;
       }
       case K_DENSE: {
@@ -1642,9 +1651,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       case K_MCPHASE:
         materialize(reg_bits(op.cl));
         r.kind = Q_PHASE;
-        r.b = 0;  // registers that meet the register part of the predicate
-        for (uint32_t j = 0; j < (1u << R); ++j)
-          if ((reg_tile_bits(j) & op.cl & cur_rs) == (op.cvl & op.cl & cur_rs)) r.b |= 1u << j;
+        r.b = regs_of(op);
         r.u.m[0] = op.pr;
         r.u.m[1] = op.pi;
         break;
@@ -1654,9 +1661,7 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
         // 16-entry tables over groups of four fixed qubits.
         materialize(reg_bits(op.cl | op.xl));
         r.kind = Q_DIAGF;
-        r.b = 0;
-        for (uint32_t j = 0; j < (1u << R); ++j)
-          if ((reg_tile_bits(j) & op.cl & cur_rs) == (op.cvl & op.cl & cur_rs)) r.b |= 1u << j;
+        r.b = regs_of(op);
         int loc[64];
         for (int &v : loc) v = -1;
         for (uint32_t b = 0; b < B; ++b) loc[spos[b]] = static_cast<int>(b);

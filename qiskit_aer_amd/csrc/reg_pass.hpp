@@ -39,7 +39,8 @@ enum RegPassOpKind : uint32_t {
   Q_LDS = 45,       // TileOp primitive extra on the LDS tile
   Q_U1 = 46,        // 2x2 matrix u.m on register bit a
   Q_U1C = 47,       // 2x2 matrix on register bit a where (l & cl) == cvl
-  Q_X = 48,         // X on register bit a where (l & cl) == cvl
+  Q_X = 48,         // X on register bit a where (l & cl) == cvl; gate passes: bit j of b:
+                    // register j meets the register part of the predicate
   Q_Y = 49,         // Y on register bit a where (l & cl) == cvl
   Q_U2 = 50,        // 4x4 matrix pool[extra..] on register bits a (matrix bit 0), b (bit 1);
                     // 16 entries in the state's precision (complex64: two per pool entry)
@@ -63,7 +64,8 @@ enum RegPassOpKind : uint32_t {
                     // phase's lane tables staged in LDS (0: none, read the tables)
   Q_CXR = 61,       // moves registers: those with bit a set change places across bit b
   // gate passes only
-  Q_SWAP = 62,      // register bits a < b change places where (l & cl) == cvl
+  Q_SWAP = 62,      // register bits a < b change places where (l & cl) == cvl; extra: the
+                    // registers that meet the register part of the predicate
   Q_U3 = 63,        // 8x8 matrix pool[extra..] on the register bits but a, the lowest as
                     // matrix bit 0: rows of complex128, or (complex64) four MFMA operands
   Q_DIAGK = 64,     // where (l & cl) == cvl: diagonal of a & 0xFF qubits, entries pool[extra..],
