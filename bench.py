@@ -28,11 +28,11 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 FP64_PEAK_TFLOPS = 78.6  # MI355X published FP64 peak (vector and matrix)
 
 # HBM bytes per tile-pass launch of the default workload (30 qubits, c128),
-# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (profiles/reg_pass_30q_brickwork_c128.md):
-# 2.0 x 8 388 975 KiB fetched (FETCH_SIZE counts half the bytes, calibrated on a
-# kernel that reads the 16 GiB state once) + 16 977 477 KiB written, averaged over
+# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (profiles/gate_pass_30q_brickwork_c128.md):
+# 2.0 x 8 388 857 KiB fetched (FETCH_SIZE counts half the bytes, calibrated on a
+# kernel that reads the 16 GiB state once) + 16 777 483 KiB written, averaged over
 # the passes of the block-fused step at width 2.
-MEASURED_TRAFFIC_30Q_C128 = (2 * 8388975 + 16977477) * 1024
+MEASURED_TRAFFIC_30Q_C128 = (2 * 8388857 + 16777483) * 1024
 
 
 def log(msg: str) -> None:
@@ -458,7 +458,8 @@ def main() -> int:
                      "unit": "GB/s", "frac": c128["kernel_gbs"] / HBM_PEAK_GBS,
                      "traffic": MEASURED_TRAFFIC_30Q_C128 if (n, args.layers) == (30, 40) else None,
                      "algorithmic_bytes_per_launch": c128["sweep_bytes"]},
-        # the same step against the FP64 vector peak (the pass's other bound)
+        # the source circuit's FP64 work against the vector peak (the pass's other
+        # bound); block fusion executes about half of it, so this can exceed 1
         "fp64_compute": {"achieved": fp64_tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": fp64_tflops / FP64_PEAK_TFLOPS,
                          "flops_per_step": u3_per_step * (1 << n) * 16},

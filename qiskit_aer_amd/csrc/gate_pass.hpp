@@ -12,11 +12,16 @@
 // The op loop is an interpreter: host-computed codes name the op together with
 // its register bits, and one comparison tree finds it.
 //
-// Bound by the FP64 units: the 30-qubit brickwork at fusion width 2 runs 24
-// passes of 11.1 ms, 91 % of whose cycles issue vector instructions (4663 per
-// wave, 3140 of them FMAs of 4x4 gates), at 118 VGPRs and four waves per SIMD.
-// Register passes on 2^11 tiles take 29 passes of 13.6 ms for it: 403 against
-// 269 ms a step.  Three waves (150 VGPRs) 281 ms; five (96 VGPRs) spill: 390 ms.
+// complex128 is bound by the FP64 units: the 30-qubit brickwork at fusion width 2
+// runs 24 passes of 10.1 ms (34.4 GB each, 3.4 TB/s), 83 % of whose cycles issue
+// vector instructions (3861 per wave, 3140 of them FMAs of 4x4 gates), at 119
+// VGPRs and four waves per SIMD.  Register passes on 2^11 tiles take 30 passes of
+// 14.1 ms for it: 425 against 244 ms a step.  At an earlier state of 269 ms, three
+// waves (150 VGPRs) took 281 ms, five (96 VGPRs, spills) 390.
+//
+// complex64 runs its 2x2, 4x4 and 8x8 gates on MFMA, at 94 VGPRs and five waves:
+// layers of SU(4) on 29 qubits 88 -> 60.5 ms (16 passes of 3.7 ms, 42 % of the
+// cycles issuing vector instructions), brickwork of 2x2 gates on 27 24.8 -> 18.3.
 #pragma once
 
 #include "reg_pass.hpp"
