@@ -1773,6 +1773,10 @@ void register_program(const std::vector<TileOp> &in, uint32_t B, uint32_t R, uin
       const size_t before = rops.size();
       emit_gate(op, rs);
       if (!gate) continue;
+      if (rops.size() == before) {  // a probe that joined the run before it, or an X that waits
+        if (!tail.empty()) tail.back().touch |= rem[i].touch;
+        continue;
+      }
       // with register moves of other ops made up before it, it touches what they do
       Tail t{rops.size() == before + 1 ? rem[i].touch : rem[i].touch | rs, 0, 0, false};
       if (is_cx(op) && rops.size() == before + 1) {

@@ -287,3 +287,35 @@ def test_replayed_launches_follow_the_probes():
         got = e.saved_expvals()[slot]
         # 4 roundings of 2^-24 of the norm per gate, doubled by the value
         assert abs(got - pauli_value(psi, label(q))) < 2 * len(c.ops) * 4 * 2.0**-24
+
+
+@pytest.mark.parametrize("precision,n,rounds", [("double", 21, 10), ("single", 13, 40)])
+def test_cx_stay_before_the_probes_they_change(precision, n, rounds):
+    """CX, then a run of probes of which a later one sees them, then gates that
+    change the layout: the layout change takes no CX past the run."""
+    print(f"case: CX before probe runs {precision} n={n}", flush=True)
+    rng = np.random.default_rng(n + rounds)
+    prefix = circuits.Circuit(n)
+    e = QubitVector(n, precision)
+    e.initialize()
+    want, slots, gates = [], [], 0
+    for r in range(rounds):
+        c = circuits.Circuit(n)
+        if r == 0:
+            for q in range(n):
+                c.gate("u3", [q], list(rng.uniform(-3, 3, 3)))
+        for q in rng.choice(12, 2, replace=False):
+            c.gate("u3", [int(q)], list(rng.uniform(-3, 3, 3)))
+        a, b, other = (int(x) for x in rng.choice(12, 3, replace=False))
+        c.gate("cx", [a, b])
+        e.apply_ops(c)
+        gates += len(c.ops)
+        prefix.ops.extend(c.ops)
+        _, psi, _ = O.run_circuit(prefix, shots=0, seed=0, fusion=False)
+        for q, p in ((other, "X"), (b, "Z"), (a, "X"), (b, "Y")):
+            lab = "".join(p if n - 1 - i == q else "I" for i in range(n))
+            slots.append(e.save_expval_pauli(list(range(n)), lab, 1.0))
+            want.append(pauli_value(psi, lab))
+    got = e.saved_expvals()[slots]
+    bound = 1e-12 if precision == "double" else 2 * gates * 4 * 2.0**-24
+    assert np.max(np.abs(got - np.array(want))) < bound
