@@ -129,8 +129,7 @@ class Circuit:
         keep = []
         if nops == 0:
             return arr, keep
-        # One list per attribute, into arrays of machine words (several times
-        # faster than numpy reading the objects), and numpy for the rest.
+        # One list per attribute, read into machine words, and numpy for the rest.
         rec = np.frombuffer(arr, dtype=_OP_DTYPE)
         chain = itertools.chain.from_iterable
         types = [o.type for o in ops]
@@ -139,10 +138,10 @@ class Circuit:
         # qubits
         qubits = [o.qubits for o in ops]
         nq = _words("q", list(map(len, qubits)))
-        qflat = array.array("Q", list(chain(qubits)) + [0])
+        qflat = _words("Q", list(chain(qubits)) + [0])
         keep.append(qflat)
         rec["num_qubits"] = nq
-        rec["qubits"] = qflat.buffer_info()[0] + 8 * (np.cumsum(nq) - nq)
+        rec["qubits"] = qflat.ctypes.data + 8 * (np.cumsum(nq) - nq)
         # real parameters: gate angles, then complex matrices as (re, im) pairs
         params = [o.params for o in ops]
         mats = []
@@ -150,10 +149,10 @@ class Circuit:
             params = [p if t == L.OP_GATE else () for p, t in zip(params, types)]
             mats = [i for i, t in enumerate(types) if t != L.OP_GATE and ops[i].matrix is not None]
         npar = _words("q", list(map(len, params)))
-        pflat = array.array("d", list(chain(params)) + [0.0])
+        pflat = _words("d", list(chain(params)) + [0.0])
         keep.append(pflat)
         rec["num_params"] = npar
-        rec["params"] = pflat.buffer_info()[0] + 8 * (np.cumsum(npar) - npar)
+        rec["params"] = pflat.ctypes.data + 8 * (np.cumsum(npar) - npar)
         for i in mats:
             m = np.array(ops[i].matrix, dtype=np.complex128)  # packed ops do not follow later changes
             keep.append(m)
@@ -185,7 +184,13 @@ class Circuit:
 
 
 def _words(code: str, values: list) -> np.ndarray:
-    return np.frombuffer(array.array(code, values), dtype=code)
+    """The values as machine words.  array.array reads a list several times
+    faster than numpy, but refuses qubits given as floats (2.0), bools or text,
+    which numpy converts."""
+    try:
+        return np.frombuffer(array.array(code, values), dtype=code)
+    except TypeError:
+        return np.fromiter(values, dtype=code, count=len(values))
 
 
 # Field layout of AerhipOp (include/aerhip.h) for filling packed records.
