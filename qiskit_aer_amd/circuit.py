@@ -154,7 +154,10 @@ class Circuit:
         rec["num_params"] = npar
         rec["params"] = pflat.ctypes.data + 8 * (np.cumsum(npar) - npar)
         for i in mats:
-            m = np.array(ops[i].matrix, dtype=np.complex128)  # packed ops do not follow later changes
+            m = ops[i].matrix
+            if m.ndim > 1 and m.size != m.shape[-1]:
+                raise ValueError("the matrix of an op is a vector, its columns one after the other")
+            m = np.array(m, dtype=np.complex128)  # packed ops do not follow later changes
             keep.append(m)
             rec["num_params"][i] = m.size
             rec["params"][i] = m.ctypes.data

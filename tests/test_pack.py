@@ -42,3 +42,26 @@ def test_negative_qubits_are_refused():
     c.pauli("X", [-1])
     with pytest.raises(OverflowError):
         c.pack()
+
+
+@pytest.mark.parametrize("shape", [(2, 2), (4, 4), (2, 8)])
+def test_square_matrices_are_refused(shape):
+    """An op's matrix is a vector; the words of a square array could be in
+    either order."""
+    c = Circuit(2)
+    c.ops = [Op(L.OP_MATRIX, "unitary", (0, 1), matrix=np.zeros(shape, dtype=complex).T.copy().T)]
+    with pytest.raises(ValueError):
+        c.pack()
+
+
+@pytest.mark.parametrize("values", [np.arange(8.0)[::-2], np.arange(8.0)[::2].astype(np.complex64),
+                                    (np.arange(4.0) + 1j).reshape(1, 4), np.array(3.0 + 4.0j)])
+def test_vectors_of_any_stride_and_type(values):
+    c = Circuit(2)
+    c.ops = [Op(L.OP_DIAGONAL, "diagonal", (0, 1), matrix=values)]
+    arr, keep = c.pack()
+    flat = values.reshape(-1)
+    assert arr[0].num_params == flat.size
+    got = [complex(arr[0].params[2 * k], arr[0].params[2 * k + 1]) for k in range(flat.size)]
+    assert got == [complex(v) for v in flat]
+    del keep
