@@ -100,8 +100,11 @@ class WorkspacePool {
       w = sets_.front();
       sets_.erase(sets_.begin());
     }
+    int device = 0;
+    (void)hipGetDevice(&device);
     (void)hipSetDevice(w.device);
     w.release();
+    (void)hipSetDevice(device);
   }
 
   void drain() {
