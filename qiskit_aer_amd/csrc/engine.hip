@@ -3081,7 +3081,6 @@ void Engine::probabilities_t(const std::vector<uint32_t> &qubits, double *out) {
   MarginalDesc md;
   std::memset(&md, 0, sizeof(md));
   md.nq = nq;
-  md.inner = 1ull << (n_ - nq);
   const uint32_t low = std::min<uint32_t>(6, n_);
   uint32_t nh = 0;  // measured qubits above the lane qubits
   for (uint32_t i = 0; i < nq; ++i) {
@@ -3095,7 +3094,7 @@ void Engine::probabilities_t(const std::vector<uint32_t> &qubits, double *out) {
   const uint64_t nchunk = std::min<uint64_t>(std::max<uint64_t>(1, inner_h / 32), std::max<uint64_t>(1, (1ull << 14) >> nh));
   md.nchunk = static_cast<uint32_t>(nchunk);
   const uint64_t items = nchunk << nh;
-  ensure_partial(outcomes * nchunk + outcomes);
+  ensure_partial(nchunk > 1 ? outcomes * nchunk + outcomes : outcomes);
   k_marginal<T><<<static_cast<uint32_t>(std::min<uint64_t>((items + 3) / 4, 1u << 16)), kThreads, 0, stream_>>>(
       sv, md, low, items, inner_h / nchunk, d_partial_);
   dout = d_partial_;
