@@ -16,14 +16,17 @@ namespace aerhip {
 
 struct BatchCircuit {
   uint64_t sv_off;      // first amplitude of the circuit's state in the batch buffer
-  uint64_t part_off;    // probe partials: partial[part_off + probe * tiles + tile]
   uint32_t num_qubits;
   uint32_t pass_begin;  // passes[pass_begin .. + pass_count)
   uint32_t pass_count;
-  uint32_t probe_base;  // saved values go to values[probe_base .. + num_probes)
-  uint32_t num_probes;
   uint32_t tile_log;    // log2 of its tiles
 };
+
+// Probes a pass of a circuit of several tiles may hold.  Their partials stand in
+// memory during the launch, a double per tile: 256 are 1/16 of the state.  On 28
+// qubits (complex128) 39 probes add 1.0 ms to a sweep of 0.7, so that cutting a
+// pass at 256 adds a tenth to it.
+constexpr uint32_t kBatchProbes = 256;
 
 // Circuits [first, first + count) of one size, whose tiles are workgroups
 // begin .. begin + (count << tile_log).
@@ -36,8 +39,7 @@ struct BatchGroups {
   BatchGroup g[kBatchGroups];
 };
 
-// |0> in every state (buffer zeroed first) and no circuit's partials unwritten:
-// every probe writes one partial per tile.
+// |0> in every state (buffer zeroed first).
 template <typename T>
 __global__ void k_batch_ones(cx<T> *__restrict__ states, const BatchCircuit *__restrict__ circ, uint64_t count) {
   const uint64_t i = blockIdx.x * (uint64_t)kThreads + threadIdx.x;
@@ -73,7 +75,7 @@ __attribute__((amdgpu_waves_per_eu(reg_pass_waves<T, B, R>()))) void k_batch(
   const PassDesc *pd = passes + c.pass_begin + p;
   if (pd->batch_class != (V == V_FULL ? 1u : 0u)) return;
   cx<T> *sv = states + c.sv_off;
-  const ProbeSink sink{partial + c.part_off, t, 1ull << tl};
+  const ProbeSink sink{partial + pd->part_off, t, 1ull << tl};
   if constexpr (V == V_PROBES) {
     reg_tile<T, B, R, 16, V_PROBES>(sv, pd, rops, tops, pool, sink, t, lds, mat, doff, red, dlt);
   } else if (pd->kind == 2) {

@@ -128,6 +128,9 @@ struct PassDesc {
   uint32_t ncomp;     // number of qubits outside the tile
   uint32_t readonly;  // 1: the pass only reads the state (probes); nothing is written back
   uint32_t batch_class; // batched circuits: 0 = runs in k_batch<V_PROBES>, 1 = in k_batch<V_FULL>
+  uint64_t part_off;    // batched circuits: the pass's probe partials, partial[part_off + row * tiles + tile],
+  uint32_t probe_at;    // whose rows' values go to values[slots[probe_at + row]],
+  uint32_t probes;      // row < probes
   uint8_t spos[16];   // tile qubits, ascending
   uint8_t comp[64];   // qubits outside the tile, ascending
 };

@@ -1907,10 +1907,16 @@ std::vector<PassPlan> Engine::gather_sweeps(std::vector<PassPlan> plans) const {
     sweep.solo = true;
     for (; i < j; ++i) {
       PassPlan &pp = plans[i];
-      if (pp.solo || (sweeps && pp.prims.size() <= 2))
-        sweep.prims.insert(sweep.prims.end(), pp.prims.begin(), pp.prims.end());
-      else
+      if (!pp.solo && !(sweeps && pp.prims.size() <= 2)) {
         out.push_back(std::move(pp));
+        continue;
+      }
+      if (sweep.prims.size() + pp.prims.size() > probe_limit_) {
+        out.push_back(std::move(sweep));
+        sweep = PassPlan();
+        sweep.solo = true;
+      }
+      sweep.prims.insert(sweep.prims.end(), pp.prims.begin(), pp.prims.end());
     }
     if (!sweep.prims.empty()) out.push_back(std::move(sweep));
   }
@@ -1982,8 +1988,9 @@ std::vector<PassPlan> Engine::plan() const {
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
         size_t count = 0;
+        uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
         for (const Pending &p : remaining) {
-          bool fits = !(p.touch & blocked) && !(p.probe && nonunitary_blocked) && (!gate || p.gate);
+          bool fits = !(p.touch & blocked) && !(p.probe && (nonunitary_blocked || !probes_left)) && (!gate || p.gate);
           if (fits) {
             const uint64_t ns = s | p.tmask;
             fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
@@ -1991,6 +1998,7 @@ std::vector<PassPlan> Engine::plan() const {
           }
           if (fits) {
             ++count;
+            probes_left -= p.probe;
             lds |= p.lds;
             if (take) take->prims.push_back(p.idx);
             continue;
@@ -3272,6 +3280,26 @@ double Engine::expval_pauli(const std::vector<uint32_t> &qubits, const std::stri
 
 namespace aerhip {
 
+// Calls f on the slot of every probe in a pass.
+template <typename F>
+void for_each_probe(Program &p, const PassDesc &d, F f) {
+  auto op = [&](TileOp &t) {
+    if (t.kind == K_PROBE) f(t.npairs);
+  };
+  if (d.kind == 0 || d.kind == 3) {
+    for (uint32_t k = 0; k < d.nops; ++k) op(p.ops[d.op_begin + k]);
+  } else if (d.kind == 2) {
+    for (uint32_t k = 0; k < d.nops; ++k) {
+      const ROp<double> &r = p.rops[d.op_begin + k];
+      const uint32_t kk = r.kind & ~F_ALL;
+      if (kk == Q_LDS) op(p.ops[r.extra]);
+      if (kk != Q_PROBE) continue;
+      RProbe *pr = reinterpret_cast<RProbe *>(p.pool.data() + r.extra);
+      for (uint32_t j = 0; j < r.a; ++j) f(pr[j].slot);
+    }
+  }
+}
+
 // Runs the queues of `count` planning engines (same precision) as one batch:
 // every circuit starts from |0>; the saved expectation values of circuit i
 // are written to values[offset_i ..], in circuit order and slot order.
@@ -3287,17 +3315,31 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   // Plan every circuit on the host threads (the handles are independent),
   // then concatenate the programs in circuit order.
   std::vector<Program> parts(count);
-  std::vector<uint32_t> nprobes(count);
+  // The kernel of every pass (PassDesc::batch_class) and its probes, numbered
+  // within it: slots[i] has their values, pass after pass.
+  std::vector<std::vector<uint32_t>> slots(count);
   parallel_for(count, [&](uint64_t i) {
-    nprobes[i] = static_cast<uint32_t>(engines[i]->probes_queued());
+    const uint64_t nprobes = engines[i]->probes_queued();
+    engines[i]->limit_probes(kBatchProbes);
     engines[i]->emit_program(parts[i]);
+    for (PassDesc &d : parts[i].passes) {
+      d.batch_class = prec == AERHIP_PRECISION_DOUBLE && d.kind == 2 &&
+                              !has_gates(pass_kernel(prec, d, parts[i].rops).variant) ? 0u : 1u;
+      d.probe_at = static_cast<uint32_t>(slots[i].size());
+      for_each_probe(parts[i], d, [&](uint32_t &slot) {
+        slots[i].push_back(slot);
+        slot = d.probes++;
+      });
+    }
+    if (slots[i].size() != nprobes) throw std::logic_error("aerhip: a probe in no pass or in two");
   });
   // Offsets of each circuit's passes / ops / register ops / pool entries in
   // the concatenated program.
   std::vector<uint64_t> pass_at(count + 1, 0), op_at(count + 1, 0), rop_at(count + 1, 0),
       pool_at(count + 1, 0);
   std::vector<BatchCircuit> circ(count);
-  uint64_t sv_off = 0, probe_off = 0, part_off = 0;
+  std::vector<uint64_t> probe_at(count + 1, 0);
+  uint64_t sv_off = 0;
   for (uint64_t i = 0; i < count; ++i) {
     const Program &p = parts[i];
     for (const PassDesc &d : p.passes)
@@ -3313,15 +3355,12 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     c.num_qubits = engines[i]->num_qubits();
     c.pass_begin = static_cast<uint32_t>(pass_at[i]);
     c.pass_count = static_cast<uint32_t>(p.passes.size());
-    c.probe_base = static_cast<uint32_t>(probe_off);
-    c.num_probes = nprobes[i];
     c.tile_log = c.num_qubits - engines[i]->tile_bits();
-    c.part_off = part_off;
     sv_off += align_up(1ull << c.num_qubits, 256);
-    part_off += static_cast<uint64_t>(c.num_probes) << c.tile_log;
-    probe_off += c.num_probes;
+    probe_at[i + 1] = probe_at[i] + slots[i].size();
   }
-  if (op_at[count] > UINT32_MAX || rop_at[count] > UINT32_MAX || pool_at[count] > UINT32_MAX)
+  const uint64_t num_probes = probe_at[count];
+  if (op_at[count] > UINT32_MAX || rop_at[count] > UINT32_MAX || pool_at[count] > UINT32_MAX || num_probes > UINT32_MAX)
     throw std::invalid_argument("aerhip: batch program too large");
   // By size, then by number of passes: the circuits of one size that have a
   // pass p are a range for every p.
@@ -3332,14 +3371,19 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   uint32_t max_passes = 0;
   for (const BatchCircuit &c : sorted) max_passes = std::max(max_passes, c.pass_count);
   // Per pass index: which kernels its passes need (bit 0 k_batch<V_PROBES>,
-  // complex128 only; bit 1 k_batch<V_FULL>).
+  // complex128 only; bit 1 k_batch<V_FULL>), and the probe partials, which take
+  // the place of those of the pass before.
   std::vector<uint32_t> classes(max_passes, 0);
-  for (Program &p : parts)
-    for (size_t k = 0; k < p.passes.size(); ++k) {
-      PassDesc &d = p.passes[k];
-      d.batch_class = prec == AERHIP_PRECISION_DOUBLE && d.kind == 2 && !has_gates(pass_kernel(prec, d, p.rops).variant) ? 0u : 1u;
+  std::vector<uint64_t> partials(max_passes, 0);
+  for (uint64_t i = 0; i < count; ++i)
+    for (size_t k = 0; k < parts[i].passes.size(); ++k) {
+      PassDesc &d = parts[i].passes[k];
       classes[k] |= 1u << d.batch_class;
+      d.probe_at += static_cast<uint32_t>(probe_at[i]);
+      d.part_off = partials[k];
+      partials[k] += static_cast<uint64_t>(d.probes) << circ[i].tile_log;
     }
+  const uint64_t part_len = max_passes ? *std::max_element(partials.begin(), partials.end()) : 0;
 
   const size_t amp = prec == AERHIP_PRECISION_DOUBLE ? 16 : 8;
   const size_t circ_bytes = count * sizeof(BatchCircuit);
@@ -3347,7 +3391,8 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   const size_t ops_off = align_up(pass_off + pass_at[count] * sizeof(PassDesc), 256);
   const size_t rops_off = align_up(ops_off + op_at[count] * sizeof(TileOp), 256);
   const size_t pool_off = align_up(rops_off + rop_at[count] * sizeof(ROp<double>), 256);
-  const size_t total = pool_off + pool_at[count] * sizeof(cd) + 16;
+  const size_t slots_off = align_up(pool_off + pool_at[count] * sizeof(cd), 256);
+  const size_t total = slots_off + num_probes * sizeof(uint32_t) + 16;
   // The upload image, written in place: each circuit's part is copied to its
   // offsets with its indices rebased (pass op ranges, TileOp pool offsets,
   // the pool offsets and TileOp indices carried by register ops).
@@ -3356,6 +3401,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   auto *hp = reinterpret_cast<PassDesc *>(h.get() + pass_off);
   auto *ho = reinterpret_cast<TileOp *>(h.get() + ops_off);
   auto *hpool = reinterpret_cast<cd *>(h.get() + pool_off);
+  auto *hslots = reinterpret_cast<uint32_t *>(h.get() + slots_off);
   parallel_for(count, [&](uint64_t i) {
     Program &p = parts[i];
     const uint32_t ob = static_cast<uint32_t>(op_at[i]), rb = static_cast<uint32_t>(rop_at[i]),
@@ -3365,6 +3411,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
       d.op_begin += d.kind == 2 || d.kind == 5 ? rb : ob;
       hp[pass_at[i] + k] = d;
     }
+    for (size_t k = 0; k < slots[i].size(); ++k) hslots[probe_at[i] + k] = static_cast<uint32_t>(probe_at[i]) + slots[i][k];
     for (size_t k = 0; k < p.ops.size(); ++k) {
       TileOp t = p.ops[k];
       t.off += pb;
@@ -3401,7 +3448,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     AERHIP_CHECK(hipEventCreate(&e0));
     AERHIP_CHECK(hipEventCreate(&e1));
     if (total > ws.program.bytes) WorkspacePool::grow(ws.program, total);
-    const size_t probe_bytes = (probe_off + part_off + 1) * sizeof(double);
+    const size_t probe_bytes = (num_probes + part_len + 1) * sizeof(double);
     if (probe_bytes > ws.probes.bytes) WorkspacePool::grow(ws.probes, probe_bytes);
     void *const d_states = ws.state.p, *const d_prog = ws.program.p;
     double *const d_probes = static_cast<double *>(ws.probes.p);
@@ -3417,6 +3464,9 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
       const auto *dr = reinterpret_cast<const ROp<T> *>(d + rops_off);
       const auto *dops = reinterpret_cast<const TileOp *>(d + ops_off);
       const auto *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
+      const auto *dslots = reinterpret_cast<const uint32_t *>(d + slots_off);
+      double *const partial = d_probes + num_probes;
+      const dim3 sums(static_cast<uint32_t>(count), std::max<uint32_t>(1, 64 / static_cast<uint32_t>(std::min<uint64_t>(count, 64))));
       k_fill_basis<T><<<grid_for(sv_off, 16384), kThreads, 0, st>>>(sv, sv_off, ~0ull);
       k_batch_ones<T><<<grid_for(count, 1u << 30), kThreads, 0, st>>>(sv, dc, count);
       for (uint32_t p = 0; p < max_passes; ++p) {
@@ -3437,12 +3487,12 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
         if constexpr (sizeof(T) == 8)
           if (classes[p] & 1u)
             k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(
-                sv, dc, gr, p, dp, dr, dops, dpool, d_probes + probe_off);
+                sv, dc, gr, p, dp, dr, dops, dpool, partial);
         if (classes[p] & 2u)
           k_batch<T, B, R, V_FULL><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops, dpool,
-                                                                                   d_probes + probe_off);
+                                                                                   partial);
+        if (partials[p]) k_batch_sums<<<sums, kThreads, 0, st>>>(dc, p, dp, dslots, partial, d_probes);
       }
-      k_batch_sums<<<static_cast<uint32_t>(count), kThreads, 0, st>>>(dc, d_probes + probe_off, d_probes);
     };
     if (prec == AERHIP_PRECISION_DOUBLE)
       run(0.0, std::integral_constant<int, kTileBitsC128>{}, std::integral_constant<int, 3>{});
@@ -3450,7 +3500,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
       run(0.0f, std::integral_constant<int, kTileBitsC64>{}, std::integral_constant<int, 4>{});
     AERHIP_CHECK(hipGetLastError());
     AERHIP_CHECK(hipEventRecord(e1, st));
-    AERHIP_CHECK(hipMemcpyAsync(values, d_probes, probe_off * sizeof(double), hipMemcpyDeviceToHost, st));
+    AERHIP_CHECK(hipMemcpyAsync(values, d_probes, num_probes * sizeof(double), hipMemcpyDeviceToHost, st));
     AERHIP_CHECK(hipStreamSynchronize(st));
     float ms = 0;
     AERHIP_CHECK(hipEventElapsedTime(&ms, e0, e1));

@@ -159,6 +159,8 @@ class Engine {
   // Gate passes for a planning handle (its program then runs through
   // launch_pass; the batched-circuit kernels do not hold them).
   void use_gate_passes() { gate_passes_ = true; }
+  // At most `count` probes in a pass over several tiles.
+  void limit_probes(uint32_t count) { probe_limit_ = count; }
 
  private:
   void check_qubits(const std::vector<uint32_t> &qubits) const;
@@ -192,6 +194,7 @@ class Engine {
   int device_;
   bool plan_only_ = false;
   bool gate_passes_ = true;
+  uint32_t probe_limit_ = ~0u;
   uint64_t size_;
   void *sv_ = nullptr;
   hipStream_t stream_ = nullptr;

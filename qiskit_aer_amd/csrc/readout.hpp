@@ -52,19 +52,24 @@ inline void sum_rows(const double *partial, uint64_t rows, uint32_t cols, double
     k_sum_rows<1024><<<static_cast<uint32_t>(rows), 1024, 0, stream>>>(partial, cols, out);
 }
 
-// values[probe_base + i] = sum of the tile partials of probe i: a workgroup per
-// circuit, a wave per probe.
-__global__ __launch_bounds__(kThreads) void k_batch_sums(const BatchCircuit *__restrict__ circ,
+// The values of the probes in pass p of every circuit, each the sum of its tile
+// partials: gridDim.y workgroups per circuit, a wave per probe.
+__global__ __launch_bounds__(kThreads) void k_batch_sums(const BatchCircuit *__restrict__ circ, uint32_t p,
+                                                      const PassDesc *__restrict__ passes,
+                                                      const uint32_t *__restrict__ slots,
                                                       const double *__restrict__ partial,
-                                                               double *__restrict__ values) {
+                                                      double *__restrict__ values) {
   const BatchCircuit &c = circ[blockIdx.x];
+  if (p >= c.pass_count) return;
+  const PassDesc &pd = passes[c.pass_begin + p];
   const uint64_t tiles = 1ull << c.tile_log;
-  for (uint32_t i = threadIdx.x >> 6; i < c.num_probes; i += kThreads / 64) {
-    const double *row = partial + c.part_off + i * tiles;
+  constexpr uint32_t NW = kThreads / 64;
+  for (uint32_t i = blockIdx.y * NW + (threadIdx.x >> 6); i < pd.probes; i += gridDim.y * NW) {
+    const double *row = partial + pd.part_off + i * tiles;
     double s = 0;
     for (uint64_t k = threadIdx.x & 63u; k < tiles; k += 64) s += row[k];
     s = wave_sum(s);
-    if ((threadIdx.x & 63u) == 0) values[c.probe_base + i] = s;
+    if ((threadIdx.x & 63u) == 0) values[slots[pd.probe_at + i]] = s;
   }
 }
 
