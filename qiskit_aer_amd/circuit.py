@@ -129,7 +129,8 @@ class Circuit:
         keep = []
         if nops == 0:
             return arr, keep
-        # One list per attribute, read into machine words, and numpy for the rest.
+        # One list per attribute, into arrays of machine words (several times
+        # faster than numpy reading the objects), and numpy for the rest.
         rec = np.frombuffer(arr, dtype=_OP_DTYPE)
         chain = itertools.chain.from_iterable
         types = [o.type for o in ops]
@@ -138,10 +139,10 @@ class Circuit:
         # qubits
         qubits = [o.qubits for o in ops]
         nq = _words("q", list(map(len, qubits)))
-        qflat = _words("Q", list(chain(qubits)) + [0])
+        qflat, at = _buffer("Q", list(chain(qubits)) + [0])
         keep.append(qflat)
         rec["num_qubits"] = nq
-        rec["qubits"] = qflat.ctypes.data + 8 * (np.cumsum(nq) - nq)
+        rec["qubits"] = at + 8 * (np.cumsum(nq) - nq)
         # real parameters: gate angles, then complex matrices as (re, im) pairs
         params = [o.params for o in ops]
         mats = []
@@ -149,10 +150,10 @@ class Circuit:
             params = [p if t == L.OP_GATE else () for p, t in zip(params, types)]
             mats = [i for i, t in enumerate(types) if t != L.OP_GATE and ops[i].matrix is not None]
         npar = _words("q", list(map(len, params)))
-        pflat = _words("d", list(chain(params)) + [0.0])
+        pflat, at = _buffer("d", list(chain(params)) + [0.0])
         keep.append(pflat)
         rec["num_params"] = npar
-        rec["params"] = pflat.ctypes.data + 8 * (np.cumsum(npar) - npar)
+        rec["params"] = at + 8 * (np.cumsum(npar) - npar)
         for i in mats:
             m = ops[i].matrix
             if m.ndim > 1 and m.size != m.shape[-1]:
@@ -187,13 +188,19 @@ class Circuit:
 
 
 def _words(code: str, values: list) -> np.ndarray:
-    """The values as machine words.  array.array reads a list several times
-    faster than numpy, but refuses qubits given as floats (2.0), bools or text,
-    which numpy converts."""
+    return np.frombuffer(array.array(code, values), dtype=code)
+
+
+def _buffer(code: str, values: list):
+    """The values as machine words, and their address.  array.array reads a list
+    several times faster than numpy, but refuses qubits given as floats (2.0),
+    bools or text, which numpy converts."""
     try:
-        return np.frombuffer(array.array(code, values), dtype=code)
+        words = array.array(code, values)
+        return words, words.buffer_info()[0]
     except TypeError:
-        return np.fromiter(values, dtype=code, count=len(values))
+        words = np.fromiter(values, dtype=code, count=len(values))
+        return words, words.ctypes.data
 
 
 # Field layout of AerhipOp (include/aerhip.h) for filling packed records.
