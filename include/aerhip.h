@@ -158,6 +158,11 @@ int aerhip_qv_set_fusion(aerhip_qv *qv, int enable, int max_qubit, int threshold
  * replayed. */
 int aerhip_qv_graph_stats(aerhip_qv *qv, uint64_t *captures, uint64_t *replays);
 
+/* No counterpart in the reference (it has one kernel per gate).  How many
+ * passes of this handle ran as gate passes (tiles of 2^12 amplitudes, 16 per
+ * thread), and how many CX and X their layout changes took along. */
+int aerhip_qv_gate_pass_stats(aerhip_qv *qv, uint64_t *passes, uint64_t *cx);
+
 /* Block fusion, the engine's form of Aer's fusion of gates into dense
  * matrices (src/transpile/fusion.hpp:849-1136, fusion_max_qubit): unitary
  * gates whose qubits stay within `width` qubits (2..5; 0 turns it off, the

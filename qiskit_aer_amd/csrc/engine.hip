@@ -2545,6 +2545,11 @@ void Engine::emit_program(Program &prog) {
       register_program(pops, ns, R, low_bits_, prec_ == AERHIP_PRECISION_SINGLE, pp.gate, pd.spos, prog.pool, rops,
                        ops, &stats_.gathers);
       pd.nops = static_cast<uint32_t>(rops.size()) - pd.op_begin;
+      if (pp.gate) {
+        ++stats_.gate_passes;
+        for (uint32_t k = 0; k < pd.nops; ++k)
+          if (rops[pd.op_begin + k].kind == Q_RELAYOUT) stats_.relayout_cx += rops[pd.op_begin + k].a;
+      }
       if (pd.readonly) rops.back().extra = 1;  // the final STORE writes nothing
       validate_register_program(rops.data() + pd.op_begin, pd.nops, ns, R, pd.spos, ops.size(),
                                 prog.pool);
@@ -4018,6 +4023,14 @@ int aerhip_qv_graph_stats(aerhip_qv *qv, uint64_t *captures, uint64_t *replays) 
     if (!captures || !replays) throw std::invalid_argument("aerhip: null argument");
     *captures = E(qv).stats().graph_captures;
     *replays = E(qv).stats().graph_replays;
+  });
+}
+
+int aerhip_qv_gate_pass_stats(aerhip_qv *qv, uint64_t *passes, uint64_t *cx) {
+  return guard([&] {
+    if (!passes || !cx) throw std::invalid_argument("aerhip: null argument");
+    *passes = E(qv).stats().gate_passes;
+    *cx = E(qv).stats().relayout_cx;
   });
 }
 

@@ -57,6 +57,8 @@ struct EngineStats {
   uint64_t fused = 0;          // gate primitives merged into fused diagonals
   uint64_t graph_captures = 0; // flushes whose pass launches were captured into a HIP graph
   uint64_t graph_replays = 0;  // flushes that replayed the captured graph
+  uint64_t gate_passes = 0;
+  uint64_t relayout_cx = 0;    // CX and X in the layout changes of gate passes
 };
 
 class Engine {

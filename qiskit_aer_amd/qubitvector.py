@@ -142,6 +142,12 @@ class QubitVector:
         L.check(self._L.aerhip_qv_graph_stats(self._h, C.byref(c), C.byref(r)))
         return int(c.value), int(r.value)
 
+    def gate_pass_stats(self) -> tuple:
+        """(passes run as gate passes, CX and X taken along by their layout changes)."""
+        p, c = C.c_uint64(), C.c_uint64()
+        L.check(self._L.aerhip_qv_gate_pass_stats(self._h, C.byref(p), C.byref(c)))
+        return int(p.value), int(c.value)
+
     def fused_count(self) -> int:
         out = C.c_uint64()
         L.check(self._L.aerhip_qv_fused_count(self._h, C.byref(out)))
