@@ -23,6 +23,13 @@ constexpr size_t kMaxQueue = 4096;      // flush threshold of the gate queue
 // fusion width 2 take 1.19 against 1.13 ms on 21 qubits, 1.65 against 1.30 on 22,
 // but 1.10 against 1.15 on 20.
 constexpr uint32_t kGateMinQubits = 21;
+// Programs of 2x2 gates, X and phases alone from 2^10 tiles on.  With fewer a
+// pass waits for its ops one after the other, which the lean register pass reads
+// one op ahead.  Kernel time of 8 layers of brickwork without block fusion, gate
+// against register passes: complex64, 14 qubits 143 against 118 us, 20 qubits 211
+// against 179, 21 qubits 247 against 194, 22 qubits 284 against 299; complex128,
+// 21 qubits 257 against 209, 22 qubits 327 against 412.
+constexpr uint64_t kLeanGateTiles = 1u << 10;
 
 inline uint64_t bit(uint32_t q) { return 1ull << q; }
 
@@ -1955,6 +1962,7 @@ std::vector<PassPlan> Engine::plan() const {
     if (!p.solo && static_cast<uint32_t>(__builtin_popcountll(p.tmask | lowmask)) > nb)
       throw std::logic_error("aerhip: a primitive mixes more qubits than a tile holds");
   const uint32_t gate_bits = gate_tile_bits();
+  const bool few_tiles = gate_bits && states_ << (n_ - gate_bits) < kLeanGateTiles;
   while (seg_begin < queue_.size()) {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
@@ -1963,15 +1971,19 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t tmask, touch;
       uint32_t idx;
       bool probe, unitary, gate;
-      bool lds;  // a register pass spills the tile for it, a gate pass does not
+      bool lds;   // a register pass spills the tile for it, a gate pass does not
+      bool lean;  // the lean register pass runs it
     };
     std::vector<Pending> remaining;
-    bool probes = false;
+    bool probes = false, all_lean = true;
     for (size_t i = seg_begin; i < seg_end; ++i) probes |= queue_[i].kind == K_PROBE;
     for (size_t i = seg_begin; i < seg_end; ++i) {
       const Prim &p = queue_[i];
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
-                                  gate_bits && gate_prim(p, probes), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2)});
+                                  gate_bits && gate_prim(p, probes), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2),
+                                  (p.kind == K_DENSE1 && p.ctrl.empty()) || p.kind == K_MCX || p.kind == K_MCPHASE ||
+                                      (p.kind == K_DIAG && p.q.size() == 1)});
+      all_lean = all_lean && remaining.back().lean;
     }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
@@ -1981,9 +1993,10 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t active = 0;
       for (const Pending &p : remaining) active |= p.touch;
       // A gate pass takes only what its kernel runs.
-      bool lds = false;  // whether the last scan took an `lds` primitive
+      bool lds = false, lean = true;  // whether the last scan took an `lds` primitive, and lean ones alone
       auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
         lds = false;
+        lean = true;
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
@@ -2000,6 +2013,7 @@ std::vector<PassPlan> Engine::plan() const {
             ++count;
             probes_left -= p.probe;
             lds |= p.lds;
+            lean = lean && p.lean;
             if (take) take->prims.push_back(p.idx);
             continue;
           }
@@ -2026,14 +2040,14 @@ std::vector<PassPlan> Engine::plan() const {
       struct Tile {
         size_t count = 0;
         uint64_t seed = 0;
-        bool lds = false;
+        bool lds = false, lean = true;
       };
       auto best_tile = [&](uint32_t c, bool g) {
         Tile t;
         t.seed = lowmask;
         auto candidate = [&](uint64_t s0) {
           const size_t k = scan(c, g, s0, nullptr, nullptr);
-          if (k > t.count) t = Tile{k, s0, lds};
+          if (k > t.count) t = Tile{k, s0, lds, lean};
         };
         candidate(lowmask);
         const uint32_t w = c - low_bits_;
@@ -2044,9 +2058,10 @@ std::vector<PassPlan> Engine::plan() const {
       Tile best = best_tile(nb, false);
       uint32_t cap = nb;
       bool gate = false;
-      if (gate_bits) {
+      if (gate_bits && !(few_tiles && all_lean)) {
         const Tile t = best_tile(gate_bits, true);
         gate = best.lds ? 2 * t.count >= best.count : t.count > best.count || (t.count == best.count && t.count > 4);
+        if (few_tiles && best.lean && t.lean) gate = false;
         if (gate) {
           best = t;
           cap = gate_bits;
@@ -3539,7 +3554,7 @@ class MultiState {
     // would move by 1e-7 with the order that gate passes use, as accurate, but
     // not the values callers have had: those states keep register passes.
     if (prec_ == AERHIP_PRECISION_DOUBLE)
-      for (Engine *e : planners_) e->use_gate_passes();
+      for (Engine *e : planners_) e->use_gate_passes(planners_.size());
     AERHIP_CHECK(hipSetDevice(device_));
     ws_ = WorkspacePool::get().take(device_, planners_.size() * (1ull << n_) * amp_bytes());
     states_ = ws_.state.p;

@@ -160,7 +160,10 @@ class Engine {
   uint64_t probes_queued() const { return probes_queued_; }
   // Gate passes for a planning handle (its program then runs through
   // launch_pass; the batched-circuit kernels do not hold them).
-  void use_gate_passes() { gate_passes_ = true; }
+  void use_gate_passes(uint64_t states) {
+    gate_passes_ = true;
+    states_ = states;
+  }
   // At most `count` probes in a pass over several tiles.
   void limit_probes(uint32_t count) { probe_limit_ = count; }
 
@@ -196,6 +199,7 @@ class Engine {
   int device_;
   bool plan_only_ = false;
   bool gate_passes_ = true;
+  uint64_t states_ = 1;  // states a pass of the program runs over
   uint32_t probe_limit_ = ~0u;
   uint64_t size_;
   void *sv_ = nullptr;

@@ -67,3 +67,40 @@ def test_probes(precision, n):
     bound = 1e-12 if precision == "double" else 2 * len(c.ops) * 16 * 2.0**-24
     assert np.max(np.abs(got - [pauli_value(psi, lab) for lab in labels])) < bound
     assert e.gate_pass_stats()[0] > 0
+
+
+def lean_gates(n, seed):
+    """Two layers of 2x2 gates, CX and phases on a window of 12 qubits."""
+    rng = np.random.default_rng(seed)
+    c = circuits.Circuit(n)
+    for layer in range(2):
+        for q in range(12):
+            c.gate("u3", [n - 1 - q], list(rng.uniform(-3, 3, 3)))
+        for q in range(layer, 11, 2):
+            c.gate("cx", [n - 1 - q, n - 2 - q])
+        for q in range(3):
+            c.gate("cp", [n - 1 - q, n - 6 - q], [float(rng.uniform(-3, 3))])
+            c.gate("rz", [n - 2 - q], [float(rng.uniform(-3, 3))])
+    return c
+
+
+@pytest.mark.parametrize("precision", ["double", "single"])
+@pytest.mark.parametrize("n,taken", [(13, False), (21, False), (22, True)])
+def test_lean_gates_from_1024_tiles_on(precision, n, taken):
+    """With fewer tiles a pass of 2x2 gates, X and phases is a register pass."""
+    print(f"case: planned lean gates {precision} n={n}", flush=True)
+    passes, _ = run(lean_gates(n, 54), n, precision)
+    assert (passes > 0) == taken
+
+
+def test_lean_passes_beside_others_with_few_tiles():
+    """The lean stretch of a circuit runs in register passes, the 4x4 gates in
+    gate passes."""
+    n = 21
+    print("case: planned lean and 4x4 gates", flush=True)
+    c = lean_gates(n, 55)
+    rng = np.random.default_rng(56)
+    for q in range(8):
+        c.unitary(D.random_unitary(4, rng), [q, q + 1])
+    passes, _ = run(c, n, "double")
+    assert passes > 0
