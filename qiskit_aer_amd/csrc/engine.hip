@@ -3166,15 +3166,15 @@ void Engine::sample_t(const std::vector<double> &rnds, uint64_t *out) {
     const uint32_t sbits = std::min<uint32_t>(blockbits, 10);
     const uint64_t nruns = size_ >> sbits;
     const uint64_t nblocks = 1ull << isz;
-    ensure_partial(nruns + 2 * nblocks);
+    const uint64_t rpb = nruns / nblocks;  // runs per index block
+    ensure_partial(nruns + (rpb > 1 ? 2 : 1) * nblocks);
     double *runs = d_partial_;
-    double *blocks = d_partial_ + nruns;
-    double *upto = blocks + nblocks;
+    double *upto = d_partial_ + nruns;
+    double *blocks = rpb > 1 ? upto + nblocks : runs;
     k_run_sums<T><<<static_cast<uint32_t>((nruns + 3) / 4), kThreads, 0, stream_>>>(sv, sbits, nruns,
                                                                                    runs);
-    const uint64_t rpb = nruns / nblocks;  // runs per index block
     if (rpb > 1) k_block_sums<<<static_cast<uint32_t>(nblocks), kThreads, 0, stream_>>>(runs, rpb, blocks);
-    k_prefix_blocks<<<1, kThreads, 0, stream_>>>(rpb > 1 ? blocks : runs, nblocks, upto);
+    k_prefix_blocks<<<1, kThreads, 0, stream_>>>(blocks, nblocks, upto);
     if (rpb > 1) k_prefix_runs<<<static_cast<uint32_t>(nblocks), kThreads, 0, stream_>>>(runs, rpb, upto);
     k_sample<T><<<static_cast<uint32_t>((shots + kDraws - 1) / kDraws), 64, 0, stream_>>>(
         sv, size_, isz, sbits, upto, runs, drnd, shots, dout);

@@ -33,3 +33,14 @@ def test_marginal_of_many_qubits():
         assert abs(p.sum() - 1.0) < 1e-12
     # one double per outcome
     assert taken(call) < 1.5 * ROW
+
+
+def test_sampling_index_of_every_amplitude():
+    print("case: memory of a fine sampling index", flush=True)
+    draws = np.random.default_rng(2).random(100)
+
+    def call(e):
+        e.set_sample_measure_index_size(N)
+        assert e.sample_measure(draws).max() < 1 << N
+    # a run and a cumulative sum per amplitude
+    assert taken(call) < 2.5 * ROW
