@@ -305,10 +305,18 @@ __global__ __launch_bounds__(64) void k_sample(const cx<T> *__restrict__ sv, uin
     if (!done) {
       const uint32_t n = static_cast<uint32_t>(min(last - sample, static_cast<uint64_t>(64)));
       uint32_t below = 0;
+      const double before = p;
 #pragma unroll 16
       for (uint32_t i = 0; i < 64; ++i) {
         p += v[q][i];
         below += rnd < p ? 0u : 1u;
+      }
+      if (p != p) {  // a NaN, maybe of a later index block: count up to it
+        double s = before;
+        for (below = 0; below < 64; ++below) {
+          s += v[q][below];
+          if (rnd < s) break;
+        }
       }
       if (below < n) {
         sample += below;
