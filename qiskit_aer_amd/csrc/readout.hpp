@@ -288,6 +288,17 @@ __global__ __launch_bounds__(64) void k_sample(const cx<T> *__restrict__ sv, uin
       }
     }
   }
+  if (!(upto[nblocks - 1u] >= 0.0)) {
+    // A NaN among the amplitudes: a window of 64 that reaches into later index
+    // blocks would count it, so these draws add one amplitude after the other.
+    if (!done)
+      for (; sample < last; ++sample) {
+        p += prob(sv[sample]);
+        if (rnd < p) break;
+      }
+    if (lane < kDraws && s < shots) out[s] = sample;
+    return;
+  }
   cx<T> a[kDraws];
   auto load = [&](uint64_t from) {
 #pragma unroll
@@ -305,18 +316,10 @@ __global__ __launch_bounds__(64) void k_sample(const cx<T> *__restrict__ sv, uin
     if (!done) {
       const uint32_t n = static_cast<uint32_t>(min(last - sample, static_cast<uint64_t>(64)));
       uint32_t below = 0;
-      const double before = p;
 #pragma unroll 16
       for (uint32_t i = 0; i < 64; ++i) {
         p += v[q][i];
         below += rnd < p ? 0u : 1u;
-      }
-      if (p != p) {  // a NaN, maybe of a later index block: count up to it
-        double s = before;
-        for (below = 0; below < 64; ++below) {
-          s += v[q][below];
-          if (rnd < s) break;
-        }
       }
       if (below < n) {
         sample += below;
