@@ -1967,23 +1967,28 @@ std::vector<PassPlan> Engine::plan() const {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
     // What the scans read of the primitives, kept together.
+    enum : uint8_t {
+      kLds = 1,   // a register pass spills the tile for it, a gate pass does not
+      kWide = 2,  // the lean register pass does not run it
+    };
     struct Pending {
       uint64_t tmask, touch;
       uint32_t idx;
       bool probe, unitary, gate;
-      bool lds;   // a register pass spills the tile for it, a gate pass does not
-      bool lean;  // the lean register pass runs it
+      uint8_t needs;
     };
     std::vector<Pending> remaining;
     bool probes = false, all_lean = true;
     for (size_t i = seg_begin; i < seg_end; ++i) probes |= queue_[i].kind == K_PROBE;
     for (size_t i = seg_begin; i < seg_end; ++i) {
       const Prim &p = queue_[i];
+      const bool spills = p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2);
+      const bool lean = (p.kind == K_DENSE1 && p.ctrl.empty()) || p.kind == K_MCX || p.kind == K_MCPHASE ||
+                        (p.kind == K_DIAG && p.q.size() == 1);
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
-                                  gate_bits && gate_prim(p, probes), p.kind == K_MCSWAP || (p.kind == K_DENSE && p.q.size() > 2),
-                                  (p.kind == K_DENSE1 && p.ctrl.empty()) || p.kind == K_MCX || p.kind == K_MCPHASE ||
-                                      (p.kind == K_DIAG && p.q.size() == 1)});
-      all_lean = all_lean && remaining.back().lean;
+                                  gate_bits && gate_prim(p, probes),
+                                  static_cast<uint8_t>((spills ? kLds : 0) | (lean ? 0 : kWide))});
+      all_lean = all_lean && lean;
     }
     while (!remaining.empty()) {
       // One candidate pass: the tile starts as `s0`, then takes the
@@ -1993,17 +1998,17 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t active = 0;
       for (const Pending &p : remaining) active |= p.touch;
       // A gate pass takes only what its kernel runs.
-      bool lds = false, lean = true;  // whether the last scan took an `lds` primitive, and lean ones alone
+      uint8_t needs = 0;  // of the primitives that the last scan took
       auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
-        lds = false;
-        lean = true;
+        needs = 0;
         uint64_t s = s0;
         uint64_t blocked = 0;
         bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
         size_t count = 0;
         uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
         for (const Pending &p : remaining) {
-          bool fits = !(p.touch & blocked) && !(p.probe && (nonunitary_blocked || !probes_left)) && (!gate || p.gate);
+          bool fits = !(p.touch & blocked) && (!gate || p.gate);
+          if (p.probe) fits = fits && !nonunitary_blocked && probes_left;
           if (fits) {
             const uint64_t ns = s | p.tmask;
             fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
@@ -2011,9 +2016,8 @@ std::vector<PassPlan> Engine::plan() const {
           }
           if (fits) {
             ++count;
-            probes_left -= p.probe;
-            lds |= p.lds;
-            lean = lean && p.lean;
+            if (p.probe) --probes_left;
+            needs |= p.needs;
             if (take) take->prims.push_back(p.idx);
             continue;
           }
@@ -2040,14 +2044,14 @@ std::vector<PassPlan> Engine::plan() const {
       struct Tile {
         size_t count = 0;
         uint64_t seed = 0;
-        bool lds = false, lean = true;
+        uint8_t needs = 0;
       };
       auto best_tile = [&](uint32_t c, bool g) {
         Tile t;
         t.seed = lowmask;
         auto candidate = [&](uint64_t s0) {
           const size_t k = scan(c, g, s0, nullptr, nullptr);
-          if (k > t.count) t = Tile{k, s0, lds, lean};
+          if (k > t.count) t = Tile{k, s0, needs};
         };
         candidate(lowmask);
         const uint32_t w = c - low_bits_;
@@ -2060,8 +2064,9 @@ std::vector<PassPlan> Engine::plan() const {
       bool gate = false;
       if (gate_bits && !(few_tiles && all_lean)) {
         const Tile t = best_tile(gate_bits, true);
-        gate = best.lds ? 2 * t.count >= best.count : t.count > best.count || (t.count == best.count && t.count > 4);
-        if (few_tiles && best.lean && t.lean) gate = false;
+        gate = best.needs & kLds ? 2 * t.count >= best.count
+                                 : t.count > best.count || (t.count == best.count && t.count > 4);
+        if (few_tiles && !((best.needs | t.needs) & kWide)) gate = false;
         if (gate) {
           best = t;
           cap = gate_bits;
