@@ -1,5 +1,6 @@
 // Host implementation of the engine and its C ABI (include/aerhip.h).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -850,6 +851,15 @@ std::vector<TileOp> fuse_phase_runs(const std::vector<TileOp> &in, const uint8_t
       out.push_back(first);
       return;
     }
+    // Fused diagonals multiply factors by 1 + 0i, and gate passes by 0 where a
+    // lane's predicate fails: with an infinite or NaN entry that is NaN, so the
+    // ops stay as they are.
+    for (const auto &m : g.members)
+      for (const cd &f : {m.second.first, m.second.second})
+        if (!std::isfinite(f.real()) || !std::isfinite(f.imag())) {
+          out.insert(out.end(), g.originals.begin(), g.originals.end());
+          return;
+        }
     TileOp op;
     std::memset(&op, 0, sizeof(op));
     op.kind = K_PHASES;
