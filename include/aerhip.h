@@ -71,6 +71,12 @@ const char *aerhip_version(void);
  * itself): free and total bytes of device memory on `device`. */
 int aerhip_device_memory(int device, uint64_t *free_out, uint64_t *total_out);
 
+/* No counterpart in the reference (its handles share nothing).  Ended handles
+ * leave their stream and buffers to later ones: at most four sets, each with a
+ * state of at most 64 MiB and four buffers of at most 8 MiB.  Frees them, for
+ * other allocators of the process; handles in use keep theirs. */
+int aerhip_release_memory(void);
+
 /* ---- lifecycle ---------------------------------------------------------- */
 
 /* QubitVector(num_qubits) + set_num_qubits (qubitvector.hpp:922-932):

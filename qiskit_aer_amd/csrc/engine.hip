@@ -3851,6 +3851,10 @@ int aerhip_device_memory(int device, uint64_t *free_out, uint64_t *total_out) {
   });
 }
 
+int aerhip_release_memory(void) {
+  return guard([] { aerhip::WorkspacePool::get().drain(); });
+}
+
 const char *aerhip_version(void) { return "aerhip 0.1.0 (gfx950)"; }
 
 // Internal to the library: planning handles and the batch runner used by

@@ -44,7 +44,8 @@ struct Workspace {
 // The sets of ended handles: at most four in a process, each with a state of at
 // most 64 MiB (22 qubits in complex128) and buffers of at most 8 MiB; what is
 // larger is freed with its handle, and all of it is freed when an allocation
-// fails.  Any thread may take or give.
+// fails or the caller asks (aerhip_release_memory).  Any thread may take, give
+// or release.
 class WorkspacePool {
  public:
   static constexpr size_t kSets = 4, kStateBytes = 64u << 20, kBufferBytes = 8u << 20;

@@ -314,6 +314,12 @@ def device_memory(device: int = 0) -> tuple:
     return free.value, total.value
 
 
+def release_memory() -> None:
+    """Frees the device and pinned memory that ended handles left for later ones
+    (at most four sets, about 400 MiB), for other allocators of the process."""
+    L.check(L.lib().aerhip_release_memory())
+
+
 def device_count() -> int:
     """Number of visible HIP devices."""
     return int(L.lib().aerhip_device_count())
