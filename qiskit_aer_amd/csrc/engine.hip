@@ -6,6 +6,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <optional>
 
 #include "aerhip.h"
 #include "engine.hpp"
@@ -3467,84 +3468,68 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
   });
 
   AERHIP_CHECK(hipSetDevice(device));
-  Workspace ws = WorkspacePool::get().take(device, sv_off * amp);
-  const hipStream_t st = ws.stream;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  auto release = [&](bool ok) {
-    ok = hipStreamSynchronize(st) == hipSuccess && ok;
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    if (ok)
-      WorkspacePool::get().give(ws);
-    else
-      ws.release();
-  };
-  try {
-    AERHIP_CHECK(hipEventCreate(&e0));
-    AERHIP_CHECK(hipEventCreate(&e1));
-    if (total > ws.program.bytes) WorkspacePool::grow(ws.program, total);
-    const size_t probe_bytes = (num_probes + part_len + 1) * sizeof(double);
-    if (probe_bytes > ws.probes.bytes) WorkspacePool::grow(ws.probes, probe_bytes);
-    void *const d_states = ws.state.p, *const d_prog = ws.program.p;
-    double *const d_probes = static_cast<double *>(ws.probes.p);
-    AERHIP_CHECK(hipMemcpyAsync(d_prog, h.get(), total, hipMemcpyHostToDevice, st));
-    char *d = static_cast<char *>(d_prog);
-    const auto *dc = reinterpret_cast<const BatchCircuit *>(d);
-    AERHIP_CHECK(hipEventRecord(e0, st));
-    auto run = [&](auto zero, auto bits, auto regs) {
-      using T = decltype(zero);
-      constexpr int B = decltype(bits)::value, R = decltype(regs)::value;
-      auto *sv = static_cast<cx<T> *>(d_states);
-      const auto *dp = reinterpret_cast<const PassDesc *>(d + pass_off);
-      const auto *dr = reinterpret_cast<const ROp<T> *>(d + rops_off);
-      const auto *dops = reinterpret_cast<const TileOp *>(d + ops_off);
-      const auto *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
-      const auto *dslots = reinterpret_cast<const uint32_t *>(d + slots_off);
-      double *const partial = d_probes + num_probes;
-      const dim3 sums(static_cast<uint32_t>(count), std::max<uint32_t>(1, 64 / static_cast<uint32_t>(std::min<uint64_t>(count, 64))));
-      k_fill_basis<T><<<grid_for(sv_off, 16384), kThreads, 0, st>>>(sv, sv_off, ~0ull);
-      k_batch_ones<T><<<grid_for(count, 1u << 30), kThreads, 0, st>>>(sv, dc, count);
-      for (uint32_t p = 0; p < max_passes; ++p) {
-        BatchGroups gr;
-        std::memset(&gr, 0, sizeof(gr));
-        uint64_t wgs = 0;
-        for (uint64_t i = 0; i < count;) {
-          uint64_t j = i, end = i;  // [i, end): one size; [i, j): those with a pass p
-          while (end < count && sorted[end].num_qubits == sorted[i].num_qubits) ++end;
-          while (j < end && sorted[j].pass_count > p) ++j;
-          if (j > i) {
-            gr.g[gr.n++] = BatchGroup{static_cast<uint32_t>(i), static_cast<uint32_t>(wgs), sorted[i].tile_log};
-            wgs += (j - i) << sorted[i].tile_log;
-          }
-          i = end;
+  WorkspaceLease ws(device, sv_off * amp);
+  const hipStream_t st = ws->stream;
+  EventPair ev;
+  ev.create();
+  if (total > ws->program.bytes) WorkspacePool::grow(ws->program, total);
+  const size_t probe_bytes = (num_probes + part_len + 1) * sizeof(double);
+  if (probe_bytes > ws->probes.bytes) WorkspacePool::grow(ws->probes, probe_bytes);
+  void *const d_states = ws->state.p, *const d_prog = ws->program.p;
+  double *const d_probes = static_cast<double *>(ws->probes.p);
+  AERHIP_CHECK(hipMemcpyAsync(d_prog, h.get(), total, hipMemcpyHostToDevice, st));
+  char *d = static_cast<char *>(d_prog);
+  const auto *dc = reinterpret_cast<const BatchCircuit *>(d);
+  AERHIP_CHECK(hipEventRecord(ev.begin, st));
+  auto run = [&](auto zero, auto bits, auto regs) {
+    using T = decltype(zero);
+    constexpr int B = decltype(bits)::value, R = decltype(regs)::value;
+    auto *sv = static_cast<cx<T> *>(d_states);
+    const auto *dp = reinterpret_cast<const PassDesc *>(d + pass_off);
+    const auto *dr = reinterpret_cast<const ROp<T> *>(d + rops_off);
+    const auto *dops = reinterpret_cast<const TileOp *>(d + ops_off);
+    const auto *dpool = reinterpret_cast<const cx<double> *>(d + pool_off);
+    const auto *dslots = reinterpret_cast<const uint32_t *>(d + slots_off);
+    double *const partial = d_probes + num_probes;
+    const dim3 sums(static_cast<uint32_t>(count), std::max<uint32_t>(1, 64 / static_cast<uint32_t>(std::min<uint64_t>(count, 64))));
+    k_fill_basis<T><<<grid_for(sv_off, 16384), kThreads, 0, st>>>(sv, sv_off, ~0ull);
+    k_batch_ones<T><<<grid_for(count, 1u << 30), kThreads, 0, st>>>(sv, dc, count);
+    for (uint32_t p = 0; p < max_passes; ++p) {
+      BatchGroups gr;
+      std::memset(&gr, 0, sizeof(gr));
+      uint64_t wgs = 0;
+      for (uint64_t i = 0; i < count;) {
+        uint64_t j = i, end = i;  // [i, end): one size; [i, j): those with a pass p
+        while (end < count && sorted[end].num_qubits == sorted[i].num_qubits) ++end;
+        while (j < end && sorted[j].pass_count > p) ++j;
+        if (j > i) {
+          gr.g[gr.n++] = BatchGroup{static_cast<uint32_t>(i), static_cast<uint32_t>(wgs), sorted[i].tile_log};
+          wgs += (j - i) << sorted[i].tile_log;
         }
-        if (wgs > 0xFFFFFFFFull / kThreads) throw std::invalid_argument("aerhip: batch too large for one launch");
-        if constexpr (sizeof(T) == 8)
-          if (classes[p] & 1u)
-            k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(
-                sv, dc, gr, p, dp, dr, dops, dpool, partial);
-        if (classes[p] & 2u)
-          k_batch<T, B, R, V_FULL><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops, dpool,
-                                                                                   partial);
-        if (partials[p]) k_batch_sums<<<sums, kThreads, 0, st>>>(dc, p, dp, dslots, partial, d_probes);
+        i = end;
       }
-    };
-    if (prec == AERHIP_PRECISION_DOUBLE)
-      run(0.0, std::integral_constant<int, kTileBitsC128>{}, std::integral_constant<int, 3>{});
-    else
-      run(0.0f, std::integral_constant<int, kTileBitsC64>{}, std::integral_constant<int, 4>{});
-    AERHIP_CHECK(hipGetLastError());
-    AERHIP_CHECK(hipEventRecord(e1, st));
-    AERHIP_CHECK(hipMemcpyAsync(values, d_probes, num_probes * sizeof(double), hipMemcpyDeviceToHost, st));
-    AERHIP_CHECK(hipStreamSynchronize(st));
-    float ms = 0;
-    AERHIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-    if (kernel_ms) *kernel_ms = ms;
-  } catch (...) {
-    release(false);
-    throw;
-  }
-  release(true);
+      if (wgs > 0xFFFFFFFFull / kThreads) throw std::invalid_argument("aerhip: batch too large for one launch");
+      if constexpr (sizeof(T) == 8)
+        if (classes[p] & 1u)
+          k_batch<T, B, R, V_PROBES><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(
+              sv, dc, gr, p, dp, dr, dops, dpool, partial);
+      if (classes[p] & 2u)
+        k_batch<T, B, R, V_FULL><<<static_cast<uint32_t>(wgs), kThreads, 0, st>>>(sv, dc, gr, p, dp, dr, dops, dpool,
+                                                                                 partial);
+      if (partials[p]) k_batch_sums<<<sums, kThreads, 0, st>>>(dc, p, dp, dslots, partial, d_probes);
+    }
+  };
+  if (prec == AERHIP_PRECISION_DOUBLE)
+    run(0.0, std::integral_constant<int, kTileBitsC128>{}, std::integral_constant<int, 3>{});
+  else
+    run(0.0f, std::integral_constant<int, kTileBitsC64>{}, std::integral_constant<int, 4>{});
+  AERHIP_CHECK(hipGetLastError());
+  AERHIP_CHECK(hipEventRecord(ev.end, st));
+  AERHIP_CHECK(hipMemcpyAsync(values, d_probes, num_probes * sizeof(double), hipMemcpyDeviceToHost, st));
+  AERHIP_CHECK(hipStreamSynchronize(st));
+  float ms = 0;
+  AERHIP_CHECK(hipEventElapsedTime(&ms, ev.begin, ev.end));
+  if (kernel_ms) *kernel_ms = ms;
 }
 
 // ---------------------------------------------------------------------------
@@ -3571,22 +3556,15 @@ class MultiState {
     if (prec_ == AERHIP_PRECISION_DOUBLE)
       for (Engine *e : planners_) e->use_gate_passes(planners_.size());
     AERHIP_CHECK(hipSetDevice(device_));
-    ws_ = WorkspacePool::get().take(device_, planners_.size() * (1ull << n_) * amp_bytes());
-    states_ = ws_.state.p;
-    st_ = ws_.stream;
-    AERHIP_CHECK(hipEventCreate(&e0_));
-    AERHIP_CHECK(hipEventCreate(&e1_));
+    ws_.emplace(device_, planners_.size() * (1ull << n_) * amp_bytes());
+    states_ = (*ws_)->state.p;
+    st_ = (*ws_)->stream;
+    ev_.create();
   }
   ~MultiState() {
     (void)hipSetDevice(device_);
-    const hipError_t e = hipStreamSynchronize(st_);
+    (void)hipStreamSynchronize(st_);
     if (d_terms_) (void)hipFree(d_terms_);
-    if (e0_) (void)hipEventDestroy(e0_);
-    if (e1_) (void)hipEventDestroy(e1_);
-    if (e == hipSuccess)
-      WorkspacePool::get().give(ws_);
-    else
-      ws_.release();
   }
   MultiState(const MultiState &) = delete;
   MultiState &operator=(const MultiState &) = delete;
@@ -3657,16 +3635,16 @@ class MultiState {
     bool together = true;
     for (uint64_t i = 1; i < cnt && together; ++i) together = same_shape(parts[0], parts[i]);
     AERHIP_CHECK(hipSetDevice(device_));
-    AERHIP_CHECK(hipEventRecord(e0_, st_));
+    AERHIP_CHECK(hipEventRecord(ev_.begin, st_));
     if (together) {
       run(parts, 0, cnt, pps, values.data());
     } else {
       for (uint64_t i = 0; i < cnt; ++i) run(parts, i, 1, pps, values.data() + i * pps);
     }
-    AERHIP_CHECK(hipEventRecord(e1_, st_));
+    AERHIP_CHECK(hipEventRecord(ev_.end, st_));
     AERHIP_CHECK(hipStreamSynchronize(st_));
     float ms = 0;
-    AERHIP_CHECK(hipEventElapsedTime(&ms, e0_, e1_));
+    AERHIP_CHECK(hipEventElapsedTime(&ms, ev_.begin, ev_.end));
     kernel_ms_ += ms;
     return values;
   }
@@ -3723,11 +3701,11 @@ class MultiState {
     else
       rops_to_float(rops.data(), rops.size(), reinterpret_cast<ROp<float> *>(h.data() + rops_off));
     if (!pool.empty()) std::memcpy(h.data() + pool_off, pool.data(), pool.size() * sizeof(cd));
-    if (total > ws_.program.bytes) {
+    if (total > (*ws_)->program.bytes) {
       AERHIP_CHECK(hipStreamSynchronize(st_));
-      WorkspacePool::grow(ws_.program, align_up(total, 1 << 16));
+      WorkspacePool::grow((*ws_)->program, align_up(total, 1 << 16));
     }
-    void *const d_prog = ws_.program.p;
+    void *const d_prog = (*ws_)->program.p;
     // pageable source: the copy is complete when hipMemcpyAsync returns
     AERHIP_CHECK(hipMemcpyAsync(d_prog, h.data(), total, hipMemcpyHostToDevice, st_));
     AERHIP_CHECK(hipStreamSynchronize(st_));
@@ -3735,9 +3713,9 @@ class MultiState {
     const uint64_t ntiles = 1ull << (n_ - tb);
     if (pps) {
       const size_t need = (cnt * pps * ntiles + cnt * pps) * sizeof(double);
-      if (need > ws_.probes.bytes) WorkspacePool::grow(ws_.probes, align_up(need, 1 << 20));
+      if (need > (*ws_)->probes.bytes) WorkspacePool::grow((*ws_)->probes, align_up(need, 1 << 20));
     }
-    double *const d_probes = static_cast<double *>(ws_.probes.p);
+    double *const d_probes = static_cast<double *>((*ws_)->probes.p);
     char *d = static_cast<char *>(d_prog);
     const DeviceProgram dp{reinterpret_cast<const PassDesc *>(d), reinterpret_cast<const TileOp *>(d + ops_off),
                            d + rops_off, reinterpret_cast<const cx<double> *>(d + pool_off),
@@ -3762,8 +3740,8 @@ class MultiState {
   std::vector<Engine *> planners_;
   void *states_ = nullptr;
   hipStream_t st_ = nullptr;
-  hipEvent_t e0_ = nullptr, e1_ = nullptr;
-  Workspace ws_;
+  std::optional<WorkspaceLease> ws_;
+  EventPair ev_;
   void *d_terms_ = nullptr;
   double kernel_ms_ = 0;
 };

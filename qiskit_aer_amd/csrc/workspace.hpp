@@ -150,4 +150,41 @@ class WorkspacePool {
   std::vector<Workspace> sets_;
 };
 
+// A set for the life of a scope or an object, also one whose constructor throws
+// later.  Back to the pool it goes when its stream is done; after an error there
+// it is freed.
+class WorkspaceLease {
+ public:
+  WorkspaceLease(int device, size_t bytes) : w_(WorkspacePool::get().take(device, bytes)) {}
+  ~WorkspaceLease() {
+    (void)hipSetDevice(w_.device);
+    if (hipStreamSynchronize(w_.stream) == hipSuccess)
+      WorkspacePool::get().give(w_);
+    else
+      w_.release();
+  }
+  WorkspaceLease(const WorkspaceLease &) = delete;
+  WorkspaceLease &operator=(const WorkspaceLease &) = delete;
+  Workspace *operator->() { return &w_; }
+
+ private:
+  Workspace w_;
+};
+
+// Two events that time what lies between them.
+struct EventPair {
+  hipEvent_t begin = nullptr, end = nullptr;
+  EventPair() = default;
+  ~EventPair() {
+    if (begin) (void)hipEventDestroy(begin);
+    if (end) (void)hipEventDestroy(end);
+  }
+  EventPair(const EventPair &) = delete;
+  EventPair &operator=(const EventPair &) = delete;
+  void create() {
+    AERHIP_CHECK(hipEventCreate(&begin));
+    AERHIP_CHECK(hipEventCreate(&end));
+  }
+};
+
 }  // namespace aerhip

@@ -2,6 +2,7 @@
 // Usage: workspace_pool CASE; prints the case and ends with 0 if it holds.
 #include <cstdio>
 #include <cstring>
+#include <optional>
 
 #include "workspace.hpp"
 
@@ -85,6 +86,41 @@ void devices() {
   EXPECT(s.foreign_frees == 0);
 }
 
+// An object that takes a set and then fails to make its events leaves the set
+// to the pool; one whose stream reports an error frees it.
+void leases() {
+  using aerhip::EventPair;
+  using aerhip::WorkspaceLease;
+  auto &s = fake::state();
+  struct Object {
+    std::optional<WorkspaceLease> ws;
+    EventPair ev;
+    explicit Object(std::size_t bytes) {
+      ws.emplace(0, bytes);
+      ev.create();
+    }
+  };
+  for (int left : {1, 2}) {  // the set's own event, then none or one of the two
+    s.events_left = left + (s.streams ? -1 : 0);
+    bool threw = false;
+    try {
+      Object o(500);
+    } catch (const std::exception &) {
+      threw = true;
+    }
+    EXPECT(threw);
+    EXPECT(s.streams == 1 && s.events == 1 && s.used() == 500 && s.syncs > 0);
+  }
+  s.events_left = 100;
+  { Object o(500); }
+  EXPECT(s.streams == 1 && s.events == 1 && s.used() == 500);
+  {
+    Object o(500);
+    s.sync_result = hipErrorUnknown;
+  }
+  EXPECT(s.streams == 0 && s.events == 0 && s.used() == 0 && s.pinned_memory.empty());
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -93,6 +129,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(name, "bounded")) bounded();
   else if (!std::strcmp(name, "out_of_memory")) out_of_memory();
   else if (!std::strcmp(name, "devices")) devices();
+  else if (!std::strcmp(name, "leases")) leases();
   else return 2;
   return failures ? 1 : 0;
 }

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["bounded", "out_of_memory", "devices"])
+@pytest.mark.parametrize("case", ["bounded", "out_of_memory", "devices", "leases"])
 def test_pool(program, case):
     r = subprocess.run([str(program), case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
