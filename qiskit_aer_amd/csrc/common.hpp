@@ -120,7 +120,8 @@ struct TileOp {
 
 struct PassDesc {
   uint32_t kind;      // 0 = tile pass, 1 = dense group pass, 2 = register pass,
-                      // 3 = probe sweep (nops K_PROBEs), 4 = qubit-permutation pass (K_QPERM)
+                      // 3 = probe sweep (nops K_PROBEs), 4 = qubit-permutation pass (K_QPERM),
+                      // 5 = gate pass (op_begin, nops: its ROps, as for 2)
   uint32_t nb;        // tile qubits
   uint32_t c;         // S contains qubits 0..c-1
   uint32_t op_begin;  // first TileOp of the pass
@@ -130,7 +131,7 @@ struct PassDesc {
   uint32_t batch_class; // batched circuits: 0 = runs in k_batch<V_PROBES>, 1 = in k_batch<V_FULL>
   uint64_t part_off;    // batched circuits: the pass's probe partials, partial[part_off + row * tiles + tile],
   uint32_t probe_at;    // whose rows' values go to values[slots[probe_at + row]],
-  uint32_t probes;      // row < probes
+  uint32_t probes;      // row < probes; in other programs, the pass's probes
   uint8_t spos[16];   // tile qubits, ascending
   uint8_t comp[64];   // qubits outside the tile, ascending
 };

@@ -2487,7 +2487,7 @@ void Engine::emit_program(Program &prog) {
       sd.nb = tile_bits_;
       sd.ncomp = n_ - tile_bits_;
       sd.op_begin = static_cast<uint32_t>(ops.size());
-      sd.nops = static_cast<uint32_t>(pp.prims.size());
+      sd.nops = sd.probes = static_cast<uint32_t>(pp.prims.size());
       for (uint32_t idx : pp.prims) {
         const Prim &p = queue_[idx];
         TileOp op;
@@ -2504,9 +2504,9 @@ void Engine::emit_program(Program &prog) {
       continue;
     }
     pd.nb = ns;
-    pd.readonly = 1;
     for (uint32_t idx : pp.prims)
-      if (queue_[idx].kind != K_PROBE) pd.readonly = 0;
+      if (queue_[idx].kind == K_PROBE) ++pd.probes;
+    pd.readonly = pd.probes == pp.prims.size();
     uint32_t c = 0;
     while (c < ns && pd.spos[c] == c) ++c;
     pd.c = c;
@@ -2764,6 +2764,10 @@ PassKernel pass_kernel(int prec, const PassDesc &pd, const std::vector<ROp<doubl
     k.probes = k.probes || kk == Q_PROBE;
     k.diag = k.diag || ((kk == Q_LOAD || kk == Q_FILL) && r.a != 0);
   }
+  if (pd.kind == 5 && k.probes)  // whose kernel holds no 8x8 gates
+    for (uint32_t i = 0; i < pd.nops; ++i)
+      if ((rops[pd.op_begin + i].kind & ~F_ALL) == Q_U3)
+        throw std::logic_error("aerhip: 8x8 gate in a gate pass with probes");
   if (prec == AERHIP_PRECISION_SINGLE && has_probes(k.variant)) k.variant = V_FULL;
   return k;
 }
@@ -3359,9 +3363,11 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
     engines[i]->limit_probes(kBatchProbes);
     engines[i]->emit_program(parts[i]);
     for (PassDesc &d : parts[i].passes) {
+      if (d.kind == 5) throw std::logic_error("aerhip: a gate pass in a batch");
       d.batch_class = prec == AERHIP_PRECISION_DOUBLE && d.kind == 2 &&
                               !has_gates(pass_kernel(prec, d, parts[i].rops).variant) ? 0u : 1u;
       d.probe_at = static_cast<uint32_t>(slots[i].size());
+      d.probes = 0;
       for_each_probe(parts[i], d, [&](uint32_t &slot) {
         slots[i].push_back(slot);
         slot = d.probes++;
@@ -3444,7 +3450,7 @@ void run_batch(Engine *const *engines, uint64_t count, int device, double *value
                    pb = static_cast<uint32_t>(pool_at[i]);
     for (size_t k = 0; k < p.passes.size(); ++k) {
       PassDesc d = p.passes[k];
-      d.op_begin += d.kind == 2 || d.kind == 5 ? rb : ob;
+      d.op_begin += d.kind == 2 ? rb : ob;
       hp[pass_at[i] + k] = d;
     }
     for (size_t k = 0; k < slots[i].size(); ++k) hslots[probe_at[i] + k] = static_cast<uint32_t>(probe_at[i]) + slots[i][k];
@@ -3628,7 +3634,9 @@ class MultiState {
       if (a.passes.size() != b.passes.size()) return false;
       for (size_t k = 0; k < a.passes.size(); ++k)
         if (a.passes[k].kind != b.passes[k].kind || a.passes[k].ncomp != b.passes[k].ncomp ||
-            a.passes[k].kind == 1)
+            a.passes[k].kind == 1 ||
+            // a gate pass with probes runs in a kernel of its own
+            (a.passes[k].kind == 5 && (a.passes[k].probes != 0) != (b.passes[k].probes != 0)))
           return false;
       return true;
     };

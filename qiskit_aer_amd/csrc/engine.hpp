@@ -75,7 +75,6 @@ class Engine {
   uint32_t num_qubits() const { return n_; }
   int precision() const { return prec_; }
   uint64_t size() const { return size_; }
-  void *device_data() { return sv_; }
   // The state's address for work on other streams.
   void *hand_out() {
     exposed_ = true;
