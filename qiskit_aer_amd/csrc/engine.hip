@@ -1978,7 +1978,7 @@ std::vector<PassPlan> Engine::plan() const {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;
     // What the scans read of the primitives, kept together.
-    enum : uint8_t {
+    enum : uint32_t {
       kLds = 1,   // a register pass spills the tile for it, a gate pass does not
       kWide = 2,  // the lean register pass does not run it
     };
@@ -1986,7 +1986,7 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t tmask, touch;
       uint32_t idx;
       bool probe, unitary, gate;
-      uint8_t needs;
+      uint32_t needs;
     };
     std::vector<Pending> remaining;
     bool probes = false, all_lean = true;
@@ -1998,7 +1998,7 @@ std::vector<PassPlan> Engine::plan() const {
                         (p.kind == K_DIAG && p.q.size() == 1);
       remaining.push_back(Pending{p.tmask, p.touch, static_cast<uint32_t>(i), p.kind == K_PROBE, p.unitary,
                                   gate_bits && gate_prim(p, probes),
-                                  static_cast<uint8_t>((spills ? kLds : 0) | (lean ? 0 : kWide))});
+                                  (spills ? kLds : 0u) | (lean ? 0u : kWide)});
       all_lean = all_lean && lean;
     }
     while (!remaining.empty()) {
@@ -2009,17 +2009,19 @@ std::vector<PassPlan> Engine::plan() const {
       uint64_t active = 0;
       for (const Pending &p : remaining) active |= p.touch;
       // A gate pass takes only what its kernel runs.
-      uint8_t needs = 0;  // of the primitives that the last scan took
-      auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
-        needs = 0;
+      uint32_t needs = 0;  // of the primitives that the last scan took
+      auto scan_of = [&](auto with_probes, uint32_t cap, bool gate, uint64_t s0, PassPlan *take,
+                         std::vector<Pending> *rest) {
+        constexpr bool P = decltype(with_probes)::value;
+        uint32_t taken = 0;
         uint64_t s = s0;
         uint64_t blocked = 0;
-        bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
+        [[maybe_unused]] bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
         size_t count = 0;
-        uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
+        [[maybe_unused]] uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
         for (const Pending &p : remaining) {
           bool fits = !(p.touch & blocked) && (!gate || p.gate);
-          if (p.probe) fits = fits && !nonunitary_blocked && probes_left;
+          if constexpr (P) fits = fits && !(p.probe && (nonunitary_blocked || !probes_left));
           if (fits) {
             const uint64_t ns = s | p.tmask;
             fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
@@ -2027,18 +2029,23 @@ std::vector<PassPlan> Engine::plan() const {
           }
           if (fits) {
             ++count;
-            if (p.probe) --probes_left;
-            needs |= p.needs;
+            if constexpr (P) probes_left -= p.probe;
+            taken |= p.needs;
             if (take) take->prims.push_back(p.idx);
             continue;
           }
           if (rest) rest->push_back(p);
           blocked |= p.touch;
-          nonunitary_blocked |= !p.unitary;
+          if constexpr (P) nonunitary_blocked |= !p.unitary;
           if (!take && (blocked & active) == active) break;
         }
         if (take) take->smask = s;
+        needs = taken;
         return count;
+      };
+      auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
+        return probes ? scan_of(std::true_type{}, cap, gate, s0, take, rest)
+                      : scan_of(std::false_type{}, cap, gate, s0, take, rest);
       };
       // Candidates: the tile seeded by nothing but the low qubits, and by
       // each window of tile_bits - low_bits consecutive qubits.  A window
@@ -2055,7 +2062,7 @@ std::vector<PassPlan> Engine::plan() const {
       struct Tile {
         size_t count = 0;
         uint64_t seed = 0;
-        uint8_t needs = 0;
+        uint32_t needs = 0;
       };
       auto best_tile = [&](uint32_t c, bool g) {
         Tile t;
