@@ -418,9 +418,10 @@ int aerhip_run_circuit(const aerhip_op *ops, uint64_t num_ops,
  *                num_qubits[i] characters (character n-1-q acts on qubit q);
  *   coeffs       one real weight per term; circuit i owns terms
  *                [term_offsets[i], term_offsets[i+1]);
- *   mode         0: every circuit in one kernel launch (one workgroup walks all
- *                passes of its circuit); 1: circuit by circuit, one launch per
- *                pass (the reference's execution order), for comparison;
+ *   mode         0: all circuits together, pass by pass (pass k of every circuit
+ *                that has one is one launch per kernel class, with a workgroup per
+ *                tile); 1: circuit by circuit, one launch per pass (the reference's
+ *                execution order), for comparison;
  *   kernel_ms    (optional) device time of the execution.
  * Dense matrices must act on at most 5 qubits. */
 int aerhip_batch_pauli_expval(const aerhip_op *ops, const uint64_t *op_offsets,

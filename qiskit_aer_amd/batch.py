@@ -1,11 +1,12 @@
-"""Many circuits with Pauli-sum expectation values in one launch.
+"""Many circuits with Pauli-sum expectation values, run together.
 
 ``batch_pauli_expval(circuits, hamiltonians)`` returns, for each circuit
 (run from |0> on its own qubit count), E_i = sum_t c_t <P_t>.  With
-``mode="batch"`` every circuit runs in a single kernel launch (one workgroup
-per circuit); ``mode="sequential"`` runs them one after the other with one
-launch per pass, the way the reference's controller executes a list of
-circuits (src/controllers/aer_controller.hpp:309-437).
+``mode="batch"`` the circuits advance pass by pass: pass k of every circuit
+that has one is one launch per kernel class, with a workgroup per tile;
+``mode="sequential"`` runs them one after the other with one launch per pass,
+the way the reference's controller executes a list of circuits
+(src/controllers/aer_controller.hpp:309-437).
 """
 from __future__ import annotations
 
