@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -32,6 +33,14 @@ constexpr uint32_t kGateMinQubits = 21;
 // against 179, 21 qubits 247 against 194, 22 qubits 284 against 299; complex128,
 // 21 qubits 257 against 209, 22 qubits 327 against 412.
 constexpr uint64_t kLeanGateTiles = 1u << 10;
+// A lean segment of few gates (16 to a pass in complex128, 20 in complex64) takes
+// gate passes only where they are fewer: it runs at the rate of its sweeps, and
+// those of larger tiles are slower where the tile's qubits are high.  12 to 24 U3
+// on the 12 highest of 27 qubits (complex128, two passes either way): 1.82 ms in
+// gate passes, 1.62 in register passes; on the 12 lowest 0.77 in one gate pass,
+// 1.48 in two register passes.  complex64, 28 qubits, a layer of brickwork 3.21
+// against 3.17 ms, two layers 4.47 against 5.15.
+constexpr uint32_t kShallowC128 = 16, kShallowC64 = 20;
 
 inline uint64_t bit(uint32_t q) { return 1ull << q; }
 
@@ -1988,6 +1997,13 @@ std::vector<PassPlan> Engine::plan() const {
       bool probe, unitary, gate;
       uint32_t needs;
     };
+    // Whether the segment has few gates for the passes its qubits take at least.
+    auto shallow = [&](const std::vector<Pending> &prims) {
+      uint64_t qubits = lowmask;
+      for (const Pending &p : prims) qubits |= p.tmask;
+      const size_t mixed = __builtin_popcountll(qubits) - low_bits_, step = gate_bits - low_bits_;
+      return prims.size() < (prec_ == AERHIP_PRECISION_DOUBLE ? kShallowC128 : kShallowC64) * std::max<size_t>(1, (mixed + step - 1) / step);
+    };
     std::vector<Pending> remaining;
     bool probes = false, all_lean = true;
     for (size_t i = seg_begin; i < seg_end; ++i) probes |= queue_[i].kind == K_PROBE;
@@ -2001,107 +2017,123 @@ std::vector<PassPlan> Engine::plan() const {
                                   (spills ? kLds : 0u) | (lean ? 0u : kWide)});
       all_lean = all_lean && lean;
     }
-    while (!remaining.empty()) {
-      // One candidate pass: the tile starts as `s0`, then takes the
-      // primitives in program order while their mixed qubits fit.  With
-      // `take` null it only counts, and stops once every qubit the remaining
-      // primitives touch is blocked.
-      uint64_t active = 0;
-      for (const Pending &p : remaining) active |= p.touch;
-      // A gate pass takes only what its kernel runs.
-      uint32_t needs = 0;  // of the primitives that the last scan took
-      auto scan_of = [&](auto with_probes, uint32_t cap, bool gate, uint64_t s0, PassPlan *take,
-                         std::vector<Pending> *rest) {
-        constexpr bool P = decltype(with_probes)::value;
-        uint32_t taken = 0;
-        uint64_t s = s0;
-        uint64_t blocked = 0;
-        [[maybe_unused]] bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
-        size_t count = 0;
-        [[maybe_unused]] uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
-        for (const Pending &p : remaining) {
-          bool fits = !(p.touch & blocked) && (!gate || p.gate);
-          if constexpr (P) fits = fits && !(p.probe && (nonunitary_blocked || !probes_left));
-          if (fits) {
-            const uint64_t ns = s | p.tmask;
-            fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
-            if (fits) s = ns;
+    // The passes of the segment; `gates`: gate passes where they are taken.
+    auto plan_segment = [&](std::vector<Pending> remaining, bool gates) {
+      std::vector<PassPlan> passes;
+      while (!remaining.empty()) {
+        // One candidate pass: the tile starts as `s0`, then takes the
+        // primitives in program order while their mixed qubits fit.  With
+        // `take` null it only counts, and stops once every qubit the remaining
+        // primitives touch is blocked.
+        uint64_t active = 0;
+        for (const Pending &p : remaining) active |= p.touch;
+        // A gate pass takes only what its kernel runs.
+        uint32_t needs = 0;  // of the primitives that the last scan took
+        auto scan_of = [&](auto with_probes, uint32_t cap, bool gate, uint64_t s0, PassPlan *take,
+                           std::vector<Pending> *rest) {
+          constexpr bool P = decltype(with_probes)::value;
+          uint32_t taken = 0;
+          uint64_t s = s0;
+          uint64_t blocked = 0;
+          [[maybe_unused]] bool nonunitary_blocked = false;  // a deferred op rescales amplitudes
+          size_t count = 0;
+          [[maybe_unused]] uint32_t probes_left = n_ > nb ? probe_limit_ : ~0u;
+          for (const Pending &p : remaining) {
+            bool fits = !(p.touch & blocked) && (!gate || p.gate);
+            if constexpr (P) fits = fits && !(p.probe && (nonunitary_blocked || !probes_left));
+            if (fits) {
+              const uint64_t ns = s | p.tmask;
+              fits = static_cast<uint32_t>(__builtin_popcountll(ns)) <= cap;
+              if (fits) s = ns;
+            }
+            if (fits) {
+              ++count;
+              if constexpr (P) probes_left -= p.probe;
+              taken |= p.needs;
+              if (take) take->prims.push_back(p.idx);
+              continue;
+            }
+            if (rest) rest->push_back(p);
+            blocked |= p.touch;
+            if constexpr (P) nonunitary_blocked |= !p.unitary;
+            if (!take && (blocked & active) == active) break;
           }
-          if (fits) {
-            ++count;
-            if constexpr (P) probes_left -= p.probe;
-            taken |= p.needs;
-            if (take) take->prims.push_back(p.idx);
-            continue;
-          }
-          if (rest) rest->push_back(p);
-          blocked |= p.touch;
-          if constexpr (P) nonunitary_blocked |= !p.unitary;
-          if (!take && (blocked & active) == active) break;
-        }
-        if (take) take->smask = s;
-        needs = taken;
-        return count;
-      };
-      auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
-        return probes ? scan_of(std::true_type{}, cap, gate, s0, take, rest)
-                      : scan_of(std::false_type{}, cap, gate, s0, take, rest);
-      };
-      // Candidates: the tile seeded by nothing but the low qubits, and by
-      // each window of tile_bits - low_bits consecutive qubits.  A window
-      // lets the pass run a whole light cone of a nearest-neighbour circuit
-      // (the 30-qubit U3+CX brickwork takes 29 passes instead of 66); the
-      // pass keeps the candidate that takes the most primitives, the first
-      // on ties.
-      // The other tile passes run every primitive; a gate pass is taken where
-      // it holds more of them, or as many but more than a few: a pass of one
-      // gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.  Where a
-      // register pass would spill the tile to LDS (swaps, 3-qubit gates), it
-      // has to hold twice as many: on 25 qubits it takes 0.73 ms, a gate pass
-      // 0.21 to 0.45.
-      struct Tile {
-        size_t count = 0;
-        uint64_t seed = 0;
-        uint32_t needs = 0;
-      };
-      auto best_tile = [&](uint32_t c, bool g) {
-        Tile t;
-        t.seed = lowmask;
-        auto candidate = [&](uint64_t s0) {
-          const size_t k = scan(c, g, s0, nullptr, nullptr);
-          if (k > t.count) t = Tile{k, s0, needs};
+          if (take) take->smask = s;
+          needs = taken;
+          return count;
         };
-        candidate(lowmask);
-        const uint32_t w = c - low_bits_;
-        if (n_ > c && w > 0)
-          for (uint32_t a = 0; a + w <= n_; ++a) candidate(lowmask | (((1ull << w) - 1ull) << a));
-        return t;
-      };
-      Tile best = best_tile(nb, false);
-      uint32_t cap = nb;
-      bool gate = false;
-      if (gate_bits && !(few_tiles && all_lean)) {
-        const Tile t = best_tile(gate_bits, true);
-        gate = best.needs & kLds ? 2 * t.count >= best.count
-                                 : t.count > best.count || (t.count == best.count && t.count > 4);
-        if (few_tiles && !((best.needs | t.needs) & kWide)) gate = false;
-        if (gate) {
-          best = t;
-          cap = gate_bits;
+        auto scan = [&](uint32_t cap, bool gate, uint64_t s0, PassPlan *take, std::vector<Pending> *rest) {
+          return probes ? scan_of(std::true_type{}, cap, gate, s0, take, rest)
+                        : scan_of(std::false_type{}, cap, gate, s0, take, rest);
+        };
+        // Candidates: the tile seeded by nothing but the low qubits, and by
+        // each window of tile_bits - low_bits consecutive qubits.  A window
+        // lets the pass run a whole light cone of a nearest-neighbour circuit
+        // (the 30-qubit U3+CX brickwork takes 29 passes instead of 66); the
+        // pass keeps the candidate that takes the most primitives, the first
+        // on ties.
+        // The other tile passes run every primitive; a gate pass is taken where
+        // it holds more of them, or as many but more than a few: a pass of one
+        // gate is the HBM sweep, 6.17 against 6.21 ms on 30 qubits.  Where a
+        // register pass would spill the tile to LDS (swaps, 3-qubit gates), it
+        // has to hold twice as many: on 25 qubits it takes 0.73 ms, a gate pass
+        // 0.21 to 0.45.
+        struct Tile {
+          size_t count = 0;
+          uint64_t seed = 0;
+          uint32_t needs = 0;
+        };
+        auto best_tile = [&](uint32_t c, bool g) {
+          Tile t;
+          t.seed = lowmask;
+          auto candidate = [&](uint64_t s0) {
+            const size_t k = scan(c, g, s0, nullptr, nullptr);
+            if (k > t.count) t = Tile{k, s0, needs};
+          };
+          candidate(lowmask);
+          const uint32_t w = c - low_bits_;
+          if (n_ > c && w > 0)
+            for (uint32_t a = 0; a + w <= n_; ++a) candidate(lowmask | (((1ull << w) - 1ull) << a));
+          return t;
+        };
+        Tile best = best_tile(nb, false);
+        uint32_t cap = nb;
+        bool gate = false;
+        if (gates) {
+          const Tile t = best_tile(gate_bits, true);
+          gate = best.needs & kLds ? 2 * t.count >= best.count
+                                   : t.count > best.count || (t.count == best.count && t.count > 4);
+          if (few_tiles && !((best.needs | t.needs) & kWide)) gate = false;
+          if (gate) {
+            best = t;
+            cap = gate_bits;
+          }
         }
+        PassPlan pp;
+        pp.gate = gate;
+        std::vector<Pending> rest;
+        scan(cap, gate, best.seed, &pp, &rest);
+        uint64_t s = pp.smask;
+        // Complete the tile with the lowest free qubits (longer contiguous runs).
+        for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < cap; ++q)
+          s |= bit(q);
+        pp.smask = s;
+        passes.push_back(std::move(pp));
+        remaining.swap(rest);
       }
-      PassPlan pp;
-      pp.gate = gate;
-      std::vector<Pending> rest;
-      scan(cap, gate, best.seed, &pp, &rest);
-      uint64_t s = pp.smask;
-      // Complete the tile with the lowest free qubits (longer contiguous runs).
-      for (uint32_t q = 0; q < n_ && static_cast<uint32_t>(__builtin_popcountll(s)) < cap; ++q)
-        s |= bit(q);
-      pp.smask = s;
-      out.push_back(std::move(pp));
-      remaining.swap(rest);
+      return passes;
+    };
+    std::vector<PassPlan> passes;
+    if (!remaining.empty() && gate_bits && all_lean && (few_tiles || shallow(remaining))) {
+      passes = plan_segment(remaining, false);
+      if (!few_tiles && gate_bits > nb) {
+        std::vector<PassPlan> with_gates = plan_segment(remaining, true);
+        if (with_gates.size() < passes.size()) passes.swap(with_gates);
+      }
+    } else {
+      passes = plan_segment(std::move(remaining), gate_bits != 0);
     }
+    std::move(passes.begin(), passes.end(), std::back_inserter(out));
     if (seg_end < queue_.size()) {
       PassPlan pp;
       pp.solo = true;

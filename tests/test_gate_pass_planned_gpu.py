@@ -104,3 +104,17 @@ def test_lean_passes_beside_others_with_few_tiles():
         c.unitary(D.random_unitary(4, rng), [q, q + 1])
     passes, _ = run(c, n, "double")
     assert passes > 0
+
+
+@pytest.mark.parametrize("precision,low,passes", [("double", True, 1), ("double", False, 0), ("single", True, 0),
+                                                  ("single", False, 0)])
+def test_shallow_lean_segments(precision, low, passes):
+    """12 gates on 12 qubits: in complex128 one gate pass instead of two register
+    passes where the tile's low bits are among them, otherwise no fewer passes."""
+    n = 23
+    print(f"case: planned shallow gates {precision} low={low}", flush=True)
+    rng = np.random.default_rng(57)
+    c = circuits.Circuit(n)
+    for q in range(12):
+        c.gate("u3", [q if low else n - 1 - q], list(rng.uniform(-3, 3, 3)))
+    assert run(c, n, precision)[0] == passes
