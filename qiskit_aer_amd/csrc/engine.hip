@@ -26,13 +26,15 @@ constexpr size_t kMaxQueue = 4096;      // flush threshold of the gate queue
 // fusion width 2 take 1.19 against 1.13 ms on 21 qubits, 1.65 against 1.30 on 22,
 // but 1.10 against 1.15 on 20.
 constexpr uint32_t kGateMinQubits = 21;
-// Programs of 2x2 gates, X and phases alone from 2^10 tiles on.  With fewer a
-// pass waits for its ops one after the other, which the lean register pass reads
-// one op ahead.  Kernel time of 8 layers of brickwork without block fusion, gate
-// against register passes: complex64, 14 qubits 143 against 118 us, 20 qubits 211
-// against 179, 21 qubits 247 against 194, 22 qubits 284 against 299; complex128,
-// 21 qubits 257 against 209, 22 qubits 327 against 412.
-constexpr uint64_t kLeanGateTiles = 1u << 10;
+// Programs of 2x2 gates, X and phases alone from 2^10 tiles on in complex128, from
+// 2^11 in complex64.  With fewer a pass waits for its ops one after the other,
+// which the lean register pass reads one op ahead.  Kernel time of 8 layers of
+// brickwork without block fusion and of a QFT, gate against register passes:
+// complex64, 14 qubits 143 against 118 and 65 against 59 us, 21 qubits 247 against
+// 194 and 116 against 112, 22 qubits 284 against 299 and 132 against 130, 23 qubits
+// 509 against 561 and 224 against 228; complex128, 21 qubits 257 against 209 and 117
+// against 106, 22 qubits 327 against 412 and 169 against 183.
+constexpr uint64_t kLeanGateTilesC128 = 1u << 10, kLeanGateTilesC64 = 1u << 11;
 // A lean segment of few gates (16 to a pass in complex128, 20 in complex64) takes
 // gate passes only where they are fewer: it runs at the rate of its sweeps, and
 // those of larger tiles are slower where the tile's qubits are high.  12 to 24 U3
@@ -1982,7 +1984,7 @@ std::vector<PassPlan> Engine::plan() const {
     if (!p.solo && static_cast<uint32_t>(__builtin_popcountll(p.tmask | lowmask)) > nb)
       throw std::logic_error("aerhip: a primitive mixes more qubits than a tile holds");
   const uint32_t gate_bits = gate_tile_bits();
-  const bool few_tiles = gate_bits && states_ << (n_ - gate_bits) < kLeanGateTiles;
+  const bool few_tiles = gate_bits && states_ << (n_ - gate_bits) < (prec_ == AERHIP_PRECISION_DOUBLE ? kLeanGateTilesC128 : kLeanGateTilesC64);
   while (seg_begin < queue_.size()) {
     size_t seg_end = seg_begin;
     while (seg_end < queue_.size() && !queue_[seg_end].solo) ++seg_end;

@@ -84,9 +84,9 @@ def lean_gates(n, seed):
     return c
 
 
-@pytest.mark.parametrize("precision", ["double", "single"])
-@pytest.mark.parametrize("n,taken", [(13, False), (21, False), (22, True)])
-def test_lean_gates_from_1024_tiles_on(precision, n, taken):
+@pytest.mark.parametrize("precision,n,taken", [("double", 13, False), ("double", 21, False), ("double", 22, True),
+                                               ("single", 13, False), ("single", 22, False), ("single", 23, True)])
+def test_lean_gates_on_few_tiles(precision, n, taken):
     """With fewer tiles a pass of 2x2 gates, X and phases is a register pass."""
     print(f"case: planned lean gates {precision} n={n}", flush=True)
     passes, _ = run(lean_gates(n, 54), n, precision)
