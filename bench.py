@@ -29,10 +29,15 @@ FP64_PEAK_TFLOPS = 78.6  # MI355X published FP64 peak (vector and matrix)
 
 # HBM bytes per tile-pass launch of the default workload (30 qubits, c128),
 # from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (profiles/gate_pass_30q_brickwork_c128.md):
-# 2.0 x 8 388 857 KiB fetched (FETCH_SIZE counts half the bytes, calibrated on a
-# kernel that reads the 16 GiB state once) + 16 777 483 KiB written, averaged over
+# 2.0 x 8 388 856 KiB fetched (FETCH_SIZE counts half the bytes, calibrated on a
+# kernel that reads the 16 GiB state once) + 16 777 507 KiB written, averaged over
 # the passes of the block-fused step at width 2.
-MEASURED_TRAFFIC_30Q_C128 = (2 * 8388857 + 16777483) * 1024
+MEASURED_TRAFFIC_30Q_C128 = (2 * 8388856 + 16777507) * 1024
+
+# FP64 operations that step executes at block-fusion width 2, from the counters
+# SQ_INSTS_VALU_FMA_F64 and SQ_INSTS_VALU_MUL_F64 (wave instructions of 64 lanes; an
+# FMA counts two).
+MEASURED_FP64_30Q_C128 = (2 * 72343355392 + 10737418240) * 64
 
 
 def log(msg: str) -> None:
@@ -358,12 +363,10 @@ def main() -> int:
             ", ".join(f"{w}: {t:.0f} ms" for w, t in times.items()))
     c128 = run_engine(n, "double", circ, args.steps, args.warmup,
                       fusion_width=widths["double"]["best_width"])
-    # FP64 work of the source circuit: each U3 costs 8 fused multiply-adds per
-    # amplitude (a complex 2x2 on each pair), CX only moves amplitudes.  Block
-    # fusion executes less: a 4x4 gate costs 16 per amplitude and replaces up to
-    # four U3s with the CX between them.
-    u3_per_step = n * args.layers
-    fp64_tflops = u3_per_step * (1 << n) * 16 / (c128["ms_per_step"] / 1e3) / 1e12
+    # FP64 operations executed, measured for the default workload at width 2
+    fp64_flops = (MEASURED_FP64_30Q_C128
+                  if (n, args.layers, widths["double"]["best_width"]) == (30, 40, 2) else None)
+    fp64_tflops = fp64_flops / (c128["ms_per_step"] / 1e3) / 1e12 if fp64_flops else None
     log(f"bench: c128 {c128['gates_per_s']:.1f} gates/s, {c128['hbm_gbs']:.0f} GB/s, "
         f"kernel {c128['kernel_gbs']:.0f} GB/s, {c128['passes_per_step']:.0f} passes, "
         f"{c128['gathers_per_step']:.0f} register layouts per step")
@@ -425,7 +428,7 @@ def main() -> int:
                 k: br[k] for k in ("gates_per_s", "ms_per_step", "hbm_gbs", "kernel_gbs", "passes_per_step")}
             extra[f"brickwork_{args.big_qubits}q_c128"]["fusion_width"] = widths["double"]["best_width"]
         bt = run_batched(args.batch_circuits, 64, seed)
-        log(f"bench: batch {bt['circuits']} circuits: one launch {bt['batch_c128']['circuits_per_s']:.0f} "
+        log(f"bench: batch {bt['circuits']} circuits: together {bt['batch_c128']['circuits_per_s']:.0f} "
             f"circuits/s (c64 {bt['batch_c64']['circuits_per_s']:.0f}), circuit by circuit "
             f"{bt['sequential_c128']['circuits_per_s']:.0f} circuits/s")
         extra["batched_hea_circuits"] = bt
@@ -458,11 +461,10 @@ def main() -> int:
                      "unit": "GB/s", "frac": c128["kernel_gbs"] / HBM_PEAK_GBS,
                      "traffic": MEASURED_TRAFFIC_30Q_C128 if (n, args.layers) == (30, 40) else None,
                      "algorithmic_bytes_per_launch": c128["sweep_bytes"]},
-        # the source circuit's FP64 work against the vector peak (the pass's other
-        # bound); block fusion executes about half of it, so this can exceed 1
+        # the FP64 work the step executes against the vector peak (the pass's other bound)
         "fp64_compute": {"achieved": fp64_tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                         "frac": fp64_tflops / FP64_PEAK_TFLOPS,
-                         "flops_per_step": u3_per_step * (1 << n) * 16},
+                         "frac": fp64_tflops / FP64_PEAK_TFLOPS if fp64_tflops else None,
+                         "flops_per_step": fp64_flops},
         "cpu_baseline": cpu,
         "extra": extra,
     }
