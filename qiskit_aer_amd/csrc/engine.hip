@@ -22,9 +22,10 @@ namespace aerhip {
 namespace {
 
 constexpr size_t kMaxQueue = 4096;      // flush threshold of the gate queue
-// Gate passes from 2^9 tiles on (two workgroups per CU): 20 layers of brickwork at
-// fusion width 2 take 1.19 against 1.13 ms on 21 qubits, 1.65 against 1.30 on 22,
-// but 1.10 against 1.15 on 20.
+// complex128 gate passes from 2^9 tiles on (two workgroups per CU).  20 layers of
+// brickwork at fusion width 2, register against gate passes: 22 qubits 1.10 against
+// 0.83 ms, 21 qubits 0.73 against 0.67, 20 qubits 0.66 against 0.63 (ten layers of
+// the mixed gate set there: 0.63 against 0.57; the line could lie lower).
 constexpr uint32_t kGateMinQubits = 21;
 // Programs of 2x2 gates, X and phases alone from 2^10 tiles on in complex128, from
 // 2^11 in complex64.  With fewer a pass waits for its ops one after the other,
