@@ -164,6 +164,15 @@ int aerhip_qv_set_fusion(aerhip_qv *qv, int enable, int max_qubit, int threshold
  * replayed. */
 int aerhip_qv_graph_stats(aerhip_qv *qv, uint64_t *captures, uint64_t *replays);
 
+/* No counterpart in the reference (it has one kernel per gate).  enable = 0 keeps
+ * the handle's gates out of gate passes (tiles of 2^12 amplitudes, 16 per thread).
+ * Those sum the products of a gate in another order than the other passes: a
+ * complex64 state moves by its own rounding, and with it, in the last digits,
+ * what FP64 sums and draws make of the state.  Handles start enabled;
+ * aerhip_run_circuit and aerhip_batch_pauli_expval keep complex64 states out of
+ * them. */
+int aerhip_qv_set_gate_passes(aerhip_qv *qv, int enable);
+
 /* No counterpart in the reference (it has one kernel per gate).  How many
  * passes of this handle ran as gate passes (tiles of 2^12 amplitudes, 16 per
  * thread), and how many CX and X their layout changes took along. */

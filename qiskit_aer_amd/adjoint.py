@@ -75,6 +75,8 @@ class AdjointEstimator:
         from .qubitvector import QubitVector
         p = np.asarray(params, dtype=np.float64).reshape(-1, self.num_params)
         qv = QubitVector(self.num_qubits, "double" if self.precision == 0 else "single", self.device)
+        if self.precision == L.PRECISION_SINGLE:
+            qv.set_gate_passes(False)  # the order of FMAs that energy() has
         labels = [self.labels[i * self.num_qubits:(i + 1) * self.num_qubits].decode()
                   for i in range(self.coeffs.size)]
         out = np.empty(p.shape[0])

@@ -430,6 +430,8 @@ int aerhip_run_circuit(const aerhip_op *ops, uint64_t num_ops, uint64_t num_qubi
     R.n = num_qubits;
     R.qv = aerhip_qv_create(num_qubits, cfg.precision, cfg.device);
     if (!R.qv) throw std::runtime_error(aerhip_last_error());
+    // the outcomes of complex64 runs depend on the order of a gate's products
+    if (cfg.precision == AERHIP_PRECISION_SINGLE) ck(aerhip_qv_set_gate_passes(R.qv, 0));
     ck(aerhip_qv_set_sample_measure_index_size(R.qv, cfg.sample_index_size));
     ck(aerhip_qv_set_fusion(R.qv, cfg.fusion_enable, std::max(2, cfg.fusion_max_qubit),
                             std::max(0, cfg.fusion_threshold)));
@@ -694,6 +696,7 @@ int aerhip_batch_pauli_expval(const aerhip_op *ops, const uint64_t *op_offsets,
           h = aerhip_qv_create(num_qubits[i], precision, device);
           if (!h) throw std::runtime_error(aerhip_last_error());
           handles.push_back(h);
+          if (precision == AERHIP_PRECISION_SINGLE) ck(aerhip_qv_set_gate_passes(h, 0));
         }
         ck(aerhip_qv_initialize(h));
         queue_circuit(h, i);

@@ -4088,6 +4088,10 @@ int aerhip_qv_graph_stats(aerhip_qv *qv, uint64_t *captures, uint64_t *replays) 
   });
 }
 
+int aerhip_qv_set_gate_passes(aerhip_qv *qv, int enable) {
+  return guard([&] { E(qv).set_gate_passes(enable != 0); });
+}
+
 int aerhip_qv_gate_pass_stats(aerhip_qv *qv, uint64_t *passes, uint64_t *cx) {
   return guard([&] {
     if (!passes || !cx) throw std::invalid_argument("aerhip: null argument");

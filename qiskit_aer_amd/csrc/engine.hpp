@@ -163,6 +163,11 @@ class Engine {
     gate_passes_ = true;
     states_ = states;
   }
+  // Whether a handle's gates may run in gate passes.
+  void set_gate_passes(bool on) {
+    flush();
+    gate_passes_ = on;
+  }
   // At most `count` probes in a pass over several tiles.
   void limit_probes(uint32_t count) { probe_limit_ = count; }
 

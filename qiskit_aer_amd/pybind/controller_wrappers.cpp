@@ -383,6 +383,7 @@ py::dict run_experiment(AerCircuit &circ, uint64_t index, const AerConfig &cfg, 
         aerhip_qv *h;
         ~Guard() { aerhip_qv_destroy(h); }
       } guard{qv};
+      if (prec == AERHIP_PRECISION_SINGLE) ck(aerhip_qv_set_gate_passes(qv, 0));
       ck(aerhip_qv_set_fusion(qv, cfg.fusion_enable ? 1 : 0,
                               static_cast<int>(cfg.fusion_max_qubit.value_or(5)),
                               static_cast<int>(cfg.fusion_threshold.value_or(14))));

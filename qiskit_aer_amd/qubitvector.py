@@ -142,6 +142,11 @@ class QubitVector:
         L.check(self._L.aerhip_qv_graph_stats(self._h, C.byref(c), C.byref(r)))
         return int(c.value), int(r.value)
 
+    def set_gate_passes(self, enable: bool = True) -> None:
+        """Whether gates may run in gate passes (default: yes), which round a
+        complex64 state in another order than the other passes."""
+        L.check(self._L.aerhip_qv_set_gate_passes(self._h, int(bool(enable))))
+
     def gate_pass_stats(self) -> tuple:
         """(passes run as gate passes, CX and X taken along by their layout changes)."""
         p, c = C.c_uint64(), C.c_uint64()
