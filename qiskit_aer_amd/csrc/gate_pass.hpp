@@ -130,16 +130,20 @@ __device__ __forceinline__ void g_u1b_mfma(Amps<float, NR> &a, float A) {
 #pragma unroll
   for (int g = 0; g < NR / 2; g += G) {
     f32x4 acc[G];
-#pragma unroll
-    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].x, zero, 4, 0, 0);
-#pragma unroll
-    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].y, acc[p], 4, 1, 0);
+    // The |1> amplitude's columns come first: U3 and U2 have a real entry (0, 0),
+    // whose one product then joins last and is rounded once.  20 layers of
+    // brickwork on 23 qubits end 9.1e-7 of the norm off so, 9.5e-7 with |0> first
+    // (register passes: 9.3e-7).
 #pragma unroll
     for (int p = 0; p < G; ++p)
-      acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p) | (1 << b)].x, acc[p], 4, 2, 0);
+      acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p) | (1 << b)].x, zero, 4, 2, 0);
 #pragma unroll
     for (int p = 0; p < G; ++p)
       acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p) | (1 << b)].y, acc[p], 4, 3, 0);
+#pragma unroll
+    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].x, acc[p], 4, 0, 0);
+#pragma unroll
+    for (int p = 0; p < G; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(A, a.v[pair_lo<b>(g + p)].y, acc[p], 4, 1, 0);
 #pragma unroll
     for (int p = 0; p < G; ++p) {
       a.v[pair_lo<b>(g + p)] = mk<float>(acc[p][0], acc[p][1]);
